@@ -2,6 +2,7 @@
 // strided-batched, with alpha/beta, per-column scale, bias and activation fused into the
 // write-back.  True fp32 multiply-accumulate throughout.
 //
+// k_sgemm, the first kernel below, is what is left for products with K below 32 (64 with int8 weights) off the 16-byte grid.
 // One workgroup owns a BM x BN tile of C and walks K in slabs of 32.  An operand whose
 // K index is contiguous in memory (A of NN/NT, B of NT) is staged as rows of 32 floats padded
 // to 36, and read back with one ds_read_b128 per 8-wide k-block: lane l takes row (l & 31),
@@ -11,7 +12,9 @@
 // multiplies the k = 4*(l>>5) + j elements of both operands, so A and B always pair up.
 // The pads make the 16 lanes a b128 read serves together, the two lane halves of a b32 read,
 // and the staging writes all fall on distinct banks (64 banks x 4 bytes).
+#include "bf16x3.h"
 #include "common.h"
+#include "gemm_staged.h"
 
 namespace {
 using namespace axhip;
@@ -31,7 +34,7 @@ struct SgemmArgs {
 };
 
 // One operand's slab: R rows (M or N extent of the tile) x BK.
-template <int R, bool KCONTIG, int T, bool GUARD, typename SRC>
+template <int R, bool KCONTIG, int T, typename SRC>
 struct Operand {
     static constexpr int STRIDE = KCONTIG ? KC_STRIDE : (R + 8);
     static constexpr int FLOATS = KCONTIG ? R * KC_STRIDE : BK * (R + 8);
@@ -55,8 +58,7 @@ struct Operand {
             if (sizeof(SRC) == 1) {                        // int8 source, K-contiguous only
                 // four elements wholly inside the row: one load at whatever alignment the row has
                 // (global memory takes unaligned vector loads)
-                const bool whole = !GUARD || (r < rows && k + 4 <= K);
-                if (whole) {
+                if (r < rows && k + 4 <= K) {
                     int w;
                     __builtin_memcpy(&w, p, 4);
                     v.x = (float)(signed char)(w & 0xff);
@@ -68,8 +70,6 @@ struct Operand {
                     for (int e = 0; e < 4; e++)
                         if (k + e < K) v[e] = (float)p[e];
                 }
-            } else if (!GUARD) {
-                v = *reinterpret_cast<const v4f *>(p);
             } else if (KCONTIG) {
                 if (r < rows) {
                     if (k + 4 <= K) __builtin_memcpy(&v, p, 16);
@@ -112,14 +112,14 @@ struct Operand {
     }
 };
 
-template <int BM, int BN, int WAVES_M, int WAVES_N, bool A_KC, bool B_KC, bool GUARD, typename BSRC>
+template <int BM, int BN, int WAVES_M, int WAVES_N, bool A_KC, bool B_KC, typename BSRC>
 __global__ void __launch_bounds__(WAVES_M *WAVES_N * 64) k_sgemm(SgemmArgs g) {
     constexpr int T = WAVES_M * WAVES_N * 64;
     constexpr int WTM = BM / WAVES_M, WTN = BN / WAVES_N;
     constexpr int TM = WTM / 32, TN = WTN / 32;
     static_assert(TM * 32 * WAVES_M == BM && TN * 32 * WAVES_N == BN, "wave tiling");
-    using OpA = Operand<BM, A_KC, T, GUARD, float>;
-    using OpB = Operand<BN, B_KC, T, GUARD, BSRC>;
+    using OpA = Operand<BM, A_KC, T, float>;
+    using OpB = Operand<BN, B_KC, T, BSRC>;
     constexpr int STAGE = OpA::FLOATS + OpB::FLOATS;
 
     extern __shared__ __attribute__((aligned(16))) float lds_f[];
@@ -190,7 +190,7 @@ __global__ void __launch_bounds__(WAVES_M *WAVES_N * 64) k_sgemm(SgemmArgs g) {
 #pragma unroll
     for (int j = 0; j < TN; j++) {
         const int64_t col = n0 + wn * WTN + j * 32 + frow;
-        const bool col_ok = !GUARD || col < g.N;
+        const bool col_ok = col < g.N;
         float cs = 1.0f, bv = 0.0f;
         if (col_ok) {
             if (g.col_scale) cs = g.col_scale[col];
@@ -201,7 +201,7 @@ __global__ void __launch_bounds__(WAVES_M *WAVES_N * 64) k_sgemm(SgemmArgs g) {
 #pragma unroll
             for (int v = 0; v < 16; v++) {
                 const int64_t row = m0 + wm * WTM + i * 32 + (v & 3) + 8 * (v >> 2) + 4 * fhalf;
-                if (GUARD && (row >= g.M || !col_ok)) continue;
+                if (row >= g.M || !col_ok) continue;
                 float r = acc[i][j][v];
                 if (g.alpha != 1.0f) r *= g.alpha;
                 if (g.col_scale) r *= cs;
@@ -214,39 +214,26 @@ __global__ void __launch_bounds__(WAVES_M *WAVES_N * 64) k_sgemm(SgemmArgs g) {
     }
 }
 
-template <int BM, int BN, bool A_KC, bool B_KC, bool GUARD, typename BSRC>
-int launch(const char *name, const SgemmArgs &g, int64_t batch) {
-    auto kern = k_sgemm<BM, BN, 2, 2, A_KC, B_KC, GUARD, BSRC>;
-    using OpA = Operand<BM, A_KC, 256, GUARD, float>;
-    using OpB = Operand<BN, B_KC, 256, GUARD, BSRC>;
-    constexpr int smem = 2 * (OpA::FLOATS + OpB::FLOATS) * (int)sizeof(float);
+template <bool A_KC, bool B_KC, typename BSRC>
+int launch_guarded(const char *name, const SgemmArgs &g, int64_t batch) {
+    auto kern = k_sgemm<64, 64, 2, 2, A_KC, B_KC, BSRC>;
+    constexpr int smem = 2 * (Operand<64, A_KC, 256, float>::FLOATS + Operand<64, B_KC, 256, BSRC>::FLOATS) * (int)sizeof(float);
     static bool attr_set = false;
     if (!attr_set) {
-        AXHIP_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
-                                          hipFuncAttributeMaxDynamicSharedMemorySize, smem),
+        AXHIP_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, smem),
                       "hipFuncSetAttribute");
         attr_set = true;
     }
-    const int64_t tiles = ((g.M + BM - 1) / BM) * ((g.N + BN - 1) / BN);
+    const int64_t tiles = ((g.M + 63) / 64) * ((g.N + 63) / 64);
     if (tiles > 0x7fffffff || batch > 65535)
-        return fail(AXHIP_ERR_SHAPE, "sgemm: grid too large (tiles=%lld batch=%lld)",
-                    (long long)tiles, (long long)batch);
+        return fail(AXHIP_ERR_SHAPE, "sgemm: grid too large (tiles=%lld batch=%lld)", (long long)tiles, (long long)batch);
     note_kernel(name);
     hipLaunchKernelGGL(kern, dim3((unsigned)tiles, (unsigned)batch), dim3(256), smem, kStream, g);
     return check_launch(name);
 }
 
-template <bool A_KC, bool B_KC, typename BSRC>
-int pick_tile(const char *const names[3], const SgemmArgs &g, int64_t batch) {
-    const int esz_b = (int)sizeof(BSRC);
-    bool aligned = (g.K % BK == 0) && g.K > 0 && ((uintptr_t)g.A % 16 == 0) &&
-                   ((uintptr_t)g.B % (esz_b == 1 ? 4 : 16) == 0) && (g.lda % 4 == 0) &&
-                   (g.ldb % 4 == 0) && (g.stride_a % 4 == 0) && (g.stride_b % 4 == 0);
-    if (aligned && g.M % 128 == 0 && g.N % 128 == 0 && (g.M / 128) * (g.N / 128) * batch >= 192)
-        return launch<128, 128, A_KC, B_KC, false, BSRC>(names[0], g, batch);
-    if (aligned && g.M % 64 == 0 && g.N % 64 == 0)
-        return launch<64, 64, A_KC, B_KC, false, BSRC>(names[1], g, batch);
-    return launch<64, 64, A_KC, B_KC, true, BSRC>(names[2], g, batch);
+StagedArgs staged_args(const SgemmArgs &g) {
+    return {g.A, g.B, g.C, g.M, g.N, g.K, g.lda, g.ldb, g.ldc, g.stride_a, g.stride_b, g.stride_c, g.K, 0, g.alpha, g.beta, g.col_scale, g.bias, g.act};
 }
 
 int validate(const char *who, int transa, int transb, int64_t M, int64_t N, int64_t K,
@@ -357,53 +344,6 @@ struct FragI8 {
                    // the even k-block's buffer, the odd one's stays unused
     __device__ __forceinline__ float get(int e) const { return (float)(signed char)(raw.x >> (8 * e)); }   // fp32 form, unused by the bf16 products
 };
-
-// fp32 x int8 products on the bf16 matrix core, with fp32 accuracy.  Every int8 value is a bf16 exactly.  An fp32
-// value a is cut into three bf16 terms: hi = a with its low 16 bits cleared, mid = (a - hi) with its low 16 bits
-// cleared, lo = a - hi - mid; both subtractions are exact and lo has at most 8 significant bits, so
-// a = hi + mid + lo exactly, every term times an int8 value is exact in fp32, and only the accumulation rounds —
-// as in the fp32 product, at a sixteenth of its matrix-core time per term.  An infinite a keeps hi = a and
-// mid = lo = 0 (a - hi would be NaN), so infinities and NaNs come out as the fp32 product gives them.
-// Cost per fp32 value: and, subtract, median (the NaN filter), and, subtract, and half of each of three packs:
-// 6.5 vector instructions; per int8 value one conversion and half a pack.
-typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
-struct Bf16x3 {
-    v4i hi, mid, lo;     // 8 k values each: a k-block's four, then the next k-block's four
-};
-__device__ __forceinline__ unsigned top_halves(unsigned second, unsigned first) {   // bf16 of two fp32, by truncation
-    return __builtin_amdgcn_perm(second, first, 0x07060302);
-}
-__device__ __forceinline__ Bf16x3 bf16x3_of(const v4f &p, const v4f &q) {
-    unsigned h[8], m[8], l[8];
-#pragma unroll
-    for (int e = 0; e < 8; e++) {
-        const float a = e < 4 ? p[e] : q[e - 4];
-        h[e] = __float_as_uint(a);
-        // a NaN whose payload sits in the low 16 bits only would be cut to an infinity: give it a quiet bit the cut keeps
-        if ((h[e] & 0x7fffffffu) > 0x7f800000u) h[e] |= 0x00400000u;
-        float r = a - __uint_as_float(h[e] & 0xffff0000u);
-        r = __builtin_amdgcn_fmed3f(r, r, 0.0f);     // NaN (a infinite or NaN) -> 0, anything else unchanged
-        m[e] = __float_as_uint(r);
-        l[e] = __float_as_uint(r - __uint_as_float(m[e] & 0xffff0000u));
-    }
-    Bf16x3 o;
-#pragma unroll
-    for (int e = 0; e < 4; e++) {
-        o.hi[e] = (int)top_halves(h[2 * e + 1], h[2 * e]);
-        o.mid[e] = (int)top_halves(m[2 * e + 1], m[2 * e]);
-        o.lo[e] = (int)top_halves(l[2 * e + 1], l[2 * e]);
-    }
-    return o;
-}
-__device__ __forceinline__ v4i bf16_of_i8(int first, int second) {   // two k-blocks of four int8 -> 8 bf16
-    unsigned f[8];
-#pragma unroll
-    for (int e = 0; e < 8; e++) f[e] = __float_as_uint((float)(signed char)((e < 4 ? first : second) >> (8 * (e & 3))));
-    v4i o;
-#pragma unroll
-    for (int e = 0; e < 4; e++) o[e] = (int)top_halves(f[2 * e + 1], f[2 * e]);
-    return o;
-}
 
 template <bool KC> struct Frag;
 template <> struct Frag<true> {
@@ -1500,17 +1440,22 @@ int try_nn_stream(const SgemmArgs &g, int64_t batch) {
 // padded row block is the cheaper choice again (224 x 11008 x 4096: 182.6 against 198.4).
 inline bool half_row_tiles(int64_t M) { return M <= 160 && ((M + 31) / 32) % 2 == 1; }
 
+// What the direct-to-LDS kernels need of an fp32 product.
+template <bool A_KC>
+bool dma_takes(const SgemmArgs &g, int64_t batch) {
+    return g.K % 4 == 0 && g.K > 0 && ((uintptr_t)g.A % 16 == 0) && ((uintptr_t)g.B % 16 == 0) &&
+           ((uintptr_t)g.C % 16 == 0) && ((uintptr_t)g.bias % 16 == 0) && g.lda % 4 == 0 &&
+           g.ldb % 4 == 0 && g.ldc % 4 == 0 && g.stride_a % 4 == 0 && g.stride_b % 4 == 0 &&
+           g.stride_c % 4 == 0 && g.lda < (1 << 20) && g.ldb < (1 << 20) && batch <= 65535 &&
+           g.N % 4 == 0 && (A_KC || g.M % 4 == 0) && ((g.M + 63) / 64) * ((g.N + 63) / 64) <= 0x7fffffff;
+}
+
 // Chooses the largest tile that still leaves about eight waves per CU; returns -1 when the
 // shape does not qualify for the fast path (the caller then uses the register-staged kernel).
 // names: 128x128, 64x64, 64x64 with the k split.
 template <bool A_KC, bool B_KC>
 int try_dma(const char *const names[3], const SgemmArgs &g, int64_t batch) {
-    const bool ok = g.K % 4 == 0 && g.K > 0 && ((uintptr_t)g.A % 16 == 0) && ((uintptr_t)g.B % 16 == 0) &&
-                    ((uintptr_t)g.C % 16 == 0) && ((uintptr_t)g.bias % 16 == 0) && g.lda % 4 == 0 &&
-                    g.ldb % 4 == 0 && g.ldc % 4 == 0 && g.stride_a % 4 == 0 && g.stride_b % 4 == 0 &&
-                    g.stride_c % 4 == 0 && g.lda < (1 << 20) && g.ldb < (1 << 20) && batch <= 65535 &&
-                    g.N % 4 == 0 && (A_KC || g.M % 4 == 0) && ((g.M + 63) / 64) * ((g.N + 63) / 64) <= 0x7fffffff;
-    if (!ok) return -1;
+    if (!dma_takes<A_KC>(g, batch)) return -1;
     if constexpr (A_KC) {
         if (half_row_tiles(g.M) && g.K >= 64 && tuning().f32_tile == 0) {
             if (g.M % 32 == 0 && g.N % 64 == 0 && g.K % 32 == 0)
@@ -1712,6 +1657,30 @@ k_splitk_finish(const float *__restrict__ part, int splits, int64_t M, int64_t N
     *dst = r;
 }
 
+}  // namespace
+
+namespace axhip {
+int splitk_finish(const float *part, int64_t splits, int64_t M, int64_t N, float alpha, float beta, const float *bias, int act,
+                  float *C, int64_t ldc) {
+    const bool vec = N % 4 == 0 && ldc % 4 == 0 && (((uintptr_t)C | (uintptr_t)bias) & 15) == 0;
+    const int64_t items = M * (vec ? N / 4 : N);
+    // enough workgroups for the chip: 16 split lanes over 16 items when the result is small
+    const bool wide = items >= 64 * 512 || splits < 8;
+    const int64_t blocks = (items + (wide ? 63 : 15)) / (wide ? 64 : 16);
+    if (blocks > 0x7fffffff) return fail(AXHIP_ERR_SHAPE, "sgemm split-k: result too large");
+#define AX_FINISH(V, L)                                                                                     \
+    hipLaunchKernelGGL((k_splitk_finish<V, L>), dim3((unsigned)blocks), dim3(256), 0, kStream, part, (int)splits, \
+                       M, N, alpha, beta, bias, act, C, ldc)
+    if (vec && wide) AX_FINISH(true, 4);
+    else if (vec) AX_FINISH(true, 16);
+    else if (wide) AX_FINISH(false, 4);
+    else AX_FINISH(false, 16);
+#undef AX_FINISH
+    return check_launch("sgemm split-k finish");
+}
+}  // namespace axhip
+
+namespace {
 int dispatch_f32(const SgemmArgs &g, int transa, int transb, int64_t batch);
 
 // how many K ranges to use (1: none).  Every range must be a whole number of 32-wide slabs.
@@ -1770,7 +1739,7 @@ bool one_launch_on_half_tiles(const SgemmArgs &g, int transa) {
 
 // returns -1 when the shape is left to the ordinary path
 template <typename BSRC>
-int try_split_k(const SgemmArgs &g, int transa, int transb, const char *name, const char *const i8_names[3]) {
+int try_split_k(const SgemmArgs &g, int transa, int transb, const char *name) {
     if (one_launch_on_half_tiles(g, transa)) return -1;
     const int64_t splits = split_count(g.M, g.N, g.K, !transa);
     if (splits < 2 || splits > 65535) return -1;
@@ -1790,33 +1759,14 @@ int try_split_k(const SgemmArgs &g, int transa, int transb, const char *name, co
     p.act = AXHIP_ACT_NONE;
     int rc;
     if (std::is_same<BSRC, float>::value) rc = dispatch_f32(p, transa, transb, splits);
-    else {
-        rc = try_dma_i8(kI8DmaNames, p, splits);
-        if (rc < 0) rc = pick_tile<true, true, int8_t>(i8_names, p, splits);
-    }
+    else rc = try_dma_i8(kI8DmaNames, p, splits);
     if (rc) return rc;
-    const bool vec = g.N % 4 == 0 && g.ldc % 4 == 0 && (((uintptr_t)g.C | (uintptr_t)g.bias) & 15) == 0;
-    const int64_t items = g.M * (vec ? g.N / 4 : g.N);
-    // enough workgroups for the chip: 16 split lanes over 16 items when the result is small
-    const bool wide = items >= 64 * 512 || splits < 8;
-    const int64_t blocks = (items + (wide ? 63 : 15)) / (wide ? 64 : 16);
-    if (blocks > 0x7fffffff) return fail(AXHIP_ERR_SHAPE, "sgemm split-k: result too large");
-#define AX_FINISH(V, L)                                                                                     \
-    hipLaunchKernelGGL((k_splitk_finish<V, L>), dim3((unsigned)blocks), dim3(256), 0, kStream, part, (int)splits, \
-                       g.M, g.N, g.alpha, g.beta, g.bias, g.act, g.C, g.ldc)
-    if (vec && wide) AX_FINISH(true, 4);
-    else if (vec) AX_FINISH(true, 16);
-    else if (wide) AX_FINISH(false, 4);
-    else AX_FINISH(false, 16);
-#undef AX_FINISH
+    rc = splitk_finish(part, splits, g.M, g.N, g.alpha, g.beta, g.bias, g.act, g.C, g.ldc);
     note_kernel(name);
-    return check_launch("sgemm split-k finish");
+    return rc;
 }
 
 int dispatch_f32(const SgemmArgs &g, int transa, int transb, int64_t batch) {
-    static const char *const nn[3] = {"sgemm_nn_128x128", "sgemm_nn_64x64", "sgemm_nn_64x64_guarded"};
-    static const char *const nt[3] = {"sgemm_nt_128x128", "sgemm_nt_64x64", "sgemm_nt_64x64_guarded"};
-    static const char *const tn[3] = {"sgemm_tn_128x128", "sgemm_tn_64x64", "sgemm_tn_64x64_guarded"};
     static const char *const nn_d[3] = {"sgemm_nn_128x128_dma", "sgemm_nn_64x64_dma", "sgemm_nn_64x64k2_dma"};
     static const char *const nt_d[3] = {"sgemm_nt_128x128_dma", "sgemm_nt_64x64_dma", "sgemm_nt_64x64k2_dma"};
     static const char *const tn_d[3] = {"sgemm_tn_128x128_dma", "sgemm_tn_64x64_dma", "sgemm_tn_64x64k2_dma"};
@@ -1828,10 +1778,11 @@ int dispatch_f32(const SgemmArgs &g, int transa, int transb, int64_t batch) {
     if (!transa && !transb) rc = try_dma<true, false>(nn_d, g, batch);
     else if (!transa && transb) rc = try_dma<true, true>(nt_d, g, batch);
     else if (transa && !transb) rc = try_dma<false, false>(tn_d, g, batch);
+    if (rc < 0) rc = staged_f32(staged_args(g), transa, transb, batch);
     if (rc >= 0) return rc;
-    if (!transa && !transb) return pick_tile<true, false, float>(nn, g, batch);
-    if (!transa && transb) return pick_tile<true, true, float>(nt, g, batch);
-    if (transa && !transb) return pick_tile<false, false, float>(tn, g, batch);
+    if (!transa && !transb) return launch_guarded<true, false, float>("sgemm_nn_64x64_guarded", g, batch);
+    if (!transa && transb) return launch_guarded<true, true, float>("sgemm_nt_64x64_guarded", g, batch);
+    if (transa && !transb) return launch_guarded<false, false, float>("sgemm_tn_64x64_guarded", g, batch);
     return fail(AXHIP_ERR_NOT_IMPLEMENTED, "sgemm: A^T * B^T is not provided");
 }
 
@@ -1851,7 +1802,7 @@ int try_interior_and_fringes(const SgemmArgs &g, int transa, int transb) {
     const float *A = static_cast<const float *>(g.A), *B = static_cast<const float *>(g.B);
     // a fringe is a strip of few tiles with the whole K: the split-K route when it qualifies
     auto fringe = [&](const SgemmArgs &f) {
-        const int rc = try_split_k<float>(f, transa, transb, "sgemm_splitk", nullptr);
+        const int rc = try_split_k<float>(f, transa, transb, "sgemm_splitk");
         return rc >= 0 ? rc : dispatch_f32(f, transa, transb, 1);
     };
     SgemmArgs p = g;
@@ -1880,16 +1831,16 @@ int try_interior_and_fringes(const SgemmArgs &g, int transa, int transb) {
 
 int run_f32(const SgemmArgs &g, int transa, int transb);
 
-// K off the 32 grid keeps a large product off every fast kernel.  It is run as the product over the
+// A large product on the tile grid whose K is a multiple of 4 but not of 32 is run as the product over the
 // first K / 32 * 32 columns (alpha and beta as given, no bias or activation yet) followed by the
 // few remaining columns accumulated on top (beta = 1) with the bias and activation of the whole.
 // Returns -1 when the shape is left alone.
 int try_k_tail(const SgemmArgs &g, int transa, int transb) {
     const int64_t Km = g.K / 32 * 32;
-    if ((transa && transb) || Km == g.K || Km < 256) return -1;
-    // K a multiple of 4 runs in one pass on the 64x64 tiles with guarded edges, which take a K tail
-    // themselves; two passes are for the other K and for shapes whose main part earns 128x128 tiles
-    if (g.K % 4 == 0 && (g.M / 128) * (g.N / 128) < 2 * (int64_t)cu_count()) return -1;
+    if (Km == g.K || Km < 256) return -1;
+    // smaller ones run in one pass on the 64x64 tiles with guarded edges, which take a K tail
+    // themselves; two passes are for shapes whose main part earns 128x128 tiles
+    if ((g.M / 128) * (g.N / 128) < 2 * (int64_t)cu_count()) return -1;
     const float *A = static_cast<const float *>(g.A), *B = static_cast<const float *>(g.B);
     SgemmArgs p = g;
     p.K = Km;
@@ -1910,7 +1861,16 @@ int try_k_tail(const SgemmArgs &g, int transa, int transb) {
 // a single product: the route for its shape
 int run_f32(const SgemmArgs &g, int transa, int transb) {
     if (!(transa && transb)) {
-        int rc = try_split_k<float>(g, transa, transb, "sgemm_splitk", nullptr);
+        int rc = -1;
+        // Off the 16-byte grid the staged tiles, which split K by themselves (us, before on guarded tiles -> staged:
+        // 372 x 2149 x 2149 127 -> 48, 222 x 434 x 1376 74 -> 13, 651 x 1862 x 2833 TN 225 -> 100, 2001 x 2003 x 2005 214 -> 135,
+        // 128 x 784 x 1023 NT 39 -> 11.5, 41 x 1113 x 92 8.7 -> 7).  On it they are ahead where K is off the 32 grid, so that the
+        // kernels below cannot cut it into ranges, and few tiles want that (128 x 1024 x 784 17.4 -> 12.0).
+        const bool on_grid = transa ? dma_takes<false>(g, 1) : dma_takes<true>(g, 1);
+        const bool wants_ranges = g.K % 32 != 0 && g.K >= 256 && ((g.M + 63) / 64) * ((g.N + 63) / 64) * 2 <= cu_count();
+        if (!on_grid || wants_ranges) rc = staged_f32(staged_args(g), transa, transb, 1);
+        if (rc >= 0) return rc;
+        rc = try_split_k<float>(g, transa, transb, "sgemm_splitk");
         if (rc >= 0) return rc;
         rc = try_interior_and_fringes(g, transa, transb);
         if (rc >= 0) return rc;
@@ -1923,37 +1883,25 @@ int run_f32(const SgemmArgs &g, int transa, int transb) {
 }  // namespace
 
 namespace axhip {
-// W8A32 through the matrix cores: B is int8 [N,K].  The direct-to-LDS tiles multiply on the bf16 matrix core
-// (try_dma_i8); shapes they do not take (K off the 32 grid, unaligned rows) convert B to fp32 while it is staged.
+// W8A32 through the matrix cores: B is int8 [N,K].
 int sgemm_i8w(int64_t M, int64_t N, int64_t K, const float *a, const int8_t *w,
               const float *w_scales, float *out) {
-    static const char *const names[3] = {"qgemm_w8a32_mfma_128x128", "qgemm_w8a32_mfma_64x64",
-                                         "qgemm_w8a32_mfma_64x64_guarded"};
     SgemmArgs g{a, w, out, M, N, K, K, K, N, 0, 0, 0, 1.0f, 0.0f, w_scales, nullptr, AXHIP_ACT_NONE};
-    auto run = [&](const SgemmArgs &p) {
-        const int rc = try_split_k<int8_t>(p, 0, 1, "qgemm_w8a32_mfma_splitk", names);
-        if (rc >= 0) return rc;
-        const int rd = try_dma_i8(kI8DmaNames, p, 1);
-        return rd >= 0 ? rd : pick_tile<true, true, int8_t>(names, p, 1);
-    };
-    // K off the 32 grid cannot be cut into ranges: the first K / 32 * 32 columns as above, then the
-    // remaining few accumulated on top (the column scale applies to each part's sum alike)
-    const int64_t Km = K / 32 * 32;
-    if (Km != K && Km >= 512) {
-        SgemmArgs p = g;
-        p.K = Km;
-        int rc = run(p);
-        if (rc != AXHIP_OK) return rc;
-        p = g;
-        p.K = K - Km;
-        p.A = a + Km;
-        p.B = w + Km;
-        p.beta = 1.0f;
-        rc = pick_tile<true, true, int8_t>(names, p, 1);
-        note_kernel("qgemm_w8a32_mfma_main+k_tail");
-        return rc;
-    }
-    return run(g);
+    // The staged tiles cut an activation into its bf16 terms once per workgroup, the direct-to-LDS ones (try_dma_i8) once
+    // per wave that multiplies it, but those are the better pipelined: from a few hundred to some 800 rows against a long K
+    // the conversions decide (us, direct -> staged: 250 x 4096 x 4096 56 -> 36, 128 x 4096 x 4096 29.6 -> 23.5, 512 x 4096 x
+    // 4096 70 -> 58, 300 x 11008 x 4096 99 -> 90, 500 x 768 x 3072 22.7 -> 18.9, 512 x 4096 x 1024 21.7 -> 18.9; but
+    // 32 x 4096 x 4096 13.7 / 13.8, 256 x 768 x 768 9.7 / 9.7, 1024 x 3072 x 768 22.2 / 22.8).
+    const bool conversions = tuning().w8a32_tile == 0 && tuning().f32_tile == 0 && tuning().f32_splitk == 0 && K % 64 == 0 &&
+                             ((K >= 1024 && M >= 129 && M <= 800) || (K >= 2048 && M >= 33 && M <= 800));
+    int rc = conversions ? staged_i8w(staged_args(g)) : -1;
+    if (rc < 0) rc = try_split_k<int8_t>(g, 0, 1, "qgemm_w8a32_mfma_splitk");
+    if (rc < 0) rc = try_dma_i8(kI8DmaNames, g, 1);
+    // ... and they take what the direct loads cannot: K off the 32 grid, rows or pointers off the 16-byte grid (us, before on
+    // guarded tiles: 516 x 3200 x 2938 176 -> 45, 833 x 11008 x 2692 645 -> 190, 28 x 2134 x 1002 48 -> 9, 383 x 1088 x 815
+    // 36 -> 12)
+    if (rc < 0) rc = staged_i8w(staged_args(g));
+    return rc >= 0 ? rc : launch_guarded<true, true, int8_t>("qgemm_w8a32_mfma_64x64_guarded", g, 1);
 }
 }  // namespace axhip
 

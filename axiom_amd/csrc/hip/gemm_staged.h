@@ -1,0 +1,27 @@
+// Interface between the GEMM dispatch and the register-staged tiles (gemm_staged.hip).
+#pragma once
+#include "common.h"
+
+namespace axhip {
+
+struct StagedArgs {
+    const void *A, *B;                          // fp32 A; B fp32, or int8 [N, K]
+    float *C;
+    int64_t M, N, K, lda, ldb, ldc;
+    int64_t stride_a, stride_b, stride_c;       // elements between batch members
+    int64_t k_range, stride_z;                  // K per range (a multiple of 64, or all of K) and elements between the ranges' outputs
+    float alpha, beta;
+    const float *col_scale, *bias;
+    int act;
+};
+
+// The register-staged tiles: any alignment, any K from 32 (fp32) or 64 (int8 weights) up; g.k_range is set to K by the caller
+// and cut into ranges here where that pays.  -1: not taken (smaller K, row pitches of 4 Mi elements and more).
+int staged_f32(const StagedArgs &g, int transa, int transb, int64_t batch);
+int staged_i8w(const StagedArgs &g);
+
+// Adds `splits` partial products [M, N] in order and applies alpha, beta, bias and activation (gemm_f32.hip).
+int splitk_finish(const float *part, int64_t splits, int64_t M, int64_t N, float alpha, float beta, const float *bias, int act,
+                  float *C, int64_t ldc);
+
+}  // namespace axhip
