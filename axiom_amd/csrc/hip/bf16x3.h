@@ -41,6 +41,22 @@ __device__ __forceinline__ Bf16x3 bf16x3_of(const v4f &p, const v4f &q) {
     }
     return o;
 }
+// fp32 x fp32 products in bf16 terms: each operand cut into three terms rounded to nearest, hi + mid + lo = a exactly (hi keeps 8
+// significant bits, a - hi at most 16, a - hi - mid at most 8).  Of the nine products of terms the three smallest (mid lo,
+// lo mid, lo lo: below 2^-25 of the product, of either sign) are left out.  Exact for magnitudes from 2^-102 up to where
+// rounding to bf16 overflows; the caller looks after the others.  Per pair: three conversions, four shifts or masks, four
+// subtractions.
+__device__ __forceinline__ void bf16x3_nearest(float a, float b, int &hi, int &mid, int &lo) {
+    typedef float v2f __attribute__((ext_vector_type(2)));
+    typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
+    auto two = [](float x, float y) { return __builtin_bit_cast(int, __builtin_convertvector(v2f{x, y}, v2bf)); };
+    auto first = [](int p) { return __uint_as_float((unsigned)p << 16); };
+    auto second = [](int p) { return __uint_as_float((unsigned)p & 0xffff0000u); };
+    hi = two(a, b);
+    const float ra = a - first(hi), rb = b - second(hi);
+    mid = two(ra, rb);
+    lo = two(ra - first(mid), rb - second(mid));
+}
 __device__ __forceinline__ v4i bf16_of_i8(int first, int second) {   // two k-blocks of four int8 -> 8 bf16
     unsigned f[8];
 #pragma unroll

@@ -1771,6 +1771,14 @@ int dispatch_f32(const SgemmArgs &g, int transa, int transb, int64_t batch) {
     static const char *const nt_d[3] = {"sgemm_nt_128x128_dma", "sgemm_nt_64x64_dma", "sgemm_nt_64x64k2_dma"};
     static const char *const tn_d[3] = {"sgemm_tn_128x128_dma", "sgemm_tn_64x64_dma", "sgemm_tn_64x64k2_dma"};
     int rc = -1;
+    // Batches in bf16 terms: from K = 256 on once there is work for the whole chip and more than one 64-wide column of tiles (us,
+    // fp32 -> split: 8 x 1024^3 155 -> 98, 64 x 1000 x 128 x 1000 153 -> 115; but 512 x 512 x 64 x 512 154 -> 171 and K = 64
+    // 193 -> 282, where the kernels for a short K or a narrow result stay).
+    const bool free_choice = tuning().f32_tile == 0 && tuning().f32_splitk == 0;
+    if (batch > 1 && free_choice && g.K >= 256 && (g.N > 128 || (g.N >= 96 && (g.M % 128 != 0 || g.K % 32 != 0))) &&
+        (double)batch * g.M * g.N * g.K >= 1.0e9)
+        rc = split_f32(staged_args(g), transa, transb, batch);
+    if (rc >= 0) return rc;
     if (!transa && transb) rc = try_nt_cols(g, batch);
     if (rc < 0 && !transa && transb) rc = try_nt_rows(g, batch);
     if (!transa && !transb) rc = try_nn_stream(g, batch);
@@ -1778,6 +1786,9 @@ int dispatch_f32(const SgemmArgs &g, int transa, int transb, int64_t batch) {
     if (!transa && !transb) rc = try_dma<true, false>(nn_d, g, batch);
     else if (!transa && transb) rc = try_dma<true, true>(nt_d, g, batch);
     else if (transa && !transb) rc = try_dma<false, false>(tn_d, g, batch);
+    // off the 16-byte grid (100 x 333 x 333 x 64 42 -> 35, 100 x 333 x 64 x 333 28 -> 24; 400 x 103 x 32 x 103 17.3 -> 18.5: the
+    // padded half of a tile costs twice)
+    if (rc < 0 && free_choice && g.K >= 64 && g.N >= 48) rc = split_f32(staged_args(g), transa, transb, batch);
     if (rc < 0) rc = staged_f32(staged_args(g), transa, transb, batch);
     if (rc >= 0) return rc;
     if (!transa && !transb) return launch_guarded<true, false, float>("sgemm_nn_64x64_guarded", g, batch);
@@ -1868,7 +1879,20 @@ int run_f32(const SgemmArgs &g, int transa, int transb) {
         // kernels below cannot cut it into ranges, and few tiles want that (128 x 1024 x 784 17.4 -> 12.0).
         const bool on_grid = transa ? dma_takes<false>(g, 1) : dma_takes<true>(g, 1);
         const bool wants_ranges = g.K % 32 != 0 && g.K >= 256 && ((g.M + 63) / 64) * ((g.N + 63) / 64) * 2 <= cu_count();
-        if (!on_grid || wants_ranges) rc = staged_f32(staged_args(g), transa, transb, 1);
+        const bool off = !on_grid || wants_ranges, whole = g.M % 64 == 0 && g.N % 64 == 0 && g.K % 32 == 0;
+        // Products in bf16 terms: wherever the staged tiles are the route and K has two slabs (0.75 to 1.0 of the fp32 ones over some
+        // hundred shapes; 1050 x 1984 x 32 8.8 -> 9.7); on the grid where the fp32 tiles hang over an edge (160 x 800 x 2656 38 -> 18,
+        // 1230 x 768 x 3072 55 -> 44, 298 x 4096 x 1024 37 -> 31; up to 160 rows their half tiles and K ranges are level or ahead) and
+        // for large whole ones (640 x 2048 x 512 17.6 -> 18.7, 1024^3 19.6 -> 20.6, 640 x 4096 x 1024 49 -> 45, 2304 x 3072 x 768 95 -> 71).  A short K is
+        // loads and write-back (2048 x 4096 x 64 16 -> 20, 128 24 -> 25; off the tile grid 4000 x 4000 x 128 53 -> 45).
+        const bool free_choice = tuning().f32_tile == 0 && tuning().f32_splitk == 0;
+        const double products = (double)g.M * g.N * g.K;
+        const bool split = off ? g.K >= 64
+                               : whole ? g.K >= 256 && products >= 1.5e9
+                                       : g.K >= 96 && (products >= 1.0e9 || (g.K >= 256 && g.M > 160 && products >= 2.0e7));
+        if (free_choice && split) rc = split_f32(staged_args(g), transa, transb, 1);
+        if (rc >= 0) return rc;
+        if (off) rc = staged_f32(staged_args(g), transa, transb, 1);
         if (rc >= 0) return rc;
         rc = try_split_k<float>(g, transa, transb, "sgemm_splitk");
         if (rc >= 0) return rc;

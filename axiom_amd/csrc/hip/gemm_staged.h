@@ -18,6 +18,8 @@ struct StagedArgs {
 // The register-staged tiles: any alignment, any K from 32 (fp32) or 64 (int8 weights) up; g.k_range is set to K by the caller
 // and cut into ranges here where that pays.  -1: not taken (smaller K, row pitches of 4 Mi elements and more).
 int staged_f32(const StagedArgs &g, int transa, int transb, int64_t batch);
+// The same products in bf16 terms on the bf16 matrix core, at fp32 accuracy.
+int split_f32(const StagedArgs &g, int transa, int transb, int64_t batch);
 int staged_i8w(const StagedArgs &g);
 
 // Adds `splits` partial products [M, N] in order and applies alpha, beta, bias and activation (gemm_f32.hip).

@@ -1,5 +1,15 @@
-// Products whose operands pass through registers on their way to LDS: fp32 matrices at any alignment and any K, and
-// W8A32 (fp32 activations against int8 weights), where the activations are cut into bf16 terms on the way.
+// Products whose operands pass through registers on their way to LDS: fp32 matrices at any alignment and any K, as they are or
+// cut into three bf16 terms each on the way, and W8A32 (fp32 activations against int8 weights), where the activations are.
+//
+// fp32 products in bf16 terms (SPLIT): six bf16 products per fp32 one (bf16x3_nearest) still take 6/16 of the matrix-core time of
+// the fp32 instructions, and as an instruction adds 16 products before it rounds, the sums are nearer to 64 bits than those of
+// the fp32 tiles on every shape measured (relative error 1024^3 4.1e-7 -> 1.2e-7 on 64x64 tiles, 2048 x 4096 x 4096 1.15e-6 ->
+// 7.0e-7 on 128x128).  us, fp32 tiles -> split: 2000 x 4096 x 1024 142 -> 99, 2000 x 1024 x 4096 134 -> 100, 2048 x 4096 x 4096
+// 466 -> 339 (203 TFLOP/s), 8192^3 7204 -> 5612, 8 x 1024^3 155 -> 98.  Bound on 128x128: matrix core busy
+// 62 % of the cycles at the 1.85 GHz that the chip then holds, LDS 31 %; 64x64: the reads of fragments from LDS.  The conversions
+// (some 8 instructions a value) are put between the products of the same wave (interleave), worth 4 to 10 %.
+// A tile whose sums are not all finite, or which met a magnitude below 2^-102, is computed again with fp32 instructions by the
+// same workgroup: infinities, NaNs, values near the largest float and very small ones come out as they did.
 //
 // Why not direct to LDS: those loads move whole 16-byte pieces to their final place, so rows that start off the 16-byte grid,
 // a K that ends inside a slab and a conversion all need the register.  A slab is fetched two slabs ahead into registers,
@@ -26,17 +36,23 @@ using namespace axhip;
 typedef int v2i __attribute__((ext_vector_type(2)));
 
 
+// How a product is formed: fp32 on the fp32 matrix core; fp32 activations in three bf16 terms against int8 weights in one;
+// both operands in three bf16 terms.
+enum Op { F32, I8W, SPLIT };
+
 // One BM x BN tile of C per workgroup of eight waves: WM x WN waves over the tile, and two sets of them (wk) that take
 // the 16-wide k-steps of a slab in turn and are added through LDS at the end.
-template <int BM, int BN, int WM, int WN, int BK, bool I8, bool A_KC, bool B_KC>
+template <int BM, int BN, int WM, int WN, int BK, Op OP>
 struct Geom {
     static_assert(WM * WN == 4, "two sets of four waves");
     static constexpr int TM = BM / WM / 32, TN = BN / WN / 32;      // 32x32 blocks per wave
-    static constexpr int ROW = BK * (I8 ? 2 : 4);                   // bytes of a row of a slab in LDS: bf16 terms, or fp32
-    static constexpr int A_PLANE = BM * ROW, A_BYTES = (I8 ? 3 : 1) * A_PLANE, B_BYTES = BN * ROW;
+    static constexpr int ROW = BK * (OP == F32 ? 4 : 2);            // bytes of a row of a slab in LDS: fp32, or bf16 terms
+    static constexpr int A_PLANE = BM * ROW, A_BYTES = (OP == F32 ? 1 : 3) * A_PLANE;
+    static constexpr int B_PLANE = BN * ROW, B_BYTES = (OP == SPLIT ? 3 : 1) * B_PLANE;
     static constexpr int STAGE = A_BYTES + B_BYTES;
     static constexpr int CPITCH = BN + 4;                           // floats per row of the tile in LDS
-    static constexpr int SMEM = 2 * STAGE > BM * CPITCH * 4 ? 2 * STAGE : BM * CPITCH * 4;
+    static constexpr int BUFFERS = 2 * STAGE > BM * CPITCH * 4 ? 2 * STAGE : BM * CPITCH * 4;
+    static constexpr int SMEM = BUFFERS + (OP == SPLIT ? 32 : 0);   // ... and a word per wave: does its part need the fp32 pass
     static_assert(SMEM <= 160 * 1024, "LDS budget");
     // Where the 16-byte chunk c of row r lies in its row: rows are spread so that the 16 lanes that a 16-byte access
     // serves together (16 rows of one chunk, or the chunks of neighbouring rows) fall on distinct banks.
@@ -45,28 +61,24 @@ struct Geom {
     }
 };
 
-template <int BM, int BN, int WM, int WN, int BK, bool I8, bool A_KC, bool B_KC, int WAVES>
-__global__ void __launch_bounds__(512, WAVES) k_gemm_staged(StagedArgs g) {
-    using G = Geom<BM, BN, WM, WN, BK, I8, A_KC, B_KC>;
+// The sum over this workgroup's range of K, into acc: per wave TM x TN blocks of 32x32, register v of lane l: row (l & 31),
+// column 8 * (v >> 2) + 4 * (l >> 5) + (v & 3).  Returns whether any wave found its part of a SPLIT product unfit.
+template <int BM, int BN, int WM, int WN, int BK, Op OP, bool A_KC, bool B_KC>
+__device__ __forceinline__ bool
+sum_range(const StagedArgs &g, unsigned char *lds, int wave, int64_t m0, int64_t n0, int64_t batch,
+          v16f (&acc)[BM / WM / 32][BN / WN / 32]) {
+    using G = Geom<BM, BN, WM, WN, BK, OP>;
+    constexpr bool I8 = OP == I8W, TERMS = OP != F32;   // int8 B; bf16 terms in LDS
     constexpr int TM = G::TM, TN = G::TN, T = 512;
     // a thread stages NTA pieces of EA k values of a row of A per slab, NTB of EB of B
     constexpr int EA = BM * BK >= 8 * T ? 8 : 4, NTA = BM * BK / T / EA;
     constexpr int EB = I8 ? (BN * BK >= 16 * T ? 16 : 8) : (BN * BK >= 8 * T ? 8 : 4), NTB = BN * BK / T / EB;
     static_assert(NTA * EA * T == BM * BK && NTB * EB * T == BN * BK, "a slab divides over the threads");
-    extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
 
     const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wk = wave >> 2, wm = (wave & 3) / WN, wn = (wave & 3) % WN;
-    const int tiles_m = (int)((g.M + BM - 1) / BM), tiles_n = (int)((g.N + BN - 1) / BN);
-    int tm, tn;
-    int64_t batch = 0;
-    if (gridDim.y == 1) tile_of_block(blockIdx.x, tiles_m, tiles_n, tm, tn);
-    else tile_of_batched_block(tiles_m, tiles_n, tm, tn, batch);
-    const int64_t m0 = (int64_t)tm * BM, n0 = (int64_t)tn * BN;
     const int64_t kbeg = (int64_t)blockIdx.z * g.k_range, kend = kbeg + g.k_range < g.K ? kbeg + g.k_range : g.K;
     const int slabs = (int)((kend - kbeg + BK - 1) / BK), last = slabs - 1;
-    float *C = g.C + batch * g.stride_c + blockIdx.z * g.stride_z;
 
     // ---- where each piece is read and written: 32-bit byte offsets from a base that is the same for the whole workgroup ----
     const char *abase = reinterpret_cast<const char *>(static_cast<const float *>(g.A) + batch * g.stride_a +
@@ -87,20 +99,16 @@ __global__ void __launch_bounds__(512, WAVES) k_gemm_staged(StagedArgs g) {
         const int q = tid + i * T, row = A_KC ? q / PER : q % BM, c = A_KC ? q % PER : q / BM;
         const unsigned r = row < mlast ? row : mlast;
         oa[i] = A_KC ? r * lda4 + c * EA * 4 : r * 4 + c * EA * lda4;
-        wa[i] = I8 ? G::at(row, c * EA / 8) + (c * EA % 8) * 2 : G::at(row, c * EA / 4);
+        wa[i] = TERMS ? G::at(row, c * EA / 8) + (c * EA % 8) * 2 : G::at(row, c * EA / 4);
     }
 #pragma unroll
     for (int i = 0; i < NTB; i++) {
         constexpr int PER = BK / EB;
         const int q = tid + i * T, row = B_KC ? q / PER : q % BN, c = B_KC ? q % PER : q / BN;
         const unsigned r = row < nlast ? row : nlast;
-        if constexpr (I8) {
-            ob[i] = r * (unsigned)g.ldb + c * EB;
-            wb[i] = G::at(row, c * EB / 8);
-        } else {
-            ob[i] = B_KC ? r * ldb4 + c * EB * 4 : r * 4 + c * EB * ldb4;
-            wb[i] = G::at(row, c * EB / 4);
-        }
+        if constexpr (I8) ob[i] = r * (unsigned)g.ldb + c * EB;
+        else ob[i] = B_KC ? r * ldb4 + c * EB * 4 : r * 4 + c * EB * ldb4;
+        wb[i] = TERMS ? G::at(row, c * EB / 8) + (c * EB % 8) * 2 : G::at(row, c * EB / 4);
     }
 
     struct Regs {
@@ -130,12 +138,30 @@ __global__ void __launch_bounds__(512, WAVES) k_gemm_staged(StagedArgs g) {
             }
         }
     };
+    // SPLIT: the smallest magnitude met, as twice its bit pattern less one (zero, which is no concern, comes out largest)
+    unsigned least = 0xffffffffu;
+    auto put_terms = [&](unsigned char *d, int plane, const auto &x, auto count) {
+        constexpr int E = decltype(count)::value;
+#pragma unroll
+        for (int e = 0; e < E; e += 2) {
+            const unsigned u = __float_as_uint(x[e]) * 2 - 1, v = __float_as_uint(x[e + 1]) * 2 - 1;
+            least = min(least, min(u, v));
+        }
+        int hi[E / 2], mid[E / 2], lo[E / 2];
+#pragma unroll
+        for (int e = 0; e < E / 2; e++) bf16x3_nearest(x[2 * e], x[2 * e + 1], hi[e], mid[e], lo[e]);
+        __builtin_memcpy(__builtin_assume_aligned(d, 2 * E), hi, 2 * E);
+        __builtin_memcpy(__builtin_assume_aligned(d + plane, 2 * E), mid, 2 * E);
+        __builtin_memcpy(__builtin_assume_aligned(d + 2 * plane, 2 * E), lo, 2 * E);
+    };
     auto stage = [&](const Regs &r, unsigned at) {   // ... into LDS buffer `at`
 #pragma unroll
         for (int i = 0; i < NTA; i++) {
             const float *x = r.a[i];
             unsigned char *d = lds + at + wa[i];
-            if constexpr (I8 && EA == 8) {
+            if constexpr (OP == SPLIT) {
+                put_terms(d, G::A_PLANE, r.a[i], std::integral_constant<int, EA>());
+            } else if constexpr (I8 && EA == 8) {
                 const Bf16x3 o = bf16x3_of(v4f{x[0], x[1], x[2], x[3]}, v4f{x[4], x[5], x[6], x[7]});
                 *reinterpret_cast<v4i *>(d) = o.hi;
                 *reinterpret_cast<v4i *>(d + G::A_PLANE) = o.mid;
@@ -157,6 +183,8 @@ __global__ void __launch_bounds__(512, WAVES) k_gemm_staged(StagedArgs g) {
 #pragma unroll
                 for (int h = 0; h < EB / 8; h++)
                     *reinterpret_cast<v4i *>(lds + at + G::A_BYTES + (wb[i] ^ (h * 16))) = bf16_of_i8(r.q[i][2 * h], r.q[i][2 * h + 1]);
+            } else if constexpr (OP == SPLIT) {
+                put_terms(lds + at + G::A_BYTES + wb[i], G::B_PLANE, r.b[i], std::integral_constant<int, EB>());
             } else {
                 const float *x = r.b[i];
 #pragma unroll
@@ -168,14 +196,25 @@ __global__ void __launch_bounds__(512, WAVES) k_gemm_staged(StagedArgs g) {
 
     // ---- LDS -> fragments -> products ----
     const int frow = lane & 31, fhalf = lane >> 5;
-    v16f acc[TM][TN];
+    // SPLIT, up to 128x64: the five smaller products in a sum of their own, so that the large one is rounded once per 16 k and not
+    // six times (relative error of 139 x 192 x 320, 288 x 3561 x 703: one sum 1.9e-7, 2.8e-7); 128x128 has no registers left for it
+    constexpr bool APART = OP == SPLIT && TM * TN < 4;
+    v16f low[APART ? TM : 1][APART ? TN : 1];
+    if constexpr (APART) {
+#pragma unroll
+        for (int i = 0; i < TM; i++)
+#pragma unroll
+            for (int j = 0; j < TN; j++)
+#pragma unroll
+                for (int v = 0; v < 16; v++) low[i][j][v] = 0.0f;
+    }
     const int arow = wm * TM * 32 + frow, brow = wn * TN * 32 + frow;     // + 32 t: the swizzle is that of the first
     // byte addresses of this lane's chunks in its wave's k-steps (wk, and wk + 2 of a 64-wide slab; fp32: the first of two)
     constexpr int STEPS = BK / 32;
     unsigned ra[STEPS], rb[STEPS];
 #pragma unroll
     for (int it = 0; it < STEPS; it++) {
-        const int ks = 2 * it + wk, c = I8 ? 2 * ks + fhalf : 4 * ks + 2 * fhalf;
+        const int ks = 2 * it + wk, c = TERMS ? 2 * ks + fhalf : 4 * ks + 2 * fhalf;
         ra[it] = G::at(arow, c);
         rb[it] = G::A_BYTES + G::at(brow, c);
     }
@@ -198,6 +237,27 @@ __global__ void __launch_bounds__(512, WAVES) k_gemm_staged(StagedArgs g) {
                         for (int j = 0; j < TN; j++)
                             acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf, fb[j]), __builtin_bit_cast(v8bf, fa[i][p]),
                                                                                 acc[i][j], 0, 0, 0);
+            } else if constexpr (OP == SPLIT) {
+                v4i fa[TM][3], fb[TN][3];
+#pragma unroll
+                for (int p = 2; p >= 0; p--) {                            // in the order of use
+#pragma unroll
+                    for (int j = 0; j < TN; j++) fb[j][2 - p] = *reinterpret_cast<const v4i *>(lds + at + rb[it] + (2 - p) * G::B_PLANE + j * 32 * G::ROW);
+#pragma unroll
+                    for (int i = 0; i < TM; i++) fa[i][p] = *reinterpret_cast<const v4i *>(lds + at + ra[it] + p * G::A_PLANE + i * 32 * G::ROW);
+                }
+#pragma unroll
+                for (int sum = 2; sum >= 0; sum--)                        // the small products first
+#pragma unroll
+                    for (int p = sum; p >= 0; p--)
+#pragma unroll
+                        for (int i = 0; i < TM; i++)
+#pragma unroll
+                            for (int j = 0; j < TN; j++) {
+                                v16f &to = APART && sum > 0 ? low[APART ? i : 0][APART ? j : 0] : acc[i][j];
+                                to = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf, fb[j][sum - p]),
+                                                                             __builtin_bit_cast(v8bf, fa[i][p]), to, 0, 0, 0);
+                            }
             } else {
                 v4f fa[TM][2], fb[TN][2];
 #pragma unroll
@@ -218,13 +278,33 @@ __global__ void __launch_bounds__(512, WAVES) k_gemm_staged(StagedArgs g) {
         }
     };
 
+    // SPLIT: the conversions go between the products of the same wave: a product keeps the matrix core for eight times as long
+    // as it takes to issue
+    auto interleave = [&]() {
+        constexpr int PRODUCTS = 6 * TM * TN, CUTS = (NTA * EA + NTB * EB) * 8 / STEPS, PER = CUTS / PRODUCTS;
+#pragma unroll
+        for (int it = 0; it < STEPS; it++) {
+            __builtin_amdgcn_sched_group_barrier(0x100, 3 * (TM + TN), 0);
+#pragma unroll
+            for (int q = 0; q < PRODUCTS; q++) {
+                __builtin_amdgcn_sched_group_barrier(0x002, PER, 0);
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            }
+        }
+    };
+
     // One slab: multiply the one in LDS, put the next one (already in registers) beside it, request the one three ahead.
     // The two wave sets of a SIMD do the first two in opposite order, so that one converts and writes while the other
     // multiplies.  No branch inside: past the last slab the last one is requested again, unused.
     auto walk = [&](auto set_number) {
         constexpr bool stage_first = decltype(set_number)::value;
         auto step = [&](int s, Regs &next, unsigned cur, unsigned nxt) {
-            if constexpr (stage_first) {
+            if constexpr (OP == SPLIT) {
+                multiply(cur);
+                stage(next, nxt);
+                load(next, s + 3);
+                interleave();
+            } else if constexpr (stage_first) {
                 stage(next, nxt);
                 load(next, s + 3);
                 multiply(cur);
@@ -261,9 +341,10 @@ __global__ void __launch_bounds__(512, WAVES) k_gemm_staged(StagedArgs g) {
         for (int q = tid; q < ROWS * 4; q += T) {
             const int row = q % ROWS, r = row < BM ? row : row - BM;
             for (int k = q / ROWS; k < skip; k += 4) {
-                if constexpr (I8) {
+                if constexpr (TERMS) {
+                    const unsigned base = end + (row < BM ? 0 : G::A_BYTES), plane = row < BM ? G::A_PLANE : G::B_PLANE;
 #pragma unroll
-                    for (int p = 0; p < 3; p++) *reinterpret_cast<unsigned short *>(lds + end + p * G::A_PLANE + G::at(r, k >> 3) + (k & 7) * 2) = 0;
+                    for (int p = 0; p < 3; p++) *reinterpret_cast<unsigned short *>(lds + base + p * plane + G::at(r, k >> 3) + (k & 7) * 2) = 0;
                 } else {
                     *reinterpret_cast<float *>(lds + end + (row < BM ? 0 : G::A_BYTES) + G::at(r, k >> 2) + (k & 3) * 4) = 0.0f;
                 }
@@ -272,10 +353,58 @@ __global__ void __launch_bounds__(512, WAVES) k_gemm_staged(StagedArgs g) {
         __syncthreads();
     }
     multiply(end);
+    if constexpr (OP != SPLIT) {
+        __syncthreads();
+        return false;
+    }
+    if constexpr (APART) {
+#pragma unroll
+        for (int i = 0; i < TM; i++)
+#pragma unroll
+            for (int j = 0; j < TN; j++) acc[i][j] += low[i][j];
+    }
+    // Terms of values below 2^-102 may fall under the smallest normal bf16 and lose bits, and infinities, NaNs and values that
+    // round past the largest bf16 leave a NaN or an infinity in every sum they enter (as, perhaps, in the fp32 product).
+    constexpr unsigned TINY = 25u << 24;              // twice the bit pattern of 2^-102
+    float finite = 0.0f;
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++)
+#pragma unroll
+            for (int v = 0; v < 16; v++) finite = __builtin_fmaf(acc[i][j][v], 0.0f, finite);
+    int *unfit = reinterpret_cast<int *>(lds + G::BUFFERS);
+    const bool bad = __builtin_amdgcn_ballot_w64(!(finite == 0.0f) || least < TINY) != 0;
+    if (lane == 0) unfit[wave] = bad;
     __syncthreads();
+    const v4i f0 = *reinterpret_cast<const v4i *>(unfit), f1 = *reinterpret_cast<const v4i *>(unfit + 4);
+    return __builtin_amdgcn_readfirstlane(f0[0] | f0[1] | f0[2] | f0[3] | f1[0] | f1[1] | f1[2] | f1[3]) != 0;
+}
+
+template <int BM, int BN, int WM, int WN, int BK, Op OP, bool A_KC, bool B_KC, int WAVES>
+__global__ void __launch_bounds__(512, WAVES) k_gemm_staged(StagedArgs g) {
+    using G = Geom<BM, BN, WM, WN, BK, OP>;
+    constexpr int TM = G::TM, TN = G::TN, T = 512;
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wk = wave >> 2, wm = (wave & 3) / WN, wn = (wave & 3) % WN;
+    const int tiles_m = (int)((g.M + BM - 1) / BM), tiles_n = (int)((g.N + BN - 1) / BN);
+    int tm, tn;
+    int64_t batch = 0;
+    if (gridDim.y == 1) tile_of_block(blockIdx.x, tiles_m, tiles_n, tm, tn);
+    else tile_of_batched_block(tiles_m, tiles_n, tm, tn, batch);
+    const int64_t m0 = (int64_t)tm * BM, n0 = (int64_t)tn * BN;
+    float *C = g.C + batch * g.stride_c + blockIdx.z * g.stride_z;
+    v16f acc[TM][TN];
+    const bool unfit = sum_range<BM, BN, WM, WN, BK, OP, A_KC, B_KC>(g, lds, wave, m0, n0, batch, acc);
+    if constexpr (OP == SPLIT) {
+        static_assert(2 * Geom<BM, BN, WM, WN, BK, F32>::STAGE <= G::BUFFERS, "the fp32 pass runs in the same LDS");
+        if (unfit) sum_range<BM, BN, WM, WN, BK, F32, A_KC, B_KC>(g, lds, wave, m0, n0, batch, acc);
+    }
 
     // ---- the two sets added in LDS, then whole rows written back ----
-    // register v of lane l: row (l & 31), column 8 * (v >> 2) + 4 * (l >> 5) + (v & 3)
+    const int frow = lane & 31, fhalf = lane >> 5, arow = wm * TM * 32 + frow;
     float *tile = reinterpret_cast<float *>(lds);
     if (wk == 1) {
 #pragma unroll
@@ -335,10 +464,10 @@ __global__ void __launch_bounds__(512, WAVES) k_gemm_staged(StagedArgs g) {
     }
 }
 
-template <int BM, int BN, int WM, int WN, int BK, bool I8, bool A_KC, bool B_KC, int WAVES>
+template <int BM, int BN, int WM, int WN, int BK, Op OP, bool A_KC, bool B_KC, int WAVES>
 int launch_staged(const char *name, const StagedArgs &g, int64_t batch, int64_t splits) {
-    using G = Geom<BM, BN, WM, WN, BK, I8, A_KC, B_KC>;
-    auto kern = k_gemm_staged<BM, BN, WM, WN, BK, I8, A_KC, B_KC, WAVES>;
+    using G = Geom<BM, BN, WM, WN, BK, OP>;
+    auto kern = k_gemm_staged<BM, BN, WM, WN, BK, OP, A_KC, B_KC, WAVES>;
     // what the kernel relies on: a last slab is fetched from further left, never from before the row; 32-bit offsets
     if (g.K < BK || g.k_range < 1 || (g.k_range % BK != 0 && g.k_range < g.K) || (splits - 1) * g.k_range >= g.K || splits * g.k_range < g.K ||
         g.lda >= (1 << 22) || g.ldb >= (1 << 22))
@@ -357,9 +486,9 @@ int launch_staged(const char *name, const StagedArgs &g, int64_t batch, int64_t 
 
 // ---- which tile, and into how many ranges of K -----------------------------------------------------------------------
 // A tile and a number of ranges are chosen by the time they should take: the rounds of workgroups over the CUs, times the
-// slabs of a range, times what a slab of that tile costs while its workgroup has the CU to itself (measured, us: fp32
-// 32-wide slabs, 64x64 0.62, 128x128 2.05; int8 weights, 64-wide slabs, 32x128 0.57, 64x128 0.90, 64x256 1.52), and for
-// more than one range the finishing launch and its traffic.
+// slabs of a range, times what a slab of that tile costs while its workgroup has the CU to itself (measured, us, in the
+// tables below), plus what a round costs besides (first loads, write-back), and for more than one range the finishing launch
+// and its traffic.
 struct Plan {
     int tile;
     int64_t splits;
@@ -367,7 +496,7 @@ struct Plan {
 };
 struct TileCost {
     int bm, bn, bk;
-    float slab_us;
+    float slab_us, round_us;
 };
 Plan plan_staged(const StagedArgs &g, int64_t batch, const TileCost *tiles, int n, bool may_split) {
     const int64_t cus = cu_count();
@@ -387,7 +516,7 @@ Plan plan_staged(const StagedArgs &g, int64_t batch, const TileCost *tiles, int 
             last = z;
             const int64_t per = (slabs + z - 1) / z;
             z = (slabs + per - 1) / per;                          // no empty range
-            float us = 3.5f + (float)((count * z + cus - 1) / cus) * (float)per * c.slab_us;
+            float us = 1.0f + (float)((count * z + cus - 1) / cus) * ((float)per * c.slab_us + c.round_us);
             if (z > 1) us += 3.0f + (float)(g.M * g.N) * (float)(z + 1) * (4.0f / 3.0e6f);
             if (best.tile < 0 || us < best.us) best = {t, z, us};
         }
@@ -416,21 +545,45 @@ int run_plan(const StagedArgs &g, const Plan &p, int bk, const char *split_name,
     return rc;
 }
 
-const TileCost kF32Tiles[] = {{64, 64, 32, 0.62f}, {128, 128, 32, 2.05f}};
-const TileCost kI8Tiles[] = {{32, 128, 64, 0.57f}, {64, 128, 64, 0.90f}, {64, 256, 64, 1.52f}};
+const TileCost kF32Tiles[] = {{64, 64, 32, 0.62f, 2.5f}, {128, 128, 32, 2.05f, 2.5f}};
+const TileCost kSplitTiles[] = {{128, 128, 32, 1.36f, 4.0f}, {128, 64, 32, 0.82f, 3.0f}, {64, 128, 32, 0.84f, 3.0f}, {64, 64, 32, 0.48f, 1.8f}};
+const TileCost kI8Tiles[] = {{32, 128, 64, 0.57f, 2.5f}, {64, 128, 64, 0.90f, 2.5f}, {64, 256, 64, 1.52f, 2.5f}};
 
 template <bool A_KC, bool B_KC>
 int run_f32(const StagedArgs &g, int64_t batch, const char *const names[2], const char *split_name) {
     const Plan p = plan_staged(g, batch, kF32Tiles, 2, batch == 1);
     if (p.tile < 0) return -1;
     return run_plan(g, p, kF32Tiles[p.tile].bk, split_name, [&](const StagedArgs &a) {
-        return p.tile == 0 ? launch_staged<64, 64, 2, 2, 32, false, A_KC, B_KC, 4>(names[0], a, batch, p.splits)
-                           : launch_staged<128, 128, 2, 2, 32, false, A_KC, B_KC, 2>(names[1], a, batch, p.splits);
+        return p.tile == 0 ? launch_staged<64, 64, 2, 2, 32, F32, A_KC, B_KC, 4>(names[0], a, batch, p.splits)
+                           : launch_staged<128, 128, 2, 2, 32, F32, A_KC, B_KC, 2>(names[1], a, batch, p.splits);
+    });
+}
+template <bool A_KC, bool B_KC>
+int run_split(const StagedArgs &g, int64_t batch, const char *const names[4], const char *split_name) {
+    const Plan p = plan_staged(g, batch, kSplitTiles, 4, batch == 1);
+    if (p.tile < 0) return -1;
+    return run_plan(g, p, kSplitTiles[p.tile].bk, split_name, [&](const StagedArgs &a) {
+        switch (p.tile) {
+            case 0: return launch_staged<128, 128, 2, 2, 32, SPLIT, A_KC, B_KC, 2>(names[0], a, batch, p.splits);
+            case 1: return launch_staged<128, 64, 2, 2, 32, SPLIT, A_KC, B_KC, 2>(names[1], a, batch, p.splits);
+            case 2: return launch_staged<64, 128, 2, 2, 32, SPLIT, A_KC, B_KC, 2>(names[2], a, batch, p.splits);
+            default: return launch_staged<64, 64, 2, 2, 32, SPLIT, A_KC, B_KC, 4>(names[3], a, batch, p.splits);
+        }
     });
 }
 }  // namespace
 
 namespace axhip {
+int split_f32(const StagedArgs &g, int transa, int transb, int64_t batch) {
+    static const char *const nn[4] = {"sgemm_nn_128x128x3_staged", "sgemm_nn_128x64x3_staged", "sgemm_nn_64x128x3_staged", "sgemm_nn_64x64x3_staged"};
+    static const char *const nt[4] = {"sgemm_nt_128x128x3_staged", "sgemm_nt_128x64x3_staged", "sgemm_nt_64x128x3_staged", "sgemm_nt_64x64x3_staged"};
+    static const char *const tn[4] = {"sgemm_tn_128x128x3_staged", "sgemm_tn_128x64x3_staged", "sgemm_tn_64x128x3_staged", "sgemm_tn_64x64x3_staged"};
+    if ((transa && transb) || g.K < 32 || g.lda >= (1 << 22) || g.ldb >= (1 << 22) || batch > 65535) return -1;
+    if (!transa && !transb) return run_split<true, false>(g, batch, nn, "sgemm_splitk");
+    if (!transa) return run_split<true, true>(g, batch, nt, "sgemm_splitk");
+    return run_split<false, false>(g, batch, tn, "sgemm_splitk");
+}
+
 int staged_f32(const StagedArgs &g, int transa, int transb, int64_t batch) {
     static const char *const nn[2] = {"sgemm_nn_64x64k2_staged", "sgemm_nn_128x128k2_staged"};
     static const char *const nt[2] = {"sgemm_nt_64x64k2_staged", "sgemm_nt_128x128k2_staged"};
@@ -447,9 +600,9 @@ int staged_i8w(const StagedArgs &g) {
     if (p.tile < 0) return -1;
     return run_plan(g, p, 64, "qgemm_w8a32_mfma_splitk", [&](const StagedArgs &a) {
         switch (p.tile) {
-            case 0: return launch_staged<32, 128, 1, 4, 64, true, true, true, 4>("qgemm_w8a32_mfma_32x128k2_staged", a, 1, p.splits);
-            case 1: return launch_staged<64, 128, 2, 2, 64, true, true, true, 4>("qgemm_w8a32_mfma_64x128k2_staged", a, 1, p.splits);
-            default: return launch_staged<64, 256, 1, 4, 64, true, true, true, 2>("qgemm_w8a32_mfma_64x256k2_staged", a, 1, p.splits);
+            case 0: return launch_staged<32, 128, 1, 4, 64, I8W, true, true, 4>("qgemm_w8a32_mfma_32x128k2_staged", a, 1, p.splits);
+            case 1: return launch_staged<64, 128, 2, 2, 64, I8W, true, true, 4>("qgemm_w8a32_mfma_64x128k2_staged", a, 1, p.splits);
+            default: return launch_staged<64, 256, 1, 4, 64, I8W, true, true, 2>("qgemm_w8a32_mfma_64x256k2_staged", a, 1, p.splits);
         }
     });
 }
