@@ -22,7 +22,7 @@ def product(hip, a, b, order):
 
 # the fp32 error bound K u sum |a||b| (u = 2^-24) holds with room for sums of random signs, see test_gpu_staged; the left-out terms
 # add at most 2^-24 of each product
-@pytest.mark.parametrize("M,N,K", [(17, 33, 64), (65, 129, 65), (129, 65, 95), (161, 516, 256), (1024, 1024, 1024), (1153, 772, 2052), (644, 4096, 1024),
+@pytest.mark.parametrize("M,N,K", [(17, 33, 64), (65, 129, 65), (129, 65, 95), (161, 516, 256), (1152, 1152, 1152), (1153, 772, 2052), (644, 4096, 1024),
                                    (2049, 1028, 260), (200, 128, 4096), (1000, 1004, 1001)])
 @pytest.mark.parametrize("order", ["nn", "nt", "tn"])
 def test_split_fp32(hip, M, N, K, order):
@@ -52,7 +52,7 @@ def test_split_batched(hip, Bn, M, N, K, transb):
     assert (np.abs(got - want) <= BOUND_FP32 * size).all()
 
 
-SHAPES = [(70, 90, 101), (200, 132, 1029), (1024, 1024, 1024)]      # one tile, ranges of K, whole tiles
+SHAPES = [(70, 90, 101), (200, 132, 1029), (1152, 1152, 1152)]      # one tile, ranges of K, whole tiles
 
 
 @pytest.mark.parametrize("M,N,K", SHAPES)
