@@ -1,104 +1,199 @@
 // Scaled dot-product attention forward: O = softmax(scale * Q K^T [+ causal mask]) V per head,
 // Q, K, V, O [BH, S, dk] row-major fp32, L [BH, S] = log-sum-exp of each score row (or NULL).
 //
-// Fused kernel (dk a multiple of 4 up to 128, on the geometry of the next size among 32, 64 and
-// 128; any S): the score matrix never leaves the chip.  A
-// workgroup of 4 waves owns 128 query rows of one head, a wave 32 of them; keys and values
-// stream through LDS in blocks of 64 (direct-to-LDS loads, two stages).  Both products run on
-// v_mfma_f32_32x32x2_f32 with the query index on the MFMA's column side, so lane l of a wave
-// owns query (l & 31) in the score tile *and* in the output accumulator:
-//   S^T tile:  A = K rows (32 keys), B = the wave's Q rows (held in registers for the whole
-//              kernel); register v of lane l = score(query l&31, key 8*(v>>2) + 4*(l>>5) + (v&3)).
+// Fused kernel (dk a multiple of 4 up to 128, on the geometry of the next size among 32, 64, 96 and
+// 128; any S): the score matrix never leaves the chip.  A workgroup of four or eight waves owns 128 or 256
+// query rows of one head, a wave 32 of them; keys and values stream through LDS in blocks of 64 (32 for dk 128).
+// Both products run on the bf16 matrix core with every fp32 operand cut into three bf16 terms (six
+// products of terms for one of values, bf16x3.h): 6/16 of the matrix-core time of the fp32 instructions,
+// which also share their lanes with the softmax's vector instructions.  K and V are cut once per
+// workgroup on their way from registers to LDS, Q once per tile, a probability when it is used.  The
+// query index is on the MFMA's column side, so lane l of a wave owns query (l & 31) in the score tile
+// *and* in the output accumulator:
+//   S^T tile:  A = K rows (32 keys), B = the wave's Q rows (terms held in registers for the whole tile);
+//              register v of lane l = score(query l&31, key 8*(v>>2) + 4*(l>>5) + (v&3)).
 //   softmax:   running maximum m and sum per query, the online form: the accumulator is
 //              rescaled by 2^(m_old - m_new) when the maximum moves.  Row reductions are within
 //              a lane plus one exchange with lane l^32.  Scores are kept in base-2 units
 //              (scale * log2(e) folded in) so the exponential is the hardware's 2^x.
-//   O^T tile:  A = V^T (lane reads V[key][d] with d = l&31), B = the probabilities exactly
-//              where the score MFMA left them: key(v, l>>5) above is also a legal pairing of
-//              the MFMA's two k indices, and a sum over keys does not care about their order.
-// K rows are XOR-swizzled in 16-byte chunks, applied on the global address side of the load, so
-// a 16-lane ds_read_b128 touches every bank once; V is laid out per load instruction with a
-// pitch (or, for dk = 32, a row order) that puts the two lane halves of a fragment read (keys 4
-// apart) on different banks.
+//   O^T tile:  A = V^T, B = the probabilities exactly where the score MFMA left them: registers 8s .. 8s+7
+//              are the eight k of a 16-key step, V^T lies in LDS in that order of keys, and a sum over
+//              keys does not care about their order.
+// V is transposed by the registers (a thread loads eight keys of one column).  Rows of both operands
+// are XOR-swizzled in 16-byte chunks, so the 16 lanes that a 16-byte access serves fall on distinct banks.
+// A tile with a sum that is not finite, or that met a magnitude below 2^-102, is computed again with fp32
+// instructions by the same workgroup: infinities, NaNs, values near the largest float and very small ones
+// come out as fp32 products give them.
+// us, fp32 instructions -> terms: 512 heads of [512, 64] 269 -> 194 (causal 178 -> 126), 64 of [1024, 128] 273 -> 174, 96 causal
+// ones of [1000, 80] 324 -> 129 (a quarter of that from the 96-wide geometry), 512 of [256, 32] 41 -> 33, 32 of [128, 64] 11.9 ->
+// 10.9.  O is nearer to 64 bits on every shape measured (relative error 4.9e-7 -> 3.7e-7 at [512, 64]).  Bound: the matrix core is
+// busy some 45 % of the time, vector instructions (cutting, softmax) about as much.  Measured and dropped: two key tiles at a time,
+// the scores of one interleaved with the exponentials of the other by instruction groups ([512, 64] 194, [1024, 96] 126 -> 128).
 //
 // Every other head size: scores through a workspace, one batched NT GEMM, a row softmax kernel and
 // one batched NN GEMM over as many heads at a time as fit 256 MiB (the structure of
 // ax_cuda_sdpa_fwd, cuda/ops_attention.cu:299-392).
-#include "common.h"
+#include "bf16x3.h"
 
 namespace {
 using namespace axhip;
 
-#define AXS_LOAD_LDS(m0val, voff, base)                                                        \
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(m0val),  \
-                 "v"(voff), "s"(base)                                                          \
-                 : "memory")
-#define AXS_VM0() __builtin_amdgcn_s_waitcnt(0 | (0 << 14) | (7 << 4) | (15 << 8))
-// at most n (a constant below 64) vector-memory loads still in flight
-#define AXS_VM(n) __builtin_amdgcn_s_waitcnt(((n) & 15) | (((n) >> 4) << 14) | (7 << 4) | (15 << 8))
+typedef int v2i __attribute__((ext_vector_type(2)));
 
-constexpr int SD_BQ = 128, SD_BKV = 64;
-
-// LDS geometry for head dimension DK (32, 64 or 128).  A direct-to-LDS load instruction moves
-// 1 KiB = RPI whole rows of DK floats.
-template <int DK>
+template <int DK, int WAVES>
 struct SdGeom {
-    static constexpr int ROWB = DK * 4;                 // bytes per row
-    static constexpr int CH = DK / 4;                   // 16-byte chunks per row
-    static constexpr int RPI = 1024 / ROWB;             // rows per load instruction
-    static constexpr int KSTAGE = SD_BKV * ROWB;        // K block, rows contiguous, chunks swizzled
-    // V block: load-instruction groups spaced so that keys k and k+4 (the two lane halves of a
-    // fragment read) fall 128 bytes apart modulo 256, i.e. on different halves of the banks
-    static constexpr int VGROUP = DK == 64 ? 1152 : DK == 128 ? 1088 : 1024;
-    static constexpr int VSTAGE = (SD_BKV / RPI) * VGROUP;
-    static constexpr int SMEM = 2 * KSTAGE + 2 * VSTAGE;
-    static constexpr int IPW = SD_BKV / RPI / 4;        // load instructions per wave and 64-row block
-    static_assert(DK == 32 || DK == 64 || DK == 128, "head dimension");
-    static_assert(2 * KSTAGE >= SD_BQ * ROWB, "the Q tile is staged through the two K stages");
-
-    // chunk swizzle key of a K/Q row: the 16 rows a ds_read_b128 serves together (same logical
-    // chunk) must land on 16 different 16-byte bank slots
-    __device__ static int swz(int row) { return CH >= 16 ? (row & 15) : ((row >> 1) & 7); }
-    // which row of its group the lane at group position `slot` fetches (V only; DK = 32 keeps
-    // rows k and k+4 next to each other)
-    __device__ static int v_row_of_slot(int slot) { return DK == 32 ? ((slot & 1) * 4 + (slot >> 1)) : slot; }
-    // byte offset of V row `key` inside a stage
-    __device__ static int v_addr(int key) {
-        if (DK == 64) return (key >> 2) * VGROUP + (key & 3) * ROWB;
-        if (DK == 128) return (key >> 1) * VGROUP + (key & 1) * ROWB;
-        return (key >> 3) * VGROUP + (((key & 3) * 2 + ((key >> 2) & 1))) * ROWB;
+    static_assert(DK == 32 || DK == 64 || DK == 96 || DK == 128, "head dimension");
+    static constexpr int BQ = 32 * WAVES;               // queries per workgroup
+    static constexpr int BKV = DK == 128 ? 32 : 64;             // keys per block
+    static constexpr int KROW = DK * 2, VROW = BKV * 2; // bytes of a row of one term: a key's, a column's
+    static constexpr int KPLANE = BKV * KROW, VPLANE = DK * VROW;
+    static constexpr int V_AT = 3 * KPLANE, STAGE = V_AT + 3 * VPLANE;
+    static constexpr bool DOUBLE = WAVES == 8;          // two blocks in LDS, or two workgroups per CU
+    static constexpr int PER_SIMD = DK == 128 && WAVES == 4 ? 1 : 2;     // waves: with two, 64 registers would spill
+    static constexpr int FLAGS_AT = (DOUBLE ? 2 : 1) * STAGE;
+    static constexpr int SMEM = FLAGS_AT + 4 * WAVES;   // a word per wave: does its part need the fp32 pass
+    static constexpr int E = BKV * DK % (512 * WAVES) == 0 ? 8 : 4;      // values of a piece that a thread stages
+    static constexpr int PIECES = BKV * DK / E / (64 * WAVES);          // pieces of K, and of V
+    static_assert(PIECES * E * 64 * WAVES == BKV * DK, "a block divides over the threads");
+    static_assert(SMEM * (DOUBLE ? 1 : 2) <= 160 * 1024, "eight waves per CU");
+    // where the 16-byte chunk c of row r lies
+    template <int ROW>
+    __device__ static unsigned at(int row, int chunk) {
+        const int key = ROW == 256 ? row & 15 : ROW == 128 ? (row >> 1) & 7 : (row >> 2) & 3;
+        return (unsigned)(row * ROW + ((chunk ^ key) << 4));
     }
+    __device__ static unsigned k_at(int row, int chunk) { return at<KROW>(row, chunk); }
+    __device__ static unsigned v_at(int col, int chunk) { return V_AT + at<VROW>(col, chunk); }
 };
 
-// RAG: S is not a multiple of 128.  Rows past the end of a head are never loaded (the load of such
-// a row is redirected to the head's last row, which keeps V finite), keys past the end are masked
-// like causal ones, and queries past the end are computed but not stored.
-// PAD: the head size dkr is below DK (a multiple of 4).  Lanes whose 16-byte chunk lies past column
-// dkr issue no load, so nothing outside a row is read; their places in the K stages are zeroed once
-// and never written again, Q's are zeroed in registers, V's feed output columns that are not stored.
-// The padded k-blocks and output tiles are multiplied like the others: branching around them
-// measured slower than the MFMAs they save (dk 96: 303 us with the branches, 268 without).
-template <int DK, bool CAUSAL, bool RAG, bool PAD>
-__global__ void __launch_bounds__(256)
+// Probabilities are kept times 2^24, so that their three terms are normal bf16 values as far down as the
+// probabilities themselves are normal floats.
+constexpr float SD_UP = 16777216.0f;
+
+// The smallest magnitude met, as twice its bit pattern less one (zero, which is no concern, comes out largest).
+constexpr unsigned SD_TINY = 25u << 24;                  // twice the bit pattern of 2^-102
+template <int E, typename T>
+__device__ __forceinline__ void cut(const float (&x)[E], T (&t)[3], unsigned *least) {
+#pragma unroll
+    for (int e = 0; e < E; e += 2) {
+        if (least) *least = min(*least, min(__float_as_uint(x[e]) * 2 - 1, __float_as_uint(x[e + 1]) * 2 - 1));
+        int hi, mid, lo;
+        bf16x3_nearest(x[e], x[e + 1], hi, mid, lo);
+        t[0][e / 2] = hi;
+        t[1][e / 2] = mid;
+        t[2][e / 2] = lo;
+    }
+}
+__device__ __forceinline__ v16f mfma_terms(const v4i &a, const v4i &b, const v16f &c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf, a), __builtin_bit_cast(v8bf, b), c, 0, 0, 0);
+}
+
+// The online softmax of a 32-key tile of scores (log2 units, masked ones -infinity): scores become
+// probabilities times `up`.  The reference point m_run of the exponentials only moves when some query's
+// maximum exceeds it by more than 2^8: until then p = 2^(s - m_run) <= 256 is safe in fp32 and exact in
+// the quotient O = sum(p v) / sum(p), and the accumulator needs no rescaling pass (which costs as many
+// vector instructions as the exponentials themselves).
+template <int DT>
+__device__ __forceinline__ void softmax_step(v16f &s, v16f (&acc_o)[DT], float &m_run, float &l_run, float up) {
+    float m_blk = -INFINITY;
+#pragma unroll
+    for (int v = 0; v < 16; v++) m_blk = fmaxf(m_blk, s[v]);
+    m_blk = fmaxf(m_blk, __shfl_xor(m_blk, 32, 64));
+    if (__builtin_amdgcn_ballot_w64(m_blk > m_run + 8.0f)) {      // wave-uniform; always taken for the first keys
+        const float m_new = fmaxf(m_run, m_blk);  // finite: key 0 is visible to every query
+        const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
+        l_run *= alpha;
+        m_run = m_new;
+#pragma unroll
+        for (int d = 0; d < DT; d++)
+#pragma unroll
+            for (int v = 0; v < 16; v++) acc_o[d][v] *= alpha;
+    }
+    float l_blk = 0.0f;
+#pragma unroll
+    for (int v = 0; v < 16; v++) {
+        const float p = __builtin_amdgcn_exp2f(s[v] - m_run) * up;
+        s[v] = p;
+        l_blk += p;
+    }
+    l_run += l_blk;
+}
+
+// A wave's 32 queries with fp32 instructions, operands straight from memory: the rare second pass.  Rows
+// past the end of the head are read as its last row, columns past dkr as zero (K, Q) or as the last one
+// (V: they feed output columns that are not stored).
+template <int DK, bool CAUSAL>
+__device__ __forceinline__ void attend_f32(const float *Qh, const float *Kh, const float *Vh, int64_t ld, int64_t S, int dkr, float scale_log2e,
+                                           int64_t wq_lo, int lane, v16f (&acc_o)[DK / 32], float &m_run, float &l_run) {
+    constexpr int DT = DK / 32;
+    const int frow = lane & 31, fhalf = lane >> 5;
+    const int64_t qg = wq_lo + frow;
+    const float *q = Qh + (qg < S ? qg : S - 1) * ld;
+    m_run = -INFINITY;
+    l_run = 0.0f;
+#pragma unroll
+    for (int d = 0; d < DT; d++)
+#pragma unroll
+        for (int v = 0; v < 16; v++) acc_o[d][v] = 0.0f;
+    const int64_t end = CAUSAL && wq_lo + 32 < S ? wq_lo + 32 : S;
+    for (int64_t k0 = 0; k0 < end; k0 += 32) {
+        const float *k = Kh + (k0 + frow < S ? k0 + frow : S - 1) * ld;
+        v16f s;
+#pragma unroll
+        for (int v = 0; v < 16; v++) s[v] = 0.0f;
+        for (int c = 4 * fhalf; c < DK; c += 8) {
+            v4f kf = {0.f, 0.f, 0.f, 0.f}, qf = kf;
+            if (c < dkr) {
+                kf = *reinterpret_cast<const v4f *>(k + c);
+                qf = *reinterpret_cast<const v4f *>(q + c) * scale_log2e;
+            }
+#pragma unroll
+            for (int e = 0; e < 4; e++) s = __builtin_amdgcn_mfma_f32_32x32x2f32(kf[e], qf[e], s, 0, 0, 0);
+        }
+        const int64_t seen = (CAUSAL && qg < S ? qg : S - 1) - k0;
+#pragma unroll
+        for (int v = 0; v < 16; v++)
+            if (8 * (v >> 2) + 4 * fhalf + (v & 3) > seen) s[v] = -INFINITY;
+        softmax_step<DT>(s, acc_o, m_run, l_run, 1.0f);
+#pragma unroll
+        for (int v = 0; v < 16; v++) {
+            const int64_t key = k0 + 8 * (v >> 2) + 4 * fhalf + (v & 3);
+            const float *row = Vh + (key < S ? key : S - 1) * ld;
+#pragma unroll
+            for (int d = 0; d < DT; d++) {
+                const int col = d * 32 + frow;
+                acc_o[d] = __builtin_amdgcn_mfma_f32_32x32x2f32(row[col < dkr ? col : dkr - 1], s[v], acc_o[d], 0, 0, 0);
+            }
+        }
+    }
+}
+
+// Rows past the end of a head are never read (such a row is redirected to the head's last row, which keeps
+// V finite), keys past the end are masked like causal ones, and queries past the end are computed but not stored.
+// PAD: the head size dkr is below DK (a multiple of 4): chunks of Q and K past column dkr are zero, columns
+// of V past it repeat the last one and feed output columns that are not stored.
+template <int DK, int WAVES, bool CAUSAL, bool PAD>
+__global__ void __launch_bounds__(64 * WAVES, (SdGeom<DK, WAVES>::PER_SIMD))
 k_sdpa(const float *__restrict__ Q, const float *__restrict__ K, const float *__restrict__ V,
        float *__restrict__ O, float *__restrict__ L, int64_t BH, int64_t S, float scale_log2e,
        int64_t H, int64_t ld, int64_t ldo, int dkr, int pair_tiles) {
-    using G = SdGeom<DK>;
-    constexpr int KB = DK / 8;                   // 8-wide k-blocks of the score product
+    using G = SdGeom<DK, WAVES>;
+    constexpr int BQ = G::BQ, BKV = G::BKV, E = G::E;
+    constexpr int KS = DK / 16;                  // 16-wide steps of the score product
     constexpr int DT = DK / 32;                  // 32-wide column tiles of the output
+    // the five smaller products of a score's terms in a sum of their own, where there are registers for it
+    constexpr bool APART = DK <= 64;
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int frow = lane & 31, fhalf = lane >> 5;
-    const int64_t nq = (S + SD_BQ - 1) / SD_BQ;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int64_t nq = (S + BQ - 1) / BQ;
     // Workgroups are handed to the 8 XCDs round-robin by linear index, and inside an XCD to its
     // CUs in a fixed rotation, so every workgroup has to carry the same amount of work.  Eight
     // heads form a group: workgroup r of a group works on head r % 8 (every query tile of a
     // head then runs on the same XCD and shares its L2 copy of K and V) and on unit r / 8.
     // A unit is one query tile, or, causal, the pair of tiles p and nq-1-p, which together
-    // visit nq+1 key blocks whatever p is (the middle tile of an odd nq stands alone).  A launch
+    // visit the same number of keys whatever p is (the middle tile of an odd nq stands alone).  A launch
     // with no more single tiles than CUs keeps them single (pair_tiles = 0): pairing would only
-    // halve the CUs at work (64 heads of 256 rows: 33.3 us paired, 22.7 single, 20.7 unmasked).
+    // halve the CUs at work.
     const bool paired = CAUSAL && pair_tiles;
     const int64_t units = paired ? (nq + 1) / 2 : nq;
     const int64_t lin = blockIdx.x, group = lin / (8 * units), left = BH - group * 8;
@@ -109,116 +204,100 @@ k_sdpa(const float *__restrict__ Q, const float *__restrict__ K, const float *__
     // and ldo (O): H = 1, ld = DK is one matrix per head; H heads side by side in rows of
     // ld >= H * DK floats is the layout a fused projection writes and the output projection reads
     const int64_t hb = head / H, hh = head - hb * H;
-    const int64_t in0 = hb * S * ld + hh * (PAD ? dkr : DK);
+    const int width = PAD ? dkr : DK;
+    const int64_t in0 = hb * S * ld + hh * width;
     const float *Qh = Q + in0, *Kh = K + in0, *Vh = V + in0;
     const unsigned rowb = (unsigned)ld * 4;      // bytes between rows in global memory
-    const unsigned lds0 = (unsigned)(uintptr_t)lds;
-    if (PAD) {                                   // the K stages' never-loaded chunks must read as zero
-        for (int o = tid * 16; o < 2 * G::KSTAGE; o += 256 * 16)
-            *reinterpret_cast<v4f *>(lds + o) = v4f{0.f, 0.f, 0.f, 0.f};
-        __syncthreads();
-    }
-
-    // per-lane byte offsets of the direct-to-LDS loads: instruction i of this wave is number
-    // 4*i + wave of a 64-row block and covers rows RPI*(4*i + wave) .. + RPI-1
-    unsigned koff[G::IPW], voff[G::IPW];
-    bool kact[G::IPW];                           // PAD: does this lane's chunk of a K / Q row exist
-    const bool vact = !PAD || (lane % G::CH) * 4 < dkr;
-#pragma unroll
-    for (int i = 0; i < G::IPW; i++) {
-        const int slot = lane / G::CH, c = lane % G::CH;
-        const int krow = G::RPI * (4 * i + wave) + slot;
-        kact[i] = !PAD || (c ^ G::swz(krow)) * 4 < dkr;
-        koff[i] = (unsigned)(krow * rowb + ((c ^ G::swz(krow)) << 4));
-        const int vrow = G::RPI * (4 * i + wave) + G::v_row_of_slot(slot);
-        voff[i] = (unsigned)(vrow * rowb + (c << 4));
-    }
-    // the same offsets for a 64-row block of which only the first `valid` (1..63) rows exist: the
-    // LDS slot (and so the swizzle) stays that of the nominal row, the source row is the last one
-    auto koff_clamped = [&](int i, int valid) {
-        const int slot = lane / G::CH, c = lane % G::CH;
-        const int krow = G::RPI * (4 * i + wave) + slot;
-        return (unsigned)((krow < valid ? krow : valid - 1) * rowb + ((c ^ G::swz(krow)) << 4));
-    };
-    auto voff_clamped = [&](int i, int valid) {
-        const int slot = lane / G::CH, c = lane % G::CH;
-        const int vrow = G::RPI * (4 * i + wave) + G::v_row_of_slot(slot);
-        return (unsigned)((vrow < valid ? vrow : valid - 1) * rowb + (c << 4));
-    };
 
     for (int pass = 0; pass < passes; pass++) {
-        const int64_t q0 = (paired && pass == 0 ? nq - 1 - unit : unit) * SD_BQ;
-        if (pass) __syncthreads();                   // the first tile's last key block has been read
-        // ---- Q tile (128 rows) through the V area, then into registers; the first key block's
-        // K rows stream into their own stage at the same time, so a workgroup pays one load
-        // latency, not two, before its first MFMA.  Its V rows follow once Q has left the V area.
-        const int64_t all_blocks = (S + SD_BKV - 1) / SD_BKV;
-        const int64_t nblocks = CAUSAL && (q0 + SD_BQ) / SD_BKV < all_blocks ? (q0 + SD_BQ) / SD_BKV : all_blocks;
-        constexpr unsigned Q_BASE = 2 * G::KSTAGE;   // 2 * KSTAGE bytes of Q fit the two V stages
-        static_assert(2 * G::KSTAGE <= 2 * G::VSTAGE, "Q staging area");
-        auto issue_k = [&](int64_t blk, int stage) {
-            const char *kg = reinterpret_cast<const char *>(Kh + blk * SD_BKV * ld);
-            const int64_t valid = S - blk * SD_BKV;
-            if (RAG && valid < SD_BKV) {
+        int t = threadIdx.x;                         // opaque: addresses are formed for each tile, not held from one to the next
+        asm volatile("" : "+v"(t));
+        const int lane = t & 63, frow = lane & 31, fhalf = lane >> 5;
+        // the pieces this thread stages of each block: E columns of a key's row of K, E keys of a column of V
+        // (a chunk holds those of registers 8s .. 8s+7 of a lane half: 16s + 4 * half + 0..3 and 8 further on)
+        int krow[G::PIECES], kcol[G::PIECES], vcol[G::PIECES], vkey[G::PIECES];
+        unsigned kput[G::PIECES], vput[G::PIECES];
 #pragma unroll
-                for (int i = 0; i < G::IPW; i++)
-                    if (kact[i]) AXS_LOAD_LDS(lds0 + stage * G::KSTAGE + (4 * i + wave) * 1024, koff_clamped(i, (int)valid), kg);
-            } else {
-#pragma unroll
-                for (int i = 0; i < G::IPW; i++)
-                    if (kact[i]) AXS_LOAD_LDS(lds0 + stage * G::KSTAGE + (4 * i + wave) * 1024, koff[i], kg);
-            }
-        };
-        auto issue_v = [&](int64_t blk, int stage) {
-            const char *vg = reinterpret_cast<const char *>(Vh + blk * SD_BKV * ld);
-            const int64_t valid = S - blk * SD_BKV;
-            if (RAG && valid < SD_BKV) {
-#pragma unroll
-                for (int i = 0; i < G::IPW; i++)
-                    if (vact) AXS_LOAD_LDS(lds0 + 2 * G::KSTAGE + stage * G::VSTAGE + (4 * i + wave) * G::VGROUP, voff_clamped(i, (int)valid), vg);
-            } else {
-#pragma unroll
-                for (int i = 0; i < G::IPW; i++)
-                    if (vact) AXS_LOAD_LDS(lds0 + 2 * G::KSTAGE + stage * G::VSTAGE + (4 * i + wave) * G::VGROUP, voff[i], vg);
-            }
-        };
-        if (RAG && q0 + SD_BQ > S) {
-            // a half with no row inside the head re-reads the first half (its queries are never stored)
-            const int64_t valid0 = S - q0 < 64 ? S - q0 : 64, left1 = S - q0 - 64;
-            const int64_t base1 = left1 > 0 ? q0 + 64 : q0, valid1 = left1 > 0 ? (left1 < 64 ? left1 : 64) : valid0;
-#pragma unroll
-            for (int i = 0; i < G::IPW; i++) {
-                if (!kact[i]) continue;
-                AXS_LOAD_LDS(lds0 + Q_BASE + (4 * i + wave) * 1024, koff_clamped(i, (int)valid0),
-                             reinterpret_cast<const char *>(Qh + q0 * ld));
-                AXS_LOAD_LDS(lds0 + Q_BASE + G::KSTAGE + (4 * i + wave) * 1024, koff_clamped(i, (int)valid1),
-                             reinterpret_cast<const char *>(Qh + base1 * ld));
-            }
-        } else {
-#pragma unroll
-            for (int i = 0; i < G::IPW; i++) {
-                if (!kact[i]) continue;
-                AXS_LOAD_LDS(lds0 + Q_BASE + (4 * i + wave) * 1024, koff[i], reinterpret_cast<const char *>(Qh + q0 * ld));
-                AXS_LOAD_LDS(lds0 + Q_BASE + G::KSTAGE + (4 * i + wave) * 1024, koff[i],
-                             reinterpret_cast<const char *>(Qh + (q0 + 64) * ld));
-            }
+        for (int i = 0; i < G::PIECES; i++) {
+            const int q = t + i * 64 * WAVES, kc = q % (DK / E), vd = q % DK, vc = q / DK;
+            krow[i] = q / (DK / E);
+            kcol[i] = kc * E;
+            kput[i] = G::k_at(krow[i], kc * E / 8) + kc * E % 8 * 2;
+            vcol[i] = PAD && vd >= dkr ? dkr - 1 : vd;
+            vkey[i] = E == 8 ? 16 * (vc >> 1) + 4 * (vc & 1) : 16 * (vc >> 2) + 4 * (vc >> 1 & 1) + 8 * (vc & 1);
+            vput[i] = G::v_at(vd, vc * E / 8) + vc * E % 8 * 2;
         }
-        issue_k(0, 0);
-        AXS_VM0();
-        __syncthreads();
-        v4f qf[KB];                                  // k-block kb: dk 8*kb + 4*fhalf .. +3 of this lane's query
+        float kr[G::PIECES][E], vr[G::PIECES][E];
+        auto load_row = [&](auto &x, const char *base, unsigned off, int col) {      // columns from `col` on
+            constexpr int N = sizeof(x) / 16;
+#pragma unroll
+            for (int h = 0; h < N; h++) {
+                v4f a = {0.f, 0.f, 0.f, 0.f};
+                if (!PAD || col + 4 * h < dkr) a = *reinterpret_cast<const v4f *>(base + off + 16 * h);
+#pragma unroll
+                for (int e = 0; e < 4; e++) x[4 * h + e] = a[e];
+            }
+        };
+        auto load = [&](int64_t blk) {
+            const char *kg = reinterpret_cast<const char *>(Kh + blk * BKV * ld), *vg = reinterpret_cast<const char *>(Vh + blk * BKV * ld);
+            const int64_t valid = S - blk * BKV;
+            if (valid >= BKV) {
+#pragma unroll
+                for (int i = 0; i < G::PIECES; i++) load_row(kr[i], kg, krow[i] * rowb + kcol[i] * 4, kcol[i]);
+#pragma unroll
+                for (int i = 0; i < G::PIECES; i++) {
+                    const unsigned off = vkey[i] * rowb + vcol[i] * 4;
+#pragma unroll
+                    for (int e = 0; e < E; e++) vr[i][e] = *reinterpret_cast<const float *>(vg + (uint64_t)(e + (e & 4)) * rowb + off);
+                }
+            } else {
+                const int end = (int)valid - 1;
+#pragma unroll
+                for (int i = 0; i < G::PIECES; i++) load_row(kr[i], kg, (krow[i] < end ? krow[i] : end) * rowb + kcol[i] * 4, kcol[i]);
+#pragma unroll
+                for (int i = 0; i < G::PIECES; i++) {
+#pragma unroll
+                    for (int e = 0; e < E; e++) {
+                        const int key = vkey[i] + e + (e & 4);
+                        vr[i][e] = *reinterpret_cast<const float *>(vg + (key < end ? key : end) * rowb + vcol[i] * 4);
+                    }
+                }
+            }
+        };
+        unsigned least;
+        auto put = [&](const float (&x)[E], unsigned at, unsigned plane) {
+            std::conditional_t<E == 8, v4i, v2i> terms[3];
+            cut(x, terms, &least);
+#pragma unroll
+            for (int p = 0; p < 3; p++) *reinterpret_cast<decltype(&terms[0])>(lds + at + p * plane) = terms[p];
+        };
+        auto stage = [&](unsigned at) {              // the block in registers, to LDS
+#pragma unroll
+            for (int i = 0; i < G::PIECES; i++) put(kr[i], at + kput[i], G::KPLANE);
+#pragma unroll
+            for (int i = 0; i < G::PIECES; i++) put(vr[i], at + vput[i], G::VPLANE);
+        };
+        const int64_t q0 = (paired && pass == 0 ? nq - 1 - unit : unit) * BQ;
+        const int64_t all_blocks = (S + BKV - 1) / BKV;
+        const int64_t nblocks = CAUSAL && (q0 + BQ) / BKV < all_blocks ? (q0 + BQ) / BKV : all_blocks;
+        const int64_t wq_lo = q0 + wave * 32, qg = wq_lo + frow;      // this wave's first query, this lane's query
+        least = 0xffffffffu;
+        load(0);
+        v4i qf[KS][3];                               // step ks: dk 16*ks + 8*fhalf .. +7 of this lane's query
         {
-            const int r = wave * 32 + frow;          // rows 64..127 sit KSTAGE bytes further on, same swizzle
-            const unsigned char *qrow = lds + Q_BASE + (r >> 6) * G::KSTAGE + (r & 63) * G::ROWB;
+            const char *q = reinterpret_cast<const char *>(Qh + (qg < S ? qg : S - 1) * ld);
 #pragma unroll
-            for (int kb = 0; kb < KB; kb++)      // scale * log2(e) goes into Q once: scores come out in log2 units
-            {
-                qf[kb] = *reinterpret_cast<const v4f *>(qrow + (((kb * 2 + fhalf) ^ G::swz(r & 63)) << 4)) * scale_log2e;
-                if (PAD && kb * 8 + 4 * fhalf >= dkr) qf[kb] = v4f{0.f, 0.f, 0.f, 0.f};   // whatever the unloaded chunk held
+            for (int ks = 0; ks < KS; ks++) {        // scale * log2(e) goes into Q once: scores come out in log2 units
+                float x[8];
+                load_row(x, q, (16 * ks + 8 * fhalf) * 4, 16 * ks + 8 * fhalf);
+#pragma unroll
+                for (int e = 0; e < 8; e++) x[e] *= scale_log2e;
+                cut(x, qf[ks], &least);
             }
         }
+        stage(0);
+        if (G::DOUBLE && nblocks > 1) load(1);
         __syncthreads();
-        issue_v(0, 0);
 
         v16f acc_o[DT];
 #pragma unroll
@@ -226,169 +305,174 @@ k_sdpa(const float *__restrict__ Q, const float *__restrict__ K, const float *__
 #pragma unroll
             for (int v = 0; v < 16; v++) acc_o[d][v] = 0.0f;
         float m_run = -INFINITY, l_run = 0.0f;       // l_run: this lane half's share of the row sum
-        const int64_t qg = q0 + wave * 32 + frow;    // this lane's query
 
-        for (int64_t blk = 0; blk < nblocks; blk++) {
-            const int stage = (int)(blk & 1);
-            if (blk > 0) {
-                AXS_VM0();
-                __syncthreads();                      // block blk has landed; stage^1 is free again
-            }
-            if (blk + 1 < nblocks) {
-                issue_k(blk + 1, stage ^ 1);
-                issue_v(blk + 1, stage ^ 1);
-            }
-            const unsigned char *ks = lds + stage * G::KSTAGE;
-            const unsigned char *vs = lds + 2 * G::KSTAGE + stage * G::VSTAGE;
+        auto attend = [&](int64_t blk, unsigned at) {
+            const int64_t kb0 = blk * BKV;
+#pragma unroll 1
+            for (int kt = 0; kt < BKV / 32; kt++) {
+                // a wave past the end of the head has nothing to do; causal: a 32-key tile entirely above this wave's 32 queries is
+                // skipped, and only tiles that straddle the diagonal pay for the mask (all wave-uniform decisions)
+                const int64_t kt0 = kb0 + 32 * kt;
+                if ((CAUSAL && kt0 > wq_lo + 31) || kt0 >= S || wq_lo >= S) break;
+                const bool need_mask = CAUSAL ? kt0 + 31 > wq_lo : kt0 + 32 > S;
 
-            // causal: a 32-key tile entirely above this wave's 32 queries is skipped, and only
-            // blocks that straddle the diagonal pay for the mask (all wave-uniform decisions)
-            const int64_t kb0 = blk * SD_BKV, wq_lo = q0 + wave * 32;
-            const bool tile_on[2] = {!CAUSAL || kb0 <= wq_lo + 31,
-                                     (!CAUSAL || kb0 + 32 <= wq_lo + 31) && (!RAG || kb0 + 32 < S)};
-            const bool need_mask = (CAUSAL && kb0 + SD_BKV - 1 > wq_lo) || (RAG && !CAUSAL && kb0 + SD_BKV > S);
-            // keys of this block with index > qrel are masked: those after the query (causal; such a
-            // query lies inside the head, so they cover the keys past its end too) or past the end
-            const int qrel = (int)((CAUSAL ? qg : S - 1) - kb0);
+                // ---- scores ----
+                v16f s, low;
+#pragma unroll
+                for (int v = 0; v < 16; v++) s[v] = low[v] = 0.0f;
+                __builtin_amdgcn_s_setprio(1);  // matrix phases go ahead of the co-resident wave's vector work
+#pragma unroll
+                for (int ks = 0; ks < KS; ks++) {
+                    v4i kf[3];
+#pragma unroll
+                    for (int p = 0; p < 3; p++)
+                        kf[p] = *reinterpret_cast<const v4i *>(lds + at + G::k_at(frow, 2 * ks + fhalf) + kt * 32 * G::KROW + p * G::KPLANE);
+#pragma unroll
+                    for (int sum = 2; sum > 0; sum--)
+#pragma unroll
+                        for (int p = sum; p >= 0; p--) (APART ? low : s) = mfma_terms(kf[sum - p], qf[ks][p], APART ? low : s);
+                    s = mfma_terms(kf[0], qf[ks][0], s);
+                }
+                __builtin_amdgcn_s_setprio(0);
+                if (APART) s += low;
+                if (need_mask) {
+                    // keys of this tile with index > qrel are masked: those after the query (causal; such a query
+                    // lies inside the head, so they cover the keys past its end too) or past the end
+                    const int qrel = (int)((CAUSAL ? qg : S - 1) - kt0);
+#pragma unroll
+                    for (int v = 0; v < 16; v++)
+                        if (8 * (v >> 2) + 4 * fhalf + (v & 3) > qrel) s[v] = -INFINITY;
+                }
+                softmax_step<DT>(s, acc_o, m_run, l_run, SD_UP);
 
-            // ---- scores of 64 keys ----
-            v16f acc_s[2];
-            __builtin_amdgcn_s_setprio(1);      // MFMA phases go ahead of the co-resident wave's VALU work
+                // ---- O^T += V^T P^T ----
 #pragma unroll
-            for (int kt = 0; kt < 2; kt++) {
+                for (int st = 0; st < 2; st++) {
+                    float x[8];
 #pragma unroll
-                for (int v = 0; v < 16; v++) acc_s[kt][v] = 0.0f;
-                if (!tile_on[kt]) continue;
-                const int r = kt * 32 + frow;
-                const unsigned char *krow = ks + r * G::ROWB;
+                    for (int e = 0; e < 8; e++) x[e] = s[8 * st + e];
+                    v4i pf[3];
+                    cut(x, pf, nullptr);
 #pragma unroll
-                for (int kb = 0; kb < KB; kb++) {
-                    const v4f kf = *reinterpret_cast<const v4f *>(krow + (((kb * 2 + fhalf) ^ G::swz(r)) << 4));
+                    for (int d = 0; d < DT; d++) {
+                        v4i vf[3];
 #pragma unroll
-                    for (int e = 0; e < 4; e++)
-                        acc_s[kt] = __builtin_amdgcn_mfma_f32_32x32x2f32(kf[e], qf[kb][e], acc_s[kt], 0, 0, 0);
+                        for (int p = 2; p >= 0; p--)
+                            vf[p] = *reinterpret_cast<const v4i *>(lds + at + G::v_at(d * 32 + frow, 4 * kt + 2 * st + fhalf) + p * G::VPLANE);
+#pragma unroll
+                        for (int sum = 2; sum >= 0; sum--)                // the small products first
+#pragma unroll
+                            for (int p = sum; p >= 0; p--) acc_o[d] = mfma_terms(vf[p], pf[sum - p], acc_o[d]);
+                    }
                 }
             }
-
-            __builtin_amdgcn_s_setprio(0);
-            // ---- online softmax ----
-            // Scores arrive in log2 units (Q was scaled once, above).  The reference point m_run
-            // of the exponentials only moves when some query's block maximum exceeds it by more
-            // than 2^8: until then p = 2^(s - m_run) <= 256 is safe in fp32 and exact in the
-            // quotient O = sum(p v) / sum(p), and the accumulator needs no rescaling pass (which
-            // costs as many vector instructions as the exponentials themselves; the fp32 MFMAs
-            // run on the same lanes as vector instructions, so every one saved is MFMA time).
-            float m_blk = -INFINITY;
-#pragma unroll
-            for (int kt = 0; kt < 2; kt++)
-#pragma unroll
-                for (int v = 0; v < 16; v++) {
-                    float s = acc_s[kt][v];
-                    if ((CAUSAL || RAG) && (!tile_on[kt] || (need_mask && kt * 32 + 8 * (v >> 2) + 4 * fhalf + (v & 3) > qrel)))
-                        s = -INFINITY;
-                    acc_s[kt][v] = s;
-                    m_blk = fmaxf(m_blk, s);
-                }
-            m_blk = fmaxf(m_blk, __shfl_xor(m_blk, 32, 64));
-            if (__builtin_amdgcn_ballot_w64(m_blk > m_run + 8.0f)) {      // wave-uniform; always taken for block 0
-                const float m_new = fmaxf(m_run, m_blk);  // finite: key 0 is visible to every query
-                const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
-                l_run *= alpha;
-                m_run = m_new;
-#pragma unroll
-                for (int d = 0; d < DT; d++)
-#pragma unroll
-                    for (int v = 0; v < 16; v++) acc_o[d][v] *= alpha;
-            }
-            float l_blk = 0.0f;
-#pragma unroll
-            for (int kt = 0; kt < 2; kt++)
-#pragma unroll
-                for (int v = 0; v < 16; v++) {
-                    const float p = __builtin_amdgcn_exp2f(acc_s[kt][v] - m_run);
-                    acc_s[kt][v] = p;
-                    l_blk += p;
-                }
-            l_run += l_blk;
-
-            if (blk == 0) {                           // the first block's V rows were issued last
-                if (nblocks > 1) AXS_VM(2 * G::IPW);      // loads return in order: all but block 1's
-                else AXS_VM0();
+        };
+        if constexpr (G::DOUBLE) {
+            // Two blocks in LDS and the next one in registers.  The two waves of a SIMD (w, w + 4) put it beside the current
+            // block before and after that is multiplied, so that one cuts while the other's products run.
+            unsigned cur = 0;
+            for (int64_t blk = 0; blk < nblocks; blk++, cur ^= G::STAGE) {
+                const bool more = blk + 1 < nblocks;
+                auto next = [&]() {
+                    stage(cur ^ G::STAGE);
+                    if (blk + 2 < nblocks) load(blk + 2);
+                };
+                if (more && wave >= 4) next();
+                attend(blk, cur);
+                if (more && wave < 4) next();
                 __syncthreads();
             }
-            // ---- O^T += V^T P^T ----
-            __builtin_amdgcn_s_setprio(1);
-#pragma unroll
-            for (int kt = 0; kt < 2; kt++) {
-                if (!tile_on[kt]) continue;
-#pragma unroll
-                for (int v = 0; v < 16; v++) {
-                    const int key = kt * 32 + 8 * (v >> 2) + 4 * fhalf + (v & 3);
-                    const float *vrow = reinterpret_cast<const float *>(vs + G::v_addr(key));
-#pragma unroll
-                    for (int d = 0; d < DT; d++)
-                        acc_o[d] = __builtin_amdgcn_mfma_f32_32x32x2f32(vrow[d * 32 + frow], acc_s[kt][v], acc_o[d], 0, 0, 0);
+        } else {
+            for (int64_t blk = 0; blk < nblocks; blk++) {
+                const bool more = blk + 1 < nblocks;
+                if (more) load(blk + 1);
+                attend(blk, 0);
+                __syncthreads();                      // the block has been read
+                if (more) {
+                    stage(0);
+                    __syncthreads();
                 }
             }
-            __builtin_amdgcn_s_setprio(0);
+        }
+
+        // ---- did every sum come out finite, and were all magnitudes such that the terms hold them? ----
+        float finite = l_run * 0.0f, up = SD_UP;
+#pragma unroll
+        for (int d = 0; d < DT; d++)
+#pragma unroll
+            for (int v = 0; v < 16; v++) finite = __builtin_fmaf(acc_o[d][v], 0.0f, finite);
+        int *unfit = reinterpret_cast<int *>(lds + G::FLAGS_AT);
+        const bool bad = __builtin_amdgcn_ballot_w64(!(finite == 0.0f) || least < SD_TINY) != 0;
+        if (lane == 0) unfit[wave] = bad;
+        __syncthreads();
+        int any = 0;
+#pragma unroll
+        for (int w = 0; w < WAVES; w++) any |= unfit[w];
+        if (__builtin_amdgcn_readfirstlane(any)) {
+            int again = lane;                        // opaque, so that no address of this pass is held through the loop above
+            asm volatile("" : "+v"(again));
+            attend_f32<DK, CAUSAL>(Qh, Kh, Vh, ld, S, width, scale_log2e, wq_lo, again, acc_o, m_run, l_run);
+            up = 1.0f;
         }
 
         // ---- normalise and write: lane owns query qg, dk columns 32*d + 8*g + 4*fhalf .. +3 ----
         const float l_tot = l_run + __shfl_xor(l_run, 32, 64);
         const float inv = 1.0f / l_tot;
-        float *orow = O + (hb * S + qg) * ldo + hh * (PAD ? dkr : DK);
-        if (!RAG || qg < S) {
+        float *orow = O + (hb * S + qg) * ldo + hh * width;
+        if (qg < S) {
 #pragma unroll
             for (int d = 0; d < DT; d++)
 #pragma unroll
                 for (int g = 0; g < 4; g++) {
-                    v4f r;
+                    v4f o;
 #pragma unroll
-                    for (int e = 0; e < 4; e++) r[e] = acc_o[d][4 * g + e] * inv;
-                    if (!PAD || d * 32 + 8 * g + 4 * fhalf < dkr) *reinterpret_cast<v4f *>(orow + d * 32 + 8 * g + 4 * fhalf) = r;
+                    for (int e = 0; e < 4; e++) o[e] = acc_o[d][4 * g + e] * inv;
+                    if (!PAD || d * 32 + 8 * g + 4 * fhalf < dkr) *reinterpret_cast<v4f *>(orow + d * 32 + 8 * g + 4 * fhalf) = o;
                 }
-            if (L && fhalf == 0) L[head * S + qg] = (m_run + __builtin_amdgcn_logf(l_tot)) * 0.6931471805599453f;
+            if (L && fhalf == 0) L[head * S + qg] = (m_run + __builtin_amdgcn_logf(l_tot / up)) * 0.6931471805599453f;
         }
     }
 }
 
-template <int DK, bool PAD>
+template <int DK, int WAVES, bool PAD>
 int launch_sdpa_p(const float *Q, const float *K, const float *V, float *O, float *L, int64_t BH, int64_t S,
                   float scale, int causal, int64_t H, int64_t ld, int64_t ldo, int dkr) {
-    using G = SdGeom<DK>;
+    using G = SdGeom<DK, WAVES>;
     static bool attr_set = false;
-    const void *kernels[4] = {reinterpret_cast<const void *>(k_sdpa<DK, false, false, PAD>),
-                              reinterpret_cast<const void *>(k_sdpa<DK, true, false, PAD>),
-                              reinterpret_cast<const void *>(k_sdpa<DK, false, true, PAD>),
-                              reinterpret_cast<const void *>(k_sdpa<DK, true, true, PAD>)};
     if (!attr_set) {
-        for (const void *k : kernels)
+        for (const void *k : {reinterpret_cast<const void *>(k_sdpa<DK, WAVES, false, PAD>), reinterpret_cast<const void *>(k_sdpa<DK, WAVES, true, PAD>)})
             AXHIP_HIP_TRY(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, G::SMEM), "hipFuncSetAttribute");
         attr_set = true;
     }
     const float sl2 = scale * 1.4426950408889634f;
-    const int64_t nq = (S + SD_BQ - 1) / SD_BQ;
+    const int64_t nq = (S + G::BQ - 1) / G::BQ;
     // causal tiles p and nq-1-p in one workgroup once there are more tiles than CUs; with a CU for every tile the
     // longest tile sets the time either way and pairing only halves the CUs at work
     const int pair = causal && nq * BH > (int64_t)cu_count();
-    dim3 grid((unsigned)((pair ? (nq + 1) / 2 : nq) * BH));
-    const bool rag = S % SD_BQ != 0;
-#define AXS_GO(C, R)                                                                                              \
-    hipLaunchKernelGGL((k_sdpa<DK, C, R, PAD>), grid, dim3(256), G::SMEM, kStream, Q, K, V, O, L, BH, S, sl2, H, ld, \
-                       ldo, dkr, pair)
-    if (causal && rag) AXS_GO(true, true);
-    else if (causal) AXS_GO(true, false);
-    else if (rag) AXS_GO(false, true);
-    else AXS_GO(false, false);
-#undef AXS_GO
+    dim3 grid((unsigned)((pair ? (nq + 1) / 2 : nq) * BH)), block(64 * WAVES);
+    if (causal)
+        hipLaunchKernelGGL((k_sdpa<DK, WAVES, true, PAD>), grid, block, G::SMEM, kStream, Q, K, V, O, L, BH, S, sl2, H, ld, ldo, dkr, pair);
+    else
+        hipLaunchKernelGGL((k_sdpa<DK, WAVES, false, PAD>), grid, block, G::SMEM, kStream, Q, K, V, O, L, BH, S, sl2, H, ld, ldo, dkr, pair);
     return check_launch("sdpa_fwd");
 }
 
 template <int DK>
 int launch_sdpa(const float *Q, const float *K, const float *V, float *O, float *L, int64_t BH, int64_t S,
                 float scale, int causal, int64_t H, int64_t ld, int64_t ldo, int dkr) {
-    return dkr == DK ? launch_sdpa_p<DK, false>(Q, K, V, O, L, BH, S, scale, causal, H, ld, ldo, dkr)
-                     : launch_sdpa_p<DK, true>(Q, K, V, O, L, BH, S, scale, causal, H, ld, ldo, dkr);
+    // Eight waves on 256 queries cut half as much of K and V for each of them, four on 128 waste less of a short head and
+    // of the diagonal.  us, four waves -> eight: 64 heads of [1024, 128] 191 -> 174 (causal 158 -> 142), 64 of [1024, 96]
+    // 141 -> 126, 96 causal ones of [1000, 80] 146 -> 129, 512 of [512, 64] 201 -> 194; but causal 126 -> 134, 512 of [256, 32]
+    // 33 -> 37, 256 causal ones of [333, 48] 49 -> 53, and with fewer tiles than CUs (64 of [128, 64]) 11.0 -> 13.9.  Geometry
+    // 128 has the registers of one wave per SIMD with four waves, so it takes eight as soon as there is more than one tile a CU.
+    if constexpr (DK > 32) {
+        const int64_t half_tiles = (S + 127) / 128, tiles = (S + 255) / 256;
+        if (DK == 128 ? half_tiles * BH > cu_count() : DK >= (causal ? 96 : 64) && tiles * BH >= cu_count() && tiles * 8 <= half_tiles * 5)
+            return dkr == DK ? launch_sdpa_p<DK, 8, false>(Q, K, V, O, L, BH, S, scale, causal, H, ld, ldo, dkr)
+                             : launch_sdpa_p<DK, 8, true>(Q, K, V, O, L, BH, S, scale, causal, H, ld, ldo, dkr);
+    }
+    return dkr == DK ? launch_sdpa_p<DK, 4, false>(Q, K, V, O, L, BH, S, scale, causal, H, ld, ldo, dkr)
+                     : launch_sdpa_p<DK, 4, true>(Q, K, V, O, L, BH, S, scale, causal, H, ld, ldo, dkr);
 }
 
 // One workgroup per score row: mask, maximum, exponentials, sum, normalise in place; L = max + log(sum).
@@ -457,7 +541,7 @@ int sdpa_unfused(const float *Q, const float *K, const float *V, float *O, float
 }  // namespace
 
 // shared by both entry points: H heads side by side in rows of ld (Q, K, V) / ldo (O) floats.  A head
-// size that is a multiple of 4 up to 128 runs on the kernel of the next size among 32, 64, 128.
+// size that is a multiple of 4 up to 128 runs on the kernel of the next size among 32, 64, 96, 128.
 static bool sdpa_fusable(int64_t dk) { return dk >= 4 && dk <= 128 && dk % 4 == 0; }
 
 static int sdpa_fused(const float *Q, const float *K, const float *V, float *O, float *L, int64_t BH, int64_t S,
@@ -469,6 +553,9 @@ static int sdpa_fused(const float *Q, const float *K, const float *V, float *O, 
     } else if (dk <= 64) {
         rc = launch_sdpa<64>(Q, K, V, O, L, BH, S, scale, causal, H, ld, ldo, (int)dk);
         axhip::note_kernel(causal ? "sdpa_fused_dk64_causal" : "sdpa_fused_dk64");
+    } else if (dk <= 96) {
+        rc = launch_sdpa<96>(Q, K, V, O, L, BH, S, scale, causal, H, ld, ldo, (int)dk);
+        axhip::note_kernel(causal ? "sdpa_fused_dk96_causal" : "sdpa_fused_dk96");
     } else {
         rc = launch_sdpa<128>(Q, K, V, O, L, BH, S, scale, causal, H, ld, ldo, (int)dk);
         axhip::note_kernel(causal ? "sdpa_fused_dk128_causal" : "sdpa_fused_dk128");
@@ -483,7 +570,7 @@ extern "C" int axhip_sdpa_fwd(const float *Q, const float *K, const float *V, fl
     if (BH < 0 || S < 0 || dk <= 0) return fail(AXHIP_ERR_SHAPE, "sdpa_fwd: bad extent");
     if (BH == 0 || S == 0) return AXHIP_OK;
     const bool aligned = ((((uintptr_t)Q | (uintptr_t)K | (uintptr_t)V | (uintptr_t)O) & 15) == 0);
-    if (sdpa_fusable(dk) && aligned && (S + SD_BQ - 1) / SD_BQ * BH <= 0x7fffffff)
+    if (sdpa_fusable(dk) && aligned && (S + 127) / 128 * BH <= 0x7fffffff)
         return sdpa_fused(Q, K, V, O, L, BH, S, dk, scale, causal, 1, dk, dk);
     return sdpa_unfused(Q, K, V, O, L, BH, S, dk, scale, causal);
 }
@@ -500,7 +587,7 @@ extern "C" int axhip_sdpa_fwd_rows(const float *Q, const float *K, const float *
     if ((((uintptr_t)Q | (uintptr_t)K | (uintptr_t)V | (uintptr_t)O) & 15) != 0)
         return fail(AXHIP_ERR_SHAPE, "sdpa_fwd_rows: tensors must be 16-byte aligned");
     if (B == 0 || S == 0) return AXHIP_OK;
-    if (B > 0x7fffffff / H || (S + SD_BQ - 1) / SD_BQ * (B * H) > 0x7fffffff)
+    if (B > 0x7fffffff / H || (S + 127) / 128 * (B * H) > 0x7fffffff)
         return fail(AXHIP_ERR_SHAPE, "sdpa_fwd_rows: too many tiles");
     return sdpa_fused(Q, K, V, O, L, B * H, S, dk, scale, causal, H, ld, ldo);
 }
