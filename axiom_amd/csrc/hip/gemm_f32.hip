@@ -1195,6 +1195,9 @@ int try_nt_cols(const SgemmArgs &g, int64_t batch) {
     if ((((uintptr_t)g.A | (uintptr_t)g.B | (uintptr_t)g.C) & 15) != 0 || g.lda % 4 != 0 || g.ldb % 4 != 0 || g.ldc % 4 != 0 ||
         g.stride_a % 4 != 0 || g.stride_b % 4 != 0 || g.stride_c % 4 != 0 || g.lda >= (1 << 20) || g.ldb >= (1 << 20))
         return -1;
+    // Batches take the same walk in bf16 terms, under the route's name (512 heads of 512 x 512, us: K = 32 109 -> 94, 64 167 -> 131; 256
+    // of them, K = 96 114 -> 94, 128 147 -> 115; 128 of 1024 x 1024, K = 128 276 -> 213)
+    if (batch > 1 && tuning().nt_walk == 0) return nt_terms(staged_args(g), batch, "sgemm_nt_cols256_dma");
     switch (g.K / 32) {
         case 1: return launch_nt_cols<1>(g, batch);
         case 2: return launch_nt_cols<2>(g, batch);
@@ -1781,6 +1784,14 @@ int dispatch_f32(const SgemmArgs &g, int transa, int transb, int64_t batch) {
     if (rc >= 0) return rc;
     if (!transa && transb) rc = try_nt_cols(g, batch);
     if (rc < 0 && !transa && transb) rc = try_nt_rows(g, batch);
+    // Batches of A B^T with a short K that neither walk takes: workgroups of 256 columns in bf16 terms, from half a workgroup per CU on
+    // (us, edge or guarded tiles -> this: 512 x 200 x 200, K = 64 55 -> 29, 256 x 333 x 333 69 -> 43, 40 x 1000 x 1000 78 -> 60, 150 x 700 x
+    // 700, K = 32 100 -> 70, 512 x 130 x 130 36 -> 20; level at 64 x 512 x 512, K = 64) while few of the columns hang over the end (130 x 260 x
+    // 260, K = 128 41 -> 56, 150 x 300 x 300, K = 32 21.7 -> 23.9, 512 x 128 x 128, K = 64 15.9 -> 15.6)
+    const int64_t nt_wide = (g.N + 255) / 256;
+    if (rc < 0 && !transa && transb && batch > 1 && free_choice && tuning().nt_walk == 0 && g.M >= 128 && nt_wide * batch >= cu_count() / 2 &&
+        ((g.K > 32 && g.N > 128 && g.N <= 256) || nt_wide * 256 * 5 <= g.N * 8))
+        rc = nt_terms(staged_args(g), batch, "sgemm_nt_cols256x3");
     if (!transa && !transb) rc = try_nn_stream(g, batch);
     if (rc >= 0) return rc;
     if (!transa && !transb) rc = try_dma<true, false>(nn_d, g, batch);
