@@ -1769,6 +1769,8 @@ int try_split_k(const SgemmArgs &g, int transa, int transb, const char *name) {
     return rc;
 }
 
+// The products of batches, and the parts of single ones.  Nothing here may use the shared workspace: its callers keep operands (the
+// score matrix of attention, also for a single head) and results (the partial sums of a K split) there.
 int dispatch_f32(const SgemmArgs &g, int transa, int transb, int64_t batch) {
     static const char *const nn_d[3] = {"sgemm_nn_128x128_dma", "sgemm_nn_64x64_dma", "sgemm_nn_64x64k2_dma"};
     static const char *const nt_d[3] = {"sgemm_nt_128x128_dma", "sgemm_nt_64x64_dma", "sgemm_nt_64x64k2_dma"};
@@ -1780,7 +1782,7 @@ int dispatch_f32(const SgemmArgs &g, int transa, int transb, int64_t batch) {
     const bool free_choice = tuning().f32_tile == 0 && tuning().f32_splitk == 0;
     if (batch > 1 && free_choice && g.K >= 256 && (g.N > 128 || (g.N >= 96 && (g.M % 128 != 0 || g.K % 32 != 0))) &&
         (double)batch * g.M * g.N * g.K >= 1.0e9)
-        rc = split_f32(staged_args(g), transa, transb, batch);
+        rc = split_f32(staged_args(g), transa, transb, batch, false);
     if (rc >= 0) return rc;
     if (!transa && transb) rc = try_nt_cols(g, batch);
     if (rc < 0 && !transa && transb) rc = try_nt_rows(g, batch);
@@ -1799,8 +1801,8 @@ int dispatch_f32(const SgemmArgs &g, int transa, int transb, int64_t batch) {
     else if (transa && !transb) rc = try_dma<false, false>(tn_d, g, batch);
     // off the 16-byte grid (100 x 333 x 333 x 64 42 -> 35, 100 x 333 x 64 x 333 28 -> 24; 400 x 103 x 32 x 103 17.3 -> 18.5: the
     // padded half of a tile costs twice)
-    if (rc < 0 && free_choice && g.K >= 64 && g.N >= 48) rc = split_f32(staged_args(g), transa, transb, batch);
-    if (rc < 0) rc = staged_f32(staged_args(g), transa, transb, batch);
+    if (rc < 0 && free_choice && g.K >= 64 && g.N >= 48) rc = split_f32(staged_args(g), transa, transb, batch, false);
+    if (rc < 0) rc = staged_f32(staged_args(g), transa, transb, batch, false);
     if (rc >= 0) return rc;
     if (!transa && !transb) return launch_guarded<true, false, float>("sgemm_nn_64x64_guarded", g, batch);
     if (!transa && transb) return launch_guarded<true, true, float>("sgemm_nt_64x64_guarded", g, batch);
@@ -1901,9 +1903,9 @@ int run_f32(const SgemmArgs &g, int transa, int transb) {
         const bool split = off ? g.K >= 64
                                : whole ? g.K >= 256 && products >= 1.5e9
                                        : g.K >= 96 && (products >= 1.0e9 || (g.K >= 256 && g.M > 160 && products >= 2.0e7));
-        if (free_choice && split) rc = split_f32(staged_args(g), transa, transb, 1);
+        if (free_choice && split) rc = split_f32(staged_args(g), transa, transb, 1, true);
         if (rc >= 0) return rc;
-        if (off) rc = staged_f32(staged_args(g), transa, transb, 1);
+        if (off) rc = staged_f32(staged_args(g), transa, transb, 1, true);
         if (rc >= 0) return rc;
         rc = try_split_k<float>(g, transa, transb, "sgemm_splitk");
         if (rc >= 0) return rc;

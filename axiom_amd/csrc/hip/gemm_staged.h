@@ -17,9 +17,11 @@ struct StagedArgs {
 
 // The register-staged tiles: any alignment, any K from 32 (fp32) or 64 (int8 weights) up; g.k_range is set to K by the caller
 // and cut into ranges here where that pays.  -1: not taken (smaller K, row pitches of 4 Mi elements and more).
-int staged_f32(const StagedArgs &g, int transa, int transb, int64_t batch);
+// may_split: K may be cut into ranges, whose sums meet in the shared workspace.  Only for a single product, and only for callers
+// that keep nothing there: attention's score matrix and the partial sums of an outer K split are operands and results there.
+int staged_f32(const StagedArgs &g, int transa, int transb, int64_t batch, bool may_split);
 // The same products in bf16 terms on the bf16 matrix core, at fp32 accuracy.
-int split_f32(const StagedArgs &g, int transa, int transb, int64_t batch);
+int split_f32(const StagedArgs &g, int transa, int transb, int64_t batch, bool may_split);
 int staged_i8w(const StagedArgs &g);
 // Batches of A * B^T with K = 32, 64, 96 or 128 in bf16 terms, B held in registers (gemm_nt_terms.hip).  -1: not taken.
 int nt_terms(const StagedArgs &g, int64_t batch, const char *name);

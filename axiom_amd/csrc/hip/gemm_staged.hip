@@ -550,8 +550,8 @@ const TileCost kSplitTiles[] = {{128, 128, 32, 1.36f, 4.0f}, {128, 64, 32, 0.82f
 const TileCost kI8Tiles[] = {{32, 128, 64, 0.57f, 2.5f}, {64, 128, 64, 0.90f, 2.5f}, {64, 256, 64, 1.52f, 2.5f}};
 
 template <bool A_KC, bool B_KC>
-int run_f32(const StagedArgs &g, int64_t batch, const char *const names[2], const char *split_name) {
-    const Plan p = plan_staged(g, batch, kF32Tiles, 2, batch == 1);
+int run_f32(const StagedArgs &g, int64_t batch, bool may_split, const char *const names[2], const char *split_name) {
+    const Plan p = plan_staged(g, batch, kF32Tiles, 2, may_split && batch == 1);
     if (p.tile < 0) return -1;
     return run_plan(g, p, kF32Tiles[p.tile].bk, split_name, [&](const StagedArgs &a) {
         return p.tile == 0 ? launch_staged<64, 64, 2, 2, 32, F32, A_KC, B_KC, 4>(names[0], a, batch, p.splits)
@@ -559,8 +559,8 @@ int run_f32(const StagedArgs &g, int64_t batch, const char *const names[2], cons
     });
 }
 template <bool A_KC, bool B_KC>
-int run_split(const StagedArgs &g, int64_t batch, const char *const names[4], const char *split_name) {
-    const Plan p = plan_staged(g, batch, kSplitTiles, 4, batch == 1);
+int run_split(const StagedArgs &g, int64_t batch, bool may_split, const char *const names[4], const char *split_name) {
+    const Plan p = plan_staged(g, batch, kSplitTiles, 4, may_split && batch == 1);
     if (p.tile < 0) return -1;
     return run_plan(g, p, kSplitTiles[p.tile].bk, split_name, [&](const StagedArgs &a) {
         switch (p.tile) {
@@ -574,24 +574,24 @@ int run_split(const StagedArgs &g, int64_t batch, const char *const names[4], co
 }  // namespace
 
 namespace axhip {
-int split_f32(const StagedArgs &g, int transa, int transb, int64_t batch) {
+int split_f32(const StagedArgs &g, int transa, int transb, int64_t batch, bool may_split) {
     static const char *const nn[4] = {"sgemm_nn_128x128x3_staged", "sgemm_nn_128x64x3_staged", "sgemm_nn_64x128x3_staged", "sgemm_nn_64x64x3_staged"};
     static const char *const nt[4] = {"sgemm_nt_128x128x3_staged", "sgemm_nt_128x64x3_staged", "sgemm_nt_64x128x3_staged", "sgemm_nt_64x64x3_staged"};
     static const char *const tn[4] = {"sgemm_tn_128x128x3_staged", "sgemm_tn_128x64x3_staged", "sgemm_tn_64x128x3_staged", "sgemm_tn_64x64x3_staged"};
     if ((transa && transb) || g.K < 32 || g.lda >= (1 << 22) || g.ldb >= (1 << 22) || batch > 65535) return -1;
-    if (!transa && !transb) return run_split<true, false>(g, batch, nn, "sgemm_splitk");
-    if (!transa) return run_split<true, true>(g, batch, nt, "sgemm_splitk");
-    return run_split<false, false>(g, batch, tn, "sgemm_splitk");
+    if (!transa && !transb) return run_split<true, false>(g, batch, may_split, nn, "sgemm_splitk");
+    if (!transa) return run_split<true, true>(g, batch, may_split, nt, "sgemm_splitk");
+    return run_split<false, false>(g, batch, may_split, tn, "sgemm_splitk");
 }
 
-int staged_f32(const StagedArgs &g, int transa, int transb, int64_t batch) {
+int staged_f32(const StagedArgs &g, int transa, int transb, int64_t batch, bool may_split) {
     static const char *const nn[2] = {"sgemm_nn_64x64k2_staged", "sgemm_nn_128x128k2_staged"};
     static const char *const nt[2] = {"sgemm_nt_64x64k2_staged", "sgemm_nt_128x128k2_staged"};
     static const char *const tn[2] = {"sgemm_tn_64x64k2_staged", "sgemm_tn_128x128k2_staged"};
     if ((transa && transb) || g.K < 32 || g.lda >= (1 << 22) || g.ldb >= (1 << 22) || batch > 65535) return -1;
-    if (!transa && !transb) return run_f32<true, false>(g, batch, nn, "sgemm_splitk");
-    if (!transa) return run_f32<true, true>(g, batch, nt, "sgemm_splitk");
-    return run_f32<false, false>(g, batch, tn, "sgemm_splitk");
+    if (!transa && !transb) return run_f32<true, false>(g, batch, may_split, nn, "sgemm_splitk");
+    if (!transa) return run_f32<true, true>(g, batch, may_split, nt, "sgemm_splitk");
+    return run_f32<false, false>(g, batch, may_split, tn, "sgemm_splitk");
 }
 
 int staged_i8w(const StagedArgs &g) {
