@@ -92,15 +92,17 @@ __device__ __forceinline__ v16f mfma_terms(const v4i &a, const v4i &b, const v16
 // probabilities times `up`.  The reference point m_run of the exponentials only moves when some query's
 // maximum exceeds it by more than 2^8: until then p = 2^(s - m_run) <= 256 is safe in fp32 and exact in
 // the quotient O = sum(p v) / sum(p), and the accumulator needs no rescaling pass (which costs as many
-// vector instructions as the exponentials themselves).
+// vector instructions as the exponentials themselves).  It starts at SD_LOWEST, the lowest finite value and not
+// -infinity: scores of -infinity then weigh nothing also where a row has met no other yet.
+constexpr float SD_LOWEST = -3.402823466e+38f;
 template <int DT>
 __device__ __forceinline__ void softmax_step(v16f &s, v16f (&acc_o)[DT], float &m_run, float &l_run, float up) {
     float m_blk = -INFINITY;
 #pragma unroll
     for (int v = 0; v < 16; v++) m_blk = fmaxf(m_blk, s[v]);
     m_blk = fmaxf(m_blk, __shfl_xor(m_blk, 32, 64));
-    if (__builtin_amdgcn_ballot_w64(m_blk > m_run + 8.0f)) {      // wave-uniform; always taken for the first keys
-        const float m_new = fmaxf(m_run, m_blk);  // finite: key 0 is visible to every query
+    if (__builtin_amdgcn_ballot_w64(m_blk > m_run + 8.0f)) {      // wave-uniform; always taken for the first finite scores
+        const float m_new = fmaxf(m_run, m_blk);
         const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
         l_run *= alpha;
         m_run = m_new;
@@ -129,7 +131,7 @@ __device__ __forceinline__ void attend_f32(const float *Qh, const float *Kh, con
     const int frow = lane & 31, fhalf = lane >> 5;
     const int64_t qg = wq_lo + frow;
     const float *q = Qh + (qg < S ? qg : S - 1) * ld;
-    m_run = -INFINITY;
+    m_run = SD_LOWEST;
     l_run = 0.0f;
 #pragma unroll
     for (int d = 0; d < DT; d++)
@@ -304,7 +306,7 @@ k_sdpa(const float *__restrict__ Q, const float *__restrict__ K, const float *__
         for (int d = 0; d < DT; d++)
 #pragma unroll
             for (int v = 0; v < 16; v++) acc_o[d][v] = 0.0f;
-        float m_run = -INFINITY, l_run = 0.0f;       // l_run: this lane half's share of the row sum
+        float m_run = SD_LOWEST, l_run = 0.0f;       // l_run: this lane half's share of the row sum
 
         auto attend = [&](int64_t blk, unsigned at) {
             const int64_t kb0 = blk * BKV;
@@ -429,7 +431,8 @@ k_sdpa(const float *__restrict__ Q, const float *__restrict__ K, const float *__
                     for (int e = 0; e < 4; e++) o[e] = acc_o[d][4 * g + e] * inv;
                     if (!PAD || d * 32 + 8 * g + 4 * fhalf < dkr) *reinterpret_cast<v4f *>(orow + d * 32 + 8 * g + 4 * fhalf) = o;
                 }
-            if (L && fhalf == 0) L[head * S + qg] = (m_run + __builtin_amdgcn_logf(l_tot / up)) * 0.6931471805599453f;
+            // (a row that saw nothing but -infinity: 0 / 0 above, and NaN here)
+            if (L && fhalf == 0) L[head * S + qg] = l_tot == 0.0f ? NAN : (m_run + __builtin_amdgcn_logf(l_tot / up)) * 0.6931471805599453f;
         }
     }
 }

@@ -99,3 +99,23 @@ def test_non_finite(hip, dk, causal):
         assert o[3, 0, 0] == top
     assert (np.abs(o - want).max(-1)[fine] <= (2 * SDPA_TOL * size * np.ones((6, S)))[fine]).all()
     assert (np.abs(l - lse)[fine] <= 1e-5 * np.maximum(1.0, np.abs(lse[fine]))).all()
+
+
+@pytest.mark.parametrize("dk", [32, 64, 80, 128])
+@pytest.mark.parametrize("causal", [0, 1])
+@pytest.mark.parametrize("S,hidden", [(200, 32), (200, 33), (200, 64), (200, 130), (520, 500)])
+def test_first_keys_hidden(hip, dk, causal, S, hidden):
+    """The first keys of every row score minus infinity: their weight is zero, and the rows that see others come out as without them;
+    rows that see no others are NaN, as the quotient of two zeros is."""
+    say("sdpa first keys hidden", dk, causal, S, hidden)
+    rng = np.random.default_rng(dk + hidden)
+    for BH in (3, 260):
+        q, k, v = (rng.uniform(-0.5, 0.5, (BH, S, dk)).astype(np.float32) for _ in range(3))
+        q[:, :, 1] = 0.5
+        k[:, :hidden, 1] = -np.inf
+        o, l = run_sdpa(hip, q, k, v, 0.3, causal)
+        some = [0, BH - 1]
+        want, lse = attention(q[some], k[some], v[some], np.float32(0.3), causal)
+        assert np.array_equal(np.isnan(o[some]), np.isnan(want)) and np.array_equal(np.isnan(l[some]), np.isnan(lse))
+        assert np.isnan(lse).any() == bool(causal)
+        assert np.nanmax(np.abs(o[some] - want)) <= SDPA_TOL and np.nanmax(np.abs(l[some] - lse)) <= 1e-5 * max(1.0, np.nanmax(np.abs(lse)))
