@@ -8,15 +8,13 @@
 // us, fp32 instructions -> this: 512 heads of 512 x 512, K = 64 167 -> 131 (4.6 TB/s; with plain stores 153), K = 128 with 256 of
 // them 147 -> 115, 128 of 1024 x 1024, K = 64 163 -> 124, K = 128 276 -> 213; off the 256 grid 256 of 333 x 333, K = 64 69 -> 43, 64 of
 // 1000 x 1000 116 -> 84, 512 of 200 x 200 55 -> 29.  Non-temporal stores where rows are no whole lines: 84 -> 111 (1000 x 1000).
-// A walk with a sum that is not finite, or that met a magnitude below 2^-102, is done again with fp32 instructions.
+// A walk with a sum that is not finite is done again with fp32 instructions.
 #include "gemm_staged.h"
 
 #include "bf16x3.h"
 
 namespace {
 using namespace axhip;
-
-typedef int v2i __attribute__((ext_vector_type(2)));
 
 template <int K>
 struct NtGeom {
@@ -30,23 +28,6 @@ struct NtGeom {
     }
 };
 
-constexpr unsigned TINY = 25u << 24;                     // twice the bit pattern of 2^-102
-template <int E, typename T>
-__device__ __forceinline__ void cut(const float (&x)[E], T (&t)[3], unsigned &least) {
-#pragma unroll
-    for (int e = 0; e < E; e += 2) {
-        // the smallest magnitude met, as twice its bit pattern less one (zero, which is no concern, comes out largest)
-        least = min(least, min(__float_as_uint(x[e]) * 2 - 1, __float_as_uint(x[e + 1]) * 2 - 1));
-        int hi, mid, lo;
-        bf16x3_nearest(x[e], x[e + 1], hi, mid, lo);
-        t[0][e / 2] = hi;
-        t[1][e / 2] = mid;
-        t[2][e / 2] = lo;
-    }
-}
-__device__ __forceinline__ v16f mfma_terms(const v4i &a, const v4i &b, const v16f &c) {
-    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf, a), __builtin_bit_cast(v8bf, b), c, 0, 0, 0);
-}
 template <int E>
 __device__ __forceinline__ void load_row(float (&x)[E], const float *p) {
 #pragma unroll
@@ -90,14 +71,13 @@ __global__ void __launch_bounds__(512, (K > 64 ? 2 : 4)) k_nt_terms(StagedArgs g
 #pragma unroll
         for (int i = 0; i < G::PIECES; i++) load_row(ar[i], reinterpret_cast<const float *>(a + ((unsigned)(prow[i] < end ? prow[i] : end) * (unsigned)g.lda + pcol[i]) * 4));
     };
-    unsigned least = 0xffffffffu;
     auto stage = [&](unsigned at) {
 #pragma unroll
         for (int i = 0; i < G::PIECES; i++) {
-            std::conditional_t<G::E == 8, v4i, v2i> t[3];
-            cut(ar[i], t, least);
+            Term<G::E> t[3];
+            cut(ar[i], TERMS_UP, t);
 #pragma unroll
-            for (int p = 0; p < 3; p++) *reinterpret_cast<decltype(&t[0])>(lds + at + put[i] + p * G::PLANE) = t[p];
+            for (int p = 0; p < 3; p++) *reinterpret_cast<Term<G::E> *>(lds + at + put[i] + p * G::PLANE) = t[p];
         }
     };
     // register v of lane l: row 8*(v>>2) + 4*(l>>5) + (v&3), column l & 31
@@ -124,12 +104,12 @@ __global__ void __launch_bounds__(512, (K > 64 ? 2 : 4)) k_nt_terms(StagedArgs g
     for (int ks = 0; ks < KS; ks++) {
         float x[8];
         load_row(x, brow + 16 * ks + 8 * fhalf);
-        cut(x, bf[ks], least);
+        cut(x, TERMS_UP, bf[ks]);
     }
     stage(0);
     if (nblocks > 1) load(1);
     __syncthreads();
-    float finite = 0.0f;
+    float seen = 0.0f;
     unsigned cur = 0;
     for (int64_t blk = 0; blk < nblocks; blk++, cur ^= G::STAGE) {
         if (blk + 1 < nblocks) {
@@ -155,21 +135,13 @@ __global__ void __launch_bounds__(512, (K > 64 ? 2 : 4)) k_nt_terms(StagedArgs g
                 acc = mfma_terms(af[0], bf[ks][0], acc);
             }
             acc += low;
-#pragma unroll
-            for (int v = 0; v < 16; v++) finite = __builtin_fmaf(acc[v], 0.0f, finite);
-            store(acc, row0);
+            look_at(acc, seen);
+            store(acc * TERMS_DOWN, row0);
         }
         __syncthreads();
     }
 
-    int *unfit = reinterpret_cast<int *>(lds + G::FLAGS_AT);
-    const bool bad = __builtin_amdgcn_ballot_w64(!(finite == 0.0f) || least < TINY) != 0;
-    if (lane == 0) unfit[wave] = bad;
-    __syncthreads();
-    int any = 0;
-#pragma unroll
-    for (int w = 0; w < 8; w++) any |= unfit[w];
-    if (!__builtin_amdgcn_readfirstlane(any) || idle) return;
+    if (!any_wave<8>(!(seen == 0.0f), lds + G::FLAGS_AT, wave) || idle) return;
     for (int64_t row0 = 0; row0 < g.M; row0 += 32) {
         const float *arow = A + (row0 + frow < g.M ? row0 + frow : g.M - 1) * g.lda;
         v16f acc;

@@ -8,8 +8,8 @@
 // 466 -> 339 (203 TFLOP/s), 8192^3 7204 -> 5612, 8 x 1024^3 155 -> 98.  Bound on 128x128: matrix core busy
 // 62 % of the cycles at the 1.85 GHz that the chip then holds, LDS 31 %; 64x64: the reads of fragments from LDS.  The conversions
 // (some 8 instructions a value) are put between the products of the same wave (interleave), worth 4 to 10 %.
-// A tile whose sums are not all finite, or which met a magnitude below 2^-102, is computed again with fp32 instructions by the
-// same workgroup: infinities, NaNs, values near the largest float and very small ones come out as they did.
+// A tile whose sums are not all finite is computed again with fp32 instructions by the same workgroup: infinities, NaNs and values
+// near the largest float come out as fp32 products give them.
 //
 // Why not direct to LDS: those loads move whole 16-byte pieces to their final place, so rows that start off the 16-byte grid,
 // a K that ends inside a slab and a conversion all need the register.  A slab is fetched two slabs ahead into registers,
@@ -33,8 +33,6 @@
 namespace {
 using namespace axhip;
 
-typedef int v2i __attribute__((ext_vector_type(2)));
-
 
 // How a product is formed: fp32 on the fp32 matrix core; fp32 activations in three bf16 terms against int8 weights in one;
 // both operands in three bf16 terms.
@@ -52,7 +50,7 @@ struct Geom {
     static constexpr int STAGE = A_BYTES + B_BYTES;
     static constexpr int CPITCH = BN + 4;                           // floats per row of the tile in LDS
     static constexpr int BUFFERS = 2 * STAGE > BM * CPITCH * 4 ? 2 * STAGE : BM * CPITCH * 4;
-    static constexpr int SMEM = BUFFERS + (OP == SPLIT ? 32 : 0);   // ... and a word per wave: does its part need the fp32 pass
+    static constexpr int SMEM = BUFFERS + (OP == SPLIT ? 32 : 0);   // ... and a word per wave: are its sums finite
     static_assert(SMEM <= 160 * 1024, "LDS budget");
     // Where the 16-byte chunk c of row r lies in its row: rows are spread so that the 16 lanes that a 16-byte access
     // serves together (16 rows of one chunk, or the chunks of neighbouring rows) fall on distinct banks.
@@ -138,21 +136,12 @@ sum_range(const StagedArgs &g, unsigned char *lds, int wave, int64_t m0, int64_t
             }
         }
     };
-    // SPLIT: the smallest magnitude met, as twice its bit pattern less one (zero, which is no concern, comes out largest)
-    unsigned least = 0xffffffffu;
-    auto put_terms = [&](unsigned char *d, int plane, const auto &x, auto count) {
-        constexpr int E = decltype(count)::value;
+    auto put_terms = [&](unsigned char *d, int plane, const auto &x) {
+        constexpr int E = sizeof(x) / sizeof(float);
+        Term<E> t[3];
+        cut(x, TERMS_UP, t);
 #pragma unroll
-        for (int e = 0; e < E; e += 2) {
-            const unsigned u = __float_as_uint(x[e]) * 2 - 1, v = __float_as_uint(x[e + 1]) * 2 - 1;
-            least = min(least, min(u, v));
-        }
-        int hi[E / 2], mid[E / 2], lo[E / 2];
-#pragma unroll
-        for (int e = 0; e < E / 2; e++) bf16x3_nearest(x[2 * e], x[2 * e + 1], hi[e], mid[e], lo[e]);
-        __builtin_memcpy(__builtin_assume_aligned(d, 2 * E), hi, 2 * E);
-        __builtin_memcpy(__builtin_assume_aligned(d + plane, 2 * E), mid, 2 * E);
-        __builtin_memcpy(__builtin_assume_aligned(d + 2 * plane, 2 * E), lo, 2 * E);
+        for (int p = 0; p < 3; p++) *reinterpret_cast<Term<E> *>(d + p * plane) = t[p];
     };
     auto stage = [&](const Regs &r, unsigned at) {   // ... into LDS buffer `at`
 #pragma unroll
@@ -160,7 +149,7 @@ sum_range(const StagedArgs &g, unsigned char *lds, int wave, int64_t m0, int64_t
             const float *x = r.a[i];
             unsigned char *d = lds + at + wa[i];
             if constexpr (OP == SPLIT) {
-                put_terms(d, G::A_PLANE, r.a[i], std::integral_constant<int, EA>());
+                put_terms(d, G::A_PLANE, r.a[i]);
             } else if constexpr (I8 && EA == 8) {
                 const Bf16x3 o = bf16x3_of(v4f{x[0], x[1], x[2], x[3]}, v4f{x[4], x[5], x[6], x[7]});
                 *reinterpret_cast<v4i *>(d) = o.hi;
@@ -184,7 +173,7 @@ sum_range(const StagedArgs &g, unsigned char *lds, int wave, int64_t m0, int64_t
                 for (int h = 0; h < EB / 8; h++)
                     *reinterpret_cast<v4i *>(lds + at + G::A_BYTES + (wb[i] ^ (h * 16))) = bf16_of_i8(r.q[i][2 * h], r.q[i][2 * h + 1]);
             } else if constexpr (OP == SPLIT) {
-                put_terms(lds + at + G::A_BYTES + wb[i], G::B_PLANE, r.b[i], std::integral_constant<int, EB>());
+                put_terms(lds + at + G::A_BYTES + wb[i], G::B_PLANE, r.b[i]);
             } else {
                 const float *x = r.b[i];
 #pragma unroll
@@ -235,8 +224,7 @@ sum_range(const StagedArgs &g, unsigned char *lds, int wave, int64_t m0, int64_t
                     for (int i = 0; i < TM; i++)
 #pragma unroll
                         for (int j = 0; j < TN; j++)
-                            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf, fb[j]), __builtin_bit_cast(v8bf, fa[i][p]),
-                                                                                acc[i][j], 0, 0, 0);
+                            acc[i][j] = mfma_terms(fb[j], fa[i][p], acc[i][j]);
             } else if constexpr (OP == SPLIT) {
                 v4i fa[TM][3], fb[TN][3];
 #pragma unroll
@@ -255,8 +243,7 @@ sum_range(const StagedArgs &g, unsigned char *lds, int wave, int64_t m0, int64_t
 #pragma unroll
                             for (int j = 0; j < TN; j++) {
                                 v16f &to = APART && sum > 0 ? low[APART ? i : 0][APART ? j : 0] : acc[i][j];
-                                to = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf, fb[j][sum - p]),
-                                                                             __builtin_bit_cast(v8bf, fa[i][p]), to, 0, 0, 0);
+                                to = mfma_terms(fb[j][sum - p], fa[i][p], to);
                             }
             } else {
                 v4f fa[TM][2], fb[TN][2];
@@ -363,22 +350,17 @@ sum_range(const StagedArgs &g, unsigned char *lds, int wave, int64_t m0, int64_t
 #pragma unroll
             for (int j = 0; j < TN; j++) acc[i][j] += low[i][j];
     }
-    // Terms of values below 2^-102 may fall under the smallest normal bf16 and lose bits, and infinities, NaNs and values that
-    // round past the largest bf16 leave a NaN or an infinity in every sum they enter (as, perhaps, in the fp32 product).
-    constexpr unsigned TINY = 25u << 24;              // twice the bit pattern of 2^-102
-    float finite = 0.0f;
+    float seen = 0.0f;
 #pragma unroll
     for (int i = 0; i < TM; i++)
 #pragma unroll
-        for (int j = 0; j < TN; j++)
+        for (int j = 0; j < TN; j++) look_at(acc[i][j], seen);
+    if (any_wave<8>(!(seen == 0.0f), lds + G::BUFFERS, wave)) return true;
 #pragma unroll
-            for (int v = 0; v < 16; v++) finite = __builtin_fmaf(acc[i][j][v], 0.0f, finite);
-    int *unfit = reinterpret_cast<int *>(lds + G::BUFFERS);
-    const bool bad = __builtin_amdgcn_ballot_w64(!(finite == 0.0f) || least < TINY) != 0;
-    if (lane == 0) unfit[wave] = bad;
-    __syncthreads();
-    const v4i f0 = *reinterpret_cast<const v4i *>(unfit), f1 = *reinterpret_cast<const v4i *>(unfit + 4);
-    return __builtin_amdgcn_readfirstlane(f0[0] | f0[1] | f0[2] | f0[3] | f1[0] | f1[1] | f1[2] | f1[3]) != 0;
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++) acc[i][j] *= TERMS_DOWN;
+    return false;
 }
 
 template <int BM, int BN, int WM, int WN, int BK, Op OP, bool A_KC, bool B_KC, int WAVES>

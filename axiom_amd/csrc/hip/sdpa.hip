@@ -21,9 +21,8 @@
 //              keys does not care about their order.
 // V is transposed by the registers (a thread loads eight keys of one column).  Rows of both operands
 // are XOR-swizzled in 16-byte chunks, so the 16 lanes that a 16-byte access serves fall on distinct banks.
-// A tile with a sum that is not finite, or that met a magnitude below 2^-102, is computed again with fp32
-// instructions by the same workgroup: infinities, NaNs, values near the largest float and very small ones
-// come out as fp32 products give them.
+// A tile with a sum that is not finite is computed again with fp32 instructions by the same workgroup:
+// infinities, NaNs and values near the largest float come out as fp32 products give them.
 // us, fp32 instructions -> terms: 512 heads of [512, 64] 269 -> 194 (causal 178 -> 126), 64 of [1024, 128] 273 -> 174, 96 causal
 // ones of [1000, 80] 324 -> 129 (a quarter of that from the 96-wide geometry), 512 of [256, 32] 41 -> 33, 32 of [128, 64] 11.9 ->
 // 10.9.  O is nearer to 64 bits on every shape measured (relative error 4.9e-7 -> 3.7e-7 at [512, 64]).  Bound: the matrix core is
@@ -38,8 +37,6 @@
 namespace {
 using namespace axhip;
 
-typedef int v2i __attribute__((ext_vector_type(2)));
-
 template <int DK, int WAVES>
 struct SdGeom {
     static_assert(DK == 32 || DK == 64 || DK == 96 || DK == 128, "head dimension");
@@ -51,7 +48,7 @@ struct SdGeom {
     static constexpr bool DOUBLE = WAVES == 8;          // two blocks in LDS, or two workgroups per CU
     static constexpr int PER_SIMD = DK == 128 && WAVES == 4 ? 1 : 2;     // waves: with two, 64 registers would spill
     static constexpr int FLAGS_AT = (DOUBLE ? 2 : 1) * STAGE;
-    static constexpr int SMEM = FLAGS_AT + 4 * WAVES;   // a word per wave: does its part need the fp32 pass
+    static constexpr int SMEM = FLAGS_AT + 4 * WAVES;   // a word per wave: are its sums finite
     static constexpr int E = BKV * DK % (512 * WAVES) == 0 ? 8 : 4;      // values of a piece that a thread stages
     static constexpr int PIECES = BKV * DK / E / (64 * WAVES);          // pieces of K, and of V
     static_assert(PIECES * E * 64 * WAVES == BKV * DK, "a block divides over the threads");
@@ -66,29 +63,7 @@ struct SdGeom {
     __device__ static unsigned v_at(int col, int chunk) { return V_AT + at<VROW>(col, chunk); }
 };
 
-// Probabilities are kept times 2^24, so that their three terms are normal bf16 values as far down as the
-// probabilities themselves are normal floats.
-constexpr float SD_UP = 16777216.0f;
-
-// The smallest magnitude met, as twice its bit pattern less one (zero, which is no concern, comes out largest).
-constexpr unsigned SD_TINY = 25u << 24;                  // twice the bit pattern of 2^-102
-template <int E, typename T>
-__device__ __forceinline__ void cut(const float (&x)[E], T (&t)[3], unsigned *least) {
-#pragma unroll
-    for (int e = 0; e < E; e += 2) {
-        if (least) *least = min(*least, min(__float_as_uint(x[e]) * 2 - 1, __float_as_uint(x[e + 1]) * 2 - 1));
-        int hi, mid, lo;
-        bf16x3_nearest(x[e], x[e + 1], hi, mid, lo);
-        t[0][e / 2] = hi;
-        t[1][e / 2] = mid;
-        t[2][e / 2] = lo;
-    }
-}
-__device__ __forceinline__ v16f mfma_terms(const v4i &a, const v4i &b, const v16f &c) {
-    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf, a), __builtin_bit_cast(v8bf, b), c, 0, 0, 0);
-}
-
-// The online softmax of a 32-key tile of scores (log2 units, masked ones -infinity): scores become
+// The online softmax of a 32-key tile of scores (log2 units once taken times `down`, masked ones -infinity): scores become
 // probabilities times `up`.  The reference point m_run of the exponentials only moves when some query's
 // maximum exceeds it by more than 2^8: until then p = 2^(s - m_run) <= 256 is safe in fp32 and exact in
 // the quotient O = sum(p v) / sum(p), and the accumulator needs no rescaling pass (which costs as many
@@ -96,11 +71,11 @@ __device__ __forceinline__ v16f mfma_terms(const v4i &a, const v4i &b, const v16
 // -infinity: scores of -infinity then weigh nothing also where a row has met no other yet.
 constexpr float SD_LOWEST = -3.402823466e+38f;
 template <int DT>
-__device__ __forceinline__ void softmax_step(v16f &s, v16f (&acc_o)[DT], float &m_run, float &l_run, float up) {
+__device__ __forceinline__ void softmax_step(v16f &s, v16f (&acc_o)[DT], float &m_run, float &l_run, float up, float down) {
     float m_blk = -INFINITY;
 #pragma unroll
     for (int v = 0; v < 16; v++) m_blk = fmaxf(m_blk, s[v]);
-    m_blk = fmaxf(m_blk, __shfl_xor(m_blk, 32, 64));
+    m_blk = fmaxf(m_blk, __shfl_xor(m_blk, 32, 64)) * down;
     if (__builtin_amdgcn_ballot_w64(m_blk > m_run + 8.0f)) {      // wave-uniform; always taken for the first finite scores
         const float m_new = fmaxf(m_run, m_blk);
         const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
@@ -114,7 +89,7 @@ __device__ __forceinline__ void softmax_step(v16f &s, v16f (&acc_o)[DT], float &
     float l_blk = 0.0f;
 #pragma unroll
     for (int v = 0; v < 16; v++) {
-        const float p = __builtin_amdgcn_exp2f(s[v] - m_run) * up;
+        const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(s[v], down, -m_run)) * up;
         s[v] = p;
         l_blk += p;
     }
@@ -156,7 +131,7 @@ __device__ __forceinline__ void attend_f32(const float *Qh, const float *Kh, con
 #pragma unroll
         for (int v = 0; v < 16; v++)
             if (8 * (v >> 2) + 4 * fhalf + (v & 3) > seen) s[v] = -INFINITY;
-        softmax_step<DT>(s, acc_o, m_run, l_run, 1.0f);
+        softmax_step<DT>(s, acc_o, m_run, l_run, 1.0f, 1.0f);
 #pragma unroll
         for (int v = 0; v < 16; v++) {
             const int64_t key = k0 + 8 * (v >> 2) + 4 * fhalf + (v & 3);
@@ -266,12 +241,11 @@ k_sdpa(const float *__restrict__ Q, const float *__restrict__ K, const float *__
                 }
             }
         };
-        unsigned least;
         auto put = [&](const float (&x)[E], unsigned at, unsigned plane) {
-            std::conditional_t<E == 8, v4i, v2i> terms[3];
-            cut(x, terms, &least);
+            Term<E> terms[3];
+            cut(x, TERMS_UP, terms);
 #pragma unroll
-            for (int p = 0; p < 3; p++) *reinterpret_cast<decltype(&terms[0])>(lds + at + p * plane) = terms[p];
+            for (int p = 0; p < 3; p++) *reinterpret_cast<Term<E> *>(lds + at + p * plane) = terms[p];
         };
         auto stage = [&](unsigned at) {              // the block in registers, to LDS
 #pragma unroll
@@ -283,7 +257,6 @@ k_sdpa(const float *__restrict__ Q, const float *__restrict__ K, const float *__
         const int64_t all_blocks = (S + BKV - 1) / BKV;
         const int64_t nblocks = CAUSAL && (q0 + BQ) / BKV < all_blocks ? (q0 + BQ) / BKV : all_blocks;
         const int64_t wq_lo = q0 + wave * 32, qg = wq_lo + frow;      // this wave's first query, this lane's query
-        least = 0xffffffffu;
         load(0);
         v4i qf[KS][3];                               // step ks: dk 16*ks + 8*fhalf .. +7 of this lane's query
         {
@@ -294,7 +267,7 @@ k_sdpa(const float *__restrict__ Q, const float *__restrict__ K, const float *__
                 load_row(x, q, (16 * ks + 8 * fhalf) * 4, 16 * ks + 8 * fhalf);
 #pragma unroll
                 for (int e = 0; e < 8; e++) x[e] *= scale_log2e;
-                cut(x, qf[ks], &least);
+                cut(x, TERMS_UP, qf[ks]);
             }
         }
         stage(0);
@@ -345,7 +318,7 @@ k_sdpa(const float *__restrict__ Q, const float *__restrict__ K, const float *__
                     for (int v = 0; v < 16; v++)
                         if (8 * (v >> 2) + 4 * fhalf + (v & 3) > qrel) s[v] = -INFINITY;
                 }
-                softmax_step<DT>(s, acc_o, m_run, l_run, SD_UP);
+                softmax_step<DT>(s, acc_o, m_run, l_run, TERMS_UP, TERMS_DOWN);
 
                 // ---- O^T += V^T P^T ----
 #pragma unroll
@@ -354,7 +327,7 @@ k_sdpa(const float *__restrict__ Q, const float *__restrict__ K, const float *__
 #pragma unroll
                     for (int e = 0; e < 8; e++) x[e] = s[8 * st + e];
                     v4i pf[3];
-                    cut(x, pf, nullptr);
+                    cut(x, 1.0f, pf);                     // (a probability is zero or from 2^-126 up, and was taken times 2^24)
 #pragma unroll
                     for (int d = 0; d < DT; d++) {
                         v4i vf[3];
@@ -397,29 +370,22 @@ k_sdpa(const float *__restrict__ Q, const float *__restrict__ K, const float *__
             }
         }
 
-        // ---- did every sum come out finite, and were all magnitudes such that the terms hold them? ----
-        float finite = l_run * 0.0f, up = SD_UP;
+        // ---- did every sum come out finite?  Scores past 2^80 below zero are infinite too: they weigh nothing, as they should,
+        // unless a row has no others ----
+        float seen = l_run * 0.0f, up = TERMS_UP, down = 1.0f / TERMS_UP;
 #pragma unroll
-        for (int d = 0; d < DT; d++)
-#pragma unroll
-            for (int v = 0; v < 16; v++) finite = __builtin_fmaf(acc_o[d][v], 0.0f, finite);
-        int *unfit = reinterpret_cast<int *>(lds + G::FLAGS_AT);
-        const bool bad = __builtin_amdgcn_ballot_w64(!(finite == 0.0f) || least < SD_TINY) != 0;
-        if (lane == 0) unfit[wave] = bad;
-        __syncthreads();
-        int any = 0;
-#pragma unroll
-        for (int w = 0; w < WAVES; w++) any |= unfit[w];
-        if (__builtin_amdgcn_readfirstlane(any)) {
+        for (int d = 0; d < DT; d++) look_at(acc_o[d], seen);
+        float l_tot = l_run + __shfl_xor(l_run, 32, 64);
+        if (any_wave<WAVES>(!(seen == 0.0f) || (l_tot == 0.0f && wq_lo < S), lds + G::FLAGS_AT, wave)) {
             int again = lane;                        // opaque, so that no address of this pass is held through the loop above
             asm volatile("" : "+v"(again));
             attend_f32<DK, CAUSAL>(Qh, Kh, Vh, ld, S, width, scale_log2e, wq_lo, again, acc_o, m_run, l_run);
-            up = 1.0f;
+            l_tot = l_run + __shfl_xor(l_run, 32, 64);
+            up = down = 1.0f;
         }
 
         // ---- normalise and write: lane owns query qg, dk columns 32*d + 8*g + 4*fhalf .. +3 ----
-        const float l_tot = l_run + __shfl_xor(l_run, 32, 64);
-        const float inv = 1.0f / l_tot;
+        const float inv = 1.0f / l_tot * down;       // the sums hold the factors of V and of the probabilities, l_tot the latter's
         float *orow = O + (hb * S + qg) * ldo + hh * width;
         if (qg < S) {
 #pragma unroll

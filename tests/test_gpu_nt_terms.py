@@ -65,3 +65,43 @@ def test_non_finite(hip, K):
     got[1, 7], a[1, 7] = 0, 0
     got[2, :, 149], b[2, 149] = 0, 0
     check(got, a, b, 1.0)
+
+
+@pytest.mark.parametrize("K", [32, 64, 96, 128])
+@pytest.mark.parametrize("scale_a,scale_b", [(2.0 ** -60, 2.0 ** -60), (2.0 ** -20, 2.0 ** -110), (2.0 ** -127, 2.0 ** 10), (2.0 ** 50, 2.0 ** 40)])
+def test_small_results(hip, K, scale_a, scale_b):
+    """Products next to the smallest normal value (and above 2^80): relative accuracy as in the middle of the range, up to fp32's own
+    smallest step."""
+    say("nt terms small results", K, scale_a, scale_b)
+    rng = np.random.default_rng(K)
+    a, b = (rng.uniform(-1, 1, (260, 140, K)) * scale_a).astype(np.float32), (rng.uniform(-1, 1, (260, 170, K)) * scale_b).astype(np.float32)
+    check(product(hip, a, b, 1.0), a, b, 1.0, 4 * 2.0 ** -149)
+
+
+@pytest.mark.parametrize("K", [32, 64, 96, 128])
+def test_small_values_among_others(hip, K):
+    """Values down to fp32's smallest beside ordinary ones are no reason for the fp32 pass: every sum comes out as with zeros in their
+    place, but for the few whose rounding is a tie."""
+    say("nt terms small values", K)
+    rng = np.random.default_rng(K)
+    a, b = rng.uniform(-1, 1, (260, 140, K)).astype(np.float32), rng.uniform(-1, 1, (260, 170, K)).astype(np.float32)
+    for x in (a, b):
+        x[rng.random(x.shape) < 0.02] = 0
+    clean = product(hip, a, b, 1.0)
+    for x in (a, b):
+        x[x == 0] = np.ldexp(1.0, rng.integers(-149, -100, (x == 0).sum())).astype(np.float32)
+    assert (product(hip, a, b, 1.0) != clean).mean() < 0.01
+
+
+@pytest.mark.parametrize("K", [32, 64, 96, 128])
+def test_single_products(hip, K):
+    """Sums with one product that is not zero, of operands with all 24 bits: the left-out terms are at most 2^-24 of it, the sum of the
+    large term and of the others is rounded once to 2^-24, the others' own five roundings are 2^-8 of that.  Any of the six products of
+    terms left out would show as 2^-18 or more in some of them."""
+    say("nt terms single products", K)
+    rng = np.random.default_rng(K)
+    a, b = np.zeros((260, 140, K), np.float32), rng.uniform(1, 2, (260, 170, K)).astype(np.float32)
+    np.put_along_axis(a, rng.integers(0, K, (260, 140, 1)), rng.uniform(1, 2, (260, 140, 1)).astype(np.float32), 2)
+    got, want = product(hip, a, b, 1.0), a.astype(np.float64) @ b.astype(np.float64).transpose(0, 2, 1)
+    err = np.abs(got - want) / want * 2.0 ** 24
+    assert (err <= 2 + 5 / 128).all(), float(err.max())

@@ -119,3 +119,38 @@ def test_first_keys_hidden(hip, dk, causal, S, hidden):
         assert np.array_equal(np.isnan(o[some]), np.isnan(want)) and np.array_equal(np.isnan(l[some]), np.isnan(lse))
         assert np.isnan(lse).any() == bool(causal)
         assert np.nanmax(np.abs(o[some] - want)) <= SDPA_TOL and np.nanmax(np.abs(l[some] - lse)) <= 1e-5 * max(1.0, np.nanmax(np.abs(lse)))
+
+
+@pytest.mark.parametrize("dk", [32, 64, 80, 128])
+def test_small_values_among_others(hip, dk):
+    """Values down to fp32's smallest beside ordinary ones are no reason for the fp32 pass: every result comes out as with zeros in their
+    place, but for the few whose rounding is a tie."""
+    say("sdpa small values", dk)
+    rng = np.random.default_rng(dk)
+    x = [rng.uniform(-0.5, 0.5, (9, 300, dk)).astype(np.float32) for _ in range(3)]
+    for y in x:
+        y[rng.random(y.shape) < 0.02] = 0
+    clean = run_sdpa(hip, *x, 0.3, 0)
+    for y in x:
+        y[y == 0] = np.ldexp(1.0, rng.integers(-149, -100, (y == 0).sum())).astype(np.float32)
+    for got, want in zip(run_sdpa(hip, *x, 0.3, 0), clean):
+        assert (got != want).mean() < 0.01
+
+
+@pytest.mark.parametrize("dk", [32, 64, 80, 128])
+@pytest.mark.parametrize("exponent", [0, -126, 90])
+def test_single_products(hip, dk, exponent):
+    """One key: O is V but for the left-out terms (2^-24), one rounding to 2^-24 of the sum of the terms, one of the quotient and the
+    division of 1 (2^-24 each), and the others' own roundings (2^-8 of that, seven at most).  L is one product of Q and K times the scale:
+    the roundings of q * scale * log2(e) (two), of the sum of terms, the left-out terms and the two on the way back."""
+    say("sdpa single products", dk, exponent)
+    rng = np.random.default_rng(dk)
+    q, k = np.zeros((500, 1, dk), np.float32), np.zeros((500, 1, dk), np.float32)
+    at = rng.integers(0, dk, (500, 1, 1))
+    np.put_along_axis(q, at, rng.uniform(1, 2, (500, 1, 1)).astype(np.float32), 2)
+    np.put_along_axis(k, at, rng.uniform(1, 2, (500, 1, 1)).astype(np.float32), 2)
+    v = np.ldexp(rng.uniform(1, 2, (500, 1, dk)), exponent).astype(np.float32)
+    o, l = run_sdpa(hip, q, k, v, 0.7, 0)
+    assert (np.abs(o - v.astype(np.float64)) <= 2.0 ** -24 * (4 + 7 / 128) * v).all()
+    want = np.float32(0.7) * (q.astype(np.float64) * k).sum(-1)
+    assert (np.abs(l - want) <= 2.0 ** -24 * 8 * want).all(), float((np.abs(l - want) / want).max() * 2 ** 24)

@@ -93,3 +93,52 @@ def test_split_non_finite(hip, M, N, K):
     rows = np.setdiff1d(np.arange(M), [1, 2, 4])
     size = np.abs(a[rows]).astype(np.float64) @ np.abs(b).astype(np.float64)
     assert (np.abs(got[rows] - ref[rows]) <= BOUND_FP32 * size).all()
+
+
+@pytest.mark.parametrize("M,N,K", SHAPES)
+@pytest.mark.parametrize("scale_a,scale_b", [(2.0 ** -60, 2.0 ** -60), (2.0 ** -55, 2.0 ** -68), (2.0 ** -20, 2.0 ** -110), (2.0 ** -127, 2.0 ** 10), (2.0 ** 50, 2.0 ** 40)])
+def test_split_small_results(hip, M, N, K, scale_a, scale_b):
+    """Ordinary or small operands whose products lie next to the smallest normal value (and above 2^80): relative accuracy as in the
+    middle of the range, up to fp32's own smallest step (one for the sum, one for each of the sums of ranges and wave sets)."""
+    say("split small results", M, N, K, scale_a, scale_b)
+    rng = np.random.default_rng(K)
+    a = (rng.uniform(-1, 1, (M, K)) * scale_a).astype(np.float32)
+    b = (rng.uniform(-1, 1, (K, N)) * scale_b).astype(np.float32)
+    got = product(hip, a, b, "nn")
+    want = a.astype(np.float64) @ b.astype(np.float64)
+    size = np.abs(a).astype(np.float64) @ np.abs(b).astype(np.float64)
+    assert (np.abs(got - want) <= BOUND_FP32 * size + 32 * 2.0 ** -149).all(), float(((np.abs(got - want) - 32 * 2.0 ** -149) / size).max())
+
+
+@pytest.mark.parametrize("M,N,K", SHAPES)
+def test_split_small_values_among_others(hip, M, N, K):
+    """Values down to fp32's smallest beside ordinary ones, as GELU and softmax leave them, are no reason for the fp32 pass: every sum
+    comes out as with zeros in their place, but for the few whose rounding is a tie.  (The fp32 instructions add in another order: they
+    would change about half of the sums.)"""
+    say("split small values", M, N, K)
+    rng = np.random.default_rng(K)
+    a, b = rng.uniform(-1, 1, (M, K)).astype(np.float32), rng.uniform(-1, 1, (K, N)).astype(np.float32)
+    for x in (a, b):
+        x[rng.random(x.shape) < 0.02] = 0
+    clean = product(hip, a, b, "nn")
+    for x in (a, b):
+        x[x == 0] = np.ldexp(1.0, rng.integers(-149, -100, (x == 0).sum())).astype(np.float32)
+    got = product(hip, a, b, "nn")
+    assert (got != clean).mean() < 0.01
+
+
+@pytest.mark.parametrize("M,N,K", SHAPES + [(65, 516, 256), (516, 65, 256)])
+@pytest.mark.parametrize("order", ["nn", "nt", "tn"])
+def test_split_single_products(hip, M, N, K, order):
+    """Sums with one product that is not zero, of operands with all 24 bits: the left-out terms are at most 2^-24 of it; the large term is
+    added to the others by a vector instruction (2^-24) or, on 128x128 tiles, by the matrix core, whose additions are taken as truncating
+    (2^-23); the others' own seven are 2^-8 of that.  Any of the six products of terms left out would show as 2^-18 or more."""
+    say("split single products", M, N, K, order)
+    rng = np.random.default_rng(K)
+    a, b = np.zeros((M, K), np.float32), np.zeros((K, N), np.float32)
+    a[np.arange(M), rng.integers(0, K, M)] = rng.uniform(1, 2, M) * rng.choice([-1, 1], M)
+    b[rng.integers(0, K, N), np.arange(N)] = rng.uniform(1, 2, N)
+    for x, y in ((a, rng.uniform(1, 2, (K, N)).astype(np.float32)), (rng.uniform(1, 2, (M, K)).astype(np.float32), b)):
+        got, want = product(hip, x, y, order), x.astype(np.float64) @ y.astype(np.float64)
+        err = np.abs(got - want) / np.abs(want) * 2.0 ** 24
+        assert (err <= 3 + 7 / 64).all(), float(err.max())
