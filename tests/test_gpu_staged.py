@@ -90,3 +90,21 @@ def test_staged_w8a32_non_finite(hip, oracle):
         ref = oracle.qgemm_w8a32(a, w, s)
     assert np.array_equal(np.isnan(got), np.isnan(ref)) and np.array_equal(np.isinf(got), np.isinf(ref))
     assert np.array_equal(np.sign(got[np.isinf(ref)]), np.sign(ref[np.isinf(ref)]))
+
+
+@pytest.mark.parametrize("order,Bn,M,N,K,kernel", [
+    ("nt", 176, 132, 131, 34, "sgemm_nt_64x64k2_staged"), ("nn", 30, 1168, 35, 32, "sgemm_nn_64x64k2_staged"), ("nt", 13, 543, 543, 32, "sgemm_nt_64x64k2_staged"),
+    ("nt", 338, 294, 294, 65, "sgemm_nt_64x64x3_staged"), ("nt", 56, 447, 449, 69, "sgemm_nt_64x64x3_staged"), ("nn", 70, 800, 22, 96, "sgemm_nn_64x64k2_staged"),
+    ("nn", 27, 1084, 85, 162, "sgemm_nn_128x128x3_staged")])
+def test_tile_of_a_short_k(hip, order, Bn, M, N, K, kernel):
+    """With a K of one to eight slabs first loads and write-back decide: 64x64 tiles, unless the large ones fill the CUs just once."""
+    say("tile of a short k", order, Bn, M, N, K)
+    rng = np.random.default_rng(Bn + M + N + K)
+    a = rng.uniform(-1, 1, (Bn, M, K)).astype(np.float32)
+    b = rng.uniform(-1, 1, (Bn, N, K) if order == "nt" else (Bn, K, N)).astype(np.float32)
+    got = hip.sgemm_batched(hip.array(a), hip.array(b), transb=order == "nt", alpha=0.25).numpy()
+    assert hip.last_kernel() == kernel
+    for h in (0, Bn // 2, Bn - 1):
+        bt = b[h].astype(np.float64).T if order == "nt" else b[h].astype(np.float64)
+        want, size = 0.25 * (a[h].astype(np.float64) @ bt), 0.25 * (np.abs(a[h]).astype(np.float64) @ np.abs(bt))
+        assert (np.abs(got[h] - want) <= BOUND_FP32 * size).all()
