@@ -1889,20 +1889,25 @@ int run_f32(const SgemmArgs &g, int transa, int transb) {
         // Off the 16-byte grid the staged tiles, which split K by themselves (us, before on guarded tiles -> staged:
         // 372 x 2149 x 2149 127 -> 48, 222 x 434 x 1376 74 -> 13, 651 x 1862 x 2833 TN 225 -> 100, 2001 x 2003 x 2005 214 -> 135,
         // 128 x 784 x 1023 NT 39 -> 11.5, 41 x 1113 x 92 8.7 -> 7).  On it they are ahead where K is off the 32 grid, so that the
-        // kernels below cannot cut it into ranges, and few tiles want that (128 x 1024 x 784 17.4 -> 12.0).
+        // kernels below cannot cut it into ranges, and few tiles want that (128 x 1024 x 784 17.4 -> 12.0, 249 x 512 x 376 NT 10.4 -> 8.9);
+        // for columns of A from K = 384 on (416 x 608 x 328 10.2 -> 10.6, 160 x 32 x 412 10.7 -> 9.4), and where their half tiles of 32
+        // rows put twice the workgroups to work from 512 on (17 x 576 x 340 7.0 -> 9.5, 160 x 20 x 472 8.2 -> 8.8, 32 x 1024 x 528 9.3 -> 9.0).
         const bool on_grid = transa ? dma_takes<false>(g, 1) : dma_takes<true>(g, 1);
-        const bool wants_ranges = g.K % 32 != 0 && g.K >= 256 && ((g.M + 63) / 64) * ((g.N + 63) / 64) * 2 <= cu_count();
+        const int64_t ranges_from = transa ? 384 : half_row_tiles(g.M) ? 512 : 256;
+        const bool wants_ranges = g.K % 32 != 0 && g.K >= ranges_from && ((g.M + 63) / 64) * ((g.N + 63) / 64) * 2 <= cu_count();
         const bool off = !on_grid || wants_ranges, whole = g.M % 64 == 0 && g.N % 64 == 0 && g.K % 32 == 0;
         // Products in bf16 terms: wherever the staged tiles are the route and K has two slabs (0.75 to 1.0 of the fp32 ones over some
         // hundred shapes; 1050 x 1984 x 32 8.8 -> 9.7); on the grid where the fp32 tiles hang over an edge (160 x 800 x 2656 38 -> 18,
         // 1230 x 768 x 3072 55 -> 44, 298 x 4096 x 1024 37 -> 31; up to 160 rows their half tiles and K ranges are level or ahead) and
         // for large whole ones (640 x 2048 x 512 17.6 -> 18.7, 1024^3 19.6 -> 20.6, 640 x 4096 x 1024 49 -> 45, 2304 x 3072 x 768 95 -> 71).  A short K is
-        // loads and write-back (2048 x 4096 x 64 16 -> 20, 128 24 -> 25; off the tile grid 4000 x 4000 x 128 53 -> 45).
+        // loads and write-back (2048 x 4096 x 64 16 -> 20, 128 24 -> 25; off the tile grid 4000 x 4000 x 128 53 -> 45).  Columns that fill
+        // less than a tile are left to the fp32 tiles where K divides into ranges of 64 (685 x 960 x 32 8.2 -> 9.5, but 501 x 992 x 64 20 -> 8.9).
         const bool free_choice = tuning().f32_tile == 0 && tuning().f32_splitk == 0;
         const double products = (double)g.M * g.N * g.K;
         const bool split = off ? g.K >= 64
                                : whole ? g.K >= 256 && products >= 1.5e9
-                                       : g.K >= 96 && (products >= 1.0e9 || (g.K >= 256 && g.M > 160 && products >= 2.0e7));
+                                       : g.K >= 96 && (products >= 1.0e9 || (g.K >= 256 && g.M > 160 && products >= 2.0e7 &&
+                                                                                (g.N >= 48 || split_count(g.M, g.N, g.K, !transa) * 64 < g.K)));
         if (free_choice && split) rc = split_f32(staged_args(g), transa, transb, 1, true);
         if (rc >= 0) return rc;
         if (off) rc = staged_f32(staged_args(g), transa, transb, 1, true);

@@ -108,3 +108,20 @@ def test_tile_of_a_short_k(hip, order, Bn, M, N, K, kernel):
         bt = b[h].astype(np.float64).T if order == "nt" else b[h].astype(np.float64)
         want, size = 0.25 * (a[h].astype(np.float64) @ bt), 0.25 * (np.abs(a[h]).astype(np.float64) @ np.abs(bt))
         assert (np.abs(got[h] - want) <= BOUND_FP32 * size).all()
+
+
+@pytest.mark.parametrize("order,M,N,K,kernel", [
+    ("nn", 17, 576, 340, "sgemm_32x64k2_dma_edge"), ("nt", 160, 20, 472, "sgemm_32x64k2_dma_edge"), ("nt", 96, 3296, 392, "sgemm_32x64k2_dma_edge"),
+    ("tn", 128, 672, 328, "sgemm_64x64k2_dma_edge"), ("nn", 249, 512, 376, "sgemm_nn_64x64x3_staged"), ("tn", 160, 32, 440, "sgemm_splitk"),
+    ("nn", 32, 1024, 540, "sgemm_splitk"), ("nn", 685, 32, 960, "sgemm_splitk")])
+def test_ranges_on_the_grid(hip, order, M, N, K, kernel):
+    """Rows on the 16-byte grid with K off the 32 grid: ranges of K on the staged tiles only where K is long enough for what the
+    direct-to-LDS tiles do in one launch."""
+    say("ranges on the grid", order, M, N, K)
+    rng = np.random.default_rng(M + N + K)
+    a, b = rng.uniform(-1, 1, (M, K)).astype(np.float32), rng.uniform(-1, 1, (K, N)).astype(np.float32)
+    da, db = hip.array(np.ascontiguousarray(a.T) if order[0] == "t" else a), hip.array(np.ascontiguousarray(b.T) if order[1] == "t" else b)
+    got = hip.sgemm(da, db, transa=order[0] == "t", transb=order[1] == "t").numpy()
+    assert hip.last_kernel() == kernel
+    want, size = a.astype(np.float64) @ b.astype(np.float64), np.abs(a).astype(np.float64) @ np.abs(b).astype(np.float64)
+    assert (np.abs(got - want) <= BOUND_FP32 * size).all()
