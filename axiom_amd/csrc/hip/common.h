@@ -219,6 +219,11 @@ __device__ __forceinline__ void turn_tile_and_store_edge(unsigned char *turn, in
             *reinterpret_cast<V4 *>(dst + (int64_t)(p * 8 + (lane >> 3)) * ld + (lane & 7) * 4) = o[p];
 }
 
+// axhip_sgemm_strided_batched for kernels that build on it.  workspace_is_free: the caller keeps nothing in workspace(), where a batch
+// of one may leave the partial sums of ranges of K (gemm_f32.hip).
+int sgemm_batched(int transa, int transb, int64_t M, int64_t N, int64_t K, float alpha, const float *A, int64_t lda, int64_t stride_a, const float *B,
+                  int64_t ldb, int64_t stride_b, float beta, float *C, int64_t ldc, int64_t stride_c, int64_t batch, bool workspace_is_free);
+
 }  // namespace axhip
 
 #define AXHIP_HIP_TRY(expr, what)                                                         \

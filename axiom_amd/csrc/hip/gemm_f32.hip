@@ -1684,7 +1684,7 @@ int splitk_finish(const float *part, int64_t splits, int64_t M, int64_t N, float
 }  // namespace axhip
 
 namespace {
-int dispatch_f32(const SgemmArgs &g, int transa, int transb, int64_t batch);
+int dispatch_f32(const SgemmArgs &g, int transa, int transb, int64_t batch, bool may_split = false);
 
 // how many K ranges to use (1: none).  Every range must be a whole number of 32-wide slabs.
 int64_t split_count(int64_t M, int64_t N, int64_t K, bool a_rows_k_contiguous) {
@@ -1769,9 +1769,9 @@ int try_split_k(const SgemmArgs &g, int transa, int transb, const char *name) {
     return rc;
 }
 
-// The products of batches, and the parts of single ones.  Nothing here may use the shared workspace: its callers keep operands (the
-// score matrix of attention, also for a single head) and results (the partial sums of a K split) there.
-int dispatch_f32(const SgemmArgs &g, int transa, int transb, int64_t batch) {
+// The products of batches, and the parts of single ones.  Without may_split nothing here may use the shared workspace: the caller keeps
+// operands (the score matrix of attention, also for a single head) or results (the partial sums of a K split) there.
+int dispatch_f32(const SgemmArgs &g, int transa, int transb, int64_t batch, bool may_split) {
     static const char *const nn_d[3] = {"sgemm_nn_128x128_dma", "sgemm_nn_64x64_dma", "sgemm_nn_64x64k2_dma"};
     static const char *const nt_d[3] = {"sgemm_nt_128x128_dma", "sgemm_nt_64x64_dma", "sgemm_nt_64x64k2_dma"};
     static const char *const tn_d[3] = {"sgemm_tn_128x128_dma", "sgemm_tn_64x64_dma", "sgemm_tn_64x64k2_dma"};
@@ -1801,8 +1801,8 @@ int dispatch_f32(const SgemmArgs &g, int transa, int transb, int64_t batch) {
     else if (transa && !transb) rc = try_dma<false, false>(tn_d, g, batch);
     // off the 16-byte grid (100 x 333 x 333 x 64 42 -> 35, 100 x 333 x 64 x 333 28 -> 24; 400 x 103 x 32 x 103 17.3 -> 18.5: the
     // padded half of a tile costs twice)
-    if (rc < 0 && free_choice && g.K >= 64 && g.N >= 48) rc = split_f32(staged_args(g), transa, transb, batch, false);
-    if (rc < 0) rc = staged_f32(staged_args(g), transa, transb, batch, false);
+    if (rc < 0 && free_choice && g.K >= 64 && g.N >= 48) rc = split_f32(staged_args(g), transa, transb, batch, may_split);
+    if (rc < 0) rc = staged_f32(staged_args(g), transa, transb, batch, may_split);
     if (rc >= 0) return rc;
     if (!transa && !transb) return launch_guarded<true, false, float>("sgemm_nn_64x64_guarded", g, batch);
     if (!transa && transb) return launch_guarded<true, true, float>("sgemm_nt_64x64_guarded", g, batch);
@@ -1964,15 +1964,10 @@ extern "C" int axhip_sgemm(int transa, int transb, int64_t M, int64_t N, int64_t
     return run_f32(g, transa, transb);
 }
 
-extern "C" int axhip_sgemm_strided_batched(int transa, int transb, int64_t M, int64_t N, int64_t K,
-                                           float alpha, const float *A, int64_t lda,
-                                           int64_t stride_a, const float *B, int64_t ldb,
-                                           int64_t stride_b, float beta, float *C, int64_t ldc,
-                                           int64_t stride_c, int64_t batch) {
-    if (int rc = axhip::ensure_ready()) return rc;
-    if (int rc = validate("sgemm_strided_batched", transa, transb, M, N, K, A, lda, B, ldb, C, ldc,
-                          AXHIP_ACT_NONE))
-        return rc;
+namespace axhip {
+int sgemm_batched(int transa, int transb, int64_t M, int64_t N, int64_t K, float alpha, const float *A, int64_t lda, int64_t stride_a, const float *B,
+                  int64_t ldb, int64_t stride_b, float beta, float *C, int64_t ldc, int64_t stride_c, int64_t batch, bool workspace_is_free) {
+    if (int rc = validate("sgemm_strided_batched", transa, transb, M, N, K, A, lda, B, ldb, C, ldc, AXHIP_ACT_NONE)) return rc;
     if (batch < 0 || stride_a < 0 || stride_b < 0 || stride_c < 0)
         return fail(AXHIP_ERR_SHAPE, "sgemm_strided_batched: negative batch or stride");
     if (M == 0 || N == 0 || batch == 0) return AXHIP_OK;
@@ -1982,7 +1977,17 @@ extern "C" int axhip_sgemm_strided_batched(int transa, int transb, int64_t M, in
         const int64_t nb = batch - b0 < kMostPerLaunch ? batch - b0 : kMostPerLaunch;
         SgemmArgs g{A + b0 * stride_a, B + b0 * stride_b, C + b0 * stride_c, M, N, K, lda, ldb, ldc, stride_a, stride_b,
                     stride_c, alpha, beta, nullptr, nullptr, AXHIP_ACT_NONE};
-        if (int rc = dispatch_f32(g, transa, transb, nb)) return rc;
+        if (int rc = dispatch_f32(g, transa, transb, nb, nb == 1 && workspace_is_free)) return rc;
     }
     return AXHIP_OK;
+}
+}  // namespace axhip
+
+extern "C" int axhip_sgemm_strided_batched(int transa, int transb, int64_t M, int64_t N, int64_t K,
+                                           float alpha, const float *A, int64_t lda,
+                                           int64_t stride_a, const float *B, int64_t ldb,
+                                           int64_t stride_b, float beta, float *C, int64_t ldc,
+                                           int64_t stride_c, int64_t batch) {
+    if (int rc = axhip::ensure_ready()) return rc;
+    return axhip::sgemm_batched(transa, transb, M, N, K, alpha, A, lda, stride_a, B, ldb, stride_b, beta, C, ldc, stride_c, batch, true);
 }

@@ -492,15 +492,13 @@ int sdpa_unfused(const float *Q, const float *K, const float *V, float *O, float
     for (int64_t h0 = 0; h0 < BH; h0 += chunk) {
         const int64_t nb = BH - h0 < chunk ? BH - h0 : chunk;
         const float *q = Q + h0 * S * dk, *k = K + h0 * S * dk, *v = V + h0 * S * dk;
-        int rc = axhip_sgemm_strided_batched(0, 1, S, S, dk, scale, q, dk, S * dk, k, dk, S * dk, 0.0f, score, S,
-                                             S * S, nb);
+        int rc = sgemm_batched(0, 1, S, S, dk, scale, q, dk, S * dk, k, dk, S * dk, 0.0f, score, S, S * S, nb, false);
         if (rc) return rc;
         if (nb * S > 0x7fffffff) return fail(AXHIP_ERR_SHAPE, "sdpa: too many score rows per chunk");
         hipLaunchKernelGGL(k_softmax_lse_rows, dim3((unsigned)(nb * S)), dim3(256), 0, kStream, score,
                            L ? L + h0 * S : nullptr, S, causal);
         if ((rc = check_launch("sdpa softmax"))) return rc;
-        rc = axhip_sgemm_strided_batched(0, 0, S, dk, S, 1.0f, score, S, S * S, v, dk, S * dk, 0.0f,
-                                         O + h0 * S * dk, dk, S * dk, nb);
+        rc = sgemm_batched(0, 0, S, dk, S, 1.0f, score, S, S * S, v, dk, S * dk, 0.0f, O + h0 * S * dk, dk, S * dk, nb, false);
         if (rc) return rc;
     }
     note_kernel("sdpa_unfused");

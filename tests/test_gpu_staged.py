@@ -125,3 +125,15 @@ def test_ranges_on_the_grid(hip, order, M, N, K, kernel):
     assert hip.last_kernel() == kernel
     want, size = a.astype(np.float64) @ b.astype(np.float64), np.abs(a).astype(np.float64) @ np.abs(b).astype(np.float64)
     assert (np.abs(got - want) <= BOUND_FP32 * size).all()
+
+
+@pytest.mark.parametrize("M,N,K,transb", [(928, 43, 928, 0), (423, 41, 1023, 1), (361, 33, 777, 0)])
+def test_batch_of_one_is_cut_like_a_product(hip, M, N, K, transb):
+    say("batch of one", M, N, K, transb)
+    rng = np.random.default_rng(M + N + K)
+    a, b = rng.uniform(-1, 1, (1, M, K)).astype(np.float32), rng.uniform(-1, 1, (1, N, K) if transb else (1, K, N)).astype(np.float32)
+    got = hip.sgemm_batched(hip.array(a), hip.array(b), transb=bool(transb), alpha=0.25).numpy()[0]
+    assert hip.last_kernel() == "sgemm_splitk"
+    bt = b[0].astype(np.float64).T if transb else b[0].astype(np.float64)
+    want, size = 0.25 * (a[0].astype(np.float64) @ bt), 0.25 * (np.abs(a[0]).astype(np.float64) @ np.abs(bt))
+    assert (np.abs(got - want) <= BOUND_FP32 * size).all()
