@@ -23,9 +23,10 @@
 // are latency: one 64x64 tile with K = 92 takes 7 us, of which 2.3 are the launch.  W8A32, 250 x 4096 x 4096 in 35 us (240
 // TFLOP/s of products, three bf16 terms each): matrix core busy 36 % of the time, LDS 44 %, vector pipe about as much; without
 // the conversions 27 us, without products 24, without global loads 27, products alone 20 - three pipes that overlap in part.
-// Measured and dropped: reading the fragments of both k-steps ahead of the products (35.7 us, 29 spills), a cut of the
-// activations without the two instructions that keep infinities (36.4 against 37.6, for a second pass over tiles with
-// non-finite sums), 64-wide fp32 slabs (2001 x 2003 x 2005 144 us against 135 with 32-wide ones).
+// Activations are cut as in SPLIT, so that small ones keep their bits (they ran on fp32 instructions before these tiles); the second
+// pass over tiles with sums that are not finite reads its operands straight from memory (no room for fp32 slabs in the same LDS).
+// Measured and dropped: reading the fragments of both k-steps ahead of the products (35.7 us, 29 spills), 64-wide fp32 slabs
+// (2001 x 2003 x 2005 144 us against 135 with 32-wide ones).
 #include "gemm_staged.h"
 
 #include "bf16x3.h"
@@ -50,7 +51,11 @@ struct Geom {
     static constexpr int STAGE = A_BYTES + B_BYTES;
     static constexpr int CPITCH = BN + 4;                           // floats per row of the tile in LDS
     static constexpr int BUFFERS = 2 * STAGE > BM * CPITCH * 4 ? 2 * STAGE : BM * CPITCH * 4;
-    static constexpr int SMEM = BUFFERS + (OP == SPLIT ? 32 : 0);   // ... and a word per wave: are its sums finite
+    // In bf16 terms a word per wave besides: are its sums finite.  Where 32 bytes more would keep a second workgroup off the CU (I8W,
+    // 64x128) the words lie in the buffers, past the tile, and are written when all waves have read the last slab.
+    static constexpr bool WORDS_INSIDE = 160 * 1024 / (BUFFERS + 32) < 160 * 1024 / BUFFERS;
+    static constexpr int SMEM = BUFFERS + (OP == F32 || WORDS_INSIDE ? 0 : 32), WORDS_AT = WORDS_INSIDE ? BUFFERS - 32 : BUFFERS;
+    static_assert(OP == F32 || BM * CPITCH * 4 <= WORDS_AT, "the words outlive the start of the write-back");
     static_assert(SMEM <= 160 * 1024, "LDS budget");
     // Where the 16-byte chunk c of row r lies in its row: rows are spread so that the 16 lanes that a 16-byte access
     // serves together (16 rows of one chunk, or the chunks of neighbouring rows) fall on distinct banks.
@@ -60,7 +65,8 @@ struct Geom {
 };
 
 // The sum over this workgroup's range of K, into acc: per wave TM x TN blocks of 32x32, register v of lane l: row (l & 31),
-// column 8 * (v >> 2) + 4 * (l >> 5) + (v & 3).  Returns whether any wave found its part of a SPLIT product unfit.
+// column 8 * (v >> 2) + 4 * (l >> 5) + (v & 3).  Returns whether any wave found its part of a product
+// in bf16 terms unfit.
 template <int BM, int BN, int WM, int WN, int BK, Op OP, bool A_KC, bool B_KC>
 __device__ __forceinline__ bool
 sum_range(const StagedArgs &g, unsigned char *lds, int wave, int64_t m0, int64_t n0, int64_t batch,
@@ -147,19 +153,8 @@ sum_range(const StagedArgs &g, unsigned char *lds, int wave, int64_t m0, int64_t
 #pragma unroll
         for (int i = 0; i < NTA; i++) {
             const float *x = r.a[i];
-            unsigned char *d = lds + at + wa[i];
-            if constexpr (OP == SPLIT) {
-                put_terms(d, G::A_PLANE, r.a[i]);
-            } else if constexpr (I8 && EA == 8) {
-                const Bf16x3 o = bf16x3_of(v4f{x[0], x[1], x[2], x[3]}, v4f{x[4], x[5], x[6], x[7]});
-                *reinterpret_cast<v4i *>(d) = o.hi;
-                *reinterpret_cast<v4i *>(d + G::A_PLANE) = o.mid;
-                *reinterpret_cast<v4i *>(d + 2 * G::A_PLANE) = o.lo;
-            } else if constexpr (I8) {
-                const Bf16x3 o = bf16x3_of(v4f{x[0], x[1], x[2], x[3]}, v4f{0.f, 0.f, 0.f, 0.f});
-                *reinterpret_cast<v2i *>(d) = v2i{o.hi[0], o.hi[1]};
-                *reinterpret_cast<v2i *>(d + G::A_PLANE) = v2i{o.mid[0], o.mid[1]};
-                *reinterpret_cast<v2i *>(d + 2 * G::A_PLANE) = v2i{o.lo[0], o.lo[1]};
+            if constexpr (TERMS) {
+                put_terms(lds + at + wa[i], G::A_PLANE, r.a[i]);
             } else {
 #pragma unroll
                 for (int h = 0; h < EA / 4; h++)
@@ -340,10 +335,8 @@ sum_range(const StagedArgs &g, unsigned char *lds, int wave, int64_t m0, int64_t
         __syncthreads();
     }
     multiply(end);
-    if constexpr (OP != SPLIT) {
-        __syncthreads();
-        return false;
-    }
+    if constexpr (OP == F32 || G::WORDS_INSIDE) __syncthreads();
+    if constexpr (OP == F32) return false;
     if constexpr (APART) {
 #pragma unroll
         for (int i = 0; i < TM; i++)
@@ -355,12 +348,50 @@ sum_range(const StagedArgs &g, unsigned char *lds, int wave, int64_t m0, int64_t
     for (int i = 0; i < TM; i++)
 #pragma unroll
         for (int j = 0; j < TN; j++) look_at(acc[i][j], seen);
-    if (any_wave<8>(!(seen == 0.0f), lds + G::BUFFERS, wave)) return true;
+    if (any_wave<8>(!(seen == 0.0f), lds + G::WORDS_AT, wave)) return true;
 #pragma unroll
     for (int i = 0; i < TM; i++)
 #pragma unroll
-        for (int j = 0; j < TN; j++) acc[i][j] *= TERMS_DOWN;
+        for (int j = 0; j < TN; j++) acc[i][j] *= I8 ? 1.0f / TERMS_UP : TERMS_DOWN;      // (an int8 value is taken as it is)
     return false;
+}
+
+// The same sum for fp32 against int8 with fp32 instructions, operands straight from memory: the rare second pass.  The wave sets
+// take pairs of k in turn.
+template <int TM, int TN, int WN>
+__device__ __forceinline__ void sum_range_i8_f32(const StagedArgs &g, int wave, int lane, int64_t m0, int64_t n0, v16f (&acc)[TM][TN]) {
+    const int wk = wave >> 2, wm = (wave & 3) / WN, wn = (wave & 3) % WN, frow = lane & 31, fhalf = lane >> 5;
+    const int64_t kbeg = (int64_t)blockIdx.z * g.k_range, kend = kbeg + g.k_range < g.K ? kbeg + g.k_range : g.K;
+    const float *a[TM];
+    const int8_t *b[TN];
+#pragma unroll
+    for (int i = 0; i < TM; i++) {
+        const int64_t row = m0 + (wm * TM + i) * 32 + frow;
+        a[i] = static_cast<const float *>(g.A) + (row < g.M ? row : g.M - 1) * g.lda;
+    }
+#pragma unroll
+    for (int j = 0; j < TN; j++) {
+        const int64_t col = n0 + (wn * TN + j) * 32 + frow;
+        b[j] = static_cast<const int8_t *>(g.B) + (col < g.N ? col : g.N - 1) * g.ldb;
+    }
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++)
+#pragma unroll
+            for (int v = 0; v < 16; v++) acc[i][j][v] = 0.0f;
+    for (int64_t k0 = kbeg + 2 * wk; k0 < kend; k0 += 4) {           // uniform
+        const int64_t k = k0 + fhalf;
+        float fa[TM], fb[TN];
+#pragma unroll
+        for (int i = 0; i < TM; i++) fa[i] = k < kend ? a[i][k] : 0.0f;
+#pragma unroll
+        for (int j = 0; j < TN; j++) fb[j] = k < kend ? (float)b[j][k] : 0.0f;
+#pragma unroll
+        for (int i = 0; i < TM; i++)
+#pragma unroll
+            for (int j = 0; j < TN; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fb[j], fa[i], acc[i][j], 0, 0, 0);
+    }
 }
 
 template <int BM, int BN, int WM, int WN, int BK, Op OP, bool A_KC, bool B_KC, int WAVES>
@@ -383,6 +414,9 @@ __global__ void __launch_bounds__(512, WAVES) k_gemm_staged(StagedArgs g) {
     if constexpr (OP == SPLIT) {
         static_assert(2 * Geom<BM, BN, WM, WN, BK, F32>::STAGE <= G::BUFFERS, "the fp32 pass runs in the same LDS");
         if (unfit) sum_range<BM, BN, WM, WN, BK, F32, A_KC, B_KC>(g, lds, wave, m0, n0, batch, acc);
+    }
+    if constexpr (OP == I8W) {
+        if (unfit) sum_range_i8_f32<TM, TN, WN>(g, wave, lane, m0, n0, acc);
     }
 
     // ---- the two sets added in LDS, then whole rows written back ----

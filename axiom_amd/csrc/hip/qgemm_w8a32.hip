@@ -11,8 +11,8 @@
 // are added over the wave together in a fixed tree order and end one per lane for the write-back.
 // Rows at any byte alignment and any K: whole 16-byte steps are fetched with one load wherever the row
 // starts (global memory takes unaligned vector loads), the last partial step byte by byte.
-// M = 1, and up to four rows against fewer than 16384 weight rows, take a form without LDS (below).  Larger M goes through the fp32 matrix-core GEMM with the
-// int8 operand converted while it is staged.
+// M = 1, and up to four rows against fewer than 16384 weight rows, take a form without LDS (below).  Larger M goes to the matrix cores
+// (sgemm_i8w), the activations in bf16 terms.
 #include "common.h"
 
 namespace axhip {
