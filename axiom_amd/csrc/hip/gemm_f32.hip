@@ -12,6 +12,8 @@
 // multiplies the k = 4*(l>>5) + j elements of both operands, so A and B always pair up.
 // The pads make the 16 lanes a b128 read serves together, the two lane halves of a b32 read,
 // and the staging writes all fall on distinct banks (64 banks x 4 bytes).
+#include <cstring>
+
 #include "bf16x3.h"
 #include "common.h"
 #include "gemm_staged.h"
@@ -1195,9 +1197,9 @@ int try_nt_cols(const SgemmArgs &g, int64_t batch) {
     if ((((uintptr_t)g.A | (uintptr_t)g.B | (uintptr_t)g.C) & 15) != 0 || g.lda % 4 != 0 || g.ldb % 4 != 0 || g.ldc % 4 != 0 ||
         g.stride_a % 4 != 0 || g.stride_b % 4 != 0 || g.stride_c % 4 != 0 || g.lda >= (1 << 20) || g.ldb >= (1 << 20))
         return -1;
-    // Batches take the same walk in bf16 terms, under the route's name (512 heads of 512 x 512, us: K = 32 109 -> 94, 64 167 -> 131; 256
+    // Batches take the same walk in bf16 terms (512 heads of 512 x 512, us: K = 32 109 -> 94, 64 167 -> 131; 256
     // of them, K = 96 114 -> 94, 128 147 -> 115; 128 of 1024 x 1024, K = 128 276 -> 213)
-    if (batch > 1 && tuning().nt_walk == 0) return nt_terms(staged_args(g), batch, "sgemm_nt_cols256_dma");
+    if (batch > 1 && tuning().nt_walk == 0) return nt_terms(staged_args(g), batch);
     switch (g.K / 32) {
         case 1: return launch_nt_cols<1>(g, batch);
         case 2: return launch_nt_cols<2>(g, batch);
@@ -1764,8 +1766,9 @@ int try_split_k(const SgemmArgs &g, int transa, int transb, const char *name) {
     if (std::is_same<BSRC, float>::value) rc = dispatch_f32(p, transa, transb, splits);
     else rc = try_dma_i8(kI8DmaNames, p, splits);
     if (rc) return rc;
+    const bool terms = std::is_same<BSRC, float>::value && strstr(axhip_last_kernel(), "x3") != nullptr;
     rc = splitk_finish(part, splits, g.M, g.N, g.alpha, g.beta, g.bias, g.act, g.C, g.ldc);
-    note_kernel(name);
+    note_kernel(terms ? kSplitTermsName : name);
     return rc;
 }
 
@@ -1793,7 +1796,7 @@ int dispatch_f32(const SgemmArgs &g, int transa, int transb, int64_t batch, bool
     const int64_t nt_wide = (g.N + 255) / 256;
     if (rc < 0 && !transa && transb && batch > 1 && free_choice && tuning().nt_walk == 0 && g.M >= 128 && nt_wide * batch >= cu_count() / 2 &&
         ((g.K > 32 && g.N > 128 && g.N <= 256) || nt_wide * 256 * 5 <= g.N * 8))
-        rc = nt_terms(staged_args(g), batch, "sgemm_nt_cols256x3");
+        rc = nt_terms(staged_args(g), batch);
     if (!transa && !transb) rc = try_nn_stream(g, batch);
     if (rc >= 0) return rc;
     if (!transa && !transb) rc = try_dma<true, false>(nn_d, g, batch);

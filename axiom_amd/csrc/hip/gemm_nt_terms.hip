@@ -157,7 +157,7 @@ __global__ void __launch_bounds__(512, (K > 64 ? 2 : 4)) k_nt_terms(StagedArgs g
 }
 
 template <int K, bool LINES>
-int launch(const StagedArgs &g, int64_t batch, const char *name) {
+int launch(const StagedArgs &g, int64_t batch) {
     using G = NtGeom<K>;
     static bool attr_set = false;
     if (!attr_set) {
@@ -165,28 +165,28 @@ int launch(const StagedArgs &g, int64_t batch, const char *name) {
                       "hipFuncSetAttribute");
         attr_set = true;
     }
-    note_kernel(name);
+    note_kernel("sgemm_nt_cols256x3");
     hipLaunchKernelGGL((k_nt_terms<K, LINES>), dim3((unsigned)((g.N + 255) / 256), (unsigned)batch), dim3(512), G::SMEM, kStream, g);
-    return check_launch(name);
+    return check_launch("sgemm_nt_cols256x3");
 }
 template <int K>
-int launch(const StagedArgs &g, int64_t batch, const char *name) {
+int launch(const StagedArgs &g, int64_t batch) {
     const bool lines = ((uintptr_t)g.C & 127) == 0 && g.ldc % 32 == 0 && g.stride_c % 32 == 0;
-    return lines ? launch<K, true>(g, batch, name) : launch<K, false>(g, batch, name);
+    return lines ? launch<K, true>(g, batch) : launch<K, false>(g, batch);
 }
 }  // namespace
 
 namespace axhip {
-int nt_terms(const StagedArgs &g, int64_t batch, const char *name) {
+int nt_terms(const StagedArgs &g, int64_t batch) {
     if (g.K % 32 != 0 || g.K < 32 || g.K > 128 || g.M < 1 || g.N < 1 || g.beta != 0.0f || g.bias || g.col_scale || g.act != AXHIP_ACT_NONE) return -1;
     if ((((uintptr_t)g.A | (uintptr_t)g.B) & 15) != 0 || g.lda % 4 != 0 || g.ldb % 4 != 0 || g.stride_a % 4 != 0 || g.stride_b % 4 != 0 ||
         g.lda >= (1 << 22) || g.ldc >= (1 << 24) || g.N >= (1 << 24) || batch > 65535 || (g.N + 255) / 256 > 0x7fffffff)
         return -1;
     switch (g.K / 32) {
-        case 1: return launch<32>(g, batch, name);
-        case 2: return launch<64>(g, batch, name);
-        case 3: return launch<96>(g, batch, name);
-        default: return launch<128>(g, batch, name);
+        case 1: return launch<32>(g, batch);
+        case 2: return launch<64>(g, batch);
+        case 3: return launch<96>(g, batch);
+        default: return launch<128>(g, batch);
     }
 }
 }  // namespace axhip

@@ -23,8 +23,10 @@ int staged_f32(const StagedArgs &g, int transa, int transb, int64_t batch, bool 
 // The same products in bf16 terms on the bf16 matrix core, at fp32 accuracy.
 int split_f32(const StagedArgs &g, int transa, int transb, int64_t batch, bool may_split);
 int staged_i8w(const StagedArgs &g);
+// What a product cut into ranges of K reports when they were formed in bf16 terms (fp32 ranges: sgemm_splitk).
+constexpr const char *kSplitTermsName = "sgemm_splitk_x3";
 // Batches of A * B^T with K = 32, 64, 96 or 128 in bf16 terms, B held in registers (gemm_nt_terms.hip).  -1: not taken.
-int nt_terms(const StagedArgs &g, int64_t batch, const char *name);
+int nt_terms(const StagedArgs &g, int64_t batch);
 
 // Adds `splits` partial products [M, N] in order and applies alpha, beta, bias and activation (gemm_f32.hip).
 int splitk_finish(const float *part, int64_t splits, int64_t M, int64_t N, float alpha, float beta, const float *bias, int act,

@@ -598,9 +598,9 @@ int split_f32(const StagedArgs &g, int transa, int transb, int64_t batch, bool m
     static const char *const nt[4] = {"sgemm_nt_128x128x3_staged", "sgemm_nt_128x64x3_staged", "sgemm_nt_64x128x3_staged", "sgemm_nt_64x64x3_staged"};
     static const char *const tn[4] = {"sgemm_tn_128x128x3_staged", "sgemm_tn_128x64x3_staged", "sgemm_tn_64x128x3_staged", "sgemm_tn_64x64x3_staged"};
     if ((transa && transb) || g.K < 32 || g.lda >= (1 << 22) || g.ldb >= (1 << 22) || batch > 65535) return -1;
-    if (!transa && !transb) return run_split<true, false>(g, batch, may_split, nn, "sgemm_splitk");
-    if (!transa) return run_split<true, true>(g, batch, may_split, nt, "sgemm_splitk");
-    return run_split<false, false>(g, batch, may_split, tn, "sgemm_splitk");
+    if (!transa && !transb) return run_split<true, false>(g, batch, may_split, nn, kSplitTermsName);
+    if (!transa) return run_split<true, true>(g, batch, may_split, nt, kSplitTermsName);
+    return run_split<false, false>(g, batch, may_split, tn, kSplitTermsName);
 }
 
 int staged_f32(const StagedArgs &g, int transa, int transb, int64_t batch, bool may_split) {

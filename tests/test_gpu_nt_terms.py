@@ -17,7 +17,7 @@ def product(hip, a, b, alpha, pad=0):
     da, db, c = hip.array(fa), hip.array(fb), hip.array(np.full((Bn, M, N + pad), 7.0, np.float32))
     hip.check(hip.L.axhip_sgemm_strided_batched(0, 1, M, N, K, alpha, da.ptr, K + pad, M * (K + pad), db.ptr, K + pad, N * (K + pad), 0.0, c.ptr,
                                                 N + pad, M * (N + pad), Bn))
-    assert hip.last_kernel().startswith("sgemm_nt_cols256"), hip.last_kernel()
+    assert hip.last_kernel() == "sgemm_nt_cols256x3"
     got = c.numpy()
     assert (got[:, :, N:] == 7.0).all()
     return got[:, :, :N]

@@ -16,7 +16,7 @@ def product(hip, a, b, order):
     hip.check(hip.L.axhip_sgemm(int(order[0] == "t"), int(order[1] == "t"), M, N, K, 1.0, da.ptr, sa.shape[1], db.ptr, sb.shape[1], 0.0, c.ptr,
                                 N, None, 0))
     kernel = hip.last_kernel()
-    assert "x3_staged" in kernel or kernel == "sgemm_splitk", kernel
+    assert kernel.endswith("x3_staged") or kernel == "sgemm_splitk_x3", kernel
     return c.numpy()
 
 
@@ -29,9 +29,6 @@ def test_split_fp32(hip, M, N, K, order):
     say("split", M, N, K, order)
     rng = np.random.default_rng(M + N + K)
     a, b = rng.uniform(-1, 1, (M, K)).astype(np.float32), rng.uniform(-1, 1, (K, N)).astype(np.float32)
-    if (M % 4 or N % 4 or K % 4) == 0 and order == "tn" and M % 64:
-        M = M // 4 * 4
-        a = a[:M]
     got = product(hip, a, b, order)
     want = a.astype(np.float64) @ b.astype(np.float64)
     size = np.abs(a).astype(np.float64) @ np.abs(b).astype(np.float64)
@@ -50,6 +47,18 @@ def test_split_batched(hip, Bn, M, N, K, transb):
     want = 0.25 * (a.astype(np.float64) @ bt)
     size = 0.25 * (np.abs(a).astype(np.float64) @ np.abs(bt))
     assert (np.abs(got - want) <= BOUND_FP32 * size).all()
+
+
+@pytest.mark.parametrize("M,N,K,tile", [(70, 90, 101, "64x64"), (501, 2053, 129, "128x64"), (513, 3583, 129, "64x128"), (1537, 1541, 129, "128x128")])
+def test_every_tile(hip, M, N, K, tile):
+    """The shapes of this file reach every tile: one row or column past whole tiles, a slab and one value more."""
+    say("split tile", M, N, K)
+    rng = np.random.default_rng(M + N + K)
+    a, b = rng.uniform(-1, 1, (M, K)).astype(np.float32), rng.uniform(-1, 1, (K, N)).astype(np.float32)
+    got = product(hip, a, b, "nn")
+    assert hip.last_kernel() == f"sgemm_nn_{tile}x3_staged"
+    size = np.abs(a).astype(np.float64) @ np.abs(b).astype(np.float64)
+    assert (np.abs(got - a.astype(np.float64) @ b.astype(np.float64)) <= BOUND_FP32 * size).all()
 
 
 SHAPES = [(70, 90, 101), (200, 132, 1029), (1152, 1152, 1152)]      # one tile, ranges of K, whole tiles
@@ -127,7 +136,7 @@ def test_split_small_values_among_others(hip, M, N, K):
     assert (got != clean).mean() < 0.01
 
 
-@pytest.mark.parametrize("M,N,K", SHAPES + [(65, 516, 256), (516, 65, 256)])
+@pytest.mark.parametrize("M,N,K", SHAPES + [(65, 517, 257), (501, 2053, 129), (513, 3583, 129)])
 @pytest.mark.parametrize("order", ["nn", "nt", "tn"])
 def test_split_single_products(hip, M, N, K, order):
     """Sums with one product that is not zero, of operands with all 24 bits: the left-out terms are at most 2^-24 of it; the large term is

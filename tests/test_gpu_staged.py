@@ -1,6 +1,7 @@
-"""The register-staged tiles (fp32 off the 16-byte grid or with K off the 32 grid, W8A32 at any alignment) against fp64, at the
-sizes where they can go wrong: one slab, a slab and one value, ranges of K that end inside a slab, tiles that hang over by all
-but one row or column, both tile sizes, every storage order, padded pitches and odd batch strides."""
+"""The register-staged tiles (products off the 16-byte grid or with K off the 32 grid: in bf16 terms from K = 64 on, on fp32 instructions
+below and for batches of few columns; W8A32 at any alignment) against fp64, at the sizes where they can go wrong: one slab, a slab and one
+value, ranges of K that end inside a slab, tiles that hang over by all but one row or column, every tile size, every storage order,
+padded pitches and odd batch strides."""
 import numpy as np
 import pytest
 
@@ -13,7 +14,8 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("M,N,K", [(17, 17, 32), (33, 65, 33), (65, 129, 63), (64, 63, 64), (129, 257, 65), (41, 1113, 92), (61, 343, 551),
-                                   (222, 434, 1376), (127, 11, 1023), (372, 2149, 257), (2001, 2003, 97), (17, 1, 4097)])
+                                   (222, 434, 1376), (127, 11, 1023), (372, 2149, 257), (2001, 2003, 97), (17, 1, 4097), (2001, 2003, 32),
+                                   (2033, 2003, 63)])
 @pytest.mark.parametrize("order", ["nn", "nt", "tn"])
 def test_staged_fp32(hip, M, N, K, order):
     say("staged", M, N, K, order)
@@ -33,7 +35,10 @@ def test_staged_fp32(hip, M, N, K, order):
     hip.check(hip.L.axhip_sgemm(int(order[0] == "t"), int(order[1] == "t"), M, N, K, 0.5, da.ptr, sa.shape[1], db.ptr, sb.shape[1], 2.0, dc.ptr,
                                 N + pad_c, dbias.ptr, 1))
     kernel = hip.last_kernel()
-    assert kernel.endswith("_staged") or kernel == "sgemm_splitk", kernel
+    if K >= 64:
+        assert kernel.endswith("x3_staged") or kernel == "sgemm_splitk_x3", kernel
+    else:
+        assert kernel == "sgemm_%s_%s_staged" % (order, "128x128k2" if M > 2000 else "64x64k2")
     full = dc.numpy()
     assert np.isnan(full[:, N:]).all()
     want = np.maximum(0.5 * (a.astype(np.float64) @ b.astype(np.float64)) + 2.0 * c + bias, 0)
@@ -41,13 +46,15 @@ def test_staged_fp32(hip, M, N, K, order):
     assert (np.abs(full[:, :N] - want) <= BOUND_FP32 * size).all(), float((np.abs(full[:, :N] - want) / size).max())
 
 
-@pytest.mark.parametrize("Bn,M,N,K,transb", [(3, 103, 103, 32, 1), (9, 67, 64, 103, 0), (17, 130, 131, 33, 1), (2, 65, 33, 129, 0)])
+@pytest.mark.parametrize("Bn,M,N,K,transb", [(3, 103, 103, 32, 1), (9, 67, 64, 103, 0), (17, 130, 131, 33, 1), (2, 65, 33, 129, 0), (9, 700, 47, 300, 0),
+                                             (16, 500, 501, 63, 1)])
 def test_staged_batched(hip, Bn, M, N, K, transb):
     say("staged batched", Bn, M, N, K, transb)
     rng = np.random.default_rng(Bn + M + K)
     a = rng.uniform(-1, 1, (Bn, M, K)).astype(np.float32)
     b = rng.uniform(-1, 1, (Bn, N, K) if transb else (Bn, K, N)).astype(np.float32)
     got = hip.sgemm_batched(hip.array(a), hip.array(b), transb=bool(transb), alpha=0.25).numpy()
+    assert hip.last_kernel().endswith("x3_staged" if K >= 64 and N >= 48 else "128x128k2_staged" if M == 500 else "64x64k2_staged")
     bt = b.astype(np.float64).transpose(0, 2, 1) if transb else b.astype(np.float64)
     want = 0.25 * (a.astype(np.float64) @ bt)
     size = 0.25 * (np.abs(a).astype(np.float64) @ np.abs(bt))
@@ -112,8 +119,8 @@ def test_tile_of_a_short_k(hip, order, Bn, M, N, K, kernel):
 
 @pytest.mark.parametrize("order,M,N,K,kernel", [
     ("nn", 17, 576, 340, "sgemm_32x64k2_dma_edge"), ("nt", 160, 20, 472, "sgemm_32x64k2_dma_edge"), ("nt", 96, 3296, 392, "sgemm_32x64k2_dma_edge"),
-    ("tn", 128, 672, 328, "sgemm_64x64k2_dma_edge"), ("nn", 249, 512, 376, "sgemm_nn_64x64x3_staged"), ("tn", 160, 32, 440, "sgemm_splitk"),
-    ("nn", 32, 1024, 540, "sgemm_splitk"), ("nn", 685, 32, 960, "sgemm_splitk")])
+    ("tn", 128, 672, 328, "sgemm_64x64k2_dma_edge"), ("nn", 249, 512, 376, "sgemm_nn_64x64x3_staged"), ("tn", 160, 32, 440, "sgemm_splitk_x3"),
+    ("nn", 32, 1024, 540, "sgemm_splitk_x3"), ("nn", 685, 32, 960, "sgemm_splitk")])
 def test_ranges_on_the_grid(hip, order, M, N, K, kernel):
     """Rows on the 16-byte grid with K off the 32 grid: ranges of K on the staged tiles only where K is long enough for what the
     direct-to-LDS tiles do in one launch."""
