@@ -1,6 +1,7 @@
-// fp32 GEMM on the fp32 matrix cores (v_mfma_f32_32x32x2_f32), NN / NT / TN, optionally
-// strided-batched, with alpha/beta, per-column scale, bias and activation fused into the
-// write-back.  True fp32 multiply-accumulate throughout.
+// fp32 GEMM, NN / NT / TN, optionally strided-batched, with alpha/beta, per-column scale, bias and
+// activation fused into the write-back: the dispatch, and the kernels on the fp32 matrix cores
+// (v_mfma_f32_32x32x2_f32).  Most large, ragged and batched products are formed in three bf16 terms per
+// operand instead, at fp32 accuracy (bf16x3.h, gemm_staged.hip, gemm_nt_terms.hip): dispatch_f32, run_f32.
 //
 // k_sgemm, the first kernel below, is what is left for products with K below 32 (64 with int8 weights) off the 16-byte grid.
 // One workgroup owns a BM x BN tile of C and walks K in slabs of 32.  An operand whose
@@ -1198,7 +1199,8 @@ int try_nt_cols(const SgemmArgs &g, int64_t batch) {
         g.stride_a % 4 != 0 || g.stride_b % 4 != 0 || g.stride_c % 4 != 0 || g.lda >= (1 << 20) || g.ldb >= (1 << 20))
         return -1;
     // Batches take the same walk in bf16 terms (512 heads of 512 x 512, us: K = 32 109 -> 94, 64 167 -> 131; 256
-    // of them, K = 96 114 -> 94, 128 147 -> 115; 128 of 1024 x 1024, K = 128 276 -> 213)
+    // of them, K = 96 114 -> 94, 128 147 -> 115; 128 of 1024 x 1024, K = 128 276 -> 213).  What is left for fp32 instructions are a
+    // forced AX_HIP_NT_WALK and single products of 131072 columns and more
     if (batch > 1 && tuning().nt_walk == 0) return nt_terms(staged_args(g), batch);
     switch (g.K / 32) {
         case 1: return launch_nt_cols<1>(g, batch);
@@ -1813,78 +1815,6 @@ int dispatch_f32(const SgemmArgs &g, int transa, int transb, int64_t batch, bool
     return fail(AXHIP_ERR_NOT_IMPLEMENTED, "sgemm: A^T * B^T is not provided");
 }
 
-// A large fp32 shape off the tile grid runs on 64x64 tiles with guarded edges (4000^3: 125
-// TFLOP/s against 141 for the large tiles on the grid).  When it is large enough for 128x128
-// tiles, its interior on that grid goes to them and only the right and bottom fringes to the
-// edge form; every block is a sub-matrix reached by pointer offsets.  Returns -1 when the shape
-// is left alone.
-int try_interior_and_fringes(const SgemmArgs &g, int transa, int transb) {
-    if ((transa && transb) || g.K % 32 != 0 || g.K <= 0) return -1;
-    if ((((uintptr_t)g.A | (uintptr_t)g.B | (uintptr_t)g.C | (uintptr_t)g.bias) & 15) != 0 || g.lda % 4 != 0 ||
-        g.ldb % 4 != 0 || g.ldc % 4 != 0)
-        return -1;                                           // the interior would not qualify for the fast kernels either
-    if ((g.M / 128) * (g.N / 128) < 2 * (int64_t)cu_count()) return -1;
-    const int64_t Mi = g.M / 128 * 128, Ni = g.N / 128 * 128;
-    if (Mi == g.M && Ni == g.N) return -1;
-    const float *A = static_cast<const float *>(g.A), *B = static_cast<const float *>(g.B);
-    // a fringe is a strip of few tiles with the whole K: the split-K route when it qualifies
-    auto fringe = [&](const SgemmArgs &f) {
-        const int rc = try_split_k<float>(f, transa, transb, "sgemm_splitk");
-        return rc >= 0 ? rc : dispatch_f32(f, transa, transb, 1);
-    };
-    SgemmArgs p = g;
-    p.M = Mi;
-    p.N = Ni;
-    int rc = dispatch_f32(p, transa, transb, 1);
-    if (rc == AXHIP_OK && Ni < g.N) {                       // columns Ni.. of the interior's rows
-        p = g;
-        p.M = Mi;
-        p.N = g.N - Ni;
-        p.B = transb ? B + Ni * g.ldb : B + Ni;
-        p.C = g.C + Ni;
-        if (g.bias) p.bias = g.bias + Ni;
-        rc = fringe(p);
-    }
-    if (rc == AXHIP_OK && Mi < g.M) {                       // rows Mi.., every column
-        p = g;
-        p.M = g.M - Mi;
-        p.A = transa ? A + Mi : A + Mi * g.lda;
-        p.C = g.C + Mi * g.ldc;
-        rc = fringe(p);
-    }
-    note_kernel("sgemm_interior+fringes");
-    return rc;
-}
-
-int run_f32(const SgemmArgs &g, int transa, int transb);
-
-// A large product on the tile grid whose K is a multiple of 4 but not of 32 is run as the product over the
-// first K / 32 * 32 columns (alpha and beta as given, no bias or activation yet) followed by the
-// few remaining columns accumulated on top (beta = 1) with the bias and activation of the whole.
-// Returns -1 when the shape is left alone.
-int try_k_tail(const SgemmArgs &g, int transa, int transb) {
-    const int64_t Km = g.K / 32 * 32;
-    if (Km == g.K || Km < 256) return -1;
-    // smaller ones run in one pass on the 64x64 tiles with guarded edges, which take a K tail
-    // themselves; two passes are for shapes whose main part earns 128x128 tiles
-    if ((g.M / 128) * (g.N / 128) < 2 * (int64_t)cu_count()) return -1;
-    const float *A = static_cast<const float *>(g.A), *B = static_cast<const float *>(g.B);
-    SgemmArgs p = g;
-    p.K = Km;
-    p.bias = nullptr;
-    p.act = AXHIP_ACT_NONE;
-    int rc = run_f32(p, transa, transb);
-    if (rc != AXHIP_OK) return rc;
-    p = g;
-    p.K = g.K - Km;
-    p.A = transa ? A + Km * g.lda : A + Km;
-    p.B = transb ? B + Km : B + Km * g.ldb;
-    p.beta = 1.0f;
-    rc = dispatch_f32(p, transa, transb, 1);
-    note_kernel("sgemm_main+k_tail");
-    return rc;
-}
-
 // a single product: the route for its shape
 int run_f32(const SgemmArgs &g, int transa, int transb) {
     if (!(transa && transb)) {
@@ -1900,7 +1830,7 @@ int run_f32(const SgemmArgs &g, int transa, int transb) {
         const bool wants_ranges = g.K % 32 != 0 && g.K >= ranges_from && ((g.M + 63) / 64) * ((g.N + 63) / 64) * 2 <= cu_count();
         const bool off = !on_grid || wants_ranges, whole = g.M % 64 == 0 && g.N % 64 == 0 && g.K % 32 == 0;
         // Products in bf16 terms: wherever the staged tiles are the route and K has two slabs (0.75 to 1.0 of the fp32 ones over some
-        // hundred shapes; 1050 x 1984 x 32 8.8 -> 9.7); on the grid where the fp32 tiles hang over an edge (160 x 800 x 2656 38 -> 18,
+        // hundred shapes; 1050 x 1984 x 32 8.8 -> 9.7); on the 16-byte grid where the fp32 tiles hang over an edge (160 x 800 x 2656 38 -> 18,
         // 1230 x 768 x 3072 55 -> 44, 298 x 4096 x 1024 37 -> 31; up to 160 rows their half tiles and K ranges are level or ahead) and
         // for large whole ones (640 x 2048 x 512 17.6 -> 18.7, 1024^3 19.6 -> 20.6, 640 x 4096 x 1024 49 -> 45, 2304 x 3072 x 768 95 -> 71).  A short K is
         // loads and write-back (2048 x 4096 x 64 16 -> 20, 128 24 -> 25; off the tile grid 4000 x 4000 x 128 53 -> 45).  Columns that fill
@@ -1916,10 +1846,6 @@ int run_f32(const SgemmArgs &g, int transa, int transb) {
         if (off) rc = staged_f32(staged_args(g), transa, transb, 1, true);
         if (rc >= 0) return rc;
         rc = try_split_k<float>(g, transa, transb, "sgemm_splitk");
-        if (rc >= 0) return rc;
-        rc = try_interior_and_fringes(g, transa, transb);
-        if (rc >= 0) return rc;
-        rc = try_k_tail(g, transa, transb);
         if (rc >= 0) return rc;
     }
     return dispatch_f32(g, transa, transb, 1);

@@ -170,10 +170,10 @@ F32_SHAPES = [(1, 1, 1), (2, 3, 2), (37, 19, 73), (64, 32, 128), (9, 500, 300), 
               (256, 3072, 2048), (192, 2816, 4096),
               # 64x64 tiles with the k split: two slabs per stage (K a multiple of 64; an odd and an even count of stages) and one (K = 160)
               (256, 512, 192), (320, 256, 448), (256, 256, 256), (256, 512, 160),
-              # off the tile grid with a large interior: fast kernels inside, guarded kernel on the fringes
+              # large and off the tile grid
               (1032, 1100, 96), (2100, 4200, 64), (1024, 1092, 160),
               (130, 257, 1027), (67, 1001, 129),                  # rows off the 16-byte grid in every form
-              (1024, 1088, 1045), (1030, 1100, 600),              # K off the 32 grid: main product, then the K tail on top
+              (1024, 1088, 1045), (1030, 1100, 600),              # K off the 32 grid
               # M or N off the 64 grid with K on the 32 grid and N % 4 == 0: direct-to-LDS tiles with guarded edges
               (65, 68, 64), (9, 4, 32), (63, 60, 96), (200, 36, 128), (500, 1000, 256), (12, 2052, 160),
               # K a multiple of 4 off the 32 grid: the last slab's tail is zero-filled in LDS
@@ -1666,7 +1666,7 @@ def test_binary_and_reductions_beyond_2_31_elements(hip, oracle, N, M):
                                         ("i8", 66001, 33000, 64)])
 def test_gemm_outputs_beyond_2_31_elements(hip, kind, M, N, K):
     """A product with more than 2^31 output elements (8.6 GB of fp32): element offsets into C must be
-    64-bit in every kernel of the route (edge tiles, interior + fringes, the persistent int8 tiles).
+    64-bit in every kernel of the route (edge tiles, bf16 terms, the persistent int8 tiles).
     Operands are small integers, so every product and every row or column sum of C is an exact fp32
     integer whatever the order: row sums of C are A . rowsum(B), column sums are colsum(A) . B, and
     rows at the start, around flat index 2^31 and at the end are read back."""

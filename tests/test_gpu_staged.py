@@ -120,10 +120,11 @@ def test_tile_of_a_short_k(hip, order, Bn, M, N, K, kernel):
 @pytest.mark.parametrize("order,M,N,K,kernel", [
     ("nn", 17, 576, 340, "sgemm_32x64k2_dma_edge"), ("nt", 160, 20, 472, "sgemm_32x64k2_dma_edge"), ("nt", 96, 3296, 392, "sgemm_32x64k2_dma_edge"),
     ("tn", 128, 672, 328, "sgemm_64x64k2_dma_edge"), ("nn", 249, 512, 376, "sgemm_nn_64x64x3_staged"), ("tn", 160, 32, 440, "sgemm_splitk_x3"),
-    ("nn", 32, 1024, 540, "sgemm_splitk_x3"), ("nn", 685, 32, 960, "sgemm_splitk")])
+    ("nn", 32, 1024, 540, "sgemm_splitk_x3"), ("nn", 685, 32, 960, "sgemm_splitk"),
+    ("nt", 3100, 3004, 64, "sgemm_64x64_dma_edge"), ("nn", 4000, 2500, 32, "sgemm_64x64_dma_edge")])
 def test_ranges_on_the_grid(hip, order, M, N, K, kernel):
     """Rows on the 16-byte grid with K off the 32 grid: ranges of K on the staged tiles only where K is long enough for what the
-    direct-to-LDS tiles do in one launch."""
+    direct-to-LDS tiles do in one launch.  A short K off the tile grid is one launch of theirs, however large the product."""
     say("ranges on the grid", order, M, N, K)
     rng = np.random.default_rng(M + N + K)
     a, b = rng.uniform(-1, 1, (M, K)).astype(np.float32), rng.uniform(-1, 1, (K, N)).astype(np.float32)
