@@ -504,10 +504,10 @@ int launch_staged(const char *name, const StagedArgs &g, int64_t batch, int64_t 
 // A tile and a number of ranges are chosen by the time they should take: what a launch costs once, and the rounds of workgroups
 // over the CUs, times the slabs of a range at what a slab of that tile costs plus what a round costs besides (first loads,
 // write-back); and for more than one range the finishing launch and its traffic.  The figures (us) of the fp32 and SPLIT tiles are
-// fitted to some 1900 products and batches, every tile timed on each, K from 32 to 3000: predictions are within 6 % (64x64) to 9 %
+// fitted to some 1900 products and batches, every tile timed on each, K from 32 to 3000: predictions are within 6 % (64x64) to 10 %
 // (128x128) on average, and the tile that is chosen within 1 % of the best one.  A round of the large tiles costs five times one of
-// 64x64, two of which share a CU: with a K of one to eight slabs that decides (us, 128x128 -> 64x64: 338 x 294 x 294, K = 64 100 ->
-// 74, 176 x 132 x 132, K = 34 32 -> 18, 383 x 279 x 279, K = 80 143 -> 101).
+// 64x64, two of which share a CU: with a K of one to eight slabs that decides (us, 128x128 -> 64x64: 338 x 294 x 294, K = 64 97 ->
+// 80, 176 x 132 x 132, K = 34 32 -> 18, 383 x 279 x 279, K = 80 140 -> 112).
 struct Plan {
     int tile;
     int64_t splits;
@@ -518,7 +518,7 @@ struct TileCost {
     float slab_us, round_us, once_us;
 };
 Plan plan_staged(const StagedArgs &g, int64_t batch, const TileCost *tiles, int n, bool may_split) {
-    const int64_t cus = cu_count();
+    const int64_t cus = cu_count(), forced = tuning().f32_splitk;     // 0: no AX_HIP_F32_SPLITK
     Plan best{-1, 1, 0.0f};
     for (int t = 0; t < n; t++) {
         const TileCost &c = tiles[t];
@@ -527,7 +527,7 @@ Plan plan_staged(const StagedArgs &g, int64_t batch, const TileCost *tiles, int 
         if (count > 0x7fffffff) continue;
         int64_t last = 0;
         for (int64_t per_cu = 0; per_cu <= 2; per_cu++) {        // no split, or as many ranges as give every CU one or two workgroups
-            int64_t z = per_cu == 0 ? 1 : per_cu * cus / count;
+            int64_t z = forced ? (count * 2 > cus ? 1 : forced) : per_cu == 0 ? 1 : per_cu * cus / count;
             if (z > g.K / 128) z = g.K / 128;
             if (z > 16) z = 16;
             if (z < 1 || (z > 1 && !may_split)) z = 1;

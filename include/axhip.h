@@ -58,7 +58,8 @@ const char *axhip_device_name(void);          /* gcnArchName of device 0, "" wit
  *   AX_HIP_I8_MFMA       16 | 32    matrix-core instruction of the persistent 256x256 W8A8 kernel: v_mfma_i32_16x16x64_i8 (what
  *                        runs by default) or v_mfma_i32_32x32x32_i8; the results are the same bits
  *   AX_HIP_F32_TILE      64x64 | 64x64k2 | 128x128   fp32 tile on the aligned fast path (k2: two wave sets split each K slab)
- *   AX_HIP_F32_SPLITK    1..4096    K ranges of the fp32 few-tile route (1: never split)
+ *   AX_HIP_F32_SPLITK    1..4096    K ranges of the fp32 few-tile route, W8A32's too (1: never split; on rows off the 16-byte grid at
+ *                        most 16, of 128 or more each)
  *   AX_HIP_NT_WALK       1 | 2      batched A B^T with K <= 128: 1, a 128-row block of A stays in LDS and the column blocks of B^T
  *                        are walked; 2, 256 rows of B stay in registers and A is walked in blocks of 32 rows (N a multiple of 256)
  *   AX_HIP_SKINNY_BLOCKS 1..65535   workgroups the skinny-M route aims for

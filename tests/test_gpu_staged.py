@@ -145,3 +145,29 @@ def test_batch_of_one_is_cut_like_a_product(hip, M, N, K, transb):
     bt = b[0].astype(np.float64).T if transb else b[0].astype(np.float64)
     want, size = 0.25 * (a[0].astype(np.float64) @ bt), 0.25 * (np.abs(a[0]).astype(np.float64) @ np.abs(bt))
     assert (np.abs(got - want) <= BOUND_FP32 * size).all()
+
+
+@pytest.mark.parametrize("splits", [1, 3, 4096])
+@pytest.mark.parametrize("M,N,K", [(372, 301, 2149), (65, 33, 257), (130, 1030, 1001)])
+def test_forced_ranges(hip, monkeypatch, M, N, K, splits):
+    """A forced number of K ranges (1: none) holds off the 16-byte grid too, for fp32 products and for int8 weights."""
+    say("forced ranges", M, N, K, splits)
+    rng = np.random.default_rng(M + N + K)
+    a, b = rng.uniform(-1, 1, (M, K)).astype(np.float32), rng.uniform(-1, 1, (K, N)).astype(np.float32)
+    w, s = rng.integers(-127, 128, (N, K), dtype=np.int8), rng.uniform(1e-3, 1e-2, N).astype(np.float32)
+    da, db, dw, ds = hip.array(a), hip.array(b), hip.array(w), hip.array(s)
+    monkeypatch.setenv("AX_HIP_F32_SPLITK", str(splits))
+    assert hip.L.axhip_tuning_reload() == 1
+    try:
+        got, kernel = hip.sgemm(da, db).numpy(), hip.last_kernel()
+        got8, kernel8 = hip.qgemm_w8a32(da, dw, ds).numpy(), hip.last_kernel()
+    finally:
+        monkeypatch.delenv("AX_HIP_F32_SPLITK")
+        assert hip.L.axhip_tuning_reload() == 0
+    if splits == 1:
+        assert kernel == "sgemm_nn_64x64k2_staged" and kernel8.endswith("k2_staged"), (kernel, kernel8)
+    else:
+        assert kernel == "sgemm_splitk" and kernel8 == "qgemm_w8a32_mfma_splitk", (kernel, kernel8)
+    size = np.abs(a).astype(np.float64)
+    assert (np.abs(got - a.astype(np.float64) @ b.astype(np.float64)) <= BOUND_FP32 * (size @ np.abs(b).astype(np.float64))).all()
+    assert (np.abs(got8 - (a.astype(np.float64) @ w.astype(np.float64).T) * s) <= BOUND_FP32 * (size @ np.abs(w).astype(np.float64).T) * s).all()
