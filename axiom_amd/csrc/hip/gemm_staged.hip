@@ -524,7 +524,7 @@ Plan plan_staged(const StagedArgs &g, int64_t batch, const TileCost *tiles, int 
         const TileCost &c = tiles[t];
         if (g.K < c.bk) continue;
         const int64_t count = ((g.M + c.bm - 1) / c.bm) * ((g.N + c.bn - 1) / c.bn) * batch, slabs = (g.K + c.bk - 1) / c.bk;
-        if (count > 0x7fffffff) continue;
+        if (count > 0x7fffff) continue;                          // 512 threads each, and a grid holds fewer than 2^32: the guarded tiles have 256
         int64_t last = 0;
         for (int64_t per_cu = 0; per_cu <= 2; per_cu++) {        // no split, or as many ranges as give every CU one or two workgroups
             int64_t z = forced ? (count * 2 > cus ? 1 : forced) : per_cu == 0 ? 1 : per_cu * cus / count;
