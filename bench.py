@@ -35,6 +35,7 @@ sys.path.insert(0, ROOT)
 
 PEAK_INT8_TOPS = 5000.0      # MI355X dense int8 MFMA, TOP/s
 PEAK_FP32_TFLOPS = 157.3     # MI355X fp32 matrix, TFLOP/s
+PEAK_BF16_TFLOPS = 2500.0    # MI355X bf16 matrix, dense; fp32 products in three bf16 terms per operand take six products each
 PEAK_HBM_GBS = 8000.0        # MI355X HBM3E, GB/s
 # Bytes that cross the L2 boundary per headline launch come from the committed counter summary of
 # `bench.py --counter-probe` (rocprofv3 --pmc FETCH_SIZE, then WRITE_SIZE, each scaled by what the same
@@ -156,14 +157,22 @@ def headline(hip, steps, warmup):
             "algorithmic_bytes": M * K + N * K + 4 * M * N + 8 * N}
 
 
+def fp32_matrix_fraction(tflops, kernel):
+    """An fp32 product's share of the matrix peak that bounds its kernel: six bf16 products for one in the kernels that work in
+    bf16 terms, the fp32 instructions otherwise."""
+    if "x3" in kernel or kernel.startswith("sdpa_fused"):
+        return {"frac_of_bf16_mfma_peak_at_6_products": 6 * tflops / PEAK_BF16_TFLOPS}
+    return {"frac_of_fp32_mfma_peak": tflops / PEAK_FP32_TFLOPS}
+
+
 def config_record(workload, flops, nbytes, time_s, bound, kernel, **extra):
     """One BASELINE configuration in the reference's record shape.  `bound` picks the roofline the
-    configuration is priced against: "hbm" (GB/s of algorithmic bytes), "mfma_fp32" (TFLOP/s) or
-    "mfma_int8" (TOP/s); roofline.achieved is the fraction of that peak."""
+    configuration is priced against: "hbm" (GB/s of algorithmic bytes), "mfma_fp32" (TFLOP/s; a sixth of the
+    bf16 peak for kernels in bf16 terms) or "mfma_int8" (TOP/s); roofline.achieved is the fraction of that peak."""
     if bound == "hbm":
         achieved, unit, peak = nbytes / time_s / 1e9, "GB/s", PEAK_HBM_GBS
     elif bound == "mfma_fp32":
-        achieved, unit, peak = flops / time_s / 1e12, "TFLOP/s", PEAK_FP32_TFLOPS
+        achieved, unit, peak = flops / time_s / 1e12, "TFLOP/s", PEAK_BF16_TFLOPS / 6 if "x3" in kernel else PEAK_FP32_TFLOPS
     else:
         achieved, unit, peak = flops / time_s / 1e12, "TOP/s", PEAK_INT8_TOPS
     rec = {"workload": workload, "algorithmic_flops": float(flops), "algorithmic_bytes": float(nbytes),
@@ -294,8 +303,7 @@ def secondary(hip):
     _, ms = time_calls(hip, lambda: hip.check(hip.L.axhip_sgemm(
         0, 0, 1024, 1024, 1024, 1.0, a.ptr, 1024, b.ptr, 1024, 0.0, c.ptr, 1024, None, 0)))
     tf = 2 * 1024 ** 3 / ms / 1e9
-    res["fp32_gemm_1024"] = {"us": ms * 1e3, "TFLOP/s": tf, "frac_of_fp32_mfma_peak": tf / PEAK_FP32_TFLOPS,
-                             "kernel": hip.last_kernel()}
+    res["fp32_gemm_1024"] = {"us": ms * 1e3, "TFLOP/s": tf, **fp32_matrix_fraction(tf, hip.last_kernel()), "kernel": hip.last_kernel()}
     result_line("axhip", "f32_nn_1024x1024x1024", "gflops", tf * 1e3)
     configs.append(config_record("configs[0]: fp32 GEMM C = A B, M=N=K=1024, row-major", 2 * 1024 ** 3, 3 * 4 * 1024 * 1024,
                                  ms * 1e-3, "mfma_fp32", hip.last_kernel(), key="config0"))
@@ -307,8 +315,7 @@ def secondary(hip):
         _, ms = time_calls(hip, lambda: hip.check(hip.L.axhip_sgemm(
             0, 0, n_, n_, n_, 1.0, a.ptr, n_, b.ptr, n_, 0.0, c.ptr, n_, None, 0)), seconds=0.4)
         tf = 2 * n_ ** 3 / ms / 1e9
-        res[f"fp32_gemm_{n_}"] = {"us": ms * 1e3, "TFLOP/s": tf, "frac_of_fp32_mfma_peak": tf / PEAK_FP32_TFLOPS,
-                                  "kernel": hip.last_kernel()}
+        res[f"fp32_gemm_{n_}"] = {"us": ms * 1e3, "TFLOP/s": tf, **fp32_matrix_fraction(tf, hip.last_kernel()), "kernel": hip.last_kernel()}
     del a, b, c
 
     # W8A32 with many rows (fp32 activations x int8 weights, fp32 accumulation): the tiles multiply on the bf16 matrix
@@ -326,7 +333,7 @@ def secondary(hip):
         tf = 2 * m_ * n_ * k_ / ms / 1e9
         res[f"w8a32_gemm_{m_}x{n_}x{k_}"] = {"us": ms * 1e3, "equivalent_TFLOP/s": tf, "fp32_gemm_us": ms32 * 1e3,
                                              "speedup_over_fp32": ms32 / ms,
-                                             "frac_of_bf16_mfma_peak_at_3_terms": 3 * tf / 2500.0, "kernel": kern}
+                                             "frac_of_bf16_mfma_peak_at_3_terms": 3 * tf / PEAK_BF16_TFLOPS, "kernel": kern}
         del xa, wq, wsc, wf, oq
 
     # config 3: FFN block 2048 x 1024 x 4096, bias + GELU fused into GEMM1, bias into GEMM2
@@ -341,14 +348,15 @@ def secondary(hip):
                                     hbuf.ptr, 4096, b1.ptr, 2))
         hip.check(hip.L.axhip_sgemm(0, 0, 2048, 1024, 4096, 1.0, hbuf.ptr, 4096, w2.ptr, 1024, 0.0,
                                     y.ptr, 1024, b2.ptr, 0))
+    hip.check(hip.L.axhip_sgemm(0, 0, 2048, 4096, 1024, 1.0, x.ptr, 1024, w1.ptr, 4096, 0.0, hbuf.ptr, 4096, b1.ptr, 2))
+    k1 = hip.last_kernel()
     _, ms = time_calls(hip, ffn)
     tf = 2 * 2 * 2048 * 1024 * 4096 / ms / 1e9
-    res["fp32_ffn_2048x1024x4096"] = {"us": ms * 1e3, "TFLOP/s": tf,
-                                      "frac_of_fp32_mfma_peak": tf / PEAK_FP32_TFLOPS}
+    res["fp32_ffn_2048x1024x4096"] = {"us": ms * 1e3, "TFLOP/s": tf, **fp32_matrix_fraction(tf, hip.last_kernel())}
     result_line("axhip", "f32_ffn_2048x1024x4096", "gflops", tf * 1e3)
     configs.append(config_record("configs[3]: fp32 FFN block, tokens 2048, d_model 1024, d_ff 4096: GEMM + bias + GELU fused, GEMM + bias",
                                  2 * 2 * 2048 * 1024 * 4096, 4 * (2048 * 1024 + 1024 * 4096 + 2 * 2048 * 4096 + 4096 * 1024 + 2048 * 1024),
-                                 ms * 1e-3, "mfma_fp32", "two launches of " + hip.last_kernel(), key="config3"))
+                                 ms * 1e-3, "mfma_fp32", k1 + " + " + hip.last_kernel(), key="config3"))
 
     # dense backward of the FFN block's first layer (X [2048,1024], W [1024,4096], dY [2048,4096]):
     # dA = dY W^T (NT), dW = X^T dY (TN), dBias = sum(dY, 0)
@@ -367,7 +375,7 @@ def secondary(hip):
         "dA_nt_us": ms * 1e3, "dA_TFLOP/s": fl / ms / 1e9, "dA_kernel": k_nt,
         "dW_tn_us": ms2 * 1e3, "dW_TFLOP/s": fl / ms2 / 1e9, "dW_kernel": k_tn,
         "dBias_us": ms3 * 1e3, "dBias_GB/s": 4 * 2048 * 4096 / ms3 / 1e6,
-        "frac_of_fp32_mfma_peak": 2 * fl / (ms + ms2) / 1e9 / PEAK_FP32_TFLOPS}
+        **fp32_matrix_fraction(2 * fl / (ms + ms2) / 1e9, k_tn)}
     del dyb, da, dw
     del x, w1, w2, hbuf, y
 
@@ -534,20 +542,20 @@ def secondary(hip):
     res["fp32_batched_pv"] = {"us": ms * 1e3, "TFLOP/s": 2 * Bn * S * S * D / ms / 1e9,
                               "GB/s": nbytes / ms / 1e6, "frac_of_hbm_peak": nbytes / ms / 1e6 / PEAK_HBM_GBS}
     res["fp32_batched_pv"]["kernel"] = hip.last_kernel()
-    # arithmetic intensity 25.6 flop/byte against a machine balance of 19.7: the roofline prices both at the matrix cores
-    # (109 us); the time the bytes alone take at 8 TB/s (84 us) is given beside it
+    # arithmetic intensity 25.6 flop/byte.  On fp32 instructions the machine balance is 19.7 and the matrix cores are the roofline
+    # (109 us); in bf16 terms it is 52, and the bytes are (84 us at 8 TB/s).  The share of the HBM peak is given for both
     for key, name, what in (("config4b_qkt", "fp32_batched_qkt", "S = Q K^T, [512,64] x [512,64]^T"),
                             ("config4b_pv", "fp32_batched_pv", "O = S V, [512,512] x [512,64]")):
         t = res[name]["us"] * 1e-6
         configs.append(config_record(f"configs[4] (b): strided-batched fp32 GEMM over 512 heads, {what}", 2 * Bn * S * S * D, nbytes, t,
-                                     "mfma_fp32", res[name]["kernel"], key=key, frac_of_hbm_peak=nbytes / t / 1e9 / PEAK_HBM_GBS))
+                                     "hbm" if "x3" in res[name]["kernel"] else "mfma_fp32", res[name]["kernel"], key=key, frac_of_hbm_peak=nbytes / t / 1e9 / PEAK_HBM_GBS))
     # fused attention forward over the same heads (both products and the softmax in one kernel,
     # no [512,512] score matrix in memory); flops counted as the two GEMMs'
     l = hip.empty((Bn, S))
     _, ms = time_calls(hip, lambda: hip.check(hip.L.axhip_sdpa_fwd(q.ptr, k.ptr, v.ptr, o.ptr, l.ptr, Bn, S, D,
                                                                   0.125, 0)))
     res["fp32_sdpa_fwd_512x512x64"] = {"us": ms * 1e3, "TFLOP/s": 4 * Bn * S * S * D / ms / 1e9,
-                                       "frac_of_fp32_mfma_peak": 4 * Bn * S * S * D / ms / 1e9 / PEAK_FP32_TFLOPS,
+                                       **fp32_matrix_fraction(4 * Bn * S * S * D / ms / 1e9, hip.last_kernel()),
                                        "kernel": hip.last_kernel(),
                                        "unfused_us": res["fp32_batched_qkt"]["us"] + res["fp32_batched_pv"]["us"]}
     _, ms = time_calls(hip, lambda: hip.check(hip.L.axhip_sdpa_fwd(q.ptr, k.ptr, v.ptr, o.ptr, l.ptr, Bn, S, D,
