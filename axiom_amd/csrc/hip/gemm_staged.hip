@@ -4,9 +4,10 @@
 // fp32 products in bf16 terms (SPLIT): six bf16 products per fp32 one (bf16x3_nearest) still take 6/16 of the matrix-core time of
 // the fp32 instructions, and as an instruction adds 16 products before it rounds, the sums are nearer to 64 bits than those of
 // the fp32 tiles on every shape measured (relative error 1024^3 4.1e-7 -> 1.2e-7 on 64x64 tiles, 2048 x 4096 x 4096 1.15e-6 ->
-// 7.0e-7 on 128x128).  us, fp32 tiles -> split: 2000 x 4096 x 1024 142 -> 99, 2000 x 1024 x 4096 134 -> 100, 2048 x 4096 x 4096
-// 466 -> 339 (203 TFLOP/s), 8192^3 7204 -> 5612, 8 x 1024^3 155 -> 98.  Bound on 128x128: matrix core busy
-// 62 % of the cycles at the 1.85 GHz that the chip then holds, LDS 31 %; 64x64: the reads of fragments from LDS.  The conversions
+// 7.0e-7 on 128x128).  us, fp32 tiles -> split: 2000 x 4096 x 1024 142 -> 98, 2000 x 1024 x 4096 134 -> 98, 4096^3 931 -> 686
+// (200 TFLOP/s), 8192^3 7370 -> 5440, 8 x 1024^3 155 -> 98, a feed-forward block 2048 x 1024 x 4096 250 -> 200.  Bound on 128x128: of
+// the cycles of that block's products the matrix core is busy 49 %, the vector pipe some 40 %, the LDS pipe 32 % (a fifth of that bank
+// conflicts); 64x64: the reads of fragments from LDS.  The conversions
 // (some 8 instructions a value) are put between the products of the same wave (interleave), worth 4 to 10 %.
 // A tile whose sums are not all finite is computed again with fp32 instructions by the same workgroup: infinities, NaNs and values
 // near the largest float come out as fp32 products give them.
@@ -17,11 +18,12 @@
 // the tile and take its 16-wide k-steps in turn; on every SIMD one wave of each set, which do the slab's two halves of work
 // (convert and write; read and multiply) in opposite order, so that vector and matrix instructions come from different waves.
 // Operands lie in LDS as rows of one slab each (an operand stored the other way is transposed by the register: a thread takes
-// consecutive k of one column), fragments are 16-byte reads, both without bank conflicts (Geom::at).
-// Bound: fp32, the matrix core: 2001 x 2003 x 2005 runs at 119 TFLOP/s (76 % of the datasheet rate; guarded 64x64 tiles without
+// consecutive k of one column), fragments are 16-byte reads; rows are spread over the banks (Geom::at).
+// Bound: fp32 instructions (forced tiles, K below 64 off the 16-byte grid, narrow batches), the matrix core: 2001 x 2003 x 2005 runs at
+// 119 TFLOP/s (76 % of the datasheet rate; guarded 64x64 tiles without
 // prefetch 75), 1024^3 at 24 us against 19.6 of the direct-to-LDS kernel, which keeps every shape it can take.  Small products
-// are latency: one 64x64 tile with K = 92 takes 7 us, of which 2.3 are the launch.  W8A32, 250 x 4096 x 4096 in 35 us (240
-// TFLOP/s of products, three bf16 terms each): matrix core busy 36 % of the time, LDS 44 %, vector pipe about as much; without
+// are latency: one 64x64 tile with K = 92 takes 7 us, of which 2.3 are the launch.  W8A32, 250 x 4096 x 4096 in 35.6 us (235
+// TFLOP/s of products, three bf16 terms each): matrix core busy 28 % of the cycles, LDS and vector pipe 24 % each, at idle clocks; without
 // the conversions 27 us, without products 24, without global loads 27, products alone 20 - three pipes that overlap in part.
 // Activations are cut as in SPLIT, so that small ones keep their bits (they ran on fp32 instructions before these tiles); the second
 // pass over tiles with sums that are not finite reads its operands straight from memory (no room for fp32 slabs in the same LDS).

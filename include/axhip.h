@@ -51,7 +51,9 @@ const char *axhip_device_name(void);          /* gcnArchName of device 0, "" wit
  * counterpart of AX_GEMM_MC / AX_GEMM_NC / AX_GEMM_KC (src/compute/backends/cpu_opt.c:512-539).
  * Read from the environment by axhip_init and again by axhip_tuning_reload (which needs no GPU and
  * returns how many variables were recognised); unset, empty or invalid values mean "choose by shape".
- * A forced choice applies only where the shape permits that kernel; results do not depend on it.
+ * A forced choice applies only where the shape permits that kernel.  Integer results do not depend on it; fp32 ones agree to
+ * fp32 accuracy, not bit for bit: AX_HIP_F32_TILE, AX_HIP_F32_SPLITK and AX_HIP_NT_WALK also keep products on fp32 instructions
+ * that would be formed in bf16 terms (axhip_sgemm), and every split adds in another order.
  *   AX_HIP_I8_TILE       64x64 | 64x64k2 | 128x64 | 128x128 | 256x256   W8A8 tile (256x256: M, N multiples of 256;
  *                        k2: two wave sets split each K slab)
  *   AX_HIP_I8_SPLITK     1..16      workgroups over K per W8A8 tile of 64x64 / 128x128 (1: never split)
@@ -124,7 +126,11 @@ int   axhip_memcpy_d2d(void *device_dst, const void *device_src, size_t bytes);
  *      transa = 0: A is [M,K] (lda >= K);  1: A is [K,M] (lda >= M)
  *      transb = 0: B is [K,N] (ldb >= N);  1: B is [N,K] (ldb >= K)
  *      bias may be NULL; beta == 0 never reads C (C may be uninitialised).
- *      True fp32 MFMA arithmetic; M <= 16 with transa = transb = 0, alpha = 1, beta = 0 takes
+ *      fp32 accuracy throughout.  Products are formed by fp32 instructions or, mostly large and ragged
+ *      ones, on the bf16 matrix core with each operand as the exact sum of three bf16 terms: six products
+ *      of terms stand for one (what they leave out is at most 2^-24 of it), added in fp32.  For every finite
+ *      operand, however small; sums that leave fp32's range or that infinities and NaNs enter come out
+ *      as fp32 instructions give them.  M <= 16 with transa = transb = 0, alpha = 1, beta = 0 takes
  *      the weight-streaming route below. ------------------------------------------------- */
 int axhip_sgemm(int transa, int transb, int64_t M, int64_t N, int64_t K, float alpha,
                 const float *A, int64_t lda, const float *B, int64_t ldb, float beta,
