@@ -52,7 +52,7 @@ __device__ __forceinline__ Bf16x3 bf16x3_of(const v4f &p, const v4f &q) {
 // are its terms: none of them is denormal, whatever the float.  Without it the cut loses bits below 2^-102, which GELU and softmax
 // produce in ordinary use; sending tiles that hold such values through fp32 instructions cost a feed-forward block on trained-like
 // activations (2048 x 1024 x 4096, pre-activations of standard deviation 2) 329 us where it takes 203.
-// What the terms cannot hold shows in the sums: operands from 2^103 up, infinities and NaNs, and sums past 2^80 leave an infinity or a
+// What the terms cannot hold shows in the sums: operands from about 2^104 up, infinities and NaNs, and sums past 2^80 leave an infinity or a
 // NaN in every sum they enter.  The kernels look at their sums (look_at, any_wave) and form such tiles again with fp32 instructions.
 // Per pair of values: two products, three conversions, four shifts or masks, four subtractions.
 typedef int v2i __attribute__((ext_vector_type(2)));
