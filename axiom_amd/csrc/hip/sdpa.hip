@@ -24,8 +24,8 @@
 // A tile with a sum that is not finite is computed again with fp32 instructions by the same workgroup:
 // infinities, NaNs and values near the largest float come out as fp32 products give them.
 // us, fp32 instructions -> terms: 512 heads of [512, 64] 269 -> 194 (causal 178 -> 126), 64 of [1024, 128] 273 -> 174, 96 causal
-// ones of [1000, 80] 324 -> 129 (a quarter of that from the 96-wide geometry), 512 of [256, 32] 41 -> 33, 32 of [128, 64] 11.9 ->
-// 10.9.  O is nearer to 64 bits on every shape measured (relative error 4.9e-7 -> 3.7e-7 at [512, 64]).  Bound: the matrix core is
+// ones of [1000, 80] 324 -> 129 (a quarter of that from the 96-wide geometry), 512 of [256, 32] 41 -> 33; with few query tiles for the
+// CUs k_sdpa_few cuts a head along its keys too (32 heads of [128, 64] 11.4 -> 6.9).  O is nearer to 64 bits on every shape measured (relative error 4.9e-7 -> 3.7e-7 at [512, 64]).  Bound: the matrix core is
 // busy 49 % of the cycles, vector instructions (cutting, softmax) take some 44 ([512, 64]; causal [1000, 80] 37 and 29).  Measured and dropped: two key tiles at a time,
 // the scores of one interleaved with the exponentials of the other by instruction groups ([512, 64] 194, [1024, 96] 126 -> 128).
 //
@@ -403,6 +403,222 @@ k_sdpa(const float *__restrict__ Q, const float *__restrict__ K, const float *__
     }
 }
 
+// Few tiles: four waves share 32 queries of one head and take its 32-key tiles in turn, each with an online softmax of its own; the
+// sets of maxima, sums and outputs meet in LDS.  Each wave reads its keys and values straight into fragment registers and cuts them itself,
+// so a key is cut once per 32 queries and not once per 128 or 256: more vector work in all, on four (or eight) times the workgroups and with
+// a quarter of the serial key tiles.
+template <int DK, bool CAUSAL, bool PAD>
+__global__ void __launch_bounds__(256, DK <= 64 ? 2 : 1)
+k_sdpa_few(const float *__restrict__ Q, const float *__restrict__ K, const float *__restrict__ V, float *__restrict__ O, float *__restrict__ L,
+           int64_t BH, int64_t S, float scale_log2e, int64_t H, int64_t ld, int64_t ldo, int dkr) {
+    constexpr int KS = DK / 16, DT = DK / 32, PIECES = 4 * DT, WAVES = 4;
+    constexpr bool APART = DK <= 64;             // as in k_sdpa
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+    auto part = reinterpret_cast<v4f (*)[PIECES][64]>(lds);              // [WAVES]: sums; then maxima and row sums; then a word per wave
+    auto ml = reinterpret_cast<float (*)[2][32]>(lds + WAVES * PIECES * 1024);
+    unsigned char *flags = lds + WAVES * (PIECES * 1024 + 256);
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = threadIdx.x & 63, frow = lane & 31, fhalf = lane >> 5;
+    const int64_t nq = (S + 31) / 32;            // workgroups as in k_sdpa: the tiles of a head on one XCD
+    const int64_t lin = blockIdx.x, group = lin / (8 * nq), left = BH - group * 8;
+    const int64_t r = lin - group * 8 * nq, hpg = left < 8 ? left : 8;
+    const int64_t head = group * 8 + r % hpg, q0 = (CAUSAL ? nq - 1 - r / hpg : r / hpg) * 32;       // causal: the longest first
+    const int64_t hb = head / H, hh = head - hb * H;
+    const int width = PAD ? dkr : DK;
+    const int64_t in0 = hb * S * ld + hh * width;
+    const float *Qh = Q + in0, *Kh = K + in0, *Vh = V + in0;
+    const unsigned rowb = (unsigned)ld * 4;
+    const int64_t qg = q0 + frow;
+    const int tiles = (int)(CAUSAL ? q0 / 32 + 1 : nq);
+
+    auto load_row = [&](float (&x)[8], const char *row, int col) {       // columns col .. col + 7, zero from width on
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            v4f a = {0.f, 0.f, 0.f, 0.f};
+            if (!PAD || col + 4 * h < dkr) a = *reinterpret_cast<const v4f *>(row + (col + 4 * h) * 4);
+#pragma unroll
+            for (int e = 0; e < 4; e++) x[4 * h + e] = a[e];
+        }
+    };
+    float kr[KS][8], vr[2][DT][8];
+    // a key past the end is read as the last one (its score is masked)
+    auto load_k = [&](int t) {
+        const int64_t key = (int64_t)t * 32 + frow;
+        const char *row = reinterpret_cast<const char *>(Kh + (key < S ? key : S - 1) * ld);
+#pragma unroll
+        for (int ks = 0; ks < KS; ks++) load_row(kr[ks], row, 16 * ks + 8 * fhalf);
+    };
+    auto load_v = [&](int t) {
+        const char *base = reinterpret_cast<const char *>(Vh + (int64_t)t * 32 * ld);
+        const int end = (int)(S - 1 - (int64_t)t * 32 < 31 ? S - 1 - (int64_t)t * 32 : 31);
+#pragma unroll
+        for (int st = 0; st < 2; st++)
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                const int key = 16 * st + 4 * fhalf + e + (e & 4);
+                const char *row = base + (unsigned)(key < end ? key : end) * rowb;
+#pragma unroll
+                for (int d = 0; d < DT; d++) {
+                    const int col = d * 32 + frow;
+                    vr[st][d][e] = *reinterpret_cast<const float *>(row + (PAD && col >= dkr ? dkr - 1 : col) * 4);
+                }
+            }
+    };
+    v4i qf[KS][3];
+    v16f acc_o[DT];
+#pragma unroll
+    for (int d = 0; d < DT; d++)
+#pragma unroll
+        for (int v = 0; v < 16; v++) acc_o[d][v] = 0.0f;
+    float m_run = SD_LOWEST, l_run = 0.0f;
+    if (wave < tiles) {
+        load_k(wave);
+        const char *q = reinterpret_cast<const char *>(Qh + (qg < S ? qg : S - 1) * ld);
+        float x[KS][8];
+#pragma unroll
+        for (int ks = 0; ks < KS; ks++) load_row(x[ks], q, 16 * ks + 8 * fhalf);
+        load_v(wave);
+#pragma unroll
+        for (int ks = 0; ks < KS; ks++) {
+#pragma unroll
+            for (int e = 0; e < 8; e++) x[ks][e] *= scale_log2e;
+            cut(x[ks], TERMS_UP, qf[ks]);
+        }
+    }
+    for (int t = wave; t < tiles; t += WAVES) {
+        const int next = t + WAVES < tiles ? t + WAVES : t;              // past the end the same tile again, unused
+        v16f s, low;
+#pragma unroll
+        for (int v = 0; v < 16; v++) s[v] = low[v] = 0.0f;
+#pragma unroll
+        for (int ks = 0; ks < KS; ks++) {
+            v4i kf[3];
+            cut(kr[ks], TERMS_UP, kf);
+#pragma unroll
+            for (int sum = 2; sum > 0; sum--)
+#pragma unroll
+                for (int p = sum; p >= 0; p--) (APART ? low : s) = mfma_terms(kf[sum - p], qf[ks][p], APART ? low : s);
+            s = mfma_terms(kf[0], qf[ks][0], s);
+        }
+        load_k(next);
+        if (APART) s += low;
+        if (CAUSAL ? t == tiles - 1 : (int64_t)t * 32 + 32 > S) {
+            const int qrel = (int)((CAUSAL ? qg : S - 1) - (int64_t)t * 32);
+#pragma unroll
+            for (int v = 0; v < 16; v++)
+                if (8 * (v >> 2) + 4 * fhalf + (v & 3) > qrel) s[v] = -INFINITY;
+        }
+        softmax_step<DT>(s, acc_o, m_run, l_run, TERMS_UP, TERMS_DOWN);
+#pragma unroll
+        for (int st = 0; st < 2; st++) {
+            float x[8];
+#pragma unroll
+            for (int e = 0; e < 8; e++) x[e] = s[8 * st + e];
+            v4i pf[3];
+            cut(x, 1.0f, pf);
+#pragma unroll
+            for (int d = 0; d < DT; d++) {
+                v4i vf[3];
+                cut(vr[st][d], TERMS_UP, vf);
+#pragma unroll
+                for (int sum = 2; sum >= 0; sum--)
+#pragma unroll
+                    for (int p = sum; p >= 0; p--) acc_o[d] = mfma_terms(vf[p], pf[sum - p], acc_o[d]);
+            }
+        }
+        load_v(next);
+    }
+
+    // ---- the waves' parts together ----
+    float seen = l_run * 0.0f;
+#pragma unroll
+    for (int d = 0; d < DT; d++) look_at(acc_o[d], seen);
+    const float l_wave = l_run + __shfl_xor(l_run, 32, 64);
+#pragma unroll
+    for (int d = 0; d < DT; d++)
+#pragma unroll
+        for (int g = 0; g < 4; g++) part[wave][d * 4 + g][lane] = v4f{acc_o[d][4 * g], acc_o[d][4 * g + 1], acc_o[d][4 * g + 2], acc_o[d][4 * g + 3]};
+    if (fhalf == 0) {
+        ml[wave][0][frow] = m_run;
+        ml[wave][1][frow] = l_wave;
+    }
+    bool unfit = any_wave<WAVES>(!(seen == 0.0f), flags, wave);
+    float m_all = ml[0][0][frow], weight[WAVES], l_all = 0.0f;
+#pragma unroll
+    for (int w = 1; w < WAVES; w++) m_all = fmaxf(m_all, ml[w][0][frow]);
+#pragma unroll
+    for (int w = 0; w < WAVES; w++) {
+        weight[w] = __builtin_amdgcn_exp2f(ml[w][0][frow] - m_all);
+        l_all += ml[w][1][frow] * weight[w];
+    }
+    unfit |= __builtin_amdgcn_ballot_w64(l_all == 0.0f && qg < S) != 0;  // the same in every wave
+    float *orow = O + (hb * S + qg) * ldo + hh * width;
+    if (unfit) {
+        if (wave != 0) return;
+        attend_f32<DK, CAUSAL>(Qh, Kh, Vh, ld, S, width, scale_log2e, q0, lane, acc_o, m_run, l_run);
+        const float l_tot = l_run + __shfl_xor(l_run, 32, 64), inv = 1.0f / l_tot;
+        if (qg >= S) return;
+#pragma unroll
+        for (int d = 0; d < DT; d++)
+#pragma unroll
+            for (int g = 0; g < 4; g++) {
+                const int col = d * 32 + 8 * g + 4 * fhalf;
+                if (!PAD || col < dkr)
+                    *reinterpret_cast<v4f *>(orow + col) = v4f{acc_o[d][4 * g] * inv, acc_o[d][4 * g + 1] * inv, acc_o[d][4 * g + 2] * inv, acc_o[d][4 * g + 3] * inv};
+            }
+        if (L && fhalf == 0) L[head * S + qg] = l_tot == 0.0f ? NAN : (m_run + __builtin_amdgcn_logf(l_tot)) * 0.6931471805599453f;
+        return;
+    }
+    if (qg >= S) return;
+    const float inv = 1.0f / l_all * (1.0f / TERMS_UP);
+    for (int piece = wave; piece < PIECES; piece += WAVES) {
+        v4f o = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int w = 0; w < WAVES; w++) o += part[w][piece][lane] * weight[w];
+        const int col = (piece >> 2) * 32 + 8 * (piece & 3) + 4 * fhalf;
+        if (!PAD || col < dkr) *reinterpret_cast<v4f *>(orow + col) = o * inv;
+    }
+    if (L && wave == 0 && fhalf == 0) L[head * S + qg] = (m_all + __builtin_amdgcn_logf(l_all / TERMS_UP)) * 0.6931471805599453f;
+}
+
+// Where the few-tiles form pays, by the key tiles that a wave walks one after the other: the longest walk is a quarter of a head's 32-key
+// tiles, all walks together are shared by the CUs, and up to some 2.25 walks of the longest kind a CU it is ahead of k_sdpa, whose
+// four waves each walk all of a head's tiles (us, k_sdpa -> this: 32 heads of [128, 64] 11.4 -> 6.9, 4 of [2048, 64] 111 -> 36, 32 of [512, 64] 33.3
+// -> 22.0, 8 causal ones of [2048, 128] 204 -> 74, 32 causal of [1024, 80] 81.6 -> 74.4; past it 64 of [512, 64] 35.7 -> 38.6, 64 causal of
+// [512, 80] 44.6 -> 55.6).  A single key tile per wave (S up to 128) is mostly start and end: one workgroup a CU, or two of the smaller
+// geometries from three tiles on (128 of [128, 64] 12.1 -> 11.5, but 128 of [128, 128] 21.3 -> 23.2, 256 of [64, 64] 8.1 -> 8.9).  A head of
+// one tile gains nothing (4.6 us either way).
+// Eight waves on 32 queries: level or behind (32 of [512, 64] 22.0 -> 27.2, 1 of [2048, 64] 32.7 -> 31.1): the vector pipe is the bound.
+template <int DK>
+bool few_tiles(int64_t BH, int64_t S, int causal) {
+    const int64_t tiles = (S + 31) / 32, walk = (tiles + 3) / 4, cus = cu_count();
+    if (tiles < 2 || BH > 4 * cus || tiles > 0xffff) return false;
+    if (walk == 1) return tiles * BH <= (DK > 64 || tiles == 2 ? 1 : 2) * cus;
+    const int64_t q = tiles / 4, all = causal ? 2 * q * (q + 1) + tiles % 4 * (q + 1) : tiles * walk;
+    return all * BH * 4 <= 9 * walk * cus;
+}
+
+template <int DK>
+int launch_sdpa_few(const float *Q, const float *K, const float *V, float *O, float *L, int64_t BH, int64_t S,
+                    float scale, int causal, int64_t H, int64_t ld, int64_t ldo, int dkr) {
+    constexpr int SMEM = 4 * (DK / 8 * 1024 + 256 + 4);
+    static bool attr_set = false;
+    if (!attr_set) {
+        for (const void *k : {reinterpret_cast<const void *>(k_sdpa_few<DK, false, false>), reinterpret_cast<const void *>(k_sdpa_few<DK, true, false>),
+                              reinterpret_cast<const void *>(k_sdpa_few<DK, false, true>), reinterpret_cast<const void *>(k_sdpa_few<DK, true, true>)})
+            AXHIP_HIP_TRY(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, SMEM), "hipFuncSetAttribute");
+        attr_set = true;
+    }
+    const float sl2 = scale * 1.4426950408889634f;
+    const dim3 grid((unsigned)((S + 31) / 32 * BH)), block(256);
+#define AX_FEW(C, P) hipLaunchKernelGGL((k_sdpa_few<DK, C, P>), grid, block, SMEM, kStream, Q, K, V, O, L, BH, S, sl2, H, ld, ldo, dkr)
+    if (causal && dkr == DK) AX_FEW(true, false);
+    else if (causal) AX_FEW(true, true);
+    else if (dkr == DK) AX_FEW(false, false);
+    else AX_FEW(false, true);
+#undef AX_FEW
+    return check_launch("sdpa_fwd");
+}
+
 template <int DK, int WAVES, bool PAD>
 int launch_sdpa_p(const float *Q, const float *K, const float *V, float *O, float *L, int64_t BH, int64_t S,
                   float scale, int causal, int64_t H, int64_t ld, int64_t ldo, int dkr) {
@@ -432,7 +648,7 @@ int launch_sdpa(const float *Q, const float *K, const float *V, float *O, float 
     // Eight waves on 256 queries cut half as much of K and V for each of them, four on 128 waste less of a short head and
     // of the diagonal.  us, four waves -> eight: 64 heads of [1024, 128] 191 -> 174 (causal 158 -> 142), 64 of [1024, 96]
     // 141 -> 126, 96 causal ones of [1000, 80] 146 -> 129, 512 of [512, 64] 201 -> 194; but causal 126 -> 134, 512 of [256, 32]
-    // 33 -> 37, 256 causal ones of [333, 48] 49 -> 53, and with fewer tiles than CUs (64 of [128, 64]) 11.0 -> 13.9.  Geometry
+    // 33 -> 37, 256 causal ones of [333, 48] 49 -> 53.  Geometry
     // 128 has the registers of one wave per SIMD with four waves, so it takes eight as soon as there is more than one tile a CU.
     if constexpr (DK > 32) {
         const int64_t half_tiles = (S + 127) / 128, tiles = (S + 255) / 256;
@@ -511,23 +727,29 @@ int sdpa_unfused(const float *Q, const float *K, const float *V, float *O, float
 // size that is a multiple of 4 up to 128 runs on the kernel of the next size among 32, 64, 96, 128.
 static bool sdpa_fusable(int64_t dk) { return dk >= 4 && dk <= 128 && dk % 4 == 0; }
 
+// A kernel's name: geometry, mask, and whether the few-tiles form runs.
+static const char *sdpa_name(int dk, int causal, bool few) {
+    static const char *const names[4][2][2] = {{{"sdpa_fused_dk32", "sdpa_fused_few_dk32"}, {"sdpa_fused_dk32_causal", "sdpa_fused_few_dk32_causal"}},
+                                               {{"sdpa_fused_dk64", "sdpa_fused_few_dk64"}, {"sdpa_fused_dk64_causal", "sdpa_fused_few_dk64_causal"}},
+                                               {{"sdpa_fused_dk96", "sdpa_fused_few_dk96"}, {"sdpa_fused_dk96_causal", "sdpa_fused_few_dk96_causal"}},
+                                               {{"sdpa_fused_dk128", "sdpa_fused_few_dk128"}, {"sdpa_fused_dk128_causal", "sdpa_fused_few_dk128_causal"}}};
+    return names[dk / 32 - 1][causal != 0][few];
+}
+
 static int sdpa_fused(const float *Q, const float *K, const float *V, float *O, float *L, int64_t BH, int64_t S,
                       int64_t dk, float scale, int causal, int64_t H, int64_t ld, int64_t ldo) {
-    int rc;
-    if (dk <= 32) {
-        rc = launch_sdpa<32>(Q, K, V, O, L, BH, S, scale, causal, H, ld, ldo, (int)dk);
-        axhip::note_kernel(causal ? "sdpa_fused_dk32_causal" : "sdpa_fused_dk32");
-    } else if (dk <= 64) {
-        rc = launch_sdpa<64>(Q, K, V, O, L, BH, S, scale, causal, H, ld, ldo, (int)dk);
-        axhip::note_kernel(causal ? "sdpa_fused_dk64_causal" : "sdpa_fused_dk64");
-    } else if (dk <= 96) {
-        rc = launch_sdpa<96>(Q, K, V, O, L, BH, S, scale, causal, H, ld, ldo, (int)dk);
-        axhip::note_kernel(causal ? "sdpa_fused_dk96_causal" : "sdpa_fused_dk96");
-    } else {
-        rc = launch_sdpa<128>(Q, K, V, O, L, BH, S, scale, causal, H, ld, ldo, (int)dk);
-        axhip::note_kernel(causal ? "sdpa_fused_dk128_causal" : "sdpa_fused_dk128");
-    }
-    return rc;
+    auto run = [&](auto geometry) {
+        constexpr int DK = decltype(geometry)::value;
+        const bool few = few_tiles<DK>(BH, S, causal);
+        const int rc = few ? launch_sdpa_few<DK>(Q, K, V, O, L, BH, S, scale, causal, H, ld, ldo, (int)dk)
+                           : launch_sdpa<DK>(Q, K, V, O, L, BH, S, scale, causal, H, ld, ldo, (int)dk);
+        axhip::note_kernel(sdpa_name(DK, causal, few));
+        return rc;
+    };
+    if (dk <= 32) return run(std::integral_constant<int, 32>());
+    if (dk <= 64) return run(std::integral_constant<int, 64>());
+    if (dk <= 96) return run(std::integral_constant<int, 96>());
+    return run(std::integral_constant<int, 128>());
 }
 
 extern "C" int axhip_sdpa_fwd(const float *Q, const float *K, const float *V, float *O, float *L, int64_t BH,
