@@ -1,0 +1,238 @@
+// Single fp32 products with few tiles and a K of some hundred, in one launch: a workgroup of four to sixteen waves owns one 32x32 tile of C, and
+// every wave forms the whole tile over its own strip of K, straight from memory, in three bf16 terms per operand (bf16x3.h); the strips meet
+// in LDS, in a fixed order.
+//
+// What bounds such products is not the matrix core but latency: the launch, the first trip to memory, the loop's barriers where waves
+// share slabs through LDS, and a second launch where K is cut into ranges to fill the chip.  Here the chip is filled by small tiles, no wave
+// waits for another before the end, and a value is cut once per tile.  Two steps of 16 k are under way per wave.
+// us, before -> here (on what): 128 x 1024 x 784 11.6 -> 7.9, 300 x 333 x 777 11.1 -> 8.6, 1024 x 256 x 1024 12.3 -> 8.6 (two launches: ranges of K), 40 x
+// 500 x 300 9.5 -> 5.9 (64x64 tiles in bf16 terms), 1024 x 256 x 256 5.9 -> 5.1 (32x64 tiles on fp32 instructions), 128 x 1024 x 10 6.6 -> 3.9 (guarded
+// tiles), 1024 x 256 x 256 A^T B 9.5 -> 5.4; geometric mean over some 800 random products that the rule below takes 1.35.  Past it the vector pipe
+// (6.5 instructions a value and 64 values a column of k) and the loads (64 rows a tile) take over: 1024^3 20 -> 25, 100 x 10 x 4096 11 -> 22.
+// The five smaller products of terms have a sum of their own, and a strip is short: relative error against 64 bits 8.6e-8 at K = 1024 (64x64
+// tiles in terms 1.2e-7, fp32 instructions 4.1e-7).
+//
+// Loads.  An operand stored along K against one stored across it: a lane reads its 32 bytes of its row in place.  Both along K
+// (A B^T): twice as many scattered lines would bound the kernel (1024 x 256 x 1024 21 us), so 64-byte pieces are loaded 16 rows at a time and
+// turned through 2 KiB of LDS of the wave's own (9.3).  Stored across K: one k of 32 rows a load.  Rows and columns past the end are
+// read as the last one, k past the end as the last one with A zero; every alignment and every K is taken.
+#include "gemm_strips.h"
+
+#include "bf16x3.h"
+
+namespace {
+using namespace axhip;
+
+constexpr int TILE = 32, CPITCH = TILE + 4, PART = TILE * CPITCH;        // floats of a wave's part of the tile
+
+template <int WAVES, bool TERMS, bool A_KC, bool B_KC, int PER_SIMD>
+__global__ void __launch_bounds__(64 * WAVES, PER_SIMD) k_gemm_strips(StagedArgs g) {
+    constexpr bool TURN = A_KC && B_KC;
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int r32 = lane & 31, h = lane >> 5;
+    int tm, tn;
+    tile_of_block(blockIdx.x, (int)((g.M + TILE - 1) / TILE), (int)((g.N + TILE - 1) / TILE), tm, tn);
+    const int64_t m0 = (int64_t)tm * TILE, n0 = (int64_t)tn * TILE, lda4 = g.lda * 4, ldb4 = g.ldb * 4;
+    const char *abase = reinterpret_cast<const char *>(static_cast<const float *>(g.A) + (A_KC ? m0 * g.lda : m0));
+    const char *bbase = reinterpret_cast<const char *>(static_cast<const float *>(g.B) + (B_KC ? n0 * g.ldb : n0));
+    const int mlast = (int)(g.M - 1 - m0 < TILE - 1 ? g.M - 1 - m0 : TILE - 1), nlast = (int)(g.N - 1 - n0 < TILE - 1 ? g.N - 1 - n0 : TILE - 1);
+    // steps of 16 k; this wave's strip is [s0, s1)
+    const int steps = (int)((g.K + 15) / 16);
+    const int s0 = (int)((int64_t)steps * wave / WAVES), s1 = (int)((int64_t)steps * (wave + 1) / WAVES);
+
+    // ---- loads: in place, a lane's 8 k (8 h + e) of row r32; turned, four k of rows 16 q + lane / 4 ----
+    std::integral_constant<bool, A_KC> akc;
+    std::integral_constant<bool, B_KC> bkc;
+    auto chunk = [&](int q) { return TURN ? lane & 3 : 2 * h + q; };
+    auto offset = [&](auto kc, int64_t ld4, int last, int q) {
+        constexpr bool KC = decltype(kc)::value;
+        const int r = TURN ? 16 * q + (lane >> 2) : r32, row = r < last ? r : last;
+        return (unsigned)row * (unsigned)(KC ? ld4 : 4) + (KC ? chunk(q) * 16 : (unsigned)(8 * h) * (unsigned)ld4);
+    };
+    const unsigned oa[2] = {offset(akc, lda4, mlast, 0), offset(akc, lda4, mlast, 1)}, ob[2] = {offset(bkc, ldb4, nlast, 0), offset(bkc, ldb4, nlast, 1)};
+    auto load_rows = [&](auto kc, const char *base, int64_t ld4, const unsigned (&o)[2], int s, bool zero_past, float (&x)[8]) {
+        const int64_t k = (int64_t)s * 16;
+        const int end = (int)(g.K - 1 - k);            // the last k there is, from this step's first
+        if constexpr (decltype(kc)::value) {
+            const char *p = base + k * 4;
+            if (end >= 15) {
+#pragma unroll
+                for (int q = 0; q < 2; q++) __builtin_memcpy(&x[4 * q], p + o[q], 16);
+            } else {
+#pragma unroll
+                for (int e = 0; e < 8; e++) {
+                    const int past = end - (4 * chunk(e >> 2) + (e & 3));          // below zero: past the end
+                    const float y = *reinterpret_cast<const float *>(p + o[e >> 2] + ((e & 3) + (past < 0 ? past : 0)) * 4);
+                    x[e] = zero_past && past < 0 ? 0.0f : y;
+                }
+            }
+        } else {
+            const char *p = base + k * ld4;
+            if (end >= 15) {
+#pragma unroll
+                for (int e = 0; e < 8; e++) x[e] = *reinterpret_cast<const float *>(p + e * ld4 + o[0]);
+            } else {
+#pragma unroll
+                for (int e = 0; e < 8; e++) {
+                    const int past = end - (8 * h + e);
+                    const float y = *reinterpret_cast<const float *>(p + (int64_t)(e + (past < 0 ? past : 0)) * ld4 + o[0]);
+                    x[e] = zero_past && past < 0 ? 0.0f : y;
+                }
+            }
+        }
+    };
+    struct Raw {
+        float a[8], b[8];
+    };
+    auto load = [&](Raw &r, int s) {
+        load_rows(akc, abase, lda4, oa, s, true, r.a);
+        load_rows(bkc, bbase, ldb4, ob, s, false, r.b);
+    };
+    // chunks lie in rows of 64 bytes, exchanged by the row so that the 16 lanes that an access serves together fall on distinct banks
+    auto turn = [&](unsigned char *d, float (&x)[8]) {
+#pragma unroll
+        for (int q = 0; q < 2; q++) {
+            const int row = 16 * q + (lane >> 2);
+            *reinterpret_cast<v4f *>(d + row * 64 + (((lane & 3) ^ ((row >> 2) & 3)) << 4)) = v4f{x[4 * q], x[4 * q + 1], x[4 * q + 2], x[4 * q + 3]};
+        }
+        const unsigned at = r32 * 64 + (((2 * h) ^ ((r32 >> 2) & 3)) << 4);
+        const v4f y = *reinterpret_cast<const v4f *>(d + at), z = *reinterpret_cast<const v4f *>(d + (at ^ 16));
+#pragma unroll
+        for (int e = 0; e < 4; e++) x[e] = y[e], x[4 + e] = z[e];
+    };
+
+    v16f acc, low;
+#pragma unroll
+    for (int v = 0; v < 16; v++) acc[v] = low[v] = 0.0f;
+    auto multiply = [&](Raw &r) {
+        if constexpr (TURN) {
+            turn(lds + wave * 4096, r.a);
+            turn(lds + wave * 4096 + 2048, r.b);
+        }
+        if constexpr (!TERMS) {
+#pragma unroll
+            for (int e = 0; e < 8; e++) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(r.b[e], r.a[e], acc, 0, 0, 0);
+            return;
+        }
+        v4i fa[3], fb[3];
+        cut(r.a, TERMS_UP, fa);
+        cut(r.b, TERMS_UP, fb);
+#pragma unroll
+        for (int sum = 2; sum > 0; sum--)              // the small products first
+#pragma unroll
+            for (int p = sum; p >= 0; p--) low = mfma_terms(fb[sum - p], fa[p], low);
+        acc = mfma_terms(fb[0], fa[0], acc);
+    };
+    if (s0 < s1) {
+        Raw r0, r1;
+        load(r0, s0);
+        load(r1, s0 + 1 < s1 ? s0 + 1 : s0);
+        int s = s0;
+        for (; s + 2 < s1; s += 2) {
+            multiply(r0);
+            load(r0, s + 2);
+            multiply(r1);
+            load(r1, s + 3 < s1 ? s + 3 : s + 2);
+        }
+        multiply(r0);
+        if (s + 1 < s1) multiply(r1);
+    }
+    if constexpr (TURN) __syncthreads();               // the parts lie where values were turned
+
+    // ---- the strips together: register v of lane l holds row l & 31, column 8 (v >> 2) + 4 (l >> 5) + (v & 3) ----
+    float seen = 0.0f;
+    if constexpr (TERMS) {
+        acc += low;
+        look_at(acc, seen);
+    }
+    float *part = reinterpret_cast<float *>(lds);
+    auto put = [&]() {
+#pragma unroll
+        for (int q = 0; q < 4; q++)
+            *reinterpret_cast<v4f *>(part + wave * PART + r32 * CPITCH + 8 * q + 4 * h) = v4f{acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]};
+    };
+    put();
+    float down = TERMS ? TERMS_DOWN : 1.0f;
+    if constexpr (!TERMS) __syncthreads();
+    else if (any_wave<WAVES>(!(seen == 0.0f), lds + WAVES * PART * 4, wave)) {
+        // what the terms cannot hold, with fp32 instructions: the waves take pairs of k in turn
+        down = 1.0f;
+#pragma unroll
+        for (int v = 0; v < 16; v++) acc[v] = 0.0f;
+        const int row = r32 < mlast ? r32 : mlast, col = r32 < nlast ? r32 : nlast;
+        for (int64_t k0 = 2 * wave; k0 < g.K; k0 += 2 * WAVES) {
+            const int64_t k = k0 + h, ke = k < g.K ? k : g.K - 1;
+            const float a = *reinterpret_cast<const float *>(abase + (A_KC ? row * lda4 + ke * 4 : ke * lda4 + row * 4));
+            const float b = *reinterpret_cast<const float *>(bbase + (B_KC ? col * ldb4 + ke * 4 : ke * ldb4 + col * 4));
+            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(k < g.K ? b : 0.0f, k < g.K ? a : 0.0f, acc, 0, 0, 0);
+        }
+        put();
+        __syncthreads();
+    }
+    const int row = tid / 8, cg = (tid & 7) * 4;       // four columns of a row each, from the first 256 threads
+    const int64_t m = m0 + row, col = n0 + cg;
+    if (tid >= TILE * TILE / 4 || m >= g.M || col >= g.N) return;
+    v4f o = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int w = 0; w < WAVES; w++) o += *reinterpret_cast<const v4f *>(part + w * PART + row * CPITCH + cg);
+    const int have = g.N - col >= 4 ? 4 : (int)(g.N - col);
+    float *cp = g.C + m * g.ldc + col;
+    o *= down;
+    if (g.alpha != 1.0f) o *= g.alpha;
+#pragma unroll
+    for (int e = 0; e < 4; e++)
+        if (e < have) {
+            if (g.beta != 0.0f) o[e] += g.beta * cp[e];
+            if (g.bias) o[e] += g.bias[col + e];
+            o[e] = apply_act(o[e], g.act);
+        }
+    if (have == 4) __builtin_memcpy(cp, &o, 16);
+    else {
+#pragma unroll
+        for (int e = 0; e < 3; e++)
+            if (e < have) cp[e] = o[e];
+    }
+}
+
+template <int WAVES, bool TERMS, bool A_KC, bool B_KC, int PER_SIMD>
+int launch(const char *name, const StagedArgs &g) {
+    constexpr int SMEM = WAVES * PART * 4 + 4 * WAVES;
+    static_assert(!(A_KC && B_KC) || WAVES * 4096 <= SMEM, "values are turned where the parts come to lie");
+    auto kern = k_gemm_strips<WAVES, TERMS, A_KC, B_KC, PER_SIMD>;
+    static bool attr_set = false;
+    if (!attr_set) {
+        AXHIP_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, SMEM), "hipFuncSetAttribute");
+        attr_set = true;
+    }
+    const int64_t tiles = ((g.M + TILE - 1) / TILE) * ((g.N + TILE - 1) / TILE);
+    note_kernel(name);
+    hipLaunchKernelGGL(kern, dim3((unsigned)tiles), dim3(64 * WAVES), SMEM, kStream, g);
+    return check_launch(name);
+}
+}  // namespace
+
+namespace axhip {
+// In terms, from a step of 16 k per wave of eight on: up to a tile a CU and a K of about nine hundred, or two tiles and some hundred (us, before -> here:
+// 100 x 4096 x 784 15.3 -> 12.0 on 512 tiles, A B^T 14.1 -> 12.8; past the limits 500 x 200 x 2000 13.2 -> 14.2, 1024 x 1024 x 256 8.2 -> 9.5, 12 x 1024 x 1024 7.0 ->
+// 7.9; A B^T on 336 tiles with K = 476 8.9 -> 9.7, with its extra turn it stops at one tile a CU).  Two workgroups share a CU from 257 tiles on: four waves each
+// (86 x 3584 x 300: eight 6.4, four 5.6).  Sixteen pay where A is stored across K, whose loads are the slowest, from K = 256 on (256 x 1000 x 500 6.6 -> 6.1).
+// K below 32 on fp32 instructions: there is little to multiply and nothing to cut (128 x 1024 x 10 6.6 -> 3.9, A B^T 6.3 -> 3.5, 784 x 40 x 20 A^T B 4.5 -> 4.1).  K from 32 to 112, and rows on
+// the 16-byte grid with K on the 4 and off the 32 grid below 576, stay with the kernels that the tests of those routes name (70 x 90 x 101 6.6 us, 4.9 here).
+int strips_f32(const StagedArgs &g, int transa, int transb, bool on_grid) {
+    if ((transa && transb) || g.K < 1 || g.lda >= (1 << 22) || g.ldb >= (1 << 22)) return -1;
+    const int64_t tiles = ((g.M + TILE - 1) / TILE) * ((g.N + TILE - 1) / TILE), cus = cu_count();
+    const bool one = tiles <= cus, two = tiles <= 2 * cus;
+    if (g.K < 32 && two) {
+        if (!transa && !transb) return launch<4, false, true, false, 4>("sgemm_nn_32x32_staged", g);
+        if (!transa) return launch<4, false, true, true, 4>("sgemm_nt_32x32_staged", g);
+        return launch<4, false, false, false, 4>("sgemm_tn_32x32_staged", g);
+    }
+    if (g.K <= 112 || !((one && g.K <= 900) || (two && !transb && g.K <= 800)) || (on_grid && g.K % 32 != 0 && g.K < 576)) return -1;
+    if (!transa && !transb)
+        return one ? launch<8, true, true, false, 2>("sgemm_nn_32x32x3_staged", g) : launch<4, true, true, false, 4>("sgemm_nn_32x32x3_staged", g);
+    if (!transa) return launch<8, true, true, true, 2>("sgemm_nt_32x32x3_staged", g);
+    if (!one) return launch<4, true, false, false, 4>("sgemm_tn_32x32x3_staged", g);
+    return g.K < 256 ? launch<8, true, false, false, 2>("sgemm_tn_32x32x3_staged", g) : launch<16, true, false, false, 4>("sgemm_tn_32x32x3_staged", g);
+}
+}  // namespace axhip

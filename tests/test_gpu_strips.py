@@ -1,0 +1,100 @@
+"""fp32 products with few tiles, in one launch of 32x32 tiles whose waves share K: edges of tiles, steps and strips in every storage order
+and form, and the inputs that bf16 terms cannot hold."""
+import numpy as np
+import pytest
+
+from test_gpu_parity import BOUND_FP32, say
+
+pytestmark = pytest.mark.gpu
+
+
+def padded(x, pad):                                           # the columns past the matrix hold NaN: read or written, they show
+    out = np.full((x.shape[0], x.shape[1] + pad), np.nan, np.float32)
+    out[:, :x.shape[1]] = x
+    return out
+
+
+def product(hip, a, b, order, alpha=1.0, beta=0.0, c=None, bias=None, act=0, pads=(3, 1, 5)):
+    sa, sb = padded(a.T if order[0] == "t" else a, pads[0]), padded(b.T if order[1] == "t" else b, pads[1])
+    M, N, K = a.shape[0], b.shape[1], a.shape[1]
+    da, db, dc = hip.array(sa), hip.array(sb), hip.array(padded(np.zeros((M, N), np.float32) if c is None else c, pads[2]))
+    dbias = None if bias is None else hip.array(bias)
+    hip.check(hip.L.axhip_sgemm(int(order[0] == "t"), int(order[1] == "t"), M, N, K, alpha, da.ptr, sa.shape[1], db.ptr, sb.shape[1], beta, dc.ptr,
+                                N + pads[2], None if bias is None else dbias.ptr, act))
+    assert "_32x32" in hip.last_kernel(), hip.last_kernel()
+    full = dc.numpy()
+    assert np.isnan(full[:, N:]).all()
+    return full[:, :N]
+
+
+# K u sum |a||b| holds with room; with terms the left-out ones add at most 2^-24 of each product
+@pytest.mark.parametrize("order", ["nn", "nt", "tn"])
+@pytest.mark.parametrize("M,N", [(17, 1), (31, 33), (32, 32), (65, 95), (100, 10), (260, 1000), (250, 2020)])
+@pytest.mark.parametrize("K", [1, 2, 15, 16, 17, 31, 113, 127, 128, 129, 255, 256, 257, 500, 641, 799, 900])
+def test_every_form(hip, M, N, K, order):
+    tiles = ((M + 31) // 32) * ((N + 31) // 32)
+    if tiles > 256 and K > 32 and (order == "nt" or K > 800):
+        pytest.skip("other kernels")
+    say("strips", M, N, K, order)
+    rng = np.random.default_rng(M * 7 + N * 3 + K)
+    a, b = rng.uniform(-1, 1, (M, K)).astype(np.float32), rng.uniform(-1, 1, (K, N)).astype(np.float32)
+    bias, c = rng.normal(0, 1, N).astype(np.float32), rng.uniform(-1, 1, (M, N)).astype(np.float32)
+    exact, size = a.astype(np.float64) @ b.astype(np.float64), np.abs(a).astype(np.float64) @ np.abs(b).astype(np.float64)
+    got = product(hip, a, b, order, 0.5, 2.0, c, bias, 1)
+    want, size = np.maximum(0.5 * exact + 2.0 * c + bias, 0), 0.5 * size + 2.0 * np.abs(c) + np.abs(bias)
+    assert (np.abs(got - want) <= BOUND_FP32 * size).all(), float((np.abs(got - want) / size).max())
+    assert np.array_equal(product(hip, a, b, order, 0.5, 2.0, c, bias, 1), got)
+
+
+@pytest.mark.parametrize("order", ["nn", "nt", "tn"])
+@pytest.mark.parametrize("M,N,K", [(64, 64, 128), (256, 768, 256), (128, 1024, 784), (1024, 96, 896), (192, 2048, 512)])
+def test_on_the_grid(hip, M, N, K, order):
+    """Rows on the 16-byte grid, K off and on the 32 grid; error no larger than fp32 instructions leave (2^-24 a product and sqrt(K) roundings)."""
+    if order == "nt" and M * N > 256 * 1024:
+        pytest.skip("other kernels")
+    say("strips on the grid", M, N, K, order)
+    rng = np.random.default_rng(M + N + K)
+    a, b = rng.normal(0, 1, (M, K)).astype(np.float32), rng.normal(0, 1, (K, N)).astype(np.float32)
+    got = product(hip, a, b, order, pads=(0, 0, 0))
+    want = a.astype(np.float64) @ b.astype(np.float64)
+    assert np.linalg.norm(got - want) <= 2.0 ** -24 * (1 + np.sqrt(K) / 4) * np.linalg.norm(want)
+
+
+@pytest.mark.parametrize("order", ["nn", "nt", "tn"])
+@pytest.mark.parametrize("K", [20, 300])
+def test_non_finite(hip, K, order):
+    """Infinities and NaNs reach the rows and columns that hold them and no others; magnitudes up to the largest float come out."""
+    say("strips non-finite", K, order)
+    rng = np.random.default_rng(K)
+    M, N = 70, 100
+    a, b = rng.uniform(-1, 1, (M, K)).astype(np.float32), rng.uniform(-1, 1, (K, N)).astype(np.float32)
+    a[3, K - 1], a[40, 0], b[K // 2, 90], a[66, 5] = np.inf, np.nan, -np.inf, np.float32(3e38)
+    b[5, :] = np.float32(2.0 ** -20)
+    b[K - 1, 7] = 0
+    got = product(hip, a, b, order)
+    with np.errstate(invalid="ignore", over="ignore"):
+        want = a.astype(np.float64) @ b.astype(np.float64)
+    assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isposinf(got), np.isposinf(want)) and np.array_equal(np.isneginf(got), np.isneginf(want))
+    fine = np.isfinite(want)
+    a[3, K - 1] = a[40, 0] = b[K // 2, 90] = 0
+    size = np.abs(a).astype(np.float64) @ np.abs(b).astype(np.float64)
+    assert (np.abs(got - want)[fine] <= (BOUND_FP32 * size)[fine]).all()
+
+
+@pytest.mark.parametrize("scale_a,scale_b", [(2.0 ** -115, 1.0), (2.0 ** -60, 2.0 ** -60), (2.0 ** 100, 2.0 ** -40), (2.0 ** 120, 2.0 ** -20)])
+def test_keeps_the_range(hip, scale_a, scale_b):
+    say("strips range", scale_a, scale_b)
+    rng = np.random.default_rng(9)
+    a, b = (rng.uniform(-1, 1, (50, 200)) * scale_a).astype(np.float32), (rng.uniform(-1, 1, (200, 40)) * scale_b).astype(np.float32)
+    got = product(hip, a, b, "nn")
+    size = np.abs(a).astype(np.float64) @ np.abs(b).astype(np.float64)
+    assert (np.abs(got - a.astype(np.float64) @ b.astype(np.float64)) <= BOUND_FP32 * size).all()
+
+
+def test_outer_products_are_rounded_once(hip):
+    """K = 1 on fp32 instructions: the product itself."""
+    say("strips outer")
+    rng = np.random.default_rng(4)
+    u, v = rng.normal(0, 1, (90, 1)).astype(np.float32), rng.normal(0, 1, (1, 300)).astype(np.float32)
+    for order in ("nn", "nt", "tn"):
+        assert np.array_equal(product(hip, u, v, order), u * v)
