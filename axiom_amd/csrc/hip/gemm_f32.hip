@@ -1800,7 +1800,8 @@ int dispatch_f32(const SgemmArgs &g, int transa, int transb, int64_t batch, bool
     if (rc < 0 && !transa && transb && batch > 1 && free_choice && tuning().nt_walk == 0 && g.M >= 128 && nt_wide * batch >= cu_count() / 2 &&
         ((g.K > 32 && g.N > 128 && g.N <= 256) || nt_wide * 256 * 5 <= g.N * 8))
         rc = nt_terms(staged_args(g), batch);
-    if (!transa && !transb) rc = try_nn_stream(g, batch);
+    if (rc < 0 && !transa && !transb && batch > 1 && free_choice) rc = nn_terms(staged_args(g), batch);
+    if (rc < 0 && !transa && !transb) rc = try_nn_stream(g, batch);
     if (rc >= 0) return rc;
     if (!transa && !transb) rc = try_dma<true, false>(nn_d, g, batch);
     else if (!transa && transb) rc = try_dma<true, true>(nt_d, g, batch);

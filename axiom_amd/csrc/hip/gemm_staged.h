@@ -27,6 +27,8 @@ int staged_i8w(const StagedArgs &g);
 constexpr const char *kSplitTermsName = "sgemm_splitk_x3";
 // Batches of A * B^T with K = 32, 64, 96 or 128 in bf16 terms, B held in registers (gemm_nt_terms.hip).  -1: not taken.
 int nt_terms(const StagedArgs &g, int64_t batch);
+// Batches of A * B with N up to 32 or 65..128 in bf16 terms, a wave over all columns (gemm_nn_terms.hip).  -1: not taken.
+int nn_terms(const StagedArgs &g, int64_t batch);
 
 // Adds `splits` partial products [M, N] in order and applies alpha, beta, bias and activation (gemm_f32.hip).
 int splitk_finish(const float *part, int64_t splits, int64_t M, int64_t N, float alpha, float beta, const float *bias, int act,
