@@ -52,14 +52,14 @@ struct LnArgs {
     float eps;
 };
 
-// KIND 0: softmax, 1: layer norm.  Thread t of a row holds columns t, t + TPR, ...
+// KIND 0: softmax, 1: layer norm.  Thread t of a row holds columns t, t + TPR, ...  back: the last workgroup takes the first rows.
 template <int TPR, int VPT, int KIND>
 __global__ void __launch_bounds__(256)
-k_rows_cached(const float *in, float *out, int64_t rows, int cols, LnArgs ln) {
+k_rows_cached(const float *in, float *out, int64_t rows, int cols, LnArgs ln, bool back) {
     __shared__ float lds[8];
     constexpr int RPB = 256 / TPR;
     const int t = threadIdx.x % TPR, wave = threadIdx.x >> 6;
-    const int64_t row = (int64_t)blockIdx.x * RPB + threadIdx.x / TPR;
+    const int64_t row = (int64_t)(back ? gridDim.x - 1 - blockIdx.x : blockIdx.x) * RPB + threadIdx.x / TPR;
     if (TPR == 64 && row >= rows) return;        // whole waves leave; a workgroup row is never partial
     const float *x = in + row * cols;
     float v[VPT];
@@ -381,6 +381,11 @@ k_rows_short(const float *in, float *out, int64_t rows, int cols, LnArgs ln) {
 
 template <int KIND>
 int launch_rows(const float *in, float *out, int64_t rows, int64_t cols, const LnArgs &ln, const char *what) {
+    // A softmax over more than the 256 MiB memory-side cache walks its rows from the last to the first: what a product before it wrote last
+    // is still there, and what it writes last, the first rows, is what a product after it reads first.  us of such a chain, from the
+    // first -> from the last: 300 heads of 500 x 500 x 64 318 -> 292, 600 654 -> 582, 100 of 1000 x 1000 416 -> 384, 32 of 2048 x 2048
+    // 526 -> 511; level where whole lines go past the cache (512 of 512 x 512 451 and 451); 96 of 1000 x 1000 x 80 530 -> 533.
+    const bool back = KIND == 0 && rows * cols * 4 > (int64_t)256 << 20;
     if (cols <= 1024) {
         const int64_t blocks = (rows + 3) / 4;
         if (blocks > 0x7fffffff) return fail(AXHIP_ERR_SHAPE, "%s: too many rows", what);
@@ -389,18 +394,18 @@ int launch_rows(const float *in, float *out, int64_t rows, int64_t cols, const L
         else if (cols <= 128)
             hipLaunchKernelGGL((k_rows_short<2, 4, KIND>), dim3((unsigned)((rows + 15) / 16)), dim3(256), 0, kStream, in, out, rows, (int)cols, ln);
         else if (cols <= 256)
-            hipLaunchKernelGGL((k_rows_cached<64, 4, KIND>), dim3((unsigned)blocks), dim3(256), 0, kStream, in, out, rows, (int)cols, ln);
+            hipLaunchKernelGGL((k_rows_cached<64, 4, KIND>), dim3((unsigned)blocks), dim3(256), 0, kStream, in, out, rows, (int)cols, ln, back);
         else if (cols <= 512)
-            hipLaunchKernelGGL((k_rows_cached<64, 8, KIND>), dim3((unsigned)blocks), dim3(256), 0, kStream, in, out, rows, (int)cols, ln);
+            hipLaunchKernelGGL((k_rows_cached<64, 8, KIND>), dim3((unsigned)blocks), dim3(256), 0, kStream, in, out, rows, (int)cols, ln, back);
         else
-            hipLaunchKernelGGL((k_rows_cached<64, 16, KIND>), dim3((unsigned)blocks), dim3(256), 0, kStream, in, out, rows, (int)cols, ln);
+            hipLaunchKernelGGL((k_rows_cached<64, 16, KIND>), dim3((unsigned)blocks), dim3(256), 0, kStream, in, out, rows, (int)cols, ln, back);
     } else {
         if (rows > 0x7fffffff) return fail(AXHIP_ERR_SHAPE, "%s: too many rows", what);
         if (cols <= 4096) {
-            hipLaunchKernelGGL((k_rows_cached<256, 16, KIND>), dim3((unsigned)rows), dim3(256), 0, kStream, in, out, rows, (int)cols, ln);
+            hipLaunchKernelGGL((k_rows_cached<256, 16, KIND>), dim3((unsigned)rows), dim3(256), 0, kStream, in, out, rows, (int)cols, ln, back);
         } else if (cols <= 6144) {
             // still in registers (24 values a thread): faster than the LDS form up to here, slower from about 8192
-            hipLaunchKernelGGL((k_rows_cached<256, 24, KIND>), dim3((unsigned)rows), dim3(256), 0, kStream, in, out, rows, (int)cols, ln);
+            hipLaunchKernelGGL((k_rows_cached<256, 24, KIND>), dim3((unsigned)rows), dim3(256), 0, kStream, in, out, rows, (int)cols, ln, back);
         } else if (cols <= 36864) {
             static bool attr_set = false;
             if (!attr_set) {
