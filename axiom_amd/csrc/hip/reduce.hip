@@ -107,7 +107,8 @@ int reduce_rows(const float *in, int64_t rows, int64_t len, float *out) {
 
 // Column reductions of [outer, axis_len, inner], inner > 1.  A workgroup is TY axis positions
 // by TX column groups of VW columns; it walks a slice of the axis TY positions at a time and
-// joins its TY partial rows through LDS.  Slice s of `splits` writes out[(o*splits + s), :].
+// joins its TY partial rows through LDS: sums as a tree (TY steps in a row were a third of a small
+// sum's time), maxima and minima in ascending order.  Slice s of `splits` writes out[(o*splits + s), :].
 template <int OP, int VW>
 __global__ void __launch_bounds__(256)
 k_reduce_cols(const float *__restrict__ in, int64_t axis_len, int64_t inner, int tx_log2, int64_t col_blocks,
@@ -158,10 +159,23 @@ k_reduce_cols(const float *__restrict__ in, int64_t axis_len, int64_t inner, int
 #pragma unroll
     for (int e = 0; e < VW; e++) join[e * 256 + threadIdx.x] = acc[e];
     __syncthreads();
-    if (ty == 0 && col < inner) {
-        for (int y = 1; y < TY; y++)
+    if (OP == AXHIP_RED_SUM) {
+        for (int half = TY >> 1; half > 0; half >>= 1) {
+            if (ty < half)
 #pragma unroll
-            for (int e = 0; e < VW; e++) acc[e] = red_join<OP>(acc[e], join[e * 256 + (y << tx_log2) + tx]);
+                for (int e = 0; e < VW; e++) join[e * 256 + threadIdx.x] += join[e * 256 + threadIdx.x + (half << tx_log2)];
+            __syncthreads();
+        }
+    }
+    if (ty == 0 && col < inner) {
+        if (OP == AXHIP_RED_SUM) {
+#pragma unroll
+            for (int e = 0; e < VW; e++) acc[e] = join[e * 256 + tx];
+        } else {
+            for (int y = 1; y < TY; y++)
+#pragma unroll
+                for (int e = 0; e < VW; e++) acc[e] = red_join<OP>(acc[e], join[e * 256 + (y << tx_log2) + tx]);
+        }
         float *dst = out + (o * splits + s) * inner + col;
 #pragma unroll
         for (int e = 0; e < VW; e++) dst[e] = acc[e];
@@ -194,10 +208,14 @@ int launch_cols(const float *in, int64_t outer, int64_t axis_len, int64_t inner,
 
 template <int OP>
 int reduce_cols(const float *in, int64_t outer, int64_t axis_len, int64_t inner, float *out) {
-    // enough workgroups to stream from every CU: cut the axis when outer x column blocks is small
+    // Sums of up to a million values down an axis of up to 1024 (a bias gradient) in one launch: narrow column blocks bring enough threads
+    // to a column, and a second launch takes longer than its slices save (us, two launches -> one: 128 x 1024 6.3 -> 3.4, 512 x 512 6.3 -> 4.3,
+    // 1024 x 1000 6.3 -> 4.0; from 2048 on the slices' sums have the smaller error, 2.9e-9 against 3.3e-9).
+    const bool one = OP == AXHIP_RED_SUM && axis_len <= 1024 && outer * axis_len * inner <= (int64_t)1 << 20;
+    // else enough workgroups to stream from every CU: cut the axis when outer x column blocks is small
     const int64_t groups = (inner + 3) / 4, col_blocks = (groups + 255) / 256;
     int64_t splits = 1;
-    if (outer * col_blocks < 2048) {
+    if (!one && outer * col_blocks < 2048) {
         splits = 2048 / (outer * col_blocks);
         const int64_t most = axis_len / (axis_len >= 8192 ? 32 : 64);       // rows per slice, at least
         if (splits > most) splits = most;
