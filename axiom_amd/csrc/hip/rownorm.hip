@@ -389,7 +389,13 @@ int launch_rows(const float *in, float *out, int64_t rows, int64_t cols, const L
     if (cols <= 1024) {
         const int64_t blocks = (rows + 3) / 4;
         if (blocks > 0x7fffffff) return fail(AXHIP_ERR_SHAPE, "%s: too many rows", what);
-        if (cols <= 64)
+        // few rows: the butterflies of a wave's rows run one after the other, so a wave takes one (us at 128 x 10, softmax 5.7 -> 3.5,
+        // 16384 x 64 6.4 -> 4.4, 8192 x 128 4.5 -> 3.5; 65536 x 128 14.3 -> 15.5)
+        if (cols <= 64 && rows <= 16384)
+            hipLaunchKernelGGL((k_rows_short<1, 1, KIND>), dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, kStream, in, out, rows, (int)cols, ln);
+        else if (cols <= 128 && rows <= 16384)
+            hipLaunchKernelGGL((k_rows_short<2, 1, KIND>), dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, kStream, in, out, rows, (int)cols, ln);
+        else if (cols <= 64)
             hipLaunchKernelGGL((k_rows_short<1, 8, KIND>), dim3((unsigned)((rows + 31) / 32)), dim3(256), 0, kStream, in, out, rows, (int)cols, ln);
         else if (cols <= 128)
             hipLaunchKernelGGL((k_rows_short<2, 4, KIND>), dim3((unsigned)((rows + 15) / 16)), dim3(256), 0, kStream, in, out, rows, (int)cols, ln);
