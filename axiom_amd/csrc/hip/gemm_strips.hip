@@ -9,8 +9,8 @@
 // 500 x 300 9.5 -> 5.9 (64x64 tiles in bf16 terms), 1024 x 256 x 256 5.9 -> 5.1 (32x64 tiles on fp32 instructions), 128 x 1024 x 10 6.6 -> 3.9 (guarded
 // tiles), 1024 x 256 x 256 A^T B 9.5 -> 5.4; geometric mean over some 800 random products that the rule below takes 1.35.  Past it the vector pipe
 // (6.5 instructions a value and 64 values a column of k) and the loads (64 rows a tile) take over: 1024^3 20 -> 25, 100 x 10 x 4096 11 -> 22.
-// The five smaller products of terms have a sum of their own, and a strip is short: relative error against 64 bits 8.6e-8 at K = 1024 (64x64
-// tiles in terms 1.2e-7, fp32 instructions 4.1e-7).
+// The five smaller products of terms have a sum of their own, the others two in turn, and the strips are added in pairs: relative error against
+// 64 bits 7.4e-8 at K = 1024 (ranges of K in terms 7.6e-8, 64x64 tiles in terms 1.2e-7, fp32 instructions 4.1e-7).
 //
 // Loads.  An operand stored along K against one stored across it: a lane reads its 32 bytes of its row in place.  Both along K
 // (A B^T): twice as many scattered lines would bound the kernel (1024 x 256 x 1024 21 us), so 64-byte pieces are loaded 16 rows at a time and
@@ -102,10 +102,12 @@ __global__ void __launch_bounds__(64 * WAVES, PER_SIMD) k_gemm_strips(StagedArgs
         for (int e = 0; e < 4; e++) x[e] = y[e], x[4 + e] = z[e];
     };
 
-    v16f acc, low;
+    // steps in turn into two sums, where there are registers for them
+    constexpr bool TURNS = TERMS && PER_SIMD <= 2;
+    v16f acc, other, low;
 #pragma unroll
-    for (int v = 0; v < 16; v++) acc[v] = low[v] = 0.0f;
-    auto multiply = [&](Raw &r) {
+    for (int v = 0; v < 16; v++) acc[v] = other[v] = low[v] = 0.0f;
+    auto multiply = [&](Raw &r, v16f &acc) {
         if constexpr (TURN) {
             turn(lds + wave * 4096, r.a);
             turn(lds + wave * 4096 + 2048, r.b);
@@ -130,19 +132,20 @@ __global__ void __launch_bounds__(64 * WAVES, PER_SIMD) k_gemm_strips(StagedArgs
         load(r1, s0 + 1 < s1 ? s0 + 1 : s0);
         int s = s0;
         for (; s + 2 < s1; s += 2) {
-            multiply(r0);
+            multiply(r0, acc);
             load(r0, s + 2);
-            multiply(r1);
+            multiply(r1, TURNS ? other : acc);
             load(r1, s + 3 < s1 ? s + 3 : s + 2);
         }
-        multiply(r0);
-        if (s + 1 < s1) multiply(r1);
+        multiply(r0, acc);
+        if (s + 1 < s1) multiply(r1, TURNS ? other : acc);
     }
     if constexpr (TURN) __syncthreads();               // the parts lie where values were turned
 
     // ---- the strips together: register v of lane l holds row l & 31, column 8 (v >> 2) + 4 (l >> 5) + (v & 3) ----
     float seen = 0.0f;
     if constexpr (TERMS) {
+        if constexpr (TURNS) acc += other;
         acc += low;
         look_at(acc, seen);
     }
@@ -173,9 +176,14 @@ __global__ void __launch_bounds__(64 * WAVES, PER_SIMD) k_gemm_strips(StagedArgs
     const int row = tid / 8, cg = (tid & 7) * 4;       // four columns of a row each, from the first 256 threads
     const int64_t m = m0 + row, col = n0 + cg;
     if (tid >= TILE * TILE / 4 || m >= g.M || col >= g.N) return;
-    v4f o = {0.f, 0.f, 0.f, 0.f};
+    v4f p[WAVES];                                      // added in pairs (sixteen in a row: error 8.9e-8 at K = 1024)
 #pragma unroll
-    for (int w = 0; w < WAVES; w++) o += *reinterpret_cast<const v4f *>(part + w * PART + row * CPITCH + cg);
+    for (int w = 0; w < WAVES; w++) p[w] = *reinterpret_cast<const v4f *>(part + w * PART + row * CPITCH + cg);
+#pragma unroll
+    for (int by = 1; by < WAVES; by *= 2)
+#pragma unroll
+        for (int w = 0; w < WAVES; w += 2 * by) p[w] += p[w + by];
+    v4f o = p[0];
     const int have = g.N - col >= 4 ? 4 : (int)(g.N - col);
     float *cp = g.C + m * g.ldc + col;
     o *= down;
@@ -213,10 +221,11 @@ int launch(const char *name, const StagedArgs &g) {
 }  // namespace
 
 namespace axhip {
-// In terms, from a step of 16 k per wave of eight on: up to a tile a CU and a K of about nine hundred, or two tiles and some hundred (us, before -> here:
+// In terms, from a step of 16 k per wave of eight on: up to a tile a CU and a K of nine hundred to fifteen hundred, or two tiles and some hundred (us, before -> here:
 // 100 x 4096 x 784 15.3 -> 12.0 on 512 tiles, A B^T 14.1 -> 12.8; past the limits 500 x 200 x 2000 13.2 -> 14.2, 1024 x 1024 x 256 8.2 -> 9.5, 12 x 1024 x 1024 7.0 ->
 // 7.9; A B^T on 336 tiles with K = 476 8.9 -> 9.7, with its extra turn it stops at one tile a CU).  Two workgroups share a CU from 257 tiles on: four waves each
-// (86 x 3584 x 300: eight 6.4, four 5.6).  Sixteen pay where A is stored across K, whose loads are the slowest, from K = 256 on (256 x 1000 x 500 6.6 -> 6.1).
+// (86 x 3584 x 300: eight 6.4, four 5.6).  Sixteen pay where A is stored across K, whose loads are the slowest, above K = 256 (256 x 1000 x 500 6.6 -> 6.1;
+// 250 x 500 x 256 4.5 -> 5.2).
 // K below 32 on fp32 instructions: there is little to multiply and nothing to cut (128 x 1024 x 10 6.6 -> 3.9, A B^T 6.3 -> 3.5, 784 x 40 x 20 A^T B 4.5 -> 4.1).  K from 32 to 112, and rows on
 // the 16-byte grid with K on the 4 and off the 32 grid below 576, stay with the kernels that the tests of those routes name (70 x 90 x 101 6.6 us, 4.9 here).
 int strips_f32(const StagedArgs &g, int transa, int transb, bool on_grid) {
@@ -228,11 +237,15 @@ int strips_f32(const StagedArgs &g, int transa, int transb, bool on_grid) {
         if (!transa) return launch<4, false, true, true, 4>("sgemm_nt_32x32_staged", g);
         return launch<4, false, false, false, 4>("sgemm_tn_32x32_staged", g);
     }
-    if (g.K <= 112 || !((one && g.K <= 900) || (two && !transb && g.K <= 800)) || (on_grid && g.K % 32 != 0 && g.K < 576)) return -1;
+    // Longer K, us: 256 x 768 x 1024 11.8 -> 8.2, A B^T 11.8 -> 8.9, 500 x 100 x 1000 10.0 -> 8.4, 100 x 10 x 1024 8.7 -> 7.6, 1000 x 128 x 1536 11.6 -> 10.6; 64 x 64 x
+    // 1024 7.4 -> 7.7, 128 x 100 x 1024 A B^T 8.0 -> 8.5, 128 x 512 x 1280 9.3 -> 9.4, 1000 x 128 x 2048 12.6 -> 12.8.
+    const bool ragged = g.M % TILE != 0 || g.N % TILE != 0;
+    const int64_t most = g.M < 96 ? 900 : tiles >= 128 ? (transb ? 1280 : 1536) : tiles > 24 || (!transb && tiles <= 8 && ragged) ? 1024 : 900;
+    if (g.K <= 112 || !((one && g.K <= most) || (two && !transb && g.K <= 800)) || (on_grid && g.K % 32 != 0 && g.K < 576)) return -1;
     if (!transa && !transb)
         return one ? launch<8, true, true, false, 2>("sgemm_nn_32x32x3_staged", g) : launch<4, true, true, false, 4>("sgemm_nn_32x32x3_staged", g);
     if (!transa) return launch<8, true, true, true, 2>("sgemm_nt_32x32x3_staged", g);
     if (!one) return launch<4, true, false, false, 4>("sgemm_tn_32x32x3_staged", g);
-    return g.K < 256 ? launch<8, true, false, false, 2>("sgemm_tn_32x32x3_staged", g) : launch<16, true, false, false, 4>("sgemm_tn_32x32x3_staged", g);
+    return g.K <= 256 ? launch<8, true, false, false, 2>("sgemm_tn_32x32x3_staged", g) : launch<16, true, false, false, 4>("sgemm_tn_32x32x3_staged", g);
 }
 }  // namespace axhip

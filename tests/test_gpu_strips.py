@@ -60,6 +60,19 @@ def test_on_the_grid(hip, M, N, K, order):
     assert np.linalg.norm(got - want) <= 2.0 ** -24 * (1 + np.sqrt(K) / 4) * np.linalg.norm(want)
 
 
+@pytest.mark.parametrize("order,M,N,K", [("nn", 100, 10, 1024), ("tn", 97, 31, 1000), ("nn", 97, 250, 901), ("nt", 250, 100, 1023), ("tn", 96, 257, 1024),
+                                         ("nt", 500, 255, 1280), ("nn", 256, 1000, 1536), ("tn", 510, 500, 1535)])
+def test_longer_k(hip, order, M, N, K):
+    say("strips of a longer K", M, N, K, order)
+    rng = np.random.default_rng(M + N + K)
+    a, b = rng.normal(0, 1, (M, K)).astype(np.float32), rng.normal(0, 1, (K, N)).astype(np.float32)
+    got = product(hip, a, b, order, 0.5, pads=(0, 0, 0)) * 2
+    want = a.astype(np.float64) @ b.astype(np.float64)
+    assert np.linalg.norm(got - want) <= 2.0 ** -24 * (1 + np.sqrt(K) / 4) * np.linalg.norm(want)
+    size = np.abs(a).astype(np.float64) @ np.abs(b).astype(np.float64)
+    assert (np.abs(got - want) <= BOUND_FP32 * size).all()
+
+
 @pytest.mark.parametrize("order", ["nn", "nt", "tn"])
 @pytest.mark.parametrize("K", [20, 300])
 def test_non_finite(hip, K, order):
