@@ -15,7 +15,8 @@
 // Loads.  An operand stored along K against one stored across it: a lane reads its 32 bytes of its row in place.  Both along K
 // (A B^T): twice as many scattered lines would bound the kernel (1024 x 256 x 1024 21 us), so 64-byte pieces are loaded 16 rows at a time and
 // turned through 2 KiB of LDS of the wave's own (9.3).  Stored across K: one k of 32 rows a load.  Rows and columns past the end are
-// read as the last one, k past the end as the last one with A zero; every alignment and every K is taken.
+// read as the last one, k past the end as the last one with A zero, and B too on fp32 instructions: zero times an infinity there would be
+// a NaN, which in terms shows in the sum and sends the tile through the second pass.  Every alignment and every K is taken.
 #include "gemm_strips.h"
 
 #include "bf16x3.h"
@@ -87,7 +88,7 @@ __global__ void __launch_bounds__(64 * WAVES, PER_SIMD) k_gemm_strips(StagedArgs
     };
     auto load = [&](Raw &r, int s) {
         load_rows(akc, abase, lda4, oa, s, true, r.a);
-        load_rows(bkc, bbase, ldb4, ob, s, false, r.b);
+        load_rows(bkc, bbase, ldb4, ob, s, !TERMS, r.b);
     };
     // chunks lie in rows of 64 bytes, exchanged by the row so that the 16 lanes that an access serves together fall on distinct banks
     auto turn = [&](unsigned char *d, float (&x)[8]) {

@@ -94,6 +94,24 @@ def test_non_finite(hip, K, order):
     assert (np.abs(got - want)[fine] <= (BOUND_FP32 * size)[fine]).all()
 
 
+@pytest.mark.parametrize("order", ["nn", "nt", "tn"])
+@pytest.mark.parametrize("K", [1, 2, 10, 15, 16, 17, 20, 31, 113, 300])
+def test_infinities_at_the_end_of_k(hip, K, order):
+    """The last k is what a step of 16 that hangs over K is filled with: an infinity there, in either operand, counts once."""
+    say("strips, infinities in the last k", K, order)
+    rng = np.random.default_rng(K)
+    M, N = 70, 100
+    a, b = rng.uniform(0.5, 1, (M, K)).astype(np.float32), rng.uniform(0.5, 1, (K, N)).astype(np.float32)
+    b[K - 1, 90], b[K - 1, 3], b[0, 64], a[41, K - 1], a[66, 0] = -np.inf, np.inf, np.inf, np.inf, -np.inf
+    a[9, K - 1] = 0
+    got = product(hip, a, b, order)
+    with np.errstate(invalid="ignore"):
+        want = a.astype(np.float64) @ b.astype(np.float64)
+    fine = np.isfinite(want)
+    assert fine.mean() > 0.9 and np.array_equal(got[~fine], want[~fine].astype(np.float32), equal_nan=True)
+    assert (np.abs(got[fine] - want[fine]) <= BOUND_FP32 * want[fine]).all()
+
+
 @pytest.mark.parametrize("scale_a,scale_b", [(2.0 ** -115, 1.0), (2.0 ** -60, 2.0 ** -60), (2.0 ** 100, 2.0 ** -40), (2.0 ** 120, 2.0 ** -20)])
 def test_keeps_the_range(hip, scale_a, scale_b):
     say("strips range", scale_a, scale_b)
