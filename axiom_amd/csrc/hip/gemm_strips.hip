@@ -151,13 +151,16 @@ __global__ void __launch_bounds__(64 * WAVES, PER_SIMD) k_gemm_strips(StagedArgs
         look_at(acc, seen);
     }
     float *part = reinterpret_cast<float *>(lds);
-    auto put = [&]() {
+    auto put = [&](float by) {
 #pragma unroll
         for (int q = 0; q < 4; q++)
-            *reinterpret_cast<v4f *>(part + wave * PART + r32 * CPITCH + 8 * q + 4 * h) = v4f{acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]};
+            *reinterpret_cast<v4f *>(part + wave * PART + r32 * CPITCH + 8 * q + 4 * h) =
+                v4f{acc[4 * q] * by, acc[4 * q + 1] * by, acc[4 * q + 2] * by, acc[4 * q + 3] * by};
     };
-    put();
-    float down = TERMS ? TERMS_DOWN : 1.0f;
+    // Strips that are finite in themselves may exceed the largest float together while they hold the factor of the terms: each gives up a
+    // WAVES-th of it first (exactly: nothing that reaches C is that small), the rest goes once they are added.
+    put(TERMS ? 1.0f / WAVES : 1.0f);
+    float down = TERMS ? TERMS_DOWN * WAVES : 1.0f;
     if constexpr (!TERMS) __syncthreads();
     else if (any_wave<WAVES>(!(seen == 0.0f), lds + WAVES * PART * 4, wave)) {
         // what the terms cannot hold, with fp32 instructions: the waves take pairs of k in turn
@@ -171,7 +174,7 @@ __global__ void __launch_bounds__(64 * WAVES, PER_SIMD) k_gemm_strips(StagedArgs
             const float b = *reinterpret_cast<const float *>(bbase + (B_KC ? col * ldb4 + ke * 4 : ke * ldb4 + col * 4));
             acc = __builtin_amdgcn_mfma_f32_32x32x2f32(k < g.K ? b : 0.0f, k < g.K ? a : 0.0f, acc, 0, 0, 0);
         }
-        put();
+        put(1.0f);
         __syncthreads();
     }
     const int row = tid / 8, cg = (tid & 7) * 4;       // four columns of a row each, from the first 256 threads

@@ -122,6 +122,19 @@ def test_keeps_the_range(hip, scale_a, scale_b):
     assert (np.abs(got - a.astype(np.float64) @ b.astype(np.float64)) <= BOUND_FP32 * size).all()
 
 
+# (order, M, N, K): forms of four, eight and sixteen waves
+@pytest.mark.parametrize("order,M,N,K", [("nn", 64, 64, 256), ("nt", 64, 64, 256), ("tn", 64, 64, 256), ("tn", 65, 97, 600), ("nn", 200, 100, 900),
+                                         ("nn", 192, 2048, 512), ("tn", 192, 2048, 512)])
+@pytest.mark.parametrize("power", [69, 71, 73, 75, 77, 79])
+def test_sums_of_one_sign_past_the_terms(hip, order, M, N, K, power):
+    """Strips whose own sums the terms hold (below 2^80) while their total is above it."""
+    say("strips, sums of one sign", M, N, K, order, power)
+    rng = np.random.default_rng(M + K + power)
+    a, b = (rng.uniform(0.5, 1, (M, K)) * 2.0 ** 37).astype(np.float32), (rng.uniform(0.5, 1, (K, N)) * 2.0 ** (power - 37)).astype(np.float32)
+    got, want = product(hip, a, b, order, pads=(0, 0, 0)), a.astype(np.float64) @ b.astype(np.float64)
+    assert (np.abs(got - want) <= BOUND_FP32 * want).all()
+
+
 def test_outer_products_are_rounded_once(hip):
     """K = 1 on fp32 instructions: the product itself."""
     say("strips outer")
