@@ -528,7 +528,9 @@ k_sdpa_few(const float *__restrict__ Q, const float *__restrict__ K, const float
         load_v(next);
     }
 
-    // ---- the waves' parts together ----
+    // ---- the waves' parts together, each at an eighth (exactly): outputs that are finite in themselves may exceed the largest float when
+    // four are added with the factors of the terms still in them ----
+    constexpr float PART_DOWN = 0.125f;
     float seen = l_run * 0.0f;
 #pragma unroll
     for (int d = 0; d < DT; d++) look_at(acc_o[d], seen);
@@ -536,7 +538,7 @@ k_sdpa_few(const float *__restrict__ Q, const float *__restrict__ K, const float
 #pragma unroll
     for (int d = 0; d < DT; d++)
 #pragma unroll
-        for (int g = 0; g < 4; g++) part[wave][d * 4 + g][lane] = v4f{acc_o[d][4 * g], acc_o[d][4 * g + 1], acc_o[d][4 * g + 2], acc_o[d][4 * g + 3]};
+        for (int g = 0; g < 4; g++) part[wave][d * 4 + g][lane] = v4f{acc_o[d][4 * g], acc_o[d][4 * g + 1], acc_o[d][4 * g + 2], acc_o[d][4 * g + 3]} * PART_DOWN;
     if (fhalf == 0) {
         ml[wave][0][frow] = m_run;
         ml[wave][1][frow] = l_wave;
@@ -569,7 +571,7 @@ k_sdpa_few(const float *__restrict__ Q, const float *__restrict__ K, const float
         return;
     }
     if (qg >= S) return;
-    const float inv = 1.0f / l_all * (1.0f / TERMS_UP);
+    const float inv = 1.0f / l_all * (1.0f / (TERMS_UP * PART_DOWN));
     for (int piece = wave; piece < PIECES; piece += WAVES) {
         v4f o = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll

@@ -48,3 +48,20 @@ def test_both_forms_on_the_same_heads(hip, S, dk, causal):
         fine = np.isfinite(o)
         assert (np.abs(o.astype(np.float64) - om[n]) / size)[fine].max() <= 2 * SDPA_TOL
         assert np.nanmax(np.abs(l - lm[n])) <= 2e-5 * max(1.0, np.nanmax(np.abs(l)))
+
+
+@pytest.mark.parametrize("BH,S,dk", [(6, 64, 20), (6, 128, 64), (3, 161, 80), (3, 512, 128)])
+@pytest.mark.parametrize("causal", [0, 1])
+@pytest.mark.parametrize("power", [70, 72, 73, 74, 75, 76, 78, 80])
+def test_values_of_one_sign_past_the_terms(hip, BH, S, dk, causal, power):
+    """Waves whose own sums the terms hold while those of all four are above what they hold; scores near each other, so that all of them count."""
+    say("sdpa few, values of one sign", BH, S, dk, causal, power)
+    rng = np.random.default_rng(S + dk + power)
+    q, k = (rng.uniform(-0.5, 0.5, (BH, S, dk)).astype(np.float32) for _ in range(2))
+    v = rng.uniform(0.5, 1, (BH, S, dk)).astype(np.float32)
+    v[0, :, 0] = 1
+    o, l = run_sdpa(hip, q, k, v * np.float32(2.0 ** power), 0.05, causal)
+    assert "few" in hip.last_kernel()
+    want, lse = attention(q, k, v, np.float32(0.05), causal)
+    assert np.abs(o.astype(np.float64) / 2.0 ** power - want).max() <= SDPA_TOL
+    assert np.abs(l - lse).max() <= 1e-5 * max(1.0, np.abs(lse).max())
