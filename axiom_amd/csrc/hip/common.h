@@ -163,6 +163,13 @@ __device__ __forceinline__ void wave_sum_spread(T (&v)[NV], int lane) {
     }
 }
 
+// Between writes and reads (or reads and later writes) of LDS through which the lanes of one wave hand each other values.  The hardware
+// keeps a wave's accesses in order; the compiler, which sees one lane's addresses, must not exchange them.
+__device__ __forceinline__ void order_in_wave() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
 // Write-back of one 32x32 MFMA result tile held in the layout "lane l owns row (l & 31), and
 // for g = 0..3 the four consecutive columns 8*g + 4*(l >> 5) + e": the wave turns the tile
 // through 4 KiB of LDS private to it so that each store instruction writes 8 rows of 128

@@ -126,6 +126,7 @@ __global__ void __launch_bounds__(64 * WAVES, NB == 1 ? 3 : 2) k_nn_terms(Staged
             const int row = 8 * q + (lane >> 3);
             *reinterpret_cast<v4f *>(turn + row * 128 + (((lane & 7) ^ ((row >> 1) & 7)) << 4)) = v4f{x[4 * q], x[4 * q + 1], x[4 * q + 2], x[4 * q + 3]};
         }
+        order_in_wave();                               // (the next writes come after a barrier of the workgroup)
 #pragma unroll
         for (int s = 0; s < 2; s++) {                  // k 16 s + 8 h + e
             const unsigned at = r32 * 128 + (((4 * s + 2 * h) ^ ((r32 >> 1) & 7)) << 4);

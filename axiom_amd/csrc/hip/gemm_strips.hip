@@ -91,16 +91,23 @@ __global__ void __launch_bounds__(64 * WAVES, PER_SIMD) k_gemm_strips(StagedArgs
         load_rows(bkc, bbase, ldb4, ob, s, !TERMS, r.b);
     };
     // chunks lie in rows of 64 bytes, exchanged by the row so that the 16 lanes that an access serves together fall on distinct banks
-    auto turn = [&](unsigned char *d, float (&x)[8]) {
+    auto turn = [&](unsigned char *d, float (&a)[8], float (&b)[8]) {
 #pragma unroll
         for (int q = 0; q < 2; q++) {
             const int row = 16 * q + (lane >> 2);
-            *reinterpret_cast<v4f *>(d + row * 64 + (((lane & 3) ^ ((row >> 2) & 3)) << 4)) = v4f{x[4 * q], x[4 * q + 1], x[4 * q + 2], x[4 * q + 3]};
+            const unsigned at = row * 64 + (((lane & 3) ^ ((row >> 2) & 3)) << 4);
+            *reinterpret_cast<v4f *>(d + at) = v4f{a[4 * q], a[4 * q + 1], a[4 * q + 2], a[4 * q + 3]};
+            *reinterpret_cast<v4f *>(d + 2048 + at) = v4f{b[4 * q], b[4 * q + 1], b[4 * q + 2], b[4 * q + 3]};
         }
-        const unsigned at = r32 * 64 + (((2 * h) ^ ((r32 >> 2) & 3)) << 4);
-        const v4f y = *reinterpret_cast<const v4f *>(d + at), z = *reinterpret_cast<const v4f *>(d + (at ^ 16));
+        order_in_wave();
 #pragma unroll
-        for (int e = 0; e < 4; e++) x[e] = y[e], x[4 + e] = z[e];
+        for (int q = 0; q < 2; q++) {
+            const unsigned at = r32 * 64 + (((2 * h + q) ^ ((r32 >> 2) & 3)) << 4);
+            const v4f y = *reinterpret_cast<const v4f *>(d + at), z = *reinterpret_cast<const v4f *>(d + 2048 + at);
+#pragma unroll
+            for (int e = 0; e < 4; e++) a[4 * q + e] = y[e], b[4 * q + e] = z[e];
+        }
+        order_in_wave();
     };
 
     // steps in turn into two sums, where there are registers for them
@@ -109,10 +116,7 @@ __global__ void __launch_bounds__(64 * WAVES, PER_SIMD) k_gemm_strips(StagedArgs
 #pragma unroll
     for (int v = 0; v < 16; v++) acc[v] = other[v] = low[v] = 0.0f;
     auto multiply = [&](Raw &r, v16f &acc) {
-        if constexpr (TURN) {
-            turn(lds + wave * 4096, r.a);
-            turn(lds + wave * 4096 + 2048, r.b);
-        }
+        if constexpr (TURN) turn(lds + wave * 4096, r.a, r.b);
         if constexpr (!TERMS) {
 #pragma unroll
             for (int e = 0; e < 8; e++) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(r.b[e], r.a[e], acc, 0, 0, 0);
