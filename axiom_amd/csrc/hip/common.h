@@ -45,6 +45,7 @@ struct Tuning {
     int i8_mfma;         // AX_HIP_I8_MFMA: 32 (v_mfma_i32_32x32x32_i8) or 16 (v_mfma_i32_16x16x64_i8) in the persistent 256x256 kernel
     int f32_tile;        // AX_HIP_F32_TILE: 64 (64x64), 642 (64x64 with the k split over two wave sets), 128 (128x128, eight waves)
     int f32_splitk;      // AX_HIP_F32_SPLITK: 1 = never split K, 2.. = that many ranges where the route applies
+    int f32_no_strips;   // AX_HIP_F32_NO_STRIPS: 1 = single fp32 products never take the one-launch strips of few tiles
     int skinny_blocks;   // AX_HIP_SKINNY_BLOCKS: workgroups the skinny-M route aims for
     int skinny_form;     // AX_HIP_SKINNY_FORM: 1 (64 columns x 256 threads), 2 (the same, the lane groups of a wave added before LDS), 3 (64 columns x 512 threads)
     int skinny_kps;      // AX_HIP_SKINNY_KPS: most rows of K one skinny-M workgroup takes (a multiple of 16)

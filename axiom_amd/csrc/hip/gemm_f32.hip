@@ -1838,7 +1838,7 @@ int run_f32(const SgemmArgs &g, int transa, int transb) {
         // loads and write-back (2048 x 4096 x 64 16 -> 20, 128 24 -> 25; off the tile grid 4000 x 4000 x 128 53 -> 45).  Columns that fill
         // less than a tile are left to the fp32 tiles where K divides into ranges of 64 (685 x 960 x 32 8.2 -> 9.5, but 501 x 992 x 64 20 -> 8.9).
         const bool free_choice = tuning().f32_tile == 0 && tuning().f32_splitk == 0;
-        if (free_choice) rc = strips_f32(staged_args(g), transa, transb, on_grid);
+        if (free_choice && !tuning().f32_no_strips) rc = strips_f32(staged_args(g), transa, transb, on_grid);
         if (rc >= 0) return rc;
         const double products = (double)g.M * g.N * g.K;
         const bool split = off ? g.K >= 64

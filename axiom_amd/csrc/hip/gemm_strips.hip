@@ -241,9 +241,9 @@ int strips_f32(const StagedArgs &g, int transa, int transb, bool on_grid) {
     const int64_t tiles = ((g.M + TILE - 1) / TILE) * ((g.N + TILE - 1) / TILE), cus = cu_count();
     const bool one = tiles <= cus, two = tiles <= 2 * cus;
     if (g.K < 32 && two) {
-        if (!transa && !transb) return launch<4, false, true, false, 4>("sgemm_nn_32x32_staged", g);
-        if (!transa) return launch<4, false, true, true, 4>("sgemm_nt_32x32_staged", g);
-        return launch<4, false, false, false, 4>("sgemm_tn_32x32_staged", g);
+        if (!transa && !transb) return launch<4, false, true, false, 4>("sgemm_nn_strips32", g);
+        if (!transa) return launch<4, false, true, true, 4>("sgemm_nt_strips32", g);
+        return launch<4, false, false, false, 4>("sgemm_tn_strips32", g);
     }
     // Longer K, us: 256 x 768 x 1024 11.8 -> 8.2, A B^T 11.8 -> 8.9, 500 x 100 x 1000 10.0 -> 8.4, 100 x 10 x 1024 8.7 -> 7.6, 1000 x 128 x 1536 11.6 -> 10.6; 64 x 64 x
     // 1024 7.4 -> 7.7, 128 x 100 x 1024 A B^T 8.0 -> 8.5, 128 x 512 x 1280 9.3 -> 9.4, 1000 x 128 x 2048 12.6 -> 12.8.
@@ -251,9 +251,9 @@ int strips_f32(const StagedArgs &g, int transa, int transb, bool on_grid) {
     const int64_t most = g.M < 96 ? 900 : tiles >= 128 ? (transb ? 1280 : 1536) : tiles > 24 || (!transb && tiles <= 8 && ragged) ? 1024 : 900;
     if (g.K <= 112 || !((one && g.K <= most) || (two && !transb && g.K <= 800)) || (on_grid && g.K % 32 != 0 && g.K < 576)) return -1;
     if (!transa && !transb)
-        return one ? launch<8, true, true, false, 2>("sgemm_nn_32x32x3_staged", g) : launch<4, true, true, false, 4>("sgemm_nn_32x32x3_staged", g);
-    if (!transa) return launch<8, true, true, true, 2>("sgemm_nt_32x32x3_staged", g);
-    if (!one) return launch<4, true, false, false, 4>("sgemm_tn_32x32x3_staged", g);
-    return g.K <= 256 ? launch<8, true, false, false, 2>("sgemm_tn_32x32x3_staged", g) : launch<16, true, false, false, 4>("sgemm_tn_32x32x3_staged", g);
+        return one ? launch<8, true, true, false, 2>("sgemm_nn_strips32x3", g) : launch<4, true, true, false, 4>("sgemm_nn_strips32x3", g);
+    if (!transa) return launch<8, true, true, true, 2>("sgemm_nt_strips32x3", g);
+    if (!one) return launch<4, true, false, false, 4>("sgemm_tn_strips32x3", g);
+    return g.K <= 256 ? launch<8, true, false, false, 2>("sgemm_tn_strips32x3", g) : launch<16, true, false, false, 4>("sgemm_tn_strips32x3", g);
 }
 }  // namespace axhip

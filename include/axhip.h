@@ -62,6 +62,8 @@ const char *axhip_device_name(void);          /* gcnArchName of device 0, "" wit
  *   AX_HIP_F32_TILE      64x64 | 64x64k2 | 128x128   fp32 tile on the aligned fast path (k2: two wave sets split each K slab)
  *   AX_HIP_F32_SPLITK    1..4096    K ranges of the fp32 few-tile route, W8A32's too (1: never split; on rows off the 16-byte grid at
  *                        most 16, of 128 or more each)
+ *   AX_HIP_F32_NO_STRIPS 1          single fp32 products with few output tiles take the tiles and K ranges of the other routes and not
+ *                        the one launch whose waves share K
  *   AX_HIP_NT_WALK       1 | 2      batched A B^T with K <= 128: 1, a 128-row block of A stays in LDS and the column blocks of B^T
  *                        are walked; 2, 256 rows of B stay in registers and A is walked in blocks of 32 rows (N a multiple of 256)
  *   AX_HIP_SKINNY_BLOCKS 1..65535   workgroups the skinny-M route aims for

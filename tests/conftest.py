@@ -33,6 +33,16 @@ def reflib():
     return RefLib()
 
 
+@pytest.fixture
+def no_strips(hip, monkeypatch):
+    """Single fp32 products on the routes that the strips of few tiles stand before: for tests of those routes at their own edges."""
+    monkeypatch.setenv("AX_HIP_F32_NO_STRIPS", "1")
+    assert hip.L.axhip_tuning_reload() == 1
+    yield
+    monkeypatch.delenv("AX_HIP_F32_NO_STRIPS")
+    assert hip.L.axhip_tuning_reload() == 0
+
+
 @pytest.fixture(scope="session")
 def hip():
     """libaxhip.so on a real GPU.  No fallback: a missing library or GPU is an error."""

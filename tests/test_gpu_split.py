@@ -22,6 +22,7 @@ def product(hip, a, b, order):
 
 # the fp32 error bound K u sum |a||b| (u = 2^-24) holds with room for sums of random signs, see test_gpu_staged; the left-out terms
 # add at most 2^-24 of each product
+@pytest.mark.usefixtures("no_strips")
 @pytest.mark.parametrize("M,N,K", [(17, 33, 64), (65, 129, 65), (129, 65, 95), (161, 516, 256), (1152, 1152, 1152), (1153, 772, 2052), (644, 4096, 1024),
                                    (2049, 1028, 260), (200, 128, 4096), (1000, 1004, 1001)])
 @pytest.mark.parametrize("order", ["nn", "nt", "tn"])
@@ -49,6 +50,7 @@ def test_split_batched(hip, Bn, M, N, K, transb):
     assert (np.abs(got - want) <= BOUND_FP32 * size).all()
 
 
+@pytest.mark.usefixtures("no_strips")
 @pytest.mark.parametrize("M,N,K,tile", [(70, 90, 101, "64x64"), (501, 2053, 129, "128x64"), (513, 3583, 129, "64x128"), (1537, 1541, 129, "128x128")])
 def test_every_tile(hip, M, N, K, tile):
     """The shapes of this file reach every tile: one row or column past whole tiles, a slab and one value more."""
@@ -64,6 +66,7 @@ def test_every_tile(hip, M, N, K, tile):
 SHAPES = [(70, 90, 101), (200, 132, 1029), (1152, 1152, 1152)]      # one tile, ranges of K, whole tiles
 
 
+@pytest.mark.usefixtures("no_strips")
 @pytest.mark.parametrize("M,N,K", SHAPES)
 @pytest.mark.parametrize("scale_a,scale_b", [(2.0 ** -115, 1.0), (2.0 ** -100, 2.0 ** 90), (2.0 ** -60, 2.0 ** -50), (2.0 ** 120, 2.0 ** -20), (1.0, 2.0 ** -118)])
 def test_split_keeps_the_range(hip, M, N, K, scale_a, scale_b):
@@ -79,6 +82,7 @@ def test_split_keeps_the_range(hip, M, N, K, scale_a, scale_b):
     assert (np.abs(got - want) <= BOUND_FP32 * size + K * 2.0 ** -149).all()
 
 
+@pytest.mark.usefixtures("no_strips")
 @pytest.mark.parametrize("M,N,K", SHAPES)
 def test_split_non_finite(hip, M, N, K):
     """Infinities, NaNs and values that round past the largest bf16 give what fp32 arithmetic gives; the other rows are untouched."""
@@ -104,6 +108,7 @@ def test_split_non_finite(hip, M, N, K):
     assert (np.abs(got[rows] - ref[rows]) <= BOUND_FP32 * size).all()
 
 
+@pytest.mark.usefixtures("no_strips")
 @pytest.mark.parametrize("M,N,K", SHAPES)
 @pytest.mark.parametrize("scale_a,scale_b", [(2.0 ** -60, 2.0 ** -60), (2.0 ** -55, 2.0 ** -68), (2.0 ** -20, 2.0 ** -110), (2.0 ** -127, 2.0 ** 10), (2.0 ** 50, 2.0 ** 40)])
 def test_split_small_results(hip, M, N, K, scale_a, scale_b):
@@ -119,6 +124,7 @@ def test_split_small_results(hip, M, N, K, scale_a, scale_b):
     assert (np.abs(got - want) <= BOUND_FP32 * size + 32 * 2.0 ** -149).all(), float(((np.abs(got - want) - 32 * 2.0 ** -149) / size).max())
 
 
+@pytest.mark.usefixtures("no_strips")
 @pytest.mark.parametrize("M,N,K", SHAPES)
 def test_split_small_values_among_others(hip, M, N, K):
     """Values down to fp32's smallest beside ordinary ones, as GELU and softmax leave them, are no reason for the fp32 pass: every sum
@@ -136,6 +142,7 @@ def test_split_small_values_among_others(hip, M, N, K):
     assert (got != clean).mean() < 0.01
 
 
+@pytest.mark.usefixtures("no_strips")
 @pytest.mark.parametrize("M,N,K", SHAPES + [(65, 517, 257), (501, 2053, 129), (513, 3583, 129)])
 @pytest.mark.parametrize("order", ["nn", "nt", "tn"])
 def test_split_single_products(hip, M, N, K, order):

@@ -13,6 +13,7 @@ pytestmark = pytest.mark.gpu
 # as sums of random signs grow with sqrt(K), the K used here by an order of magnitude
 
 
+@pytest.mark.usefixtures("no_strips")
 @pytest.mark.parametrize("M,N,K", [(17, 17, 32), (33, 65, 33), (65, 129, 63), (64, 63, 64), (129, 257, 65), (41, 1113, 92), (61, 343, 551),
                                    (222, 434, 1376), (127, 11, 1023), (372, 2149, 257), (2001, 2003, 97), (17, 1, 4097), (2001, 2003, 32),
                                    (2033, 2003, 63)])
@@ -117,6 +118,7 @@ def test_tile_of_a_short_k(hip, order, Bn, M, N, K, kernel):
         assert (np.abs(got[h] - want) <= BOUND_FP32 * size).all()
 
 
+@pytest.mark.usefixtures("no_strips")
 @pytest.mark.parametrize("order,M,N,K,kernel", [
     ("nn", 17, 576, 340, "sgemm_32x64k2_dma_edge"), ("nt", 160, 20, 472, "sgemm_32x64k2_dma_edge"), ("nt", 96, 3296, 392, "sgemm_32x64k2_dma_edge"),
     ("tn", 128, 672, 328, "sgemm_64x64k2_dma_edge"), ("nn", 249, 512, 376, "sgemm_nn_64x64x3_staged"), ("tn", 160, 32, 440, "sgemm_splitk_x3"),

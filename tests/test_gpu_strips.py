@@ -21,7 +21,7 @@ def product(hip, a, b, order, alpha=1.0, beta=0.0, c=None, bias=None, act=0, pad
     dbias = None if bias is None else hip.array(bias)
     hip.check(hip.L.axhip_sgemm(int(order[0] == "t"), int(order[1] == "t"), M, N, K, alpha, da.ptr, sa.shape[1], db.ptr, sb.shape[1], beta, dc.ptr,
                                 N + pads[2], None if bias is None else dbias.ptr, act))
-    assert "_32x32" in hip.last_kernel(), hip.last_kernel()
+    assert "_strips32" in hip.last_kernel(), hip.last_kernel()
     full = dc.numpy()
     assert np.isnan(full[:, N:]).all()
     return full[:, :N]
