@@ -229,11 +229,16 @@ int launch(const char *name, const StagedArgs &g) {
 }  // namespace
 
 namespace axhip {
-// In terms, from a step of 16 k per wave of eight on: up to a tile a CU and a K of nine hundred to fifteen hundred, or two tiles and some hundred (us, before -> here:
-// 100 x 4096 x 784 15.3 -> 12.0 on 512 tiles, A B^T 14.1 -> 12.8; past the limits 500 x 200 x 2000 13.2 -> 14.2, 1024 x 1024 x 256 8.2 -> 9.5, 12 x 1024 x 1024 7.0 ->
-// 7.9; A B^T on 336 tiles with K = 476 8.9 -> 9.7, with its extra turn it stops at one tile a CU).  Two workgroups share a CU from 257 tiles on: four waves each
-// (86 x 3584 x 300: eight 6.4, four 5.6).  Sixteen pay where A is stored across K, whose loads are the slowest, above K = 256 (256 x 1000 x 500 6.6 -> 6.1;
-// 250 x 500 x 256 4.5 -> 5.2).
+// In terms from K = 113 on, with limits to K from operands that are cached and operands from HBM (the strips have two steps under way and
+// wait longer for memory than the kernels before).  us, before -> here, cached / from HBM: 1024 x 256 x 1024 12.3 / 12.7 -> 8.5 / 10.1, 384 x 128 x
+// 700 10.5 / 11.0 -> 7.3 / 9.0, A B^T 256 x 768 x 896 11.5 / 12.5 -> 8.3 / 9.6, 500 x 300 x 640 11.0 / 11.9 -> 7.1 / 8.4, A^T B 1024 x 256 x 1280 13.1 / 13.5 ->
+// 10.4 / 11.7; past the limits 1588 x 22 x 973 9.8 / 10.5 -> 8.6 / 12.0, 1446 x 65 x 1208 11.8 / 12.8 -> 10.2 / 14.0, A B^T 57 x 1598 x 893 9.9 / 11.3 -> 8.9 / 12.7;
+// 1024 x 1024 x 256 cached 8.2 -> 9.5, and A B^T on 336 tiles with K = 476, with its extra turn, 8.9 -> 9.7.
+// Two workgroups share a CU from 257 tiles on: four waves each (86 x 3584 x 300: eight 6.4, four 5.6).  Off the 16-byte grid four too up to K = 176,
+// where eight strips of a step or two leave a larger error than the staged tiles in terms that they stand before (geometric means over some
+// hundred products: eight 1.05 of theirs at K = 129..144, 1.02 at 145..160, 1.01 at 161..168, 0.99 from 177 on, four 0.99, 0.98, 0.96), and none up to
+// K = 128 (four 1.07 at 64..80, 1.01 at 113..120).  On the grid the kernels before were on fp32 instructions, with three times the error.
+// Sixteen pay where A is stored across K, whose loads are the slowest, above K = 256 (256 x 1000 x 500 6.6 -> 6.1; 250 x 500 x 256 4.5 -> 5.2).
 // K below 32 on fp32 instructions: there is little to multiply and nothing to cut (128 x 1024 x 10 6.6 -> 3.9, A B^T 6.3 -> 3.5, 784 x 40 x 20 A^T B 4.5 -> 4.1).  K from 32 to 112, and rows on
 // the 16-byte grid with K on the 4 and off the 32 grid below 576, stay with the kernels that the tests of those routes name (70 x 90 x 101 6.6 us, 4.9 here).
 int strips_f32(const StagedArgs &g, int transa, int transb, bool on_grid) {
@@ -245,15 +250,14 @@ int strips_f32(const StagedArgs &g, int transa, int transb, bool on_grid) {
         if (!transa) return launch<4, false, true, true, 4>("sgemm_nt_strips32", g);
         return launch<4, false, false, false, 4>("sgemm_tn_strips32", g);
     }
-    // Longer K, us: 256 x 768 x 1024 11.8 -> 8.2, A B^T 11.8 -> 8.9, 500 x 100 x 1000 10.0 -> 8.4, 100 x 10 x 1024 8.7 -> 7.6, 1000 x 128 x 1536 11.6 -> 10.6; 64 x 64 x
-    // 1024 7.4 -> 7.7, 128 x 100 x 1024 A B^T 8.0 -> 8.5, 128 x 512 x 1280 9.3 -> 9.4, 1000 x 128 x 2048 12.6 -> 12.8.
-    const bool ragged = g.M % TILE != 0 || g.N % TILE != 0;
-    const int64_t most = g.M < 96 ? 900 : tiles >= 128 ? (transb ? 1280 : 1536) : tiles > 24 || (!transb && tiles <= 8 && ragged) ? 1024 : 900;
-    if (g.K <= 112 || !((one && g.K <= most) || (two && !transb && g.K <= 800)) || (on_grid && g.K % 32 != 0 && g.K < 576)) return -1;
+    const bool many = tiles >= 128;
+    const int64_t most = transb ? (many ? 896 : 640) : !many ? 800 : transa ? 1280 : 1024;
+    if (g.K <= (on_grid ? 112 : 128) || !((one && g.K <= most) || (two && !transb && g.K <= 800)) || (on_grid && g.K % 32 != 0 && g.K < 576)) return -1;
+    const bool four = !one || (!on_grid && g.K <= 176);
     if (!transa && !transb)
-        return one ? launch<8, true, true, false, 2>("sgemm_nn_strips32x3", g) : launch<4, true, true, false, 4>("sgemm_nn_strips32x3", g);
-    if (!transa) return launch<8, true, true, true, 2>("sgemm_nt_strips32x3", g);
-    if (!one) return launch<4, true, false, false, 4>("sgemm_tn_strips32x3", g);
+        return four ? launch<4, true, true, false, 4>("sgemm_nn_strips32x3", g) : launch<8, true, true, false, 2>("sgemm_nn_strips32x3", g);
+    if (!transa) return four ? launch<4, true, true, true, 4>("sgemm_nt_strips32x3", g) : launch<8, true, true, true, 2>("sgemm_nt_strips32x3", g);
+    if (four) return launch<4, true, false, false, 4>("sgemm_tn_strips32x3", g);
     return g.K <= 256 ? launch<8, true, false, false, 2>("sgemm_tn_strips32x3", g) : launch<16, true, false, false, 4>("sgemm_tn_strips32x3", g);
 }
 }  // namespace axhip
