@@ -236,8 +236,8 @@ namespace axhip {
 // 1024 x 1024 x 256 cached 8.2 -> 9.5, and A B^T on 336 tiles with K = 476, with its extra turn, 8.9 -> 9.7.
 // Two workgroups share a CU from 257 tiles on: four waves each (86 x 3584 x 300: eight 6.4, four 5.6).  Off the 16-byte grid four too up to K = 176,
 // where eight strips of a step or two leave a larger error than the staged tiles in terms that they stand before (geometric means over some
-// hundred products: eight 1.05 of theirs at K = 129..144, 1.02 at 145..160, 1.01 at 161..168, 0.99 from 177 on, four 0.99, 0.98, 0.96), and none up to
-// K = 128 (four 1.07 at 64..80, 1.01 at 113..120).  On the grid the kernels before were on fp32 instructions, with three times the error.
+// hundred products: eight 1.05 of theirs at K = 129..144, 1.02 at 145..160, 1.01 at 161..168, 0.99 from 177 on, four 0.99, 0.98, 0.96 and, of
+// uniform values, 1.00 at 121..128), and none up to K = 120 (four 1.07 at 64..80, 1.01 at 113..120).  On the grid the kernels before were on fp32 instructions, with three times the error.
 // Sixteen pay where A is stored across K, whose loads are the slowest, above K = 256 (256 x 1000 x 500 6.6 -> 6.1; 250 x 500 x 256 4.5 -> 5.2).
 // K below 32 on fp32 instructions: there is little to multiply and nothing to cut (128 x 1024 x 10 6.6 -> 3.9, A B^T 6.3 -> 3.5, 784 x 40 x 20 A^T B 4.5 -> 4.1).  K from 32 to 112, and rows on
 // the 16-byte grid with K on the 4 and off the 32 grid below 576, stay with the kernels that the tests of those routes name (70 x 90 x 101 6.6 us, 4.9 here).
@@ -252,7 +252,7 @@ int strips_f32(const StagedArgs &g, int transa, int transb, bool on_grid) {
     }
     const bool many = tiles >= 128;
     const int64_t most = transb ? (many ? 896 : 640) : !many ? 800 : transa ? 1280 : 1024;
-    if (g.K <= (on_grid ? 112 : 128) || !((one && g.K <= most) || (two && !transb && g.K <= 800)) || (on_grid && g.K % 32 != 0 && g.K < 576)) return -1;
+    if (g.K <= (on_grid ? 112 : 120) || !((one && g.K <= most) || (two && !transb && g.K <= 800)) || (on_grid && g.K % 32 != 0 && g.K < 576)) return -1;
     const bool four = !one || (!on_grid && g.K <= 176);
     if (!transa && !transb)
         return four ? launch<4, true, true, false, 4>("sgemm_nn_strips32x3", g) : launch<8, true, true, false, 2>("sgemm_nn_strips32x3", g);
