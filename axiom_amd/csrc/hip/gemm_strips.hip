@@ -234,7 +234,10 @@ namespace axhip {
 // 700 10.5 / 11.0 -> 7.3 / 9.0, A B^T 256 x 768 x 896 11.5 / 12.5 -> 8.3 / 9.6, 500 x 300 x 640 11.0 / 11.9 -> 7.1 / 8.4, A^T B 1024 x 256 x 1280 13.1 / 13.5 ->
 // 10.4 / 11.7; past the limits 1588 x 22 x 973 9.8 / 10.5 -> 8.6 / 12.0, 1446 x 65 x 1208 11.8 / 12.8 -> 10.2 / 14.0, A B^T 57 x 1598 x 893 9.9 / 11.3 -> 8.9 / 12.7;
 // 1024 x 1024 x 256 cached 8.2 -> 9.5, and A B^T on 336 tiles with K = 476, with its extra turn, 8.9 -> 9.7.
-// Two workgroups share a CU from 257 tiles on: four waves each (86 x 3584 x 300: eight 6.4, four 5.6).  Off the 16-byte grid four too up to K = 176,
+// Two workgroups share a CU from 257 tiles on: four waves each (86 x 3584 x 300: eight 6.4, four 5.6); but
+// eight on up to a third of the CUs with K above 400, where ranges of K on 64x64 tiles would have the smaller error than four long strips (geometric
+// mean over 51 products 1.03 of theirs with four, at most 1.09; 0.94 with eight, times 1.05 in A B and 0.96 in A^T B of four's), and none there above
+// K = 640 (127 x 2125 x 705 13.7 -> 15.3, 2186 x 104 x 699 from HBM 13.0 -> 14.9).  Off the 16-byte grid four too up to K = 176,
 // where eight strips of a step or two leave a larger error than the staged tiles in terms that they stand before (geometric means over some
 // hundred products: eight 1.05 of theirs at K = 129..144, 1.02 at 145..160, 1.01 at 161..168, 0.99 from 177 on, four 0.99, 0.98, 0.96 and, of
 // uniform values, 1.00 at 121..128), and none up to K = 120 (four 1.07 at 64..80, 1.01 at 113..120).  On the grid the kernels before were on fp32 instructions, with three times the error.
@@ -252,7 +255,11 @@ int strips_f32(const StagedArgs &g, int transa, int transb, bool on_grid) {
     }
     const bool many = tiles >= 128;
     const int64_t most = transb ? (many ? 896 : 640) : !many ? 800 : transa ? 1280 : 1024;
-    if (g.K <= (on_grid ? 112 : 120) || !((one && g.K <= most) || (two && !transb && g.K <= 800)) || (on_grid && g.K % 32 != 0 && g.K < 576)) return -1;
+    const bool third = tiles * 3 <= cus * 4;                   // two workgroups on a third of the CUs at most
+    if (g.K <= (on_grid ? 112 : 120) || !((one && g.K <= most) || (two && !transb && g.K <= (third ? 640 : 800))) || (on_grid && g.K % 32 != 0 && g.K < 576))
+        return -1;
+    if (!one && third && g.K > 400)
+        return transa ? launch<8, true, false, false, 4>("sgemm_tn_strips32x3", g) : launch<8, true, true, false, 4>("sgemm_nn_strips32x3", g);
     const bool four = !one || (!on_grid && g.K <= 176);
     if (!transa && !transb)
         return four ? launch<4, true, true, false, 4>("sgemm_nn_strips32x3", g) : launch<8, true, true, false, 2>("sgemm_nn_strips32x3", g);

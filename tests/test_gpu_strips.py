@@ -34,7 +34,7 @@ def tiles(M, N):
 def most(order, M, N):
     """The largest K that the strips take (256 CUs)."""
     if tiles(M, N) > 256:
-        return 0 if order == "nt" else 800
+        return 0 if order == "nt" else 640 if tiles(M, N) <= 341 else 800
     return {"nn": (800, 1024), "nt": (640, 896), "tn": (800, 1280)}[order][tiles(M, N) >= 128]
 
 
@@ -152,7 +152,7 @@ def test_outer_products_are_rounded_once(hip):
         assert np.array_equal(product(hip, u, v, order), u * v)
 
 
-@pytest.mark.parametrize("order,M,N", [("nn", 100, 100), ("nn", 130, 1000), ("nt", 100, 100), ("nt", 130, 1000), ("tn", 100, 100), ("tn", 130, 1000), ("nn", 200, 2000)])
+@pytest.mark.parametrize("order,M,N", [("nn", 100, 100), ("nn", 130, 1000), ("nn", 330, 990), ("tn", 352, 992), ("nt", 100, 100), ("nt", 130, 1000), ("tn", 100, 100), ("tn", 130, 1000), ("nn", 200, 2000)])
 def test_where_k_ends(hip, order, M, N):
     """The last K that the strips take and the next one, which takes another route."""
     K = most(order, M, N)
@@ -166,14 +166,13 @@ def test_where_k_ends(hip, order, M, N):
         assert (np.abs(got - a.astype(np.float64) @ b.astype(np.float64)) <= BOUND_FP32 * (np.abs(a).astype(np.float64) @ np.abs(b).astype(np.float64))).all()
 
 
-@pytest.mark.parametrize("order", ["nn", "nt", "tn"])
-@pytest.mark.parametrize("K", [121, 128, 150, 176, 177])
-def test_error_of_short_k_off_the_grid(hip, monkeypatch, order, K):
+@pytest.mark.parametrize("order,M,N,K", [(o, 255, 1021, K) for o in ("nn", "nt", "tn") for K in (121, 128, 150, 176, 177)] +
+                         [(o, 321, 865, K) for o in ("nn", "tn") for K in (401, 600)])
+def test_error_is_that_of_the_staged_tiles_or_less(hip, monkeypatch, order, M, N, K):
     """No larger than what the staged tiles in terms leave on the same operands, which the strips stand before; 1 % for the luck of the draw: over a quarter of a
     million sums whose errors are independent a norm is known to some 0.15 %."""
-    say("strips, error of a short k", order, K)
+    say("strips, error", order, M, N, K)
     rng = np.random.default_rng(K)
-    M, N = 255, 1021
     a, b = rng.uniform(-1, 1, (M, K)).astype(np.float32), rng.uniform(-1, 1, (K, N)).astype(np.float32)
     want = a.astype(np.float64) @ b.astype(np.float64)
     strips = np.linalg.norm(product(hip, a, b, order) - want)
@@ -182,7 +181,7 @@ def test_error_of_short_k_off_the_grid(hip, monkeypatch, order, K):
     try:
         da, db = hip.array(a.T if order[0] == "t" else a), hip.array(b.T if order[1] == "t" else b)
         staged = np.linalg.norm(hip.sgemm(da, db, transa=order[0] == "t", transb=order[1] == "t").numpy() - want)
-        assert hip.last_kernel().endswith("x3_staged")
+        assert hip.last_kernel().endswith("x3_staged") or hip.last_kernel() == "sgemm_splitk_x3"
     finally:
         monkeypatch.delenv("AX_HIP_F32_NO_STRIPS")
         assert hip.L.axhip_tuning_reload() == 0
