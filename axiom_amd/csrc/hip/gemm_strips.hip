@@ -242,13 +242,15 @@ namespace axhip {
 // hundred products: eight 1.05 of theirs at K = 129..144, 1.02 at 145..160, 1.01 at 161..168, 0.99 from 177 on, four 0.99, 0.98, 0.96 and, of
 // uniform values, 1.00 at 121..128), and none up to K = 120 (four 1.07 at 64..80, 1.01 at 113..120).  On the grid the kernels before were on fp32 instructions, with three times the error.
 // Sixteen pay where A is stored across K, whose loads are the slowest, above K = 256 (256 x 1000 x 500 6.6 -> 6.1; 250 x 500 x 256 4.5 -> 5.2).
-// K below 32 on fp32 instructions: there is little to multiply and nothing to cut (128 x 1024 x 10 6.6 -> 3.9, A B^T 6.3 -> 3.5, 784 x 40 x 20 A^T B 4.5 -> 4.1).  K from 32 to 112, and rows on
-// the 16-byte grid with K on the 4 and off the 32 grid below 576, stay with the kernels that the tests of those routes name (70 x 90 x 101 6.6 us, 4.9 here).
+// On fp32 instructions up to K = 63 off the grid and 112 on it, where the kernels before are on them too: there is little to multiply and nothing to
+// cut.  Four waves, up to two tiles a CU (geometric means over some hundred products a range, cached / from HBM, and the error over that of the
+// kernels before: K below 32 1.3 / 1.3, 0.99; 32..63 off the grid 1.31 / 1.29, 0.86, on it 1.22 / 1.21, 0.74; 64..112 on the grid 1.32 / 1.31, 0.64; strips in
+// terms 1.17 / 1.18 there.  us: 128 x 1024 x 10 6.6 -> 3.9, A B^T 6.3 -> 3.5, 784 x 40 x 20 A^T B 4.5 -> 4.1).
 int strips_f32(const StagedArgs &g, int transa, int transb, bool on_grid) {
     if ((transa && transb) || g.K < 1 || g.lda >= (1 << 22) || g.ldb >= (1 << 22)) return -1;
     const int64_t tiles = ((g.M + TILE - 1) / TILE) * ((g.N + TILE - 1) / TILE), cus = cu_count();
     const bool one = tiles <= cus, two = tiles <= 2 * cus;
-    if (g.K < 32 && two) {
+    if (two && g.K < (on_grid ? 113 : 64)) {
         if (!transa && !transb) return launch<4, false, true, false, 4>("sgemm_nn_strips32", g);
         if (!transa) return launch<4, false, true, true, 4>("sgemm_nt_strips32", g);
         return launch<4, false, false, false, 4>("sgemm_tn_strips32", g);
@@ -256,8 +258,7 @@ int strips_f32(const StagedArgs &g, int transa, int transb, bool on_grid) {
     const bool many = tiles >= 128;
     const int64_t most = transb ? (many ? 896 : 640) : !many ? 800 : transa ? 1280 : 1024;
     const bool third = tiles * 3 <= cus * 4;                   // two workgroups on a third of the CUs at most
-    if (g.K <= (on_grid ? 112 : 120) || !((one && g.K <= most) || (two && !transb && g.K <= (third ? 640 : 800))) || (on_grid && g.K % 32 != 0 && g.K < 576))
-        return -1;
+    if (g.K <= (on_grid ? 112 : 120) || !((one && g.K <= most) || (two && !transb && g.K <= (third ? 640 : 800)))) return -1;
     if (!one && third && g.K > 400)
         return transa ? launch<8, true, false, false, 4>("sgemm_tn_strips32x3", g) : launch<8, true, true, false, 4>("sgemm_nn_strips32x3", g);
     const bool four = !one || (!on_grid && g.K <= 176);

@@ -39,7 +39,7 @@ def most(order, M, N):
 
 
 FORMS = [(order, M, N, K) for order in ("nn", "nt", "tn") for M, N in [(17, 1), (31, 33), (32, 32), (65, 95), (100, 10), (260, 1000), (250, 2020)]
-         for K in (1, 2, 15, 16, 17, 31, 121, 128, 129, 143, 144, 145, 176, 177, 255, 256, 257, 500, 640, 641, 799) if K < 32 or K <= most(order, M, N)]
+         for K in (1, 2, 15, 16, 17, 31, 32, 47, 63, 121, 128, 129, 143, 144, 145, 176, 177, 255, 256, 257, 500, 640, 641, 799) if K < 64 or K <= most(order, M, N)]
 
 
 # K u sum |a||b| holds with room; with terms the left-out ones add at most 2^-24 of each product
@@ -57,7 +57,8 @@ def test_every_form(hip, M, N, K, order):
 
 
 @pytest.mark.parametrize("order,M,N,K", [(o, M, N, K) for o in ("nn", "nt", "tn") for M, N, K in [(64, 64, 128), (256, 768, 256), (128, 1024, 784),
-                                                                                                 (1024, 96, 640), (192, 2048, 512)] if K <= most(o, M, N)])
+    (1024, 96, 640), (192, 2048, 512), (20, 36, 32), (36, 1000, 44), (100, 2048, 60), (64, 64, 64), (96, 260, 100), (192, 2048, 112), (68, 100, 116), (160, 96, 132),
+    (32, 1024, 340), (128, 672, 328), (160, 20, 572)] if K < 113 or K <= most(o, M, N)])
 def test_on_the_grid(hip, M, N, K, order):
     """Rows on the 16-byte grid, K off and on the 32 grid; error no larger than fp32 instructions leave (2^-24 a product and sqrt(K) roundings)."""
     say("strips on the grid", M, N, K, order)
@@ -82,7 +83,7 @@ def test_longer_k(hip, order, M, N, K):
 
 
 @pytest.mark.parametrize("order", ["nn", "nt", "tn"])
-@pytest.mark.parametrize("K", [20, 300])
+@pytest.mark.parametrize("K", [20, 60, 300])
 def test_non_finite(hip, K, order):
     """Infinities and NaNs reach the rows and columns that hold them and no others; magnitudes up to the largest float come out."""
     say("strips non-finite", K, order)
