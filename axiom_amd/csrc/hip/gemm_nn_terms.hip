@@ -244,16 +244,20 @@ int nn_terms(const StagedArgs &g, int64_t batch) {
         return -1;
     // Under 96 rows idle waves cost more than the tiles (N = 32, 256 of 64 x 500 13.8 -> 16.1, 16 x 1024 22.5 -> 24.7).
     const int64_t cus = cu_count(), tiles4 = (g.M + 127) / 128 * batch, tiles8 = (g.M + 255) / 256 * batch;
-    // Off the 16-byte grid from K = 128 on: the staged tiles take fewer of the products into one sum there and their error is the smaller one
-    // (N = 80, 70 x 70 4.8e-8 against 6.6e-8; N <= 32 keeps the same line, 512 of 100 x 100, N = 17 17.5 and 9.5).
-    const bool on_grid = g.K % 4 == 0 && g.N % 4 == 0;
-    if (!on_grid && g.K < 128) return -1;
-    // N <= 32 from three quarters of the CUs on (1000 x 1000, 32 of them 39 -> 32; 64 of 256 x 256, 128 workgroups, level)
-    if (g.N <= 32) return tiles4 * 4 >= cus * 3 ? launch<1, 4>(g, batch) : -1;
+    // whether the kernels before load straight to LDS, and are on fp32 instructions
+    const bool on_grid = (g.K | g.N | g.lda | g.ldb | g.ldc | g.stride_a | g.stride_b | g.stride_c) % 4 == 0 &&
+                         ((uintptr_t)g.A | (uintptr_t)g.B | (uintptr_t)g.C) % 16 == 0;
+    // N <= 32 from three quarters of the CUs on (1000 x 1000, 32 of them 39 -> 32; 64 of 256 x 256, 128 workgroups, level), off the grid from
+    // K = 128 on (512 of 100 x 100, N = 17 17.5 and 9.5)
+    if (g.N <= 32) return tiles4 * 4 >= cus * 3 && (on_grid || g.K >= 128) ? launch<1, 4>(g, batch) : -1;
     // N = 33..64 as above.  Wider ones need 0.7 of two workgroups a CU (N = 80, 64 of 512 x 512, half of them, 0.97; 96 of 384 x 384,
     // 0.56, 1.16; off the grid, where the kernels before are faster, 0.75), N > 96 K >= 256 (256 of 1024 x 128 82.5 -> 84.1, 200 x 200
     // 109 -> 111).
     if (g.N <= 64 || tiles4 * 20 <= 2 * cus * (on_grid ? 14 : 15) || (g.N > 96 && g.K < 256)) return -1;
+    // Off the grid they stand before tiles in terms, whose error is the larger one on 128x128 tiles only: elsewhere those have the five smaller
+    // products in a sum of their own over all of K (129 of 959 x 181, N = 69 9.6e-8 here and 5.9e-8 there, 284 of 176 x 990, N = 73 2.2e-7 and
+    // 1.15e-7; on 128x128 tiles 1.4 to 1.5 times the error here).
+    if (!on_grid && !split_is_128x128(g, batch)) return -1;
     // Four waves or eight: rounds of workgroups over the chip, of which one with a workgroup on each CU at most is 0.72 (N = 80: 96 of
     // 640 x 640 82 with eight and 59 with four, 64 of 1000 x 1000 86 and 100).
     const int64_t left = tiles4 % (2 * cus), cost4 = tiles4 / (2 * cus) * 107 + (left == 0 ? 0 : left <= cus ? 72 : 105);

@@ -22,6 +22,8 @@ struct StagedArgs {
 int staged_f32(const StagedArgs &g, int transa, int transb, int64_t batch, bool may_split);
 // The same products in bf16 terms on the bf16 matrix core, at fp32 accuracy.
 int split_f32(const StagedArgs &g, int transa, int transb, int64_t batch, bool may_split);
+// Whether split_f32 would form this batch on its 128x128 tiles.
+bool split_is_128x128(const StagedArgs &g, int64_t batch);
 int staged_i8w(const StagedArgs &g);
 // What a product cut into ranges of K reports when they were formed in bf16 terms (fp32 ranges: sgemm_splitk).
 constexpr const char *kSplitTermsName = "sgemm_splitk_x3";

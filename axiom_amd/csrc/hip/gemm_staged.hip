@@ -605,6 +605,8 @@ int split_f32(const StagedArgs &g, int transa, int transb, int64_t batch, bool m
     return run_split<false, false>(g, batch, may_split, tn, kSplitTermsName);
 }
 
+bool split_is_128x128(const StagedArgs &g, int64_t batch) { return g.K >= 64 && plan_staged(g, batch, kSplitTiles, 4, false).tile == 0; }
+
 int staged_f32(const StagedArgs &g, int transa, int transb, int64_t batch, bool may_split) {
     static const char *const nn[2] = {"sgemm_nn_64x64k2_staged", "sgemm_nn_128x128k2_staged"};
     static const char *const nt[2] = {"sgemm_nt_64x64k2_staged", "sgemm_nt_128x128k2_staged"};

@@ -27,15 +27,18 @@ def products(hip, a, b, alpha=1.0, pads=(0, 0, 0)):
     return full[:, :, :N], hip.last_kernel()
 
 
+KS = (64, 65, 95, 96, 128, 159, 256, 291)
+# up to 32 columns, any alignment; more of them on the 16-byte grid (from 96 on with K >= 256 whole tiles only); off it where the staged tiles would be 128x128
+FORMS = [(-(-400 // -(-M // 128)), M, N, K, pads) for pads in [(0, 0, 0), (1, 3, 5)] for M, N in [(96, 1), (128, 17), (129, 32), (300, 31)] for K in KS
+         if K >= 128 or (K % 4 == 0 and N % 4 == 0 and pads[0] == 0)]
+FORMS += [(-(-400 // -(-M // 128)), M, N, K, pads) for pads in [(0, 0, 0), (4, 8, 4)] for M, N in [(128, 80), (257, 96), (256, 128), (385, 72)] for K in KS
+          if K % 4 == 0 and not (N > 96 and K < 256) and not (N >= 96 and K >= 256 and M % 128)]
+FORMS += [(134, 338, 90, 146, (1, 3, 5)), (206, 345, 76, 133, (0, 0, 0)), (62, 966, 76, 210, (1, 3, 5)), (108, 458, 92, 286, (0, 0, 0))]
+
+
 # K u sum |a||b| holds with room; with terms the left-out ones add at most 2^-24 of each product
-@pytest.mark.parametrize("pads", [(0, 0, 0), (1, 3, 5)])
-@pytest.mark.parametrize("M,N", [(96, 1), (128, 17), (129, 32), (300, 31), (97, 65), (128, 80), (257, 96), (200, 97), (256, 128), (385, 100)])
-@pytest.mark.parametrize("K", [64, 65, 95, 96, 128, 159, 256, 291])
-def test_every_form(hip, M, N, K, pads):
-    on_grid = K % 4 == 0 and N % 4 == 0
-    if (not on_grid and K < 128) or (N > 96 and K < 256) or (N >= 96 and K >= 256 and (M % 128 or K % 32)):
-        pytest.skip("other kernels")
-    H = -(-200 if N <= 32 else -400) // -(-M // 128)
+@pytest.mark.parametrize("H,M,N,K,pads", FORMS)
+def test_every_form(hip, H, M, N, K, pads):
     say("narrow batches", H, M, N, K, pads)
     rng = np.random.default_rng(M * 7 + N * 3 + K)
     a, b = rng.uniform(-1, 1, (H, M, K)).astype(np.float32), rng.uniform(-1, 1, (H, K, N)).astype(np.float32)
@@ -46,6 +49,21 @@ def test_every_form(hip, M, N, K, pads):
     sums = got.astype(np.float64).sum(axis=2) - 0.5 * np.matmul(a.astype(np.float64), b.astype(np.float64).sum(axis=2, keepdims=True))[:, :, 0]
     size = 0.5 * np.matmul(np.abs(a).astype(np.float64), np.abs(b).astype(np.float64).sum(axis=2, keepdims=True))[:, :, 0]
     assert (np.abs(sums) <= BOUND_FP32 * size).all()
+
+
+@pytest.mark.parametrize("H,M,N,K,taken", [
+    (242, 175, 94, 134, False), (288, 227, 74, 199, False), (134, 338, 90, 146, True),     # off the grid, before 64x64 tiles in terms and before 128x128
+    (192, 128, 20, 132, True), (191, 128, 20, 132, False)])                                # workgroups a CU
+def test_where_it_runs(hip, H, M, N, K, taken):
+    """Both sides of the limits of the rule (256 CUs)."""
+    say("narrow batches, limits", H, M, N, K)
+    rng = np.random.default_rng(H + M + N)
+    a, b = rng.normal(0, 1, (H, M, K)).astype(np.float32), rng.normal(0, 1, (H, K, N)).astype(np.float32)
+    got = hip.sgemm_batched(hip.array(a), hip.array(b)).numpy()
+    assert (hip.last_kernel() in KERNELS) == taken, hip.last_kernel()
+    for h in (0, H - 1):
+        want, size = a[h].astype(np.float64) @ b[h].astype(np.float64), np.abs(a[h]).astype(np.float64) @ np.abs(b[h]).astype(np.float64)
+        assert (np.abs(got[h] - want) <= BOUND_FP32 * size).all()
 
 
 @pytest.mark.parametrize("H,M,N,name", [(256, 128, 24, KERNELS[0]), (420, 128, 80, KERNELS[0]), (256, 250, 80, KERNELS[1])])
