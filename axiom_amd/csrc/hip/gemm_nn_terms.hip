@@ -247,9 +247,13 @@ int nn_terms(const StagedArgs &g, int64_t batch) {
     // whether the kernels before load straight to LDS, and are on fp32 instructions
     const bool on_grid = (g.K | g.N | g.lda | g.ldb | g.ldc | g.stride_a | g.stride_b | g.stride_c) % 4 == 0 &&
                          ((uintptr_t)g.A | (uintptr_t)g.B | (uintptr_t)g.C) % 16 == 0;
-    // N <= 32 from three quarters of the CUs on (1000 x 1000, 32 of them 39 -> 32; 64 of 256 x 256, 128 workgroups, level), off the grid from
-    // K = 128 on (512 of 100 x 100, N = 17 17.5 and 9.5)
-    if (g.N <= 32) return tiles4 * 4 >= cus * 3 && (on_grid || g.K >= 128) ? launch<1, 4>(g, batch) : -1;
+    if (g.N <= 32) {
+        // From three quarters of the CUs on (1000 x 1000, 32 of them 39 -> 32; 64 of 256 x 256, 128 workgroups, level); from one and a half
+        // where three of eight waves would have no rows and the kernels before have 32-row tiles (132 x 936, N = 4, 99 of them 22.0 -> 28.8, 144 x 144,
+        // N = 4, 146 of them 8.7 -> 11.3).  Cached operands gain more than such from HBM (497 random batches, any N: 1.34 and 1.23).
+        const bool short_rows = on_grid && g.M > 128 && g.M <= 160;
+        return tiles4 * 4 >= cus * (short_rows ? 6 : 3) ? launch<1, 4>(g, batch) : -1;
+    }
     // N = 33..64 as above.  Wider ones need 0.7 of two workgroups a CU (N = 80, 64 of 512 x 512, half of them, 0.97; 96 of 384 x 384,
     // 0.56, 1.16; off the grid, where the kernels before are faster, 0.75), N > 96 K >= 256 (256 of 1024 x 128 82.5 -> 84.1, 200 x 200
     // 109 -> 111).

@@ -29,8 +29,7 @@ def products(hip, a, b, alpha=1.0, pads=(0, 0, 0)):
 
 KS = (64, 65, 95, 96, 128, 159, 256, 291)
 # up to 32 columns, any alignment; more of them on the 16-byte grid (from 96 on with K >= 256 whole tiles only); off it where the staged tiles would be 128x128
-FORMS = [(-(-400 // -(-M // 128)), M, N, K, pads) for pads in [(0, 0, 0), (1, 3, 5)] for M, N in [(96, 1), (128, 17), (129, 32), (300, 31)] for K in KS
-         if K >= 128 or (K % 4 == 0 and N % 4 == 0 and pads[0] == 0)]
+FORMS = [(-(-400 // -(-M // 128)), M, N, K, pads) for pads in [(0, 0, 0), (1, 3, 5)] for M, N in [(96, 1), (128, 17), (129, 32), (300, 31)] for K in KS]
 FORMS += [(-(-400 // -(-M // 128)), M, N, K, pads) for pads in [(0, 0, 0), (4, 8, 4)] for M, N in [(128, 80), (257, 96), (256, 128), (385, 72)] for K in KS
           if K % 4 == 0 and not (N > 96 and K < 256) and not (N >= 96 and K >= 256 and M % 128)]
 FORMS += [(134, 338, 90, 146, (1, 3, 5)), (206, 345, 76, 133, (0, 0, 0)), (62, 966, 76, 210, (1, 3, 5)), (108, 458, 92, 286, (0, 0, 0))]
@@ -53,7 +52,8 @@ def test_every_form(hip, H, M, N, K, pads):
 
 @pytest.mark.parametrize("H,M,N,K,taken", [
     (242, 175, 94, 134, False), (288, 227, 74, 199, False), (134, 338, 90, 146, True),     # off the grid, before 64x64 tiles in terms and before 128x128
-    (192, 128, 20, 132, True), (191, 128, 20, 132, False)])                                # workgroups a CU
+    (146, 144, 4, 144, False), (200, 144, 4, 144, True), (192, 128, 20, 132, True), (191, 128, 20, 132, False),   # rows that exist, workgroups a CU
+    (191, 100, 30, 66, False), (192, 100, 30, 66, True)])                                  # a K of three units, off the grid
 def test_where_it_runs(hip, H, M, N, K, taken):
     """Both sides of the limits of the rule (256 CUs)."""
     say("narrow batches, limits", H, M, N, K)

@@ -102,7 +102,7 @@ def test_staged_w8a32_non_finite(hip, oracle):
 
 @pytest.mark.parametrize("order,Bn,M,N,K,kernel", [
     ("nt", 176, 132, 131, 34, "sgemm_nt_64x64k2_staged"), ("nn", 30, 1168, 35, 32, "sgemm_nn_64x64k2_staged"), ("nt", 13, 543, 543, 32, "sgemm_nt_64x64k2_staged"),
-    ("nt", 338, 294, 294, 65, "sgemm_nt_64x64x3_staged"), ("nt", 56, 447, 449, 69, "sgemm_nt_64x64x3_staged"), ("nn", 70, 800, 22, 96, "sgemm_nn_64x64k2_staged"),
+    ("nt", 338, 294, 294, 65, "sgemm_nt_64x64x3_staged"), ("nt", 56, 447, 449, 69, "sgemm_nt_64x64x3_staged"), ("nn", 70, 800, 34, 96, "sgemm_nn_64x64k2_staged"),
     ("nn", 27, 1084, 85, 162, "sgemm_nn_128x128x3_staged")])
 def test_tile_of_a_short_k(hip, order, Bn, M, N, K, kernel):
     """With a K of one to eight slabs first loads and write-back decide: 64x64 tiles, unless the large ones fill the CUs just once."""
