@@ -583,12 +583,15 @@ k_sdpa_few(const float *__restrict__ Q, const float *__restrict__ K, const float
 }
 
 // Where the few-tiles form pays, by the key tiles that a wave walks one after the other: the longest walk is a quarter of a head's 32-key
-// tiles, all walks together are shared by the CUs, and up to some 2.25 walks of the longest kind a CU it is ahead of k_sdpa, whose
-// four waves each walk all of a head's tiles (us, k_sdpa -> this: 32 heads of [128, 64] 11.4 -> 6.9, 4 of [2048, 64] 111 -> 36, 32 of [512, 64] 33.3
-// -> 22.0, 8 causal ones of [2048, 128] 204 -> 74, 32 causal of [1024, 80] 81.6 -> 74.4; past it 64 of [512, 64] 35.7 -> 38.6, 64 causal of
-// [512, 80] 44.6 -> 55.6).  A single key tile per wave (S up to 128) is mostly start and end: one workgroup a CU, or two of the smaller
-// geometries from three tiles on (128 of [128, 64] 12.1 -> 11.5, but 128 of [128, 128] 21.3 -> 23.2, 256 of [64, 64] 8.1 -> 8.9).  A head of
-// one tile gains nothing (4.6 us either way).
+// tiles, and all walks together are shared by the CUs.  `limit` is four times the longest walks a CU up to which it is ahead of k_sdpa, whose
+// four waves each walk all of a head's tiles: two rounds of workgroups and a little where two share a CU (geometries 32 and 64), two where one has
+// it, one where a walk is two tiles and mostly start and end; causal walks differ in length, and the shorter they all are the sooner the
+// longer geometries fall behind (us, k_sdpa -> this: 32 heads of [128, 64] 11.4 -> 6.9, 4 of [2048, 64] 111 -> 36, 32 of [512, 64] 33.3 -> 22.0, 8 causal ones of
+// [2048, 128] 204 -> 74, 32 causal of [1024, 80] 81.6 -> 74.4; past it 64 of [512, 64] 35.7 -> 38.6, 64 causal of [512, 80] 44.6 -> 55.6, 81 of [216, 128]
+// 30.4 -> 43.2, 100 of [160, 128] 23.6 -> 28.7, 53 of [294, 96] 29.8 -> 37.7, causal 113 of [208, 80] 23.8 -> 34.1, 57 of [507, 128] 60.6 -> 70.8; over 2804 random
+// ones within it 0.91 to 2.8 times as fast).  A single key tile per wave (S up to 128): one workgroup a CU, or two of the smaller geometries from three
+// tiles on (128 of [128, 64] 12.1 -> 11.5, but 128 of [128, 128] 21.3 -> 23.2, 256 of [64, 64] 8.1 -> 8.9).  A head of one tile gains nothing (4.6 us
+// either way).
 // Eight waves on 32 queries: level or behind (32 of [512, 64] 22.0 -> 27.2, 1 of [2048, 64] 32.7 -> 31.1): the vector pipe is the bound.
 template <int DK>
 bool few_tiles(int64_t BH, int64_t S, int causal) {
@@ -596,7 +599,12 @@ bool few_tiles(int64_t BH, int64_t S, int causal) {
     if (tiles < 2 || BH > 4 * cus || tiles > 0xffff) return false;
     if (walk == 1) return tiles * BH <= (DK > 64 || tiles == 2 ? 1 : 2) * cus;
     const int64_t q = tiles / 4, all = causal ? 2 * q * (q + 1) + tiles % 4 * (q + 1) : tiles * walk;
-    return all * BH * 4 <= 9 * walk * cus;
+    int64_t limit = 9;
+    if (causal && DK > 64) limit = walk + (DK == 96 ? 2 : 1) < 7 ? walk + (DK == 96 ? 2 : 1) : 7;
+    else if (causal && DK == 64 && walk == 2) limit = 5;
+    else if (!causal && DK > 64) limit = walk == 2 ? 4 : 8;
+    else if (!causal && DK == 64 && walk <= 3) limit = 8;
+    return all * BH * 4 <= limit * walk * cus;
 }
 
 template <int DK>

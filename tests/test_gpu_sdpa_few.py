@@ -11,7 +11,11 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("BH,S,dk,causal,few", [(256, 32, 64, 0, False), (128, 64, 64, 0, True), (129, 64, 64, 1, False),
                                                 (128, 128, 64, 0, True), (129, 128, 32, 0, False), (64, 97, 96, 1, True), (65, 128, 128, 0, False),
-                                                (36, 512, 64, 0, True), (37, 512, 80, 0, False), (57, 512, 128, 1, True), (58, 512, 64, 1, False)])
+                                                (36, 512, 64, 0, True), (37, 512, 80, 0, False), (57, 512, 64, 1, True), (58, 512, 64, 1, False),
+                                                (32, 512, 128, 1, True), (33, 512, 128, 1, False), (36, 224, 96, 0, True), (37, 224, 96, 0, False),
+                                                (51, 300, 128, 0, True), (52, 300, 128, 0, False), (53, 256, 64, 1, True), (54, 256, 64, 1, False),
+                                                (85, 150, 80, 1, True), (86, 150, 80, 1, False), (64, 256, 64, 0, True), (65, 256, 64, 0, False),
+                                                (25, 993, 96, 1, False), (36, 512, 32, 1, True)])
 def test_where_it_runs(hip, BH, S, dk, causal, few):
     """Both sides of each limit of the rule (256 CUs)."""
     say("sdpa few", BH, S, dk, causal)
