@@ -232,7 +232,7 @@ namespace axhip {
 // In terms from K = 113 on, with limits to K from operands that are cached and operands from HBM (the strips have two steps under way and
 // wait longer for memory than the kernels before).  us, before -> here, cached / from HBM: 1024 x 256 x 1024 12.3 / 12.7 -> 8.5 / 10.1, 384 x 128 x
 // 700 10.5 / 11.0 -> 7.3 / 9.0, A B^T 256 x 768 x 896 11.5 / 12.5 -> 8.3 / 9.6, 500 x 300 x 640 11.0 / 11.9 -> 7.1 / 8.4, A^T B 1024 x 256 x 1280 13.1 / 13.5 ->
-// 10.4 / 11.7; past the limits 1588 x 22 x 973 9.8 / 10.5 -> 8.6 / 12.0, 1446 x 65 x 1208 11.8 / 12.8 -> 10.2 / 14.0, A B^T 57 x 1598 x 893 9.9 / 11.3 -> 8.9 / 12.7;
+// 10.4 / 11.7, up to eight tiles 128 x 10 x 1024 9.4 / 9.6 -> 7.8 / 8.4, A^T B 97 x 31 x 1000 9.9 / 10.1 -> 8.3 / 8.9; past the limits 1588 x 22 x 973 9.8 / 10.5 -> 8.6 / 12.0, 1446 x 65 x 1208 11.8 / 12.8 -> 10.2 / 14.0, A B^T 57 x 1598 x 893 9.9 / 11.3 -> 8.9 / 12.7;
 // 1024 x 1024 x 256 cached 8.2 -> 9.5, and A B^T on 336 tiles with K = 476, with its extra turn, 8.9 -> 9.7.
 // Two workgroups share a CU from 257 tiles on: four waves each (86 x 3584 x 300: eight 6.4, four 5.6); but
 // eight on up to a third of the CUs with K above 400, where ranges of K on 64x64 tiles would have the smaller error than four long strips (geometric
@@ -256,7 +256,8 @@ int strips_f32(const StagedArgs &g, int transa, int transb, bool on_grid) {
         return launch<4, false, false, false, 4>("sgemm_tn_strips32", g);
     }
     const bool many = tiles >= 128;
-    const int64_t most = transb ? (many ? 896 : 640) : !many ? 800 : transa ? 1280 : 1024;
+    const bool ranges_in_terms = !on_grid || g.K % 32 != 0;      // what stands behind a longer K: ranges on the staged tiles in terms, or on fp32 ones
+    const int64_t most = transb ? (many ? 896 : 640) : many ? (transa ? 1280 : 1024) : ranges_in_terms && (transa || tiles <= 8) ? 1024 : 800;
     const bool third = tiles * 3 <= cus * 4;                   // two workgroups on a third of the CUs at most
     if (g.K <= (on_grid ? 112 : 120) || !((one && g.K <= most) || (two && !transb && g.K <= (third ? 640 : 800)))) return -1;
     if (!one && third && g.K > 400)
