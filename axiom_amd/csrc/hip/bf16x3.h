@@ -88,7 +88,7 @@ __device__ __forceinline__ void look_at(const v16f &sum, float &seen) {
 #pragma unroll
     for (int v = 0; v < 16; v++) seen = __builtin_fmaf(sum[v], 0.0f, seen);
 }
-// Whether any lane of the workgroup's WAVES waves (4 or 8) says so, through a word of LDS per wave.  Every wave calls it; it holds a barrier.
+// Whether any lane of the workgroup's WAVES waves (a multiple of four) says so, through a word of LDS per wave.  Every wave calls it; it holds a barrier.
 template <int WAVES>
 __device__ __forceinline__ bool any_wave(bool says, unsigned char *words, int wave) {
     int *word = reinterpret_cast<int *>(words);

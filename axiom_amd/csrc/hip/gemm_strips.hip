@@ -5,12 +5,15 @@
 // What bounds such products is not the matrix core but latency: the launch, the first trip to memory, the loop's barriers where waves
 // share slabs through LDS, and a second launch where K is cut into ranges to fill the chip.  Here the chip is filled by small tiles, no wave
 // waits for another before the end, and a value is cut once per tile.  Two steps of 16 k are under way per wave.
-// us, before -> here (on what): 128 x 1024 x 784 11.6 -> 7.9, 300 x 333 x 777 11.1 -> 8.6, 1024 x 256 x 1024 12.3 -> 8.6 (two launches: ranges of K), 40 x
+// us, before -> here (on what), cached operands: 128 x 1024 x 784 11.6 -> 7.9, 300 x 333 x 777 11.1 -> 8.6, 1024 x 256 x 1024 12.3 -> 8.6 (two launches: ranges of K), 40 x
 // 500 x 300 9.5 -> 5.9 (64x64 tiles in bf16 terms), 1024 x 256 x 256 5.9 -> 5.1 (32x64 tiles on fp32 instructions), 128 x 1024 x 10 6.6 -> 3.9 (guarded
-// tiles), 1024 x 256 x 256 A^T B 9.5 -> 5.4; geometric mean over some 800 random products that the rule below takes 1.35.  Past it the vector pipe
-// (6.5 instructions a value and 64 values a column of k) and the loads (64 rows a tile) take over: 1024^3 20 -> 25, 100 x 10 x 4096 11 -> 22.
-// The five smaller products of terms have a sum of their own, the others two in turn, and the strips are added in pairs: relative error against
-// 64 bits 7.4e-8 at K = 1024 (ranges of K in terms 7.6e-8, 64x64 tiles in terms 1.2e-7, fp32 instructions 4.1e-7).
+// tiles), 1024 x 256 x 256 A^T B 9.5 -> 5.0; geometric mean over 2818 random products that the rule below takes 1.29, operands from HBM 1.28 (in terms 1.39
+// and 1.36).  Past it the vector pipe (6.5 instructions a value and 64 values a column of k) and the loads (64 rows a tile) take over: 1024^3 20 ->
+// 25, 100 x 10 x 4096 11 -> 22.
+// The five smaller products of terms have a sum of their own, the others one, or two in turn where a wave has the registers (eight waves with one
+// tile a CU), and the strips are added in pairs: relative error against 64 bits 7.1e-8 at K = 1024 on eight or sixteen waves (ranges of K in terms
+// 7.6e-8, 64x64 tiles in terms 1.2e-7, fp32 instructions 4.1e-7), on four 8.1e-8 at K = 784 (ranges 8.1e-8).  A sum with a single product that is
+// not zero is off by up to 1.7 units of 2^-24, where fp32 instructions round it (1.0).
 //
 // Loads.  An operand stored along K against one stored across it: a lane reads its 32 bytes of its row in place.  Both along K
 // (A B^T): twice as many scattered lines would bound the kernel (1024 x 256 x 1024 21 us), so 64-byte pieces are loaded 16 rows at a time and

@@ -129,7 +129,7 @@ int   axhip_memcpy_d2d(void *device_dst, const void *device_src, size_t bytes);
  *      transb = 0: B is [K,N] (ldb >= N);  1: B is [N,K] (ldb >= K)
  *      bias may be NULL; beta == 0 never reads C (C may be uninitialised).
  *      fp32 accuracy throughout.  Products are formed by fp32 instructions or, mostly large and ragged
- *      ones, on the bf16 matrix core with each operand as the exact sum of three bf16 terms: six products
+ *      ones and those with few tiles and K from about 120 up, on the bf16 matrix core with each operand as the exact sum of three bf16 terms: six products
  *      of terms stand for one (what they leave out is at most 2^-24 of it), added in fp32.  For every finite
  *      operand, however small; sums that leave fp32's range or that infinities and NaNs enter come out
  *      as fp32 instructions give them.  M <= 16 with transa = transb = 0, alpha = 1, beta = 0 takes
