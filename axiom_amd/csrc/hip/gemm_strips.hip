@@ -7,8 +7,8 @@
 // waits for another before the end, and a value is cut once per tile.  Two steps of 16 k are under way per wave.
 // us, before -> here (on what), cached operands: 128 x 1024 x 784 11.6 -> 7.9, 300 x 333 x 777 11.1 -> 8.6, 1024 x 256 x 1024 12.3 -> 8.6 (two launches: ranges of K), 40 x
 // 500 x 300 9.5 -> 5.9 (64x64 tiles in bf16 terms), 1024 x 256 x 256 5.9 -> 5.1 (32x64 tiles on fp32 instructions), 128 x 1024 x 10 6.6 -> 3.9 (guarded
-// tiles), 1024 x 256 x 256 A^T B 9.5 -> 5.0; geometric mean over 2818 random products that the rule below takes 1.29, operands from HBM 1.28 (in terms 1.39
-// and 1.36).  Past it the vector pipe (6.5 instructions a value and 64 values a column of k) and the loads (64 rows a tile) take over: 1024^3 20 ->
+// tiles), 1024 x 256 x 256 A^T B 9.5 -> 5.0; geometric mean over 2612 random products that the rule below takes 1.33, operands from HBM 1.31 (in terms 1.41
+// and 1.38).  Past it the vector pipe (6.5 instructions a value and 64 values a column of k) and the loads (64 rows a tile) take over: 1024^3 20 ->
 // 25, 100 x 10 x 4096 11 -> 22.
 // The five smaller products of terms have a sum of their own, the others one, or two in turn where a wave has the registers (eight waves with one
 // tile a CU), and the strips are added in pairs: relative error against 64 bits 7.1e-8 at K = 1024 on eight or sixteen waves (ranges of K in terms
@@ -232,10 +232,12 @@ int launch(const char *name, const StagedArgs &g) {
 }  // namespace
 
 namespace axhip {
-// In terms from K = 113 on, with limits to K from operands that are cached and operands from HBM (the strips have two steps under way and
-// wait longer for memory than the kernels before).  us, before -> here, cached / from HBM: 1024 x 256 x 1024 12.3 / 12.7 -> 8.5 / 10.1, 384 x 128 x
-// 700 10.5 / 11.0 -> 7.3 / 9.0, A B^T 256 x 768 x 896 11.5 / 12.5 -> 8.3 / 9.6, 500 x 300 x 640 11.0 / 11.9 -> 7.1 / 8.4, A^T B 1024 x 256 x 1280 13.1 / 13.5 ->
-// 10.4 / 11.7, up to eight tiles 128 x 10 x 1024 9.4 / 9.6 -> 7.8 / 8.4, A^T B 97 x 31 x 1000 9.9 / 10.1 -> 8.3 / 8.9; past the limits 1588 x 22 x 973 9.8 / 10.5 -> 8.6 / 12.0, 1446 x 65 x 1208 11.8 / 12.8 -> 10.2 / 14.0, A B^T 57 x 1598 x 893 9.9 / 11.3 -> 8.9 / 12.7;
+// In terms from K = 113 on.  The limits to K lie where the geometric mean of the gains with operands cached and operands from HBM falls to one: two
+// steps under way wait longer for memory than the kernels behind, which gain as much there as they lose cached, and have a second launch to be issued
+// (a training step of a 384-896-216 classifier, batch 160, 70.6 us with 160 x 216 x 896 here and 74.3 on ranges of K).  us, before -> here, cached / from
+// HBM: 1024 x 256 x 1024 12.3 / 12.7 -> 8.5 / 10.1, 384 x 128 x 700 10.5 / 11.0 -> 7.3 / 9.0, 128 x 10 x 1024 9.4 / 9.6 -> 7.8 / 8.4, A B^T 256 x 768 x 896 11.5 / 12.5
+// -> 8.3 / 9.6, 500 x 300 x 640 11.0 / 11.9 -> 7.1 / 8.4, A^T B 1024 x 256 x 1280 13.1 / 13.5 -> 10.4 / 11.7, 97 x 31 x 1000 9.9 / 10.1 -> 8.3 / 8.9; near the limits 1588 x
+// 22 x 973 9.8 / 10.5 -> 8.6 / 12.0, 1446 x 65 x 1208 11.8 / 12.8 -> 10.2 / 14.0, past them A B^T 57 x 1598 x 893 9.9 / 11.3 -> 8.9 / 12.7, 96 x 64 x 896 7.3 / 7.4 -> 7.8 / 8.2, 72 x 1354 x 1317 12.3 / 13.6 -> 13.4 / 14.7;
 // 1024 x 1024 x 256 cached 8.2 -> 9.5, and A B^T on 336 tiles with K = 476, with its extra turn, 8.9 -> 9.7.
 // Two workgroups share a CU from 257 tiles on: four waves each (86 x 3584 x 300: eight 6.4, four 5.6); but
 // eight on up to a third of the CUs with K above 400, where ranges of K on 64x64 tiles would have the smaller error than four long strips (geometric
@@ -260,7 +262,10 @@ int strips_f32(const StagedArgs &g, int transa, int transb, bool on_grid) {
     }
     const bool many = tiles >= 128;
     const bool ranges_in_terms = !on_grid || g.K % 32 != 0;      // what stands behind a longer K: ranges on the staged tiles in terms, or on fp32 ones
-    const int64_t most = transb ? (many ? 896 : 640) : many ? (transa ? 1280 : 1024) : ranges_in_terms && (transa || tiles <= 8) ? 1024 : 800;
+    const int64_t most = many              ? (transb ? 1088 : g.M < 96 ? 1024 : 1536)
+                         : ranges_in_terms ? (transb ? 864 : 1024)
+                         : tiles > 24      ? (transb ? 832 : 896)
+                                           : (transb ? 800 : 864);
     const bool third = tiles * 3 <= cus * 4;                   // two workgroups on a third of the CUs at most
     if (g.K <= (on_grid ? 112 : 120) || !((one && g.K <= most) || (two && !transb && g.K <= (third ? 640 : 800)))) return -1;
     if (!one && third && g.K > 400)
