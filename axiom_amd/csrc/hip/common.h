@@ -18,6 +18,11 @@ int cu_count();
 void note_kernel(const char *name);
 // Checks the launch that was just issued on the null stream.
 int check_launch(const char *what);
+// What the workspace holds from axhip_init on: 288 GB of memory make room for the planes of terms of every product that pays for them up to
+// 2048 x 4096 x 4096 (gemm_planes.hip).
+constexpr size_t kWorkspaceStart = size_t(160) << 20;
+// What it holds now.
+size_t workspace_bytes();
 // A device workspace of at least `bytes`, owned by the runtime (grown on demand), or NULL.
 void *workspace(size_t bytes);
 // `n` zero-initialised device ints owned by the runtime.  Kernels that use them as arrival counters

@@ -22,6 +22,13 @@ struct StagedArgs {
 int staged_f32(const StagedArgs &g, int transa, int transb, int64_t batch, bool may_split);
 // The same products in bf16 terms on the bf16 matrix core, at fp32 accuracy.
 int split_f32(const StagedArgs &g, int transa, int transb, int64_t batch, bool may_split);
+// What split_f32 would choose for a single product whose K may be cut into ranges, and the time that it reckons with.
+struct StagedChoice {
+    bool is_128x128;
+    int64_t ranges;
+    float us;
+};
+StagedChoice split_choice(const StagedArgs &g);
 // Whether split_f32 would form this batch on its 128x128 tiles.
 bool split_is_128x128(const StagedArgs &g, int64_t batch);
 int staged_i8w(const StagedArgs &g);

@@ -605,6 +605,10 @@ int split_f32(const StagedArgs &g, int transa, int transb, int64_t batch, bool m
     return run_split<false, false>(g, batch, may_split, tn, kSplitTermsName);
 }
 
+StagedChoice split_choice(const StagedArgs &g) {
+    const Plan p = plan_staged(g, 1, kSplitTiles, 4, true);
+    return {p.tile == 0, p.splits, p.us};
+}
 bool split_is_128x128(const StagedArgs &g, int64_t batch) { return g.K >= 64 && plan_staged(g, batch, kSplitTiles, 4, false).tile == 0; }
 
 int staged_f32(const StagedArgs &g, int transa, int transb, int64_t batch, bool may_split) {

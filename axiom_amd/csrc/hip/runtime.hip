@@ -125,6 +125,8 @@ int check_launch(const char *what) {
     return AXHIP_OK;
 }
 
+size_t workspace_bytes() { return g_ws_bytes; }
+
 void *workspace(size_t bytes) {
     if (bytes <= g_ws_bytes) return g_ws;
     if (g_ws) {
@@ -262,9 +264,9 @@ int axhip_init(void) {
         return fail(AXHIP_ERR_BACKEND, "device 0 is %s; this library holds gfx950 code only",
                     prop.gcnArchName);
     if (int rc = axhip::skinny_setup()) return rc;
-    // the shared workspace and the arrival counters exist from the start (64 MiB, 4096 counters): a first
-    // call at a new shape then pays no allocation or device-wide wait unless it needs more than that
-    if (!axhip::workspace(size_t(64) << 20) || !axhip::strip_counters(4096)) return AXHIP_ERR_ALLOC;
+    // the shared workspace and the arrival counters exist from the start (160 MiB, or 64 on a device that is nearly full; 4096 counters): a
+    // first call at a new shape then pays no allocation or device-wide wait unless it needs more than that
+    if ((!axhip::workspace(axhip::kWorkspaceStart) && !axhip::workspace(size_t(64) << 20)) || !axhip::strip_counters(4096)) return AXHIP_ERR_ALLOC;
     g_ready = 1;
     return AXHIP_OK;
 }

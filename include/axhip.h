@@ -103,7 +103,7 @@ void  axhip_reset_alloc_stats(void);
 /* Bytes of device memory the driver reports free on the current device (hipMemGetInfo), or -1 without
  * a device.  The counterpart of what cudaMemGetInfo gives a caller of the reference's CUDA backend. */
 int64_t axhip_device_free_bytes(void);
-/* The shared device workspace (split-K partial sums, reduction partials, padded operand copies) is 64 MiB
+/* The shared device workspace (split-K partial sums, reduction partials, operands cut into bf16 terms, padded copies) is 160 MiB
  * from axhip_init on and grows when a call needs more; growing waits for the device, frees the old block and asks the
  * driver for a new one, which costs the first call at a larger shape some tens of microseconds that later
  * calls do not pay.  axhip_workspace_reserve grows it ahead of time (at model load, before a timed or
