@@ -24,9 +24,9 @@
 // A tile with a sum that is not finite is computed again with fp32 instructions by the same workgroup:
 // infinities, NaNs and values near the largest float come out as fp32 products give them.
 // us, fp32 instructions -> terms: 512 heads of [512, 64] 269 -> 194 (causal 178 -> 126), 64 of [1024, 128] 273 -> 174, 96 causal
-// ones of [1000, 80] 324 -> 129 (a quarter of that from the 96-wide geometry), 512 of [256, 32] 41 -> 33; with few query tiles for the
+// ones of [1000, 80] 324 -> 108 (a quarter of that from the 96-wide geometry), 512 of [256, 32] 41 -> 33; with few query tiles for the
 // CUs k_sdpa_few cuts a head along its keys too (32 heads of [128, 64] 11.4 -> 6.9).  O is nearer to 64 bits on every shape measured (relative error 4.9e-7 -> 3.7e-7 at [512, 64]).  Bound: the matrix core is
-// busy 49 % of the cycles, vector instructions (cutting, softmax) take some 44 ([512, 64]; causal [1000, 80] 37 and 29, whose 192 workgroups of paired tiles leave a quarter of the CUs without one).  Measured and dropped: two key tiles at a time,
+// busy 49 % of the cycles, vector instructions (cutting, softmax) take some 44 ([512, 64]).  Measured and dropped: two key tiles at a time,
 // the scores of one interleaved with the exponentials of the other by instruction groups ([512, 64] 194, [1024, 96] 126 -> 128).
 //
 // Every other head size: scores through a workspace, one batched NT GEMM, a row softmax kernel and
@@ -163,19 +163,27 @@ k_sdpa(const float *__restrict__ Q, const float *__restrict__ K, const float *__
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     const int64_t nq = (S + BQ - 1) / BQ;
-    // Workgroups are handed to the 8 XCDs round-robin by linear index, and inside an XCD to its
-    // CUs in a fixed rotation, so every workgroup has to carry the same amount of work.  Eight
+    // Workgroups go to the 8 XCDs round-robin by linear index, inside an XCD to whichever CU has room.  Eight
     // heads form a group: workgroup r of a group works on head r % 8 (every query tile of a
-    // head then runs on the same XCD and shares its L2 copy of K and V) and on unit r / 8.
-    // A unit is one query tile, or, causal, the pair of tiles p and nq-1-p, which together
-    // visit the same number of keys whatever p is (the middle tile of an odd nq stands alone).  A launch
-    // with no more single tiles than CUs keeps them single (pair_tiles = 0): pairing would only
-    // halve the CUs at work.
+    // head then runs on the same XCD and shares its L2 copy of K and V) and on unit r / 8, a query tile.
+    // Causal tiles visit more keys the later they are: single ones go out longest first over all heads, so that the short ones even out the
+    // ends (us, pairs -> this, both on eight waves unless said: 96 heads of [1000, 80] 122 -> 108, 61 of [1472, 80] 162 -> 146, 218 of [655, 128] 286 -> 227; on four
+    // 145 of [192, 32] 16.2 -> 11.1, 193 of [832, 64] 159 -> 121; 2 % of that is from L2 copies no longer shared).
+    // pair_tiles: a unit is the pair of tiles p and nq-1-p, which together visit the same number of keys whatever p is (the
+    // middle tile of an odd nq stands alone).
     const bool paired = CAUSAL && pair_tiles;
     const int64_t units = paired ? (nq + 1) / 2 : nq;
-    const int64_t lin = blockIdx.x, group = lin / (8 * units), left = BH - group * 8;
-    const int64_t r = lin - group * 8 * units, hpg = left < 8 ? left : 8;
-    const int64_t head = group * 8 + r % hpg, unit = r / hpg;
+    int64_t head, unit;
+    if (CAUSAL && !paired) {
+        const unsigned longer = blockIdx.x / (unsigned)BH;
+        unit = nq - 1 - longer;
+        head = blockIdx.x - longer * (unsigned)BH;
+    } else {
+        const int64_t lin = blockIdx.x, group = lin / (8 * units), left = BH - group * 8;
+        const int64_t r = lin - group * 8 * units, hpg = left < 8 ? left : 8;
+        head = group * 8 + r % hpg;
+        unit = r / hpg;
+    }
     const int passes = (paired && unit != nq - 1 - unit) ? 2 : 1;
     // head b * H + h starts at row b * S, column h * DK of matrices with row pitch ld (Q, K, V)
     // and ldo (O): H = 1, ld = DK is one matrix per head; H heads side by side in rows of
@@ -641,9 +649,10 @@ int launch_sdpa_p(const float *Q, const float *K, const float *V, float *O, floa
     }
     const float sl2 = scale * 1.4426950408889634f;
     const int64_t nq = (S + G::BQ - 1) / G::BQ;
-    // causal tiles p and nq-1-p in one workgroup once there are more tiles than CUs; with a CU for every tile the
-    // longest tile sets the time either way and pairing only halves the CUs at work
-    const int pair = causal && nq * BH > (int64_t)cu_count();
+    // causal tiles p and nq-1-p in one workgroup where the pairs give every CU the same number of keys, or nearly: [512, 64] x 512, [2048, 64] x 32 and
+    // [1024, 128] x 64 single 128.4, 129.2, 136.5 us, paired 127.4, 126.8, 134.2 (the 96-wide geometry [1024, 96] x 64 100.9 against 108)
+    const int64_t cus = cu_count(), pairs = (nq + 1) / 2 * BH, rounds = (pairs + cus - 1) / cus;
+    const int pair = causal && WAVES == 4 && (DK == 64 || DK == 128) && rounds * cus * 30 <= nq * BH * 16;
     dim3 grid((unsigned)((pair ? (nq + 1) / 2 : nq) * BH)), block(64 * WAVES);
     if (causal)
         hipLaunchKernelGGL((k_sdpa<DK, WAVES, true, PAD>), grid, block, G::SMEM, kStream, Q, K, V, O, L, BH, S, sl2, H, ld, ldo, dkr, pair);
@@ -656,13 +665,26 @@ template <int DK>
 int launch_sdpa(const float *Q, const float *K, const float *V, float *O, float *L, int64_t BH, int64_t S,
                 float scale, int causal, int64_t H, int64_t ld, int64_t ldo, int dkr) {
     // Eight waves on 256 queries cut half as much of K and V for each of them, four on 128 waste less of a short head and
-    // of the diagonal.  us, four waves -> eight: 64 heads of [1024, 128] 191 -> 174 (causal 158 -> 142), 64 of [1024, 96]
-    // 141 -> 126, 96 causal ones of [1000, 80] 146 -> 129, 512 of [512, 64] 201 -> 194; but causal 126 -> 134, 512 of [256, 32]
-    // 33 -> 37, 256 causal ones of [333, 48] 49 -> 53.  Geometry
+    // of the diagonal.  us, four waves -> eight: 64 heads of [1024, 128] 191 -> 174, 64 of [1024, 96]
+    // 141 -> 126, 96 causal ones of [1000, 80] 116 -> 108, 512 of [512, 64] 201 -> 194; but causal 128 -> 142, 512 of [256, 32]
+    // 33 -> 37, 256 causal ones of [333, 48] 40 -> 44.  Geometry
     // 128 has the registers of one wave per SIMD with four waves, so it takes eight as soon as there is more than one tile a CU.
     if constexpr (DK > 32) {
-        const int64_t half_tiles = (S + 127) / 128, tiles = (S + 255) / 256;
-        if (DK == 128 ? half_tiles * BH > cu_count() : DK >= (causal ? 96 : 64) && tiles * BH >= cu_count() && tiles * 8 <= half_tiles * 5)
+        const int64_t half_tiles = (S + 127) / 128, tiles = (S + 255) / 256, cus = cu_count();
+        const bool fits = tiles * 8 <= half_tiles * 5;
+        bool eight;
+        if (!causal) eight = DK == 128 ? half_tiles * BH > cus : DK >= 64 && tiles * BH >= cus && fits;
+        else {
+            // single causal tiles: three of 128 queries or two of 256, where the latter have a CU each (us, four -> eight: 99 heads of [381, 96] 40 -> 31, 95 of
+            // [322, 64] 27 -> 23, 120 of [314, 128] 57 -> 49 but 50 of [316, 128], whose three have one too, 43 -> 48; 129 of [280, 80] 35 -> 48); geometry 128
+            // a little under two rounds of them, too (219 of [384, 128] 103 -> 97, 186 of [448, 128] 119 -> 113), and from nine blocks of 128 x 128 a CU on (238 of [512, 128] 163 -> 134, 60 of [832, 128] 109 -> 113)
+            // geometry 128 two or one by their rounds (178 of [192, 128] 46 -> 37, 430 of [208, 128] 98 -> 87, but 124 of [190, 128] 28 -> 37)
+            eight = half_tiles == 3 && 2 * BH <= cus && (DK != 128 || 3 * BH > cus);
+            if (DK == 128 && half_tiles == 2) eight = (BH + cus - 1) / cus * 5 < (2 * BH + cus - 1) / cus * 3;
+            else if (DK == 128) eight = eight || (half_tiles == 3 && BH <= cus && 6 * BH > 5 * cus) || (half_tiles == 4 && 10 * BH >= 7 * cus) || (half_tiles + 1) * half_tiles * BH > 18 * cus;
+            if (DK == 96) eight = eight || ((tiles == 1 ? BH > cus : tiles * BH * 2 >= cus) && fits);
+        }
+        if (eight)
             return dkr == DK ? launch_sdpa_p<DK, 8, false>(Q, K, V, O, L, BH, S, scale, causal, H, ld, ldo, dkr)
                              : launch_sdpa_p<DK, 8, true>(Q, K, V, O, L, BH, S, scale, causal, H, ld, ldo, dkr);
     }
