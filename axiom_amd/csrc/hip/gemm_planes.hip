@@ -8,9 +8,10 @@
 // power cap (2000 x 4096 x 1024 the product alone 80 -> 72 us, 1.4 PFLOP/s of bf16 products; with 64 of 256 CUs at work it is at 87 % of the peak).
 // us, staged tiles -> this, both launches, back to back: 2000 x 4096 x 1024 99 -> 82, 2000 x 3072 x 1024 106 -> 73, 2048 x 4096 x 4096 352 -> 286, A B^T
 // 2112 x 2432 x 2403 206 -> 149, A^T B 1288 x 3985 x 767 82 -> 59.
-// Bound: power with every CU at work on 256x128 tiles; 128x64 ones the LDS pipe (read 18 KiB a wave and 48 products, 48 bytes a cycle written beside it).
-// Measured and dropped: four waves of 128x64 on a 256x128 tile (one wave a SIMD leaves its waits bare: 72 -> 92), 128x128 on four waves (86), and two
-// sets of waves over K on 128x64 for one tile a CU (a stage then arrives later than it is wanted: 1024^3 31, 2000 x 1024 x 4096 98).
+// Bound: 256x128 tiles, power with every CU at work; 128x64 ones, what L2 hands to the CUs (36 KiB per tile and 32 k: 2000 x 3072 x 1024 906 MB in 59 us, 15.4
+// TB/s; the same rate where A's fragments go to registers without LDS, where sets of waves share K, and with a ring of four stages).
+// Measured and dropped: four waves of 128x64 on a 256x128 tile (one wave a SIMD leaves its waits bare: 72 -> 92), 128x128 on four waves (86), and for one
+// 128x64 tile a CU two sets of waves over K, or fragments of A straight to registers (2000 x 1024 x 4096 98 and 117 where the staged tiles take 104).
 #include "gemm_planes.h"
 
 #include "bf16x3.h"

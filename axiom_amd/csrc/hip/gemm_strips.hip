@@ -1,6 +1,6 @@
-// Single fp32 products with few tiles and a K of some hundred, in one launch: a workgroup of four to sixteen waves owns one 32x32 tile of C, and
+// Single fp32 products with few tiles, in one launch: a workgroup of four to sixteen waves owns one 32x32 tile of C, or one range of K of it, and
 // every wave forms the whole tile over its own strip of K, straight from memory, in three bf16 terms per operand (bf16x3.h); the strips meet
-// in LDS, in a fixed order.
+// in LDS, in a fixed order, and the ranges in memory, where the last workgroup of a tile to arrive adds them, in a fixed order too.
 //
 // What bounds such products is not the matrix core but latency: the launch, the first trip to memory, the loop's barriers where waves
 // share slabs through LDS, and a second launch where K is cut into ranges to fill the chip.  Here the chip is filled by small tiles, no wave
@@ -29,8 +29,14 @@ using namespace axhip;
 
 constexpr int TILE = 32, CPITCH = TILE + 4, PART = TILE * CPITCH;        // floats of a wave's part of the tile
 
-template <int WAVES, bool TERMS, bool A_KC, bool B_KC, int PER_SIMD>
-__global__ void __launch_bounds__(64 * WAVES, PER_SIMD) k_gemm_strips(StagedArgs g) {
+struct Meeting {                 // of ranges of K: a part of each tile for each, a counter for each tile
+    float *parts;
+    int *arrivals;
+};
+
+// RANGES: the workgroup has the range blockIdx.y of K (an argument of the kernel without it costs one with K = 256 0.3 us).
+template <int WAVES, bool TERMS, bool A_KC, bool B_KC, int PER_SIMD, bool RANGES>
+__global__ void __launch_bounds__(64 * WAVES, PER_SIMD) k_gemm_strips(StagedArgs g, std::conditional_t<RANGES, Meeting, int> meeting) {
     constexpr bool TURN = A_KC && B_KC;
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -41,9 +47,14 @@ __global__ void __launch_bounds__(64 * WAVES, PER_SIMD) k_gemm_strips(StagedArgs
     const char *abase = reinterpret_cast<const char *>(static_cast<const float *>(g.A) + (A_KC ? m0 * g.lda : m0));
     const char *bbase = reinterpret_cast<const char *>(static_cast<const float *>(g.B) + (B_KC ? n0 * g.ldb : n0));
     const int mlast = (int)(g.M - 1 - m0 < TILE - 1 ? g.M - 1 - m0 : TILE - 1), nlast = (int)(g.N - 1 - n0 < TILE - 1 ? g.N - 1 - n0 : TILE - 1);
-    // steps of 16 k; this wave's strip is [s0, s1)
-    const int steps = (int)((g.K + 15) / 16);
-    const int s0 = (int)((int64_t)steps * wave / WAVES), s1 = (int)((int64_t)steps * (wave + 1) / WAVES);
+    // steps of 16 k; this workgroup's are `steps` from `first` on, this wave's strip of them is [s0, s1)
+    int first = 0, steps = (int)((g.K + 15) / 16);
+    if constexpr (RANGES) {
+        const int64_t all = steps;
+        first = (int)(all * blockIdx.y / gridDim.y);
+        steps = (int)(all * (blockIdx.y + 1) / gridDim.y) - first;
+    }
+    const int s0 = first + (int)((int64_t)steps * wave / WAVES), s1 = first + (int)((int64_t)steps * (wave + 1) / WAVES);
 
     // ---- loads: in place, a lane's 8 k (8 h + e) of row r32; turned, four k of rows 16 q + lane / 4 ----
     std::integral_constant<bool, A_KC> akc;
@@ -175,18 +186,19 @@ __global__ void __launch_bounds__(64 * WAVES, PER_SIMD) k_gemm_strips(StagedArgs
 #pragma unroll
         for (int v = 0; v < 16; v++) acc[v] = 0.0f;
         const int row = r32 < mlast ? r32 : mlast, col = r32 < nlast ? r32 : nlast;
-        for (int64_t k0 = 2 * wave; k0 < g.K; k0 += 2 * WAVES) {
-            const int64_t k = k0 + h, ke = k < g.K ? k : g.K - 1;
+        const int64_t kend = RANGES && (int64_t)(first + steps) * 16 < g.K ? (int64_t)(first + steps) * 16 : g.K;
+        for (int64_t k0 = (int64_t)first * 16 + 2 * wave; k0 < kend; k0 += 2 * WAVES) {
+            const int64_t k = k0 + h, ke = k < kend ? k : kend - 1;
             const float a = *reinterpret_cast<const float *>(abase + (A_KC ? row * lda4 + ke * 4 : ke * lda4 + row * 4));
             const float b = *reinterpret_cast<const float *>(bbase + (B_KC ? col * ldb4 + ke * 4 : ke * ldb4 + col * 4));
-            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(k < g.K ? b : 0.0f, k < g.K ? a : 0.0f, acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(k < kend ? b : 0.0f, k < kend ? a : 0.0f, acc, 0, 0, 0);
         }
         put(1.0f);
         __syncthreads();
     }
     const int row = tid / 8, cg = (tid & 7) * 4;       // four columns of a row each, from the first 256 threads
     const int64_t m = m0 + row, col = n0 + cg;
-    if (tid >= TILE * TILE / 4 || m >= g.M || col >= g.N) return;
+    if (tid >= TILE * TILE / 4) return;                // (whole waves: they no longer count at barriers)
     v4f p[WAVES];                                      // added in pairs (sixteen in a row: error 8.9e-8 at K = 1024)
 #pragma unroll
     for (int w = 0; w < WAVES; w++) p[w] = *reinterpret_cast<const v4f *>(part + w * PART + row * CPITCH + cg);
@@ -195,9 +207,47 @@ __global__ void __launch_bounds__(64 * WAVES, PER_SIMD) k_gemm_strips(StagedArgs
 #pragma unroll
         for (int w = 0; w < WAVES; w += 2 * by) p[w] += p[w + by];
     v4f o = p[0];
+    o *= down;
+    if constexpr (RANGES) {
+        // The ranges meet in memory: every workgroup leaves its part, and the last one to arrive on the tile's counter adds them in order.  Parts, counter
+        // and the reads below are device-scope accesses (the workgroups run on XCDs with an L2 each); the wait makes a thread's stores complete before the
+        // barrier, the barrier orders them before thread 0's increment.
+        typedef float v2f __attribute__((ext_vector_type(2)));
+        const int ranges = gridDim.y;
+        int64_t *slots = reinterpret_cast<int64_t *>(meeting.parts + (int64_t)blockIdx.x * ranges * (TILE * TILE)) + 2 * tid;
+        constexpr int STRIDE = TILE * TILE / 2;
+        __hip_atomic_store(slots + blockIdx.y * STRIDE, __builtin_bit_cast(int64_t, v2f{o[0], o[1]}), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(slots + blockIdx.y * STRIDE + 1, __builtin_bit_cast(int64_t, v2f{o[2], o[3]}), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        int *last = reinterpret_cast<int *>(lds + WAVES * PART * 4);
+        __builtin_amdgcn_s_waitcnt(0);
+        __syncthreads();
+        if (tid == 0) *last = __hip_atomic_fetch_add(meeting.arrivals + blockIdx.x, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == ranges - 1;
+        __syncthreads();
+        if (!*last) return;
+        o = v4f{0.f, 0.f, 0.f, 0.f};
+        for (int r0 = 0; r0 < ranges; r0 += 8) {
+            v2f x[8][2];
+#pragma unroll
+            for (int u = 0; u < 8; u++) {
+                const int r = r0 + u < ranges ? r0 + u : ranges - 1;
+#pragma unroll
+                for (int e = 0; e < 2; e++) x[u][e] = __builtin_bit_cast(v2f, __hip_atomic_load(slots + r * STRIDE + e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+                if (r0 + u >= ranges) x[u][0] = x[u][1] = v2f{0.f, 0.f};
+            }
+#pragma unroll
+            for (int by = 1; by < 8; by *= 2)
+#pragma unroll
+                for (int u = 0; u < 8; u += 2 * by) {
+                    x[u][0] += x[u + by][0];
+                    x[u][1] += x[u + by][1];
+                }
+            o += v4f{x[0][0][0], x[0][0][1], x[0][1][0], x[0][1][1]};
+        }
+        if (tid == 0) __hip_atomic_store(meeting.arrivals + blockIdx.x, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);      // ready for the next launch
+    }
+    if (m >= g.M || col >= g.N) return;
     const int have = g.N - col >= 4 ? 4 : (int)(g.N - col);
     float *cp = g.C + m * g.ldc + col;
-    o *= down;
     if (g.alpha != 1.0f) o *= g.alpha;
 #pragma unroll
     for (int e = 0; e < 4; e++)
@@ -214,19 +264,25 @@ __global__ void __launch_bounds__(64 * WAVES, PER_SIMD) k_gemm_strips(StagedArgs
     }
 }
 
-template <int WAVES, bool TERMS, bool A_KC, bool B_KC, int PER_SIMD>
-int launch(const char *name, const StagedArgs &g) {
+template <int WAVES, bool TERMS, bool A_KC, bool B_KC, int PER_SIMD, bool RANGES = false>
+int launch(const char *name, const StagedArgs &g, int64_t ranges = 1) {
     constexpr int SMEM = WAVES * PART * 4 + 4 * WAVES;
     static_assert(!(A_KC && B_KC) || WAVES * 4096 <= SMEM, "values are turned where the parts come to lie");
-    auto kern = k_gemm_strips<WAVES, TERMS, A_KC, B_KC, PER_SIMD>;
+    auto kern = k_gemm_strips<WAVES, TERMS, A_KC, B_KC, PER_SIMD, RANGES>;
     static bool attr_set = false;
     if (!attr_set) {
         AXHIP_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, SMEM), "hipFuncSetAttribute");
         attr_set = true;
     }
     const int64_t tiles = ((g.M + TILE - 1) / TILE) * ((g.N + TILE - 1) / TILE);
+    std::conditional_t<RANGES, Meeting, int> meeting{};
+    if constexpr (RANGES) {
+        meeting.parts = static_cast<float *>(workspace((size_t)(tiles * ranges * TILE * TILE) * sizeof(float)));
+        meeting.arrivals = strip_counters((size_t)tiles);
+        if (!meeting.parts || !meeting.arrivals) return AXHIP_ERR_ALLOC;
+    }
     note_kernel(name);
-    hipLaunchKernelGGL(kern, dim3((unsigned)tiles), dim3(64 * WAVES), SMEM, kStream, g);
+    hipLaunchKernelGGL(kern, dim3((unsigned)tiles, (unsigned)ranges), dim3(64 * WAVES), SMEM, kStream, g, meeting);
     return check_launch(name);
 }
 }  // namespace
@@ -247,6 +303,12 @@ namespace axhip {
 // hundred products: eight 1.05 of theirs at K = 129..144, 1.02 at 145..160, 1.01 at 161..168, 0.99 from 177 on, four 0.99, 0.98, 0.96 and, of
 // uniform values, 1.00 at 121..128), and none up to K = 120 (four 1.07 at 64..80, 1.01 at 113..120).  On the grid the kernels before were on fp32 instructions, with three times the error.
 // Sixteen pay where A is stored across K, whose loads are the slowest, above K = 256 (256 x 1000 x 500 6.6 -> 6.1; 250 x 500 x 256 4.5 -> 5.2).
+// A K past that, or past 760 with up to 64 tiles, in ranges, which meet in the same launch: for a narrow result two launches had cost their floor twice, and a few
+// workgroups of eight waves each wait for memory through their strip.  us, before -> here: 100 x 10 x 4096 10.8 -> 7.9, 128 x 10 x 1024 8.6 -> 5.7, 64 x
+// 256 x 2048 A^T B 8.7 -> 7.7, 100 x 100 x 4096 9.2 -> 8.9.  Geometric means over 800 random products, before over here, and the error over that of before: up to 32 tiles
+// K = 761..960 1.18 to 1.28 (four ranges of four waves, 1.00 of the strips' and 0.7 of the others' error), ..1300 1.36 to 1.45 (eight), ..4608 1.14 to 1.43
+// (eight of eight waves, 0.6 to 0.8); 33 to 64 tiles ..1024 1.07 to 1.36, ..2600 1.12 to 1.31; 65 to 100 tiles 961..2600 1.08 to 1.17.  Below K = 760 the parts are
+// so short that adding them costs accuracy (1.01 to 1.05 for 1.0 to 1.2 of the speed), past 100 tiles the chip is full (0.7 to 1.0); sixteen ranges 0.8 to 1.0 of eight.
 // On fp32 instructions up to K = 63 off the grid and 112 on it, where the kernels before are on them too: there is little to multiply and nothing to
 // cut.  Four waves, up to two tiles a CU (geometric means over some hundred products a range, cached / from HBM, and the error over that of the
 // kernels before: K below 32 1.3 / 1.3, 0.99; 32..63 off the grid 1.31 / 1.29, 0.86, on it 1.22 / 1.21, 0.74; 64..112 on the grid 1.32 / 1.31, 0.64; strips in
@@ -267,7 +329,24 @@ int strips_f32(const StagedArgs &g, int transa, int transb, bool on_grid) {
                          : tiles > 24      ? (transb ? 832 : 896)
                                            : (transb ? 800 : 864);
     const bool third = tiles * 3 <= cus * 4;                   // two workgroups on a third of the CUs at most
-    if (g.K <= (on_grid ? 112 : 120) || !((one && g.K <= most) || (two && !transb && g.K <= (third ? 640 : 800)))) return -1;
+    const bool strips = (one && g.K <= most) || (two && !transb && g.K <= (third ? 640 : 800));
+    // Few tiles and a long K: ranges of it, four to eight workgroups a tile.  (Their name holds that of the strips where those are what stands behind.)
+    const int64_t waves = tiles <= 32 ? (g.K > 1300 ? 8 : 4) : tiles <= 64 && g.K > 1024 ? 8 : 4;
+    const int64_t ranges = g.K <= 760                ? 1
+                           : tiles <= 32             ? (g.K <= 960 ? 4 : g.K <= 4608 ? 8 : 1)
+                           : tiles <= 64             ? (g.K <= 2600 ? 4 : 1)
+                           : tiles <= 100            ? (g.K > 960 && g.K <= 2600 ? 8 : 1)
+                                                     : 1;
+    if (ranges > 1) {
+        static const char *const names[3][2] = {{"sgemm_nn_ranges32x3", "sgemm_nn_strips32x3_ranges"},
+                                                {"sgemm_nt_ranges32x3", "sgemm_nt_strips32x3_ranges"},
+                                                {"sgemm_tn_ranges32x3", "sgemm_tn_strips32x3_ranges"}};
+        const char *name = names[transa ? 2 : transb ? 1 : 0][strips];
+        if (!transa && !transb) return waves == 8 ? launch<8, true, true, false, 2, true>(name, g, ranges) : launch<4, true, true, false, 4, true>(name, g, ranges);
+        if (!transa) return waves == 8 ? launch<8, true, true, true, 2, true>(name, g, ranges) : launch<4, true, true, true, 4, true>(name, g, ranges);
+        return waves == 8 ? launch<8, true, false, false, 2, true>(name, g, ranges) : launch<4, true, false, false, 4, true>(name, g, ranges);
+    }
+    if (g.K <= (on_grid ? 112 : 120) || !strips) return -1;
     if (!one && third && g.K > 400)
         return transa ? launch<8, true, false, false, 4>("sgemm_tn_strips32x3", g) : launch<8, true, true, false, 4>("sgemm_nn_strips32x3", g);
     const bool four = !one || (!on_grid && g.K <= 176);
