@@ -493,7 +493,7 @@ k_sdpa_few(const float *__restrict__ Q, const float *__restrict__ K, const float
         }
     }
     for (int t = wave; t < tiles; t += WAVES) {
-        const int next = t + WAVES < tiles ? t + WAVES : t;              // past the end the same tile again, unused
+        const int next = t + WAVES;
         v16f s, low;
 #pragma unroll
         for (int v = 0; v < 16; v++) s[v] = low[v] = 0.0f;
@@ -507,7 +507,7 @@ k_sdpa_few(const float *__restrict__ Q, const float *__restrict__ K, const float
                 for (int p = sum; p >= 0; p--) (APART ? low : s) = mfma_terms(kf[sum - p], qf[ks][p], APART ? low : s);
             s = mfma_terms(kf[0], qf[ks][0], s);
         }
-        load_k(next);
+        if (next < tiles) load_k(next);
         if (APART) s += low;
         if (CAUSAL ? t == tiles - 1 : (int64_t)t * 32 + 32 > S) {
             const int qrel = (int)((CAUSAL ? qg : S - 1) - (int64_t)t * 32);
@@ -533,7 +533,7 @@ k_sdpa_few(const float *__restrict__ Q, const float *__restrict__ K, const float
                     for (int p = sum; p >= 0; p--) acc_o[d] = mfma_terms(vf[p], pf[sum - p], acc_o[d]);
             }
         }
-        load_v(next);
+        if (next < tiles) load_v(next);
     }
 
     // ---- the waves' parts together, each at an eighth (exactly): outputs that are finite in themselves may exceed the largest float when
