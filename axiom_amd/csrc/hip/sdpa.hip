@@ -605,19 +605,23 @@ k_sdpa_few(const float *__restrict__ Q, const float *__restrict__ K, const float
 // ones within it 0.91 to 2.8 times as fast).  A single key tile per wave (S up to 128): one workgroup a CU, or two of the smaller geometries from three
 // tiles on (128 of [128, 64] 12.1 -> 11.5, but 128 of [128, 128] 21.3 -> 23.2, 256 of [64, 64] 8.1 -> 8.9).  A head of one tile gains nothing (4.6 us
 // either way).
+// With the last tile apart from the loop the line moved out: of 60 random ones with walks of ten tiles and more, up to 1.3 times the limit, all but one were 1.0 to 1.65 times as
+// fast (geometric mean 1.11; 39 of [1166, 32] causal 46.3 -> 46.8), except unmasked ones of the two larger geometries and walks of nine (0.95 to 1.03), which stay; at 1.4 times and
+// beyond 0.7 to 1.3.  One tile a wave of the geometry 96 with four tiles: 21 random ones 1.05 (78 of [99, 96] causal 16.1 -> 14.0, 127 of [100, 80] causal 14.9 -> 15.2).
 // Eight waves on 32 queries: level or behind (32 of [512, 64] 22.0 -> 27.2, 1 of [2048, 64] 32.7 -> 31.1): the vector pipe is the bound.
 template <int DK>
 bool few_tiles(int64_t BH, int64_t S, int causal) {
     const int64_t tiles = (S + 31) / 32, walk = (tiles + 3) / 4, cus = cu_count();
     if (tiles < 2 || BH > 4 * cus || tiles > 0xffff) return false;
-    if (walk == 1) return tiles * BH <= (DK > 64 || tiles == 2 ? 1 : 2) * cus;
+    if (walk == 1) return tiles * BH <= (tiles == 4 ? (DK < 128 ? 2 : 1) : tiles == 3 && DK <= 64 ? 2 : 1) * cus;
     const int64_t q = tiles / 4, all = causal ? 2 * q * (q + 1) + tiles % 4 * (q + 1) : tiles * walk;
     int64_t limit = 9;
     if (causal && DK > 64) limit = walk + (DK == 96 ? 2 : 1) < 7 ? walk + (DK == 96 ? 2 : 1) : 7;
     else if (causal && DK == 64 && walk == 2) limit = 5;
     else if (!causal && DK > 64) limit = walk == 2 ? 4 : 8;
     else if (!causal && DK == 64 && walk <= 3) limit = 8;
-    return all * BH * 4 <= limit * walk * cus;
+    const bool further = walk > 9 && (causal || DK <= 64);
+    return all * BH * 40 <= limit * (further ? 13 : 10) * walk * cus;
 }
 
 template <int DK>
