@@ -605,9 +605,10 @@ k_sdpa_few(const float *__restrict__ Q, const float *__restrict__ K, const float
 // ones within it 0.91 to 2.8 times as fast).  A single key tile per wave (S up to 128): one workgroup a CU, or two of the smaller geometries from three
 // tiles on (128 of [128, 64] 12.1 -> 11.5, but 128 of [128, 128] 21.3 -> 23.2, 256 of [64, 64] 8.1 -> 8.9).  A head of one tile gains nothing (4.6 us
 // either way).
-// With the last tile apart from the loop the line moved out: of 60 random ones with walks of ten tiles and more, up to 1.3 times the limit, all but one were 1.0 to 1.65 times as
-// fast (geometric mean 1.11; 39 of [1166, 32] causal 46.3 -> 46.8), except unmasked ones of the two larger geometries and walks of nine (0.95 to 1.03), which stay; at 1.4 times and
-// beyond 0.7 to 1.3.  One tile a wave of the geometry 96 with four tiles: 21 random ones 1.05 (78 of [99, 96] causal 16.1 -> 14.0, 127 of [100, 80] causal 14.9 -> 15.2).
+// With the last tile apart from the loop the line moved out: random ones of the two smaller geometries with walks of ten tiles and more, up to 1.3 times the limit, 0.99 to 1.65
+// times as fast (17 of [1256, 32] 47.7 -> 36.8, 14 of [1571, 32] 58.6 -> 48.3, causal 28 of [1386, 32] 53.1 -> 47.6, 39 of [1166, 32] 46.3 -> 46.8); walks of nine 0.95 to 1.2, the larger geometries
+// 0.93 to 1.3 (causal 18 of [1908, 112] 192 -> 206), at 1.4 times and beyond 0.7 to 1.3: these stay.  One tile a wave of the geometry 96 with four tiles: 24 random
+// ones 0.98 to 1.16 (78 of [99, 96] causal 16.1 -> 14.0, 127 of [100, 80] causal 14.9 -> 15.2).
 // Eight waves on 32 queries: level or behind (32 of [512, 64] 22.0 -> 27.2, 1 of [2048, 64] 32.7 -> 31.1): the vector pipe is the bound.
 template <int DK>
 bool few_tiles(int64_t BH, int64_t S, int causal) {
@@ -620,7 +621,7 @@ bool few_tiles(int64_t BH, int64_t S, int causal) {
     else if (causal && DK == 64 && walk == 2) limit = 5;
     else if (!causal && DK > 64) limit = walk == 2 ? 4 : 8;
     else if (!causal && DK == 64 && walk <= 3) limit = 8;
-    const bool further = walk > 9 && (causal || DK <= 64);
+    const bool further = walk > 9 && DK <= 64;
     return all * BH * 40 <= limit * (further ? 13 : 10) * walk * cus;
 }
 

@@ -9,7 +9,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("BH,S,dk,causal,few", [(31, 1400, 64, 1, True), (32, 1400, 64, 1, False), (18, 1300, 32, 0, True), (19, 1300, 32, 0, False),
-                                                (27, 1300, 128, 1, True), (28, 1300, 128, 1, False), (12, 1300, 80, 0, True), (13, 1300, 80, 0, False),
+                                                (21, 1300, 128, 1, True), (22, 1300, 128, 1, False), (12, 1300, 80, 0, True), (13, 1300, 80, 0, False),
                                                 (128, 128, 96, 0, True), (129, 128, 96, 0, False), (128, 97, 80, 1, True)])
 def test_where_it_runs(hip, BH, S, dk, causal, few):
     """256 CUs."""
