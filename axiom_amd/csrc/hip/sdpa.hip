@@ -25,7 +25,7 @@
 // infinities, NaNs and values near the largest float come out as fp32 products give them.
 // us, fp32 instructions -> terms: 512 heads of [512, 64] 269 -> 194 (causal 178 -> 126), 64 of [1024, 128] 273 -> 174, 96 causal
 // ones of [1000, 80] 324 -> 108 (a quarter of that from the 96-wide geometry), 512 of [256, 32] 41 -> 33; with few query tiles for the
-// CUs k_sdpa_few cuts a head along its keys too (32 heads of [128, 64] 11.4 -> 6.9).  O is nearer to 64 bits on every shape measured (relative error 4.9e-7 -> 3.7e-7 at [512, 64]).  Bound: the matrix core is
+// CUs k_sdpa_few cuts a head along its keys too (32 heads of [128, 64] 11.4 -> 6.6).  O is nearer to 64 bits on every shape measured (relative error 4.9e-7 -> 3.7e-7 at [512, 64]).  Bound: the matrix core is
 // busy 49 % of the cycles, vector instructions (cutting, softmax) take some 44 ([512, 64]).  Measured and dropped: two key tiles at a time,
 // the scores of one interleaved with the exponentials of the other by instruction groups ([512, 64] 194, [1024, 96] 126 -> 128).
 //
@@ -599,7 +599,7 @@ k_sdpa_few(const float *__restrict__ Q, const float *__restrict__ K, const float
 // tiles, and all walks together are shared by the CUs.  `limit` is four times the longest walks a CU up to which it is ahead of k_sdpa, whose
 // four waves each walk all of a head's tiles: two rounds of workgroups and a little where two share a CU (geometries 32 and 64), two where one has
 // it, one where a walk is two tiles and mostly start and end; causal walks differ in length, and the shorter they all are the sooner the
-// longer geometries fall behind (us, k_sdpa -> this: 32 heads of [128, 64] 11.4 -> 6.9, 4 of [2048, 64] 111 -> 36, 32 of [512, 64] 33.3 -> 22.0, 8 causal ones of
+// longer geometries fall behind (us, k_sdpa -> this as it was before its last tile stood apart: 32 heads of [128, 64] 11.4 -> 6.9, 4 of [2048, 64] 111 -> 36, 32 of [512, 64] 33.3 -> 22.0, 8 causal ones of
 // [2048, 128] 204 -> 74, 32 causal of [1024, 80] 81.6 -> 74.4; past it 64 of [512, 64] 35.7 -> 38.6, 64 causal of [512, 80] 44.6 -> 55.6, 81 of [216, 128]
 // 30.4 -> 43.2, 100 of [160, 128] 23.6 -> 28.7, 53 of [294, 96] 29.8 -> 37.7, causal 113 of [208, 80] 23.8 -> 34.1, 57 of [507, 128] 60.6 -> 70.8; over 2804 random
 // ones within it 0.91 to 2.8 times as fast).  A single key tile per wave (S up to 128): one workgroup a CU, or two of the smaller geometries from three
@@ -608,7 +608,8 @@ k_sdpa_few(const float *__restrict__ Q, const float *__restrict__ K, const float
 // With the last tile apart from the loop the line moved out: random ones of the two smaller geometries with walks of ten tiles and more, up to 1.3 times the limit, 0.99 to 1.65
 // times as fast (17 of [1256, 32] 47.7 -> 36.8, 14 of [1571, 32] 58.6 -> 48.3, causal 28 of [1386, 32] 53.1 -> 47.6, 39 of [1166, 32] 46.3 -> 46.8); walks of nine 0.95 to 1.2, the larger geometries
 // 0.93 to 1.3 (causal 18 of [1908, 112] 192 -> 206), at 1.4 times and beyond 0.7 to 1.3: these stay.  One tile a wave of the geometry 96 with four tiles: 24 random
-// ones 0.98 to 1.16 (78 of [99, 96] causal 16.1 -> 14.0, 127 of [100, 80] causal 14.9 -> 15.2).
+// ones 0.98 to 1.16 (78 of [99, 96] causal 16.1 -> 14.0, 127 of [100, 80] causal 14.9 -> 15.2); the geometry 128 keeps one (four tiles would gain 2 to 13 %, three lose 5: 150 of
+// [96, 128] 17.0 -> 17.9).
 // Eight waves on 32 queries: level or behind (32 of [512, 64] 22.0 -> 27.2, 1 of [2048, 64] 32.7 -> 31.1): the vector pipe is the bound.
 template <int DK>
 bool few_tiles(int64_t BH, int64_t S, int causal) {
