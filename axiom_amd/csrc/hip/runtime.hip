@@ -127,22 +127,32 @@ int check_launch(const char *what) {
 
 size_t workspace_bytes() { return g_ws_bytes; }
 
-void *workspace(size_t bytes) {
-    if (bytes <= g_ws_bytes) return g_ws;
+// hipMalloc, or NULL.  The runtime keeps a refusal until it is asked for: left there it would be reported by the next launch's check.
+static void *device_block(size_t bytes) {
+    void *p = nullptr;
+    if (hipMalloc(&p, bytes) == hipSuccess) return p;
+    (void)hipGetLastError();
+    return nullptr;
+}
+
+// The workspace at `bytes` or more, without a message where there is no room.
+static bool grow_workspace(size_t bytes) {
+    if (bytes <= g_ws_bytes) return true;
     if (g_ws) {
         (void)hipDeviceSynchronize();
         (void)hipFree(g_ws);
-        g_ws = nullptr;
         g_ws_bytes = 0;
     }
-    size_t want = bytes < (size_t(8) << 20) ? (size_t(8) << 20) : bytes;
-    if (hipMalloc(&g_ws, want) != hipSuccess) {
-        g_ws = nullptr;
-        fail(AXHIP_ERR_ALLOC, "workspace of %zu bytes: out of device memory", want);
-        return nullptr;
-    }
-    g_ws_bytes = want;
-    return g_ws;
+    const size_t want = bytes < (size_t(8) << 20) ? (size_t(8) << 20) : bytes;
+    g_ws = device_block(want);
+    if (g_ws) g_ws_bytes = want;
+    return g_ws != nullptr;
+}
+
+void *workspace(size_t bytes) {
+    if (grow_workspace(bytes)) return g_ws;
+    fail(AXHIP_ERR_ALLOC, "workspace of %zu bytes: out of device memory", bytes);
+    return nullptr;
 }
 
 float *ones_vector(size_t n) {
@@ -154,8 +164,8 @@ float *ones_vector(size_t n) {
         g_ones_n = 0;
     }
     size_t want = n < 65536 ? 65536 : n;
-    if (hipMalloc(reinterpret_cast<void **>(&g_ones), want * sizeof(float)) != hipSuccess) {
-        g_ones = nullptr;
+    g_ones = static_cast<float *>(device_block(want * sizeof(float)));
+    if (!g_ones) {
         fail(AXHIP_ERR_ALLOC, "ones vector (%zu floats): out of device memory", want);
         return nullptr;
     }
@@ -178,8 +188,10 @@ int *strip_counters(size_t n) {
         g_ctr_n = 0;
     }
     size_t want = n < 4096 ? 4096 : n;
-    if (hipMalloc(reinterpret_cast<void **>(&g_ctr), want * sizeof(int)) != hipSuccess ||
-        hipMemset(g_ctr, 0, want * sizeof(int)) != hipSuccess) {
+    g_ctr = static_cast<int *>(device_block(want * sizeof(int)));
+    if (!g_ctr || hipMemset(g_ctr, 0, want * sizeof(int)) != hipSuccess) {
+        if (g_ctr) (void)hipFree(g_ctr);
+        (void)hipGetLastError();
         g_ctr = nullptr;
         fail(AXHIP_ERR_ALLOC, "arrival counters (%zu ints): out of device memory", want);
         return nullptr;
@@ -266,7 +278,7 @@ int axhip_init(void) {
     if (int rc = axhip::skinny_setup()) return rc;
     // the shared workspace and the arrival counters exist from the start (160 MiB, or 64 on a device that is nearly full; 4096 counters): a
     // first call at a new shape then pays no allocation or device-wide wait unless it needs more than that
-    if ((!axhip::workspace(axhip::kWorkspaceStart) && !axhip::workspace(size_t(64) << 20)) || !axhip::strip_counters(4096)) return AXHIP_ERR_ALLOC;
+    if ((!axhip::grow_workspace(axhip::kWorkspaceStart) && !axhip::workspace(size_t(64) << 20)) || !axhip::strip_counters(4096)) return AXHIP_ERR_ALLOC;
     g_ready = 1;
     return AXHIP_OK;
 }
