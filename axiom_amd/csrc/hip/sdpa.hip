@@ -664,12 +664,23 @@ int launch_sdpa_p(const float *Q, const float *K, const float *V, float *O, floa
     // [1024, 128] x 64 single 128.4, 129.2, 136.5 us, paired 127.4, 126.8, 134.2 (the 96-wide geometry [1024, 96] x 64 100.9 against 108)
     const int64_t cus = cu_count(), pairs = (nq + 1) / 2 * BH, rounds = (pairs + cus - 1) / cus;
     const int pair = causal && WAVES == 4 && (DK == 64 || DK == 128) && rounds * cus * 30 <= nq * BH * 16;
-    dim3 grid((unsigned)((pair ? (nq + 1) / 2 : nq) * BH)), block(64 * WAVES);
-    if (causal)
-        hipLaunchKernelGGL((k_sdpa<DK, WAVES, true, PAD>), grid, block, G::SMEM, kStream, Q, K, V, O, L, BH, S, sl2, H, ld, ldo, dkr, pair);
-    else
-        hipLaunchKernelGGL((k_sdpa<DK, WAVES, false, PAD>), grid, block, G::SMEM, kStream, Q, K, V, O, L, BH, S, sl2, H, ld, ldo, dkr, pair);
-    return check_launch("sdpa_fwd");
+    const dim3 block(64 * WAVES);
+    // A grid holds fewer than 2^32 threads: more heads go in pieces, of whole batches where those fit (head h of a launch lies in batch h / H of its pointers).
+    const int64_t a_head = pair ? (nq + 1) / 2 : nq;
+    int64_t most = 0xffffffffll / (64 * WAVES) / a_head;
+    if (most < 1) return fail(AXHIP_ERR_SHAPE, "sdpa_fwd: too many tiles");
+    if (most > H) most -= most % H;
+    for (int64_t h0 = 0, n; h0 < BH; h0 += n) {
+        n = BH - h0 < most ? BH - h0 : most;
+        if (most < H && n > H - h0 % H) n = H - h0 % H;
+        const int64_t in = h0 / H * S * ld + h0 % H * dkr, out = h0 / H * S * ldo + h0 % H * dkr;
+        const dim3 grid((unsigned)(a_head * n));
+        float *lse = L ? L + h0 * S : nullptr;
+        if (causal) hipLaunchKernelGGL((k_sdpa<DK, WAVES, true, PAD>), grid, block, G::SMEM, kStream, Q + in, K + in, V + in, O + out, lse, n, S, sl2, H, ld, ldo, dkr, pair);
+        else hipLaunchKernelGGL((k_sdpa<DK, WAVES, false, PAD>), grid, block, G::SMEM, kStream, Q + in, K + in, V + in, O + out, lse, n, S, sl2, H, ld, ldo, dkr, pair);
+        if (int rc = check_launch("sdpa_fwd")) return rc;
+    }
+    return AXHIP_OK;
 }
 
 template <int DK>

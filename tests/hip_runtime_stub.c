@@ -12,7 +12,7 @@
 typedef struct {
     char kernel[256];
     uint32_t grid[3], block[3];
-    uint64_t shared;
+    uint64_t shared, args[7];      /* of attention: Q, K, V, O, L, heads, sequence */
 } Launch;
 static Launch launches[MOST];
 static int count;
@@ -60,7 +60,7 @@ hipError_t __hipPopCallConfiguration(dim3 *grid, dim3 *block, size_t *shared, hi
     return hipSuccess;
 }
 hipError_t hipLaunchKernel(const void *function, dim3 grid, dim3 block, void **args, size_t shared, hipStream_t stream) {
-    (void)args, (void)stream;
+    (void)stream;
     const uint64_t most = (uint64_t)1 << 32;
     if (!grid.x || !grid.y || !grid.z || (uint64_t)block.x * block.y * block.z > 1024 || shared > 160 * 1024) return note(hipErrorInvalidConfiguration);
     if ((uint64_t)grid.x * block.x >= most || (uint64_t)grid.y * block.y >= most || (uint64_t)grid.z * block.z >= most) return note(hipErrorInvalidConfiguration);
@@ -72,6 +72,7 @@ hipError_t hipLaunchKernel(const void *function, dim3 grid, dim3 block, void **a
         l->grid[0] = grid.x, l->grid[1] = grid.y, l->grid[2] = grid.z;
         l->block[0] = block.x, l->block[1] = block.y, l->block[2] = block.z;
         l->shared = shared;
+        for (int i = 0; i < 7 && strstr(l->kernel, "k_sdpa"); i++) memcpy(&l->args[i], args[i], 8);
     }
     count++;
     return hipSuccess;

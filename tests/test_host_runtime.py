@@ -13,7 +13,7 @@ PRELUDE = """
 import ctypes as C, sys
 sys.path.insert(0, %r)
 class Launch(C.Structure):
-    _fields_ = [("kernel", C.c_char * 256), ("grid", C.c_uint32 * 3), ("block", C.c_uint32 * 3), ("shared", C.c_uint64)]
+    _fields_ = [("kernel", C.c_char * 256), ("grid", C.c_uint32 * 3), ("block", C.c_uint32 * 3), ("shared", C.c_uint64), ("args", C.c_uint64 * 7)]
 stub = C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)
 stub.stub_launch.restype, stub.stub_set_free.argtypes = C.POINTER(Launch), [C.c_size_t]
 from axiom_amd import AxHip
@@ -77,3 +77,29 @@ hip.check(L.axhip_fill_f32(A, 1.0, 1000))
 assert L.axhip_sum_axis(A, 1, 100 * MIB, 2048, D) == 2 and "ones" in hip.last_error()
 hip.check(L.axhip_fill_f32(A, 1.0, 1000))
 """)
+
+
+@pytest.mark.parametrize("S,dk,H,B", [(129, 4, 1, 8500001), (129, 36, 1, 9000000), (129, 68, 1, 9000000), (129, 100, 1, 9000000), (200, 32, 7, 1300000), (4096, 4, 1 << 20, 1),
+                                      (2049, 4, 999999, 3), (128, 8, 1, 20000000)])
+@pytest.mark.parametrize("causal", [0, 1])
+def test_attention_over_more_tiles_than_a_grid_holds(stub, S, dk, H, B, causal):
+    """2^24 workgroups of 256 threads are 2^32 threads, one more than a launch may have: the heads go in pieces, of whole batches or within one."""
+    run(stub, """
+S, dk, H, B, causal = %r
+hip.check(L.axhip_init())
+O, lse = 1 << 48, 1 << 49
+if H == 1:
+    hip.check(L.axhip_sdpa_fwd(A, B_ptr, D, O, lse, B, S, dk, 0.5, causal))
+else:
+    hip.check(L.axhip_sdpa_fwd_rows(A, B_ptr, D, H * dk, O, H * dk, lse, B, H, S, dk, 0.5, causal))
+at = 0                                              # heads so far
+for x in launched():
+    b, h = divmod(at, H)
+    assert list(x.args[:4]) == [p + 4 * (b * S * H + h) * dk for p in (A, 1 << 46, D, O)] and x.args[4] == lse + 4 * at * S and x.args[6] == S
+    n = x.args[5]
+    assert n %% H == 0 or h + n <= H
+    a_head = -(-S // (x.block[0] // 2))
+    assert x.grid[0] in (a_head * n, (a_head + 1) // 2 * n)
+    at += n
+assert at == B * H
+""".replace("B_ptr", "1 << 46") % ((S, dk, H, B, causal),))
