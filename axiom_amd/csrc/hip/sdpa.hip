@@ -33,6 +33,7 @@
 // one batched NN GEMM over as many heads at a time as fit 256 MiB (the structure of
 // ax_cuda_sdpa_fwd, cuda/ops_attention.cu:299-392).
 #include "bf16x3.h"
+#include "sdpa_order.h"
 
 namespace {
 using namespace axhip;
@@ -145,6 +146,9 @@ __device__ __forceinline__ void attend_f32(const float *Qh, const float *Kh, con
     }
 }
 
+constexpr int64_t FAR = 7168;                            // queries: K and V of such a head are more than an XCD's L2 holds
+constexpr int ORDER_GROUPS = -1, ORDER_PAIRS = -2;       // of query tiles, where they go out in groups of eight heads
+
 // Rows past the end of a head are never read (such a row is redirected to the head's last row, which keeps
 // V finite), keys past the end are masked like causal ones, and queries past the end are computed but not stored.
 // PAD: the head size dkr is below DK (a multiple of 4): chunks of Q and K past column dkr are zero, columns
@@ -153,7 +157,7 @@ template <int DK, int WAVES, bool CAUSAL, bool PAD>
 __global__ void __launch_bounds__(64 * WAVES, (SdGeom<DK, WAVES>::PER_SIMD))
 k_sdpa(const float *__restrict__ Q, const float *__restrict__ K, const float *__restrict__ V,
        float *__restrict__ O, float *__restrict__ L, int64_t BH, int64_t S, float scale_log2e,
-       int64_t H, int64_t ld, int64_t ldo, int dkr, int pair_tiles) {
+       int64_t H, int64_t ld, int64_t ldo, int dkr, int order) {
     using G = SdGeom<DK, WAVES>;
     constexpr int BQ = G::BQ, BKV = G::BKV, E = G::E;
     constexpr int KS = DK / 16;                  // 16-wide steps of the score product
@@ -163,22 +167,17 @@ k_sdpa(const float *__restrict__ Q, const float *__restrict__ K, const float *__
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     const int64_t nq = (S + BQ - 1) / BQ;
-    // Workgroups go to the 8 XCDs round-robin by linear index, inside an XCD to whichever CU has room.  Eight
-    // heads form a group: workgroup r of a group works on head r % 8 (every query tile of a
-    // head then runs on the same XCD and shares its L2 copy of K and V) and on unit r / 8, a query tile.
-    // Causal tiles visit more keys the later they are: single ones go out longest first over all heads, so that the short ones even out the
-    // ends (us, pairs -> this, both on eight waves unless said: 96 heads of [1000, 80] 122 -> 108, 61 of [1472, 80] 162 -> 146, 218 of [655, 128] 286 -> 227; on four
-    // 145 of [192, 32] 16.2 -> 11.1, 193 of [832, 64] 159 -> 121; 2 % of that is from L2 copies no longer shared).
-    // pair_tiles: a unit is the pair of tiles p and nq-1-p, which together visit the same number of keys whatever p is (the
-    // middle tile of an odd nq stands alone).
-    const bool paired = CAUSAL && pair_tiles;
-    const int64_t units = paired ? (nq + 1) / 2 : nq;
+    // Workgroups go to the 8 XCDs round-robin by linear index.  Eight heads form a group: workgroup r of a group works on head r % 8 (every query tile of a
+    // head then runs on the same XCD and shares its L2 copy of K and V) and on unit r / 8: a query tile, or a pair of causal tiles p and nq - 1 - p, which together
+    // visit the same number of keys whatever p is (the middle tile of an odd nq stands alone).  `order` >= 0: single causal tiles in the order of sdpa_order.h.
+    const bool paired = CAUSAL && order == ORDER_PAIRS;
     int64_t head, unit;
-    if (CAUSAL && !paired) {
-        const unsigned longer = blockIdx.x / (unsigned)BH;
-        unit = nq - 1 - longer;
-        head = blockIdx.x - longer * (unsigned)BH;
+    if (CAUSAL && order >= 0) {
+        const CausalTile o = causal_tile(blockIdx.x, (unsigned)BH, (unsigned)nq, (unsigned)order);
+        head = o.head;
+        unit = o.tile;
     } else {
+        const int64_t units = paired ? (nq + 1) / 2 : nq;
         const int64_t lin = blockIdx.x, group = lin / (8 * units), left = BH - group * 8;
         const int64_t r = lin - group * 8 * units, hpg = left < 8 ? left : 8;
         head = group * 8 + r % hpg;
@@ -660,10 +659,13 @@ int launch_sdpa_p(const float *Q, const float *K, const float *V, float *O, floa
     }
     const float sl2 = scale * 1.4426950408889634f;
     const int64_t nq = (S + G::BQ - 1) / G::BQ;
-    // causal tiles p and nq-1-p in one workgroup where the pairs give every CU the same number of keys, or nearly: [512, 64] x 512, [2048, 64] x 32 and
-    // [1024, 128] x 64 single 128.4, 129.2, 136.5 us, paired 127.4, 126.8, 134.2 (the 96-wide geometry [1024, 96] x 64 100.9 against 108)
+    // Causal tiles p and nq - 1 - p in one workgroup where there are more tiles than CUs and the pairs, up to two a CU, give every CU the same number of keys or
+    // nearly ([8192, 64] x 8 single 486 us, paired 462, [16384, 64] x 8 1520 and 1416, [1024, 128] x 64 136.5 and 134.2; but [8192, 32] x 16 433 and 457); and up to one a CU
+    // where K and V of a head are more than an XCD's L2 holds ([7662, 80] x 12 734 and 696, [8192, 96] x 12 802 and 776, [7000, 80] x 12 648 and 652, but [6000, 80] x 12 524
+    // and 548).  With a CU for every tile there is nothing to even out.
     const int64_t cus = cu_count(), pairs = (nq + 1) / 2 * BH, rounds = (pairs + cus - 1) / cus;
-    const int pair = causal && WAVES == 4 && (DK == 64 || DK == 128) && rounds * cus * 30 <= nq * BH * 16;
+    const bool even = WAVES == 4 && (DK == 64 || DK == 128) && rounds <= 2 && rounds * cus * 30 <= nq * BH * 16, far = DK >= 96 && rounds == 1 && S > FAR;
+    const bool pair = causal && nq * BH > cus && (even || far);
     const dim3 block(64 * WAVES);
     // A grid holds fewer than 2^32 threads: more heads go in pieces, of whole batches where those fit (head h of a launch lies in batch h / H of its pointers).
     const int64_t a_head = pair ? (nq + 1) / 2 : nq;
@@ -675,9 +677,10 @@ int launch_sdpa_p(const float *Q, const float *K, const float *V, float *O, floa
         if (most < H && n > H - h0 % H) n = H - h0 % H;
         const int64_t in = h0 / H * S * ld + h0 % H * dkr, out = h0 / H * S * ldo + h0 % H * dkr;
         const dim3 grid((unsigned)(a_head * n));
+        const int order = pair ? ORDER_PAIRS : nq * n > cus ? (int)causal_last(n, nq, cus * (WAVES == 8 || DK == 128 ? 1 : 2)) : ORDER_GROUPS;
         float *lse = L ? L + h0 * S : nullptr;
-        if (causal) hipLaunchKernelGGL((k_sdpa<DK, WAVES, true, PAD>), grid, block, G::SMEM, kStream, Q + in, K + in, V + in, O + out, lse, n, S, sl2, H, ld, ldo, dkr, pair);
-        else hipLaunchKernelGGL((k_sdpa<DK, WAVES, false, PAD>), grid, block, G::SMEM, kStream, Q + in, K + in, V + in, O + out, lse, n, S, sl2, H, ld, ldo, dkr, pair);
+        if (causal) hipLaunchKernelGGL((k_sdpa<DK, WAVES, true, PAD>), grid, block, G::SMEM, kStream, Q + in, K + in, V + in, O + out, lse, n, S, sl2, H, ld, ldo, dkr, order);
+        else hipLaunchKernelGGL((k_sdpa<DK, WAVES, false, PAD>), grid, block, G::SMEM, kStream, Q + in, K + in, V + in, O + out, lse, n, S, sl2, H, ld, ldo, dkr, order);
         if (int rc = check_launch("sdpa_fwd")) return rc;
     }
     return AXHIP_OK;

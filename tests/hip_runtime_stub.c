@@ -13,6 +13,7 @@ typedef struct {
     char kernel[256];
     uint32_t grid[3], block[3];
     uint64_t shared, args[7];      /* of attention: Q, K, V, O, L, heads, sequence */
+    int32_t order;                 /* and in which its tiles go out */
 } Launch;
 static Launch launches[MOST];
 static int count;
@@ -73,6 +74,7 @@ hipError_t hipLaunchKernel(const void *function, dim3 grid, dim3 block, void **a
         l->block[0] = block.x, l->block[1] = block.y, l->block[2] = block.z;
         l->shared = shared;
         for (int i = 0; i < 7 && strstr(l->kernel, "k_sdpa"); i++) memcpy(&l->args[i], args[i], 8);
+        if (strstr(l->kernel, "k_sdpaI")) memcpy(&l->order, args[12], 4);
     }
     count++;
     return hipSuccess;

@@ -13,7 +13,7 @@ PRELUDE = """
 import ctypes as C, sys
 sys.path.insert(0, %r)
 class Launch(C.Structure):
-    _fields_ = [("kernel", C.c_char * 256), ("grid", C.c_uint32 * 3), ("block", C.c_uint32 * 3), ("shared", C.c_uint64), ("args", C.c_uint64 * 7)]
+    _fields_ = [("kernel", C.c_char * 256), ("grid", C.c_uint32 * 3), ("block", C.c_uint32 * 3), ("shared", C.c_uint64), ("args", C.c_uint64 * 7), ("order", C.c_int32)]
 stub = C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)
 stub.stub_launch.restype, stub.stub_set_free.argtypes = C.POINTER(Launch), [C.c_size_t]
 from axiom_amd import AxHip
