@@ -707,7 +707,10 @@ int launch_sdpa(const float *Q, const float *K, const float *V, float *O, float 
             eight = half_tiles == 3 && 2 * BH <= cus && (DK != 128 || 3 * BH > cus);
             if (DK == 128 && half_tiles == 2) eight = (BH + cus - 1) / cus * 5 < (2 * BH + cus - 1) / cus * 3;
             else if (DK == 128) eight = eight || (half_tiles == 3 && BH <= cus && 6 * BH > 5 * cus) || (half_tiles == 4 && 10 * BH >= 7 * cus) || (half_tiles + 1) * half_tiles * BH > 18 * cus;
-            if (DK == 96) eight = eight || ((tiles == 1 ? BH > cus : tiles * BH * 2 >= cus) && fits);
+            // geometry 96 from half a tile of 256 a CU on, with more than three tiles a head from three quarters on, and where heads are so long that tiles of 128 go out in pairs (launch_sdpa_p)
+            // from one (four -> eight: 90 of [400, 96] 47 -> 44, 90 of [595, 96] 71 -> 64, 34 of [1786, 96] 177 -> 173, but 32 of [1024, 96] 85 -> 95, 14 of [3002, 80] 245 -> 260, 24 of [2000, 96] 178 -> 185,
+            // 8 of [7662, 80] 590 -> 650)
+            if (DK == 96) eight = eight || ((tiles == 1 ? BH > cus : tiles <= 3 ? tiles * BH * 2 >= cus : S > FAR ? tiles * BH >= cus : tiles * BH * 4 > cus * 3) && fits);
         }
         if (eight)
             return dkr == DK ? launch_sdpa_p<DK, 8, false>(Q, K, V, O, L, BH, S, scale, causal, H, ld, ldo, dkr)

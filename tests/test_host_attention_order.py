@@ -40,3 +40,18 @@ assert x.order == order, x.order
 tiles = -(-S // (x.block[0] // 2))
 assert x.grid[0] == heads * ((tiles + 1) // 2 if order == -2 else tiles)
 """ % ((heads, S, dk, order),))
+
+
+# (heads, S, head size, waves a workgroup): geometry 96 under the mask, both sides of each line
+WAVES = [(32, 1024, 96, 4), (24, 2000, 96, 4), (25, 1793, 96, 8), (17, 2358, 80, 4), (90, 400, 96, 8), (44, 600, 80, 8), (42, 600, 80, 4), (8, 7662, 80, 4), (9, 7662, 80, 8), (28, 1786, 96, 8)]
+
+
+@pytest.mark.parametrize("heads,S,dk,waves", WAVES)
+def test_waves_of_geometry_96(stub, heads, S, dk, waves):  # noqa: F811
+    run(stub, """
+heads, S, dk, waves = %r
+hip.check(L.axhip_init())
+hip.check(L.axhip_sdpa_fwd(A, 1 << 46, D, 1 << 48, None, heads, S, dk, 0.5, 1))
+x, = launched()
+assert "few" not in x.kernel.decode() and x.block[0] == 64 * waves, (x.kernel, x.block[0])
+""" % ((heads, S, dk, waves),))
