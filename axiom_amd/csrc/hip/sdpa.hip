@@ -491,7 +491,7 @@ k_sdpa_few(const float *__restrict__ Q, const float *__restrict__ K, const float
             cut(x[ks], TERMS_UP, qf[ks]);
         }
     }
-    auto attend = [&](int t, auto more) {            // more: this wave's next tile is fetched meanwhile
+    auto attend = [&](int t, auto more, int next) {  // more: tile `next` is fetched meanwhile
         v16f s, low;
 #pragma unroll
         for (int v = 0; v < 16; v++) s[v] = low[v] = 0.0f;
@@ -505,7 +505,7 @@ k_sdpa_few(const float *__restrict__ Q, const float *__restrict__ K, const float
                 for (int p = sum; p >= 0; p--) (APART ? low : s) = mfma_terms(kf[sum - p], qf[ks][p], APART ? low : s);
             s = mfma_terms(kf[0], qf[ks][0], s);
         }
-        if constexpr (decltype(more)::value) load_k(t + WAVES);
+        if constexpr (decltype(more)::value) load_k(next);
         if (APART) s += low;
         if (CAUSAL ? t == tiles - 1 : (int64_t)t * 32 + 32 > S) {
             const int qrel = (int)((CAUSAL ? qg : S - 1) - (int64_t)t * 32);
@@ -531,14 +531,19 @@ k_sdpa_few(const float *__restrict__ Q, const float *__restrict__ K, const float
                     for (int p = sum; p >= 0; p--) acc_o[d] = mfma_terms(vf[p], pf[sum - p], acc_o[d]);
             }
         }
-        if constexpr (decltype(more)::value) load_v(t + WAVES);
+        if constexpr (decltype(more)::value) load_v(next);
     };
     // The last tile stands apart and fetches nothing: with one tile a wave, fetching it again was half of all loads, and a branch about the fetch cuts
     // the loop in two for the scheduler.  us, fetched again -> branch -> apart: 32 heads of [128, 64] 6.85 -> 6.60 -> 6.55, 16 of [128, 128] 11.8 -> 10.9 -> 10.1, 32
     // of [500, 128] 49.6 -> 47.9 -> 45.6, 8 of [288, 32] 7.05 -> 7.18 -> 6.95, 4 of [2048, 64] 40.0 -> 40.9 -> 39.0.
+    // Only geometry 96 at its full width under the mask is slower apart: more registers than a wave addresses directly (9 of [2312, 96] 119 -> 125, 5 of [2206, 96] 53 -> 56).
     int t = wave;
-    for (; t + WAVES < tiles; t += WAVES) attend(t, std::true_type());
-    if (t < tiles) attend(t, std::false_type());
+    if constexpr (DK == 96 && CAUSAL && !PAD) {
+        for (; t < tiles; t += WAVES) attend(t, std::true_type(), t + WAVES < tiles ? t + WAVES : t);
+    } else {
+        for (; t + WAVES < tiles; t += WAVES) attend(t, std::true_type(), t + WAVES);
+        if (t < tiles) attend(t, std::false_type(), t);
+    }
 
     // ---- the waves' parts together, each at an eighth (exactly): outputs that are finite in themselves may exceed the largest float when
     // four are added with the factors of the terms still in them ----
