@@ -410,6 +410,18 @@ k_sdpa(const float *__restrict__ Q, const float *__restrict__ K, const float *__
     }
 }
 
+// A kernel's name: geometry, mask, waves (four unless it says eight), and whether tiles go out in pairs; or the form for few tiles.
+enum Form { FOUR, EIGHT, FOUR_PAIRS, EIGHT_PAIRS, FEW };
+const char *sdpa_name(int dk, int causal, Form form) {
+#define AX_NAMES(DK)                                                                                                                          \
+    {{"sdpa_fused_dk" DK, "sdpa_fused_dk" DK "_w8", "", "", "sdpa_fused_few_dk" DK},                                                             \
+     {"sdpa_fused_dk" DK "_causal", "sdpa_fused_dk" DK "_causal_w8", "sdpa_fused_dk" DK "_causal_pairs", "sdpa_fused_dk" DK "_causal_w8_pairs",   \
+      "sdpa_fused_few_dk" DK "_causal"}}
+    static const char *const names[4][2][5] = {AX_NAMES("32"), AX_NAMES("64"), AX_NAMES("96"), AX_NAMES("128")};
+#undef AX_NAMES
+    return names[dk / 32 - 1][causal != 0][form];
+}
+
 // Few tiles: four waves share 32 queries of one head and take its 32-key tiles in turn, each with an online softmax of its own; the
 // sets of maxima, sums and outputs meet in LDS.  Each wave reads its keys and values straight into fragment registers and cuts them itself,
 // so a key is cut once per 32 queries and not once per 128 or 256: more vector work in all, on four (or eight) times the workgroups and with
@@ -643,6 +655,7 @@ int launch_sdpa_few(const float *Q, const float *K, const float *V, float *O, fl
     }
     const float sl2 = scale * 1.4426950408889634f;
     const dim3 grid((unsigned)((S + 31) / 32 * BH)), block(256);
+    note_kernel(sdpa_name(DK, causal, FEW));
 #define AX_FEW(C, P) hipLaunchKernelGGL((k_sdpa_few<DK, C, P>), grid, block, SMEM, kStream, Q, K, V, O, L, BH, S, sl2, H, ld, ldo, dkr)
     if (causal && dkr == DK) AX_FEW(true, false);
     else if (causal) AX_FEW(true, true);
@@ -676,6 +689,7 @@ int launch_sdpa_p(const float *Q, const float *K, const float *V, float *O, floa
     const int64_t a_head = pair ? (nq + 1) / 2 : nq;
     int64_t most = 0xffffffffll / (64 * WAVES) / a_head;
     if (most < 1) return fail(AXHIP_ERR_SHAPE, "sdpa_fwd: too many tiles");
+    note_kernel(sdpa_name(DK, causal, pair ? (WAVES == 8 ? EIGHT_PAIRS : FOUR_PAIRS) : WAVES == 8 ? EIGHT : FOUR));
     if (most > H) most -= most % H;
     for (int64_t h0 = 0, n; h0 < BH; h0 += n) {
         n = BH - h0 < most ? BH - h0 : most;
@@ -792,24 +806,12 @@ int sdpa_unfused(const float *Q, const float *K, const float *V, float *O, float
 // size that is a multiple of 4 up to 128 runs on the kernel of the next size among 32, 64, 96, 128.
 static bool sdpa_fusable(int64_t dk) { return dk >= 4 && dk <= 128 && dk % 4 == 0; }
 
-// A kernel's name: geometry, mask, and whether the few-tiles form runs.
-static const char *sdpa_name(int dk, int causal, bool few) {
-    static const char *const names[4][2][2] = {{{"sdpa_fused_dk32", "sdpa_fused_few_dk32"}, {"sdpa_fused_dk32_causal", "sdpa_fused_few_dk32_causal"}},
-                                               {{"sdpa_fused_dk64", "sdpa_fused_few_dk64"}, {"sdpa_fused_dk64_causal", "sdpa_fused_few_dk64_causal"}},
-                                               {{"sdpa_fused_dk96", "sdpa_fused_few_dk96"}, {"sdpa_fused_dk96_causal", "sdpa_fused_few_dk96_causal"}},
-                                               {{"sdpa_fused_dk128", "sdpa_fused_few_dk128"}, {"sdpa_fused_dk128_causal", "sdpa_fused_few_dk128_causal"}}};
-    return names[dk / 32 - 1][causal != 0][few];
-}
-
 static int sdpa_fused(const float *Q, const float *K, const float *V, float *O, float *L, int64_t BH, int64_t S,
                       int64_t dk, float scale, int causal, int64_t H, int64_t ld, int64_t ldo) {
     auto run = [&](auto geometry) {
         constexpr int DK = decltype(geometry)::value;
-        const bool few = few_tiles<DK>(BH, S, causal);
-        const int rc = few ? launch_sdpa_few<DK>(Q, K, V, O, L, BH, S, scale, causal, H, ld, ldo, (int)dk)
-                           : launch_sdpa<DK>(Q, K, V, O, L, BH, S, scale, causal, H, ld, ldo, (int)dk);
-        axhip::note_kernel(sdpa_name(DK, causal, few));
-        return rc;
+        return few_tiles<DK>(BH, S, causal) ? launch_sdpa_few<DK>(Q, K, V, O, L, BH, S, scale, causal, H, ld, ldo, (int)dk)
+                                            : launch_sdpa<DK>(Q, K, V, O, L, BH, S, scale, causal, H, ld, ldo, (int)dk);
     };
     if (dk <= 32) return run(std::integral_constant<int, 32>());
     if (dk <= 64) return run(std::integral_constant<int, 64>());
