@@ -411,9 +411,9 @@ int planes_f32(const StagedArgs &g, int transa, int transb) {
         constexpr bool A_KC = decltype(a_kc)::value, B_KC = decltype(b_kc)::value;
         return tile == 0 ? launch_planes<4, 2, 4, 4, false, A_KC, B_KC>(names[0], p) : launch_planes<2, 2, 4, 2, true, A_KC, B_KC>(names[1], p);
     };
-    static const char *const nn[2] = {"sgemm_nn_planes256x128x3_staged", "sgemm_nn_planes128x64x3_staged"};
-    static const char *const nt[2] = {"sgemm_nt_planes256x128x3_staged", "sgemm_nt_planes128x64x3_staged"};
-    static const char *const tn[2] = {"sgemm_tn_planes256x128x3_staged", "sgemm_tn_planes128x64x3_staged"};
+    static const char *const nn[2] = {"sgemm_nn_planes256x128x3", "sgemm_nn_planes128x64x3"};
+    static const char *const nt[2] = {"sgemm_nt_planes256x128x3", "sgemm_nt_planes128x64x3"};
+    static const char *const tn[2] = {"sgemm_tn_planes256x128x3", "sgemm_tn_planes128x64x3"};
     const std::true_type yes;
     const std::false_type no;
     if (!transa && !transb) return launch(yes, no, nn);

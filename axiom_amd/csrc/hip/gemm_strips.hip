@@ -326,11 +326,10 @@ int strips_f32(const StagedArgs &g, int transa, int transb, bool on_grid) {
     const bool ranges_in_terms = !on_grid || g.K % 32 != 0;      // what stands behind a longer K: ranges on the staged tiles in terms, or on fp32 ones
     const int64_t most = many              ? (transb ? 1088 : g.M < 96 ? 1024 : 1536)
                          : ranges_in_terms ? (transb ? 864 : 1024)
-                         : tiles > 24      ? (transb ? 832 : 896)
-                                           : (transb ? 800 : 864);
+                                           : (transb ? 832 : 896);
     const bool third = tiles * 3 <= cus * 4;                   // two workgroups on a third of the CUs at most
     const bool strips = (one && g.K <= most) || (two && !transb && g.K <= (third ? 640 : 800));
-    // Few tiles and a long K: ranges of it, four to eight workgroups a tile.  (Their name holds that of the strips where those are what stands behind.)
+    // Few tiles and a long K: ranges of it, four to eight workgroups a tile.
     const int64_t waves = tiles <= 32 ? (g.K > 1300 ? 8 : 4) : tiles <= 64 && g.K > 1024 ? 8 : 4;
     const int64_t ranges = g.K <= 760                ? 1
                            : tiles <= 32             ? (g.K <= 960 ? 4 : g.K <= 4608 ? 8 : 1)
@@ -338,10 +337,7 @@ int strips_f32(const StagedArgs &g, int transa, int transb, bool on_grid) {
                            : tiles <= 100            ? (g.K > 960 && g.K <= 2600 ? 8 : 1)
                                                      : 1;
     if (ranges > 1) {
-        static const char *const names[3][2] = {{"sgemm_nn_ranges32x3", "sgemm_nn_strips32x3_ranges"},
-                                                {"sgemm_nt_ranges32x3", "sgemm_nt_strips32x3_ranges"},
-                                                {"sgemm_tn_ranges32x3", "sgemm_tn_strips32x3_ranges"}};
-        const char *name = names[transa ? 2 : transb ? 1 : 0][strips];
+        const char *name = transa ? "sgemm_tn_ranges32x3" : transb ? "sgemm_nt_ranges32x3" : "sgemm_nn_ranges32x3";
         if (!transa && !transb) return waves == 8 ? launch<8, true, true, false, 2, true>(name, g, ranges) : launch<4, true, true, false, 4, true>(name, g, ranges);
         if (!transa) return waves == 8 ? launch<8, true, true, true, 2, true>(name, g, ranges) : launch<4, true, true, true, 4, true>(name, g, ranges);
         return waves == 8 ? launch<8, true, false, false, 2, true>(name, g, ranges) : launch<4, true, false, false, 4, true>(name, g, ranges);

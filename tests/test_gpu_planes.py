@@ -7,7 +7,7 @@ from test_gpu_parity import BOUND_FP32, say
 
 pytestmark = pytest.mark.gpu
 
-LARGE, SMALL = "planes256x128x3_staged", "planes128x64x3_staged"
+LARGE, SMALL = "planes256x128x3", "planes128x64x3"
 
 
 def padded(x, pad, off=0):

@@ -1,4 +1,4 @@
-"""fp32 products with few tiles, in one launch of 32x32 tiles whose waves share K: edges of tiles, steps and strips in every storage order
+"""fp32 products with few tiles, in one launch of 32x32 tiles whose waves share K (or, past the longest K of that, a range of it): edges of tiles, steps and strips in every storage order
 and form, and the inputs that bf16 terms cannot hold."""
 import numpy as np
 import pytest
@@ -21,7 +21,7 @@ def product(hip, a, b, order, alpha=1.0, beta=0.0, c=None, bias=None, act=0, pad
     dbias = None if bias is None else hip.array(bias)
     hip.check(hip.L.axhip_sgemm(int(order[0] == "t"), int(order[1] == "t"), M, N, K, alpha, da.ptr, sa.shape[1], db.ptr, sb.shape[1], beta, dc.ptr,
                                 N + pads[2], None if bias is None else dbias.ptr, act))
-    assert "_strips32" in hip.last_kernel(), hip.last_kernel()
+    assert ("_ranges32x3" if in_ranges(M, N, K) else "_strips32") in hip.last_kernel(), hip.last_kernel()
     full = dc.numpy()
     assert np.isnan(full[:, N:]).all()
     return full[:, :N]
@@ -31,17 +31,22 @@ def tiles(M, N):
     return ((M + 31) // 32) * ((N + 31) // 32)
 
 
+def in_ranges(M, N, K):
+    """A longer K on few tiles: ranges of it in workgroups of their own (test_gpu_strips_ranges.py)."""
+    return K > 760 and tiles(M, N) <= 64 or K > 960 and tiles(M, N) <= 100
+
+
 def most(order, M, N):
     """The largest K that the strips take off the 16-byte grid (256 CUs)."""
     if tiles(M, N) > 256:
         return 0 if order == "nt" else 640 if tiles(M, N) <= 341 else 800
     if tiles(M, N) >= 128:
         return 1088 if order == "nt" else 1024 if M < 96 else 1536
-    return 864 if order == "nt" else 1024
+    return 760 if tiles(M, N) <= 64 else 864 if order == "nt" else 960 if tiles(M, N) <= 100 else 1024
 
 
 FORMS = [(order, M, N, K) for order in ("nn", "nt", "tn") for M, N in [(17, 1), (31, 33), (32, 32), (65, 95), (100, 10), (260, 1000), (250, 2020)]
-         for K in (1, 2, 15, 16, 17, 31, 32, 47, 63, 121, 128, 129, 143, 144, 145, 176, 177, 255, 256, 257, 500, 640, 641, 799) if K < 64 or K <= most(order, M, N)]
+         for K in (1, 2, 15, 16, 17, 31, 32, 47, 63, 121, 128, 129, 143, 144, 145, 176, 177, 255, 256, 257, 500, 640, 641, 760, 799) if K < 64 or K <= most(order, M, N)]
 
 
 # K u sum |a||b| holds with room; with terms the left-out ones add at most 2^-24 of each product
@@ -72,7 +77,8 @@ def test_on_the_grid(hip, M, N, K, order):
 
 
 @pytest.mark.parametrize("order,M,N,K", [("nn", 100, 10, 1024), ("tn", 97, 31, 1000), ("nn", 97, 250, 1023), ("nt", 250, 100, 863), ("tn", 96, 257, 1024),
-                                         ("nt", 500, 255, 1088), ("nn", 256, 1000, 1536), ("tn", 510, 500, 1535)])
+                                         ("nn", 100, 10, 760), ("tn", 97, 31, 757), ("nn", 97, 250, 759), ("nt", 250, 100, 760), ("nt", 250, 257, 863), ("nn", 250, 257, 960),
+                                         ("tn", 250, 257, 959), ("tn", 330, 300, 1024), ("nt", 500, 255, 1088), ("nn", 256, 1000, 1536), ("tn", 510, 500, 1535)])
 def test_longer_k(hip, order, M, N, K):
     say("strips of a longer K", M, N, K, order)
     rng = np.random.default_rng(M + N + K)
@@ -134,7 +140,7 @@ def test_keeps_the_range(hip, scale_a, scale_b):
 
 
 # (order, M, N, K): forms of four, eight and sixteen waves
-@pytest.mark.parametrize("order,M,N,K", [("nn", 64, 64, 256), ("nt", 64, 64, 256), ("tn", 64, 64, 256), ("tn", 65, 97, 600), ("nn", 200, 100, 800),
+@pytest.mark.parametrize("order,M,N,K", [("nn", 64, 64, 256), ("nt", 64, 64, 256), ("tn", 64, 64, 256), ("tn", 65, 97, 600), ("nn", 200, 100, 760), ("nn", 200, 100, 800),
                                          ("nn", 192, 2048, 512), ("tn", 192, 2048, 512)])
 @pytest.mark.parametrize("power", [69, 71, 73, 75, 77, 79])
 def test_sums_of_one_sign_past_the_terms(hip, order, M, N, K, power):
@@ -155,7 +161,7 @@ def test_outer_products_are_rounded_once(hip):
         assert np.array_equal(product(hip, u, v, order), u * v)
 
 
-@pytest.mark.parametrize("order,M,N", [("nn", 50, 10), ("nn", 101, 99), ("nn", 130, 1002), ("nn", 70, 1602), ("nn", 330, 990), ("tn", 351, 991), ("nt", 101, 99), ("nt", 130, 1002), ("tn", 101, 99),
+@pytest.mark.parametrize("order,M,N", [("nn", 50, 10), ("nn", 101, 99), ("nn", 250, 257), ("nt", 250, 257), ("tn", 330, 300), ("nn", 130, 1002), ("nn", 70, 1602), ("nn", 330, 990), ("tn", 351, 991), ("nt", 101, 99), ("nt", 130, 1002), ("tn", 101, 99),
                                        ("tn", 130, 1002), ("nn", 200, 2002)])
 def test_where_k_ends(hip, order, M, N):
     """The last K that the strips take and the next one, which takes another route."""

@@ -24,7 +24,7 @@ def test_ranges(hip, M, N, K, taken, order):
     exact, size = a.astype(np.float64) @ b.astype(np.float64), np.abs(a).astype(np.float64) @ np.abs(b).astype(np.float64)
     for pads, off in (((3, 1, 5), 1), ((0, 0, 0), 0)):
         got = product(hip, a, b, order, c=c, alpha=0.5, beta=2.0, bias=bias, act=1, pads=pads, off=off)
-        assert ("ranges" in hip.last_kernel()) == taken, hip.last_kernel()
+        assert (hip.last_kernel() == f"sgemm_{order}_ranges32x3") == taken, hip.last_kernel()
         want = np.maximum(0.5 * exact + 2.0 * c + bias, 0)
         assert (np.abs(got - want) <= BOUND_FP32 * (0.5 * size + 2.0 * np.abs(c) + np.abs(bias))).all()
         assert np.array_equal(product(hip, a, b, order, c=c, alpha=0.5, beta=2.0, bias=bias, act=1, pads=pads, off=off), got)
