@@ -376,9 +376,12 @@ int launch_planes(const char *name, const PlanesArgs &p) {
 }  // namespace
 
 namespace axhip {
-// Tiles of 256x128 (a workgroup a CU) and 128x64 (two a CU), each priced by a line fitted to 420 products of 1.2e9 to 4e10 multiply-adds in every
-// storage order, timed back to back (mean error 3 %), and taken where that is a twentieth below what the staged tiles should take (plan_staged; those
-// are within 10 %).  A hundred of the 420 are: geometric mean 1.20, none slower (K below 480, left out: 2122 x 3008 x 320 35.4 -> 38.0).  Elsewhere
+// Tiles of 256x128 (a workgroup a CU) and 128x64 (two a CU), each priced by a line fitted to 420 products of 1.2e9 to 4e10 multiply-adds in every storage order, and
+// taken where that is a twentieth below the price of the staged tiles (plan_staged).  The prices are for this comparison; as times both are too low where the chip runs into its
+// power cap (2048 x 4096 x 4096 241 for 311 us, staged 320 for 366; over 79 products of up to 2e11 multiply-adds 0.70 to 0.98, staged 0.77 to 1.05).  On these
+// 79 planes are 1.24 times as fast (0.99 to 1.43), on 145 more near the line, of K up to 7300, 1.15 (0.999 and more).  Near the line with a K above 4096 planes of 128x64 are
+// behind but for A^T B (A B^T 1498 x 2020 x 7312 270 -> 292, 2208 x 1248 x 6112 218 -> 238, A B 2368 x 1248 x 6304 245 -> 256; A^T B 1495 x 1819 x 5230 226 -> 215, A B
+// 1706 x 3467 x 5049, priced at 0.90, 456 -> 388): a twelfth there.  K below 480, left out: 2122 x 3008 x 320 35.4 -> 38.0.  Elsewhere
 // cutting costs what it saves: up to a tile or two a CU (1024^3 21 -> 34, 2000 x 1024 x 1024 31 -> 37), and a long K with few columns (2000 x 1024 x 4096
 // 104 -> 113; its planes take 20).
 // The error against 64 bits is no larger than before on any of them: 128x64 has as many sums as the staged 128x64 and 64x64 tiles (1.19e-7 at K = 1024,
@@ -395,7 +398,7 @@ int planes_f32(const StagedArgs &g, int transa, int transb) {
     const float us[2] = {4.6f + 0.357f * cut_mb + large * (1.042f * slabs + 13.7f),
                          8.7f + 0.207f * cut_mb + pairs * (0.851f * slabs + 5.6f) + single * (0.567f * slabs + 3.3f)};
     const int tile = staged.is_128x128 && us[0] < us[1] ? 0 : 1, kblocks = (int)up(g.K, 32);
-    if (us[tile] > 0.95f * staged.us) return -1;
+    if (us[tile] > (tile == 1 && !transa && g.K > 4096 ? 0.92f : 0.95f) * staged.us) return -1;
     PlanesArgs p{g, nullptr, nullptr, (int)up(g.M, 16), (int)up(g.N, 16), kblocks};
     const size_t a_bytes = (size_t)p.a_blocks * kblocks * BLOCK, b_bytes = (size_t)p.b_blocks * kblocks * BLOCK;
     if (a_bytes + b_bytes > kWorkspaceStart || a_bytes + b_bytes > workspace_bytes()) return -1;     // never grown for planes
