@@ -79,3 +79,19 @@ def test_ranges_large_sums(hip, M, N, K):
     assert want.max() < np.finfo(np.float32).max
     got = product(hip, a, b, "nn")
     assert "ranges" in hip.last_kernel() and (np.abs(got - want) <= BOUND_FP32 * want).all()
+
+
+@pytest.mark.parametrize("M,N,K", [(100, 12, 4096), (64, 300, 1024), (300, 320, 1312), (50, 10, 777)])
+@pytest.mark.parametrize("order", ["nn", "nt", "tn"])
+def test_ranges_single_products(hip, M, N, K, order):
+    """Sums with one product that is not zero, of operands with all 24 bits, in any of the ranges: the left-out terms are at most 2^-24 of it, the matrix core's own
+    addition truncates (2^-23), the others' are 2^-8 of that.  Any of the six products of terms left out would show as 2^-18 or more."""
+    say("ranges single products", M, N, K, order)
+    rng = np.random.default_rng(K)
+    a = np.zeros((M, K), np.float32)
+    a[np.arange(M), rng.integers(0, K, M)] = rng.uniform(1, 2, M) * rng.choice([-1, 1], M)
+    b = rng.uniform(1, 2, (K, N)).astype(np.float32)
+    got, want = product(hip, a, b, order), a.astype(np.float64) @ b.astype(np.float64)
+    assert hip.last_kernel() == f"sgemm_{order}_ranges32x3"
+    err = np.abs(got - want) / np.abs(want) * 2.0 ** 24
+    assert (err <= 3 + 7 / 64).all(), float(err.max())
