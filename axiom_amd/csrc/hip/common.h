@@ -18,8 +18,7 @@ int cu_count();
 void note_kernel(const char *name);
 // Checks the launch that was just issued on the null stream.
 int check_launch(const char *what);
-// What the workspace holds from axhip_init on: 288 GB of memory make room for the planes of terms of every product that pays for them up to
-// 2048 x 4096 x 4096 (gemm_planes.hip).
+// What the workspace holds from axhip_init on, and the most that planes of terms take of it (gemm_planes.hip): those of 2048 x 4096 x 4096 are 151 MB.
 constexpr size_t kWorkspaceStart = size_t(160) << 20;
 // What it holds now.
 size_t workspace_bytes();
@@ -51,6 +50,7 @@ struct Tuning {
     int f32_tile;        // AX_HIP_F32_TILE: 64 (64x64), 642 (64x64 with the k split over two wave sets), 128 (128x128, eight waves)
     int f32_splitk;      // AX_HIP_F32_SPLITK: 1 = never split K, 2.. = that many ranges where the route applies
     int f32_no_strips;   // AX_HIP_F32_NO_STRIPS: 1 = single fp32 products never take the one-launch strips of few tiles
+    int f32_no_planes;   // AX_HIP_F32_NO_PLANES: 1 = large single fp32 products never go over planes of terms
     int skinny_blocks;   // AX_HIP_SKINNY_BLOCKS: workgroups the skinny-M route aims for
     int skinny_form;     // AX_HIP_SKINNY_FORM: 1 (64 columns x 256 threads), 2 (the same, the lane groups of a wave added before LDS), 3 (64 columns x 512 threads)
     int skinny_kps;      // AX_HIP_SKINNY_KPS: most rows of K one skinny-M workgroup takes (a multiple of 16)

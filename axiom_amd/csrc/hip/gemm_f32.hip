@@ -1846,7 +1846,7 @@ int run_f32(const SgemmArgs &g, int transa, int transb) {
                                : whole ? g.K >= 256 && products >= 1.5e9
                                        : g.K >= 96 && (products >= 1.0e9 || (g.K >= 256 && g.M > 160 && products >= 2.0e7 &&
                                                                                 (g.N >= 48 || split_count(g.M, g.N, g.K, !transa) * 64 < g.K)));
-        if (free_choice && split) rc = planes_f32(staged_args(g), transa, transb);
+        if (free_choice && split && !tuning().f32_no_planes) rc = planes_f32(staged_args(g), transa, transb);
         if (rc < 0 && free_choice && split) rc = split_f32(staged_args(g), transa, transb, 1, true);
         if (rc >= 0) return rc;
         if (off) rc = staged_f32(staged_args(g), transa, transb, 1, true);

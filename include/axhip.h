@@ -64,6 +64,7 @@ const char *axhip_device_name(void);          /* gcnArchName of device 0, "" wit
  *                        most 16, of 128 or more each)
  *   AX_HIP_F32_NO_STRIPS 1          single fp32 products with few output tiles take the tiles and K ranges of the other routes and not
  *                        the one launch whose waves share K
+ *   AX_HIP_F32_NO_PLANES 1          large single fp32 products are not cut into planes of bf16 terms first: the tiles cut what they read
  *   AX_HIP_NT_WALK       1 | 2      batched A B^T with K <= 128: 1, a 128-row block of A stays in LDS and the column blocks of B^T
  *                        are walked; 2, 256 rows of B stay in registers and A is walked in blocks of 32 rows (N a multiple of 256)
  *   AX_HIP_SKINNY_BLOCKS 1..65535   workgroups the skinny-M route aims for
@@ -108,7 +109,8 @@ int64_t axhip_device_free_bytes(void);
  * driver for a new one, which costs the first call at a larger shape some tens of microseconds that later
  * calls do not pay.  axhip_workspace_reserve grows it ahead of time (at model load, before a timed or
  * latency-bound loop) to at least `bytes` and reports the size it then has in *have (may be NULL); bytes = 0
- * only reports.  It never shrinks.  No counterpart in the reference, whose CUDA backend grows its score
+ * only reports.  It never shrinks.  Single fp32 products that go over planes of terms take at most the 160 MiB of the start, however
+ * much there is, so that a product takes the same way whatever was reserved or called before it.  No counterpart in the reference, whose CUDA backend grows its score
  * buffer on demand in the same way (cuda/ops_attention.cu:305-318) and offers no call to do it ahead of
  * time.  Same threading rule as the compute entry points. */
 int   axhip_workspace_reserve(size_t bytes, size_t *have);

@@ -100,3 +100,25 @@ def test_planes_non_finite(hip, M, N, K, order):
     rows = np.setdiff1d(np.arange(M), [1, 2, 4, M - 1])
     size = np.abs(a[rows]).astype(np.float64) @ np.abs(b).astype(np.float64)
     assert (np.abs(got[rows] - ref[rows]) <= BOUND_FP32 * size).all()
+
+
+@pytest.mark.parametrize("M,N,K", [(1793, 3969, 545), (1665, 3009, 545), (2000, 2432, 2016)])
+@pytest.mark.parametrize("order", ["nn", "nt", "tn"])
+def test_error_is_that_of_the_staged_tiles_or_less(hip, monkeypatch, M, N, K, order):
+    """No larger than what the tiles that planes stand before leave on the same operands; 1 % for the luck of the draw: over four million sums and more whose
+    errors are independent a norm is known to some 0.05 %."""
+    say("planes, error", M, N, K, order)
+    rng = np.random.default_rng(K)
+    a, b = rng.uniform(-1, 1, (M, K)).astype(np.float32), rng.uniform(-1, 1, (K, N)).astype(np.float32)
+    want = a.astype(np.float64) @ b.astype(np.float64)
+    planes = np.linalg.norm(product(hip, a, b, order) - want)
+    assert "planes" in hip.last_kernel()
+    monkeypatch.setenv("AX_HIP_F32_NO_PLANES", "1")
+    assert hip.L.axhip_tuning_reload() == 1
+    try:
+        staged = np.linalg.norm(product(hip, a, b, order) - want)
+        assert hip.last_kernel().endswith("x3_staged") or hip.last_kernel() == "sgemm_splitk_x3"
+    finally:
+        monkeypatch.delenv("AX_HIP_F32_NO_PLANES")
+        assert hip.L.axhip_tuning_reload() == 0
+    assert planes <= 1.01 * staged, (planes, staged)
