@@ -305,10 +305,11 @@ namespace axhip {
 // Sixteen pay where A is stored across K, whose loads are the slowest, above K = 256 (256 x 1000 x 500 6.6 -> 6.1; 250 x 500 x 256 4.5 -> 5.2).
 // A K past that, or past 760 with up to 64 tiles, in ranges, which meet in the same launch: for a narrow result two launches had cost their floor twice, and a few
 // workgroups of eight waves each wait for memory through their strip.  us, before -> here: 100 x 10 x 4096 10.8 -> 7.9, 128 x 10 x 1024 8.6 -> 5.7, 64 x
-// 256 x 2048 A^T B 8.7 -> 7.7, 100 x 100 x 4096 9.2 -> 8.9.  Geometric means over 800 random products, before over here, and the error over that of before: up to 32 tiles
+// 256 x 2048 A^T B 8.7 -> 7.7, 100 x 100 x 4096 9.2 -> 8.9 (on the 16-byte grid with whole K from fp32 instructions: fewer bits in a sum of one product, 1.7 in place of 1 unit of 2^-24).  Geometric means over 800 random products, before over here, and the error over that of before: up to 32 tiles
 // K = 761..960 1.18 to 1.28 (four ranges of four waves, 1.00 of the strips' and 0.7 of the others' error), ..1300 1.36 to 1.45 (eight), ..4608 1.14 to 1.43
 // (eight of eight waves, 0.6 to 0.8); 33 to 64 tiles ..1024 1.07 to 1.36, ..2600 1.12 to 1.31; 65 to 100 tiles 961..2600 1.08 to 1.17.  Below K = 760 the parts are
-// so short that adding them costs accuracy (1.01 to 1.05 for 1.0 to 1.2 of the speed), past 100 tiles the chip is full (0.7 to 1.0); sixteen ranges 0.8 to 1.0 of eight.
+// so short that adding them costs accuracy (1.01 to 1.05 for 1.0 to 1.2 of the speed), past 100 tiles the chip is full (0.7 to 1.0); sixteen ranges 0.8 to 1.0 of eight.  A longer K on
+// 33 to 100 tiles is behind (2610 to 3320 0.92 to 1.09, 4700 to 8000 0.72 to 0.93); up to 32 tiles it is ahead still (49 of 50 up to 15900 1.06 to 1.45), but its error is not compared there.
 // On fp32 instructions up to K = 63 off the grid and 112 on it, where the kernels before are on them too: there is little to multiply and nothing to
 // cut.  Four waves, up to two tiles a CU (geometric means over some hundred products a range, cached / from HBM, and the error over that of the
 // kernels before: K below 32 1.3 / 1.3, 0.99; 32..63 off the grid 1.31 / 1.29, 0.86, on it 1.22 / 1.21, 0.74; 64..112 on the grid 1.32 / 1.31, 0.64; strips in

@@ -24,7 +24,7 @@
 // A tile with a sum that is not finite is computed again with fp32 instructions by the same workgroup:
 // infinities, NaNs and values near the largest float come out as fp32 products give them.
 // us, fp32 instructions -> terms: 512 heads of [512, 64] 269 -> 194 (causal 178 -> 126), 64 of [1024, 128] 273 -> 174, 96 causal
-// ones of [1000, 80] 324 -> 108 (a quarter of that from the 96-wide geometry), 512 of [256, 32] 41 -> 33; with few query tiles for the
+// ones of [1000, 80] 324 -> 113 (a quarter of that from the 96-wide geometry; the matrix core is busy 43 % of the cycles, vector instructions some 34, and on zeros it takes 97), 512 of [256, 32] 41 -> 33; with few query tiles for the
 // CUs k_sdpa_few cuts a head along its keys too (32 heads of [128, 64] 11.4 -> 6.6).  O is nearer to 64 bits on every shape measured (relative error 4.9e-7 -> 3.7e-7 at [512, 64]).  Bound: the matrix core is
 // busy 49 % of the cycles, vector instructions (cutting, softmax) take some 44 ([512, 64]).  Measured and dropped: two key tiles at a time,
 // the scores of one interleaved with the exponentials of the other by instruction groups ([512, 64] 194, [1024, 96] 126 -> 128).
