@@ -6,7 +6,7 @@
 // left is what the int8 kernels do: loads straight to LDS, reads of whole fragments without a bank conflict, products; no vector instruction in the loop.
 // v_mfma_f32_16x16x32_bf16, not 32x32x16: its accumulators are read and written half as often, and at full load the matrix core runs into the
 // power cap (2000 x 4096 x 1024 the product alone 80 -> 72 us, 1.4 PFLOP/s of bf16 products; with 64 of 256 CUs at work it is at 87 % of the peak).
-// us, staged tiles -> this, both launches, back to back, one box: 2000 x 4096 x 1024 105 -> 85, 2000 x 3072 x 1024 98 -> 79, 2048 x 4096 x 4096 366 -> 311, A B^T
+// us, staged tiles -> this, both launches, back to back, on one card: 2000 x 4096 x 1024 105 -> 85, 2000 x 3072 x 1024 98 -> 79, 2048 x 4096 x 4096 366 -> 311, A B^T
 // 2112 x 2432 x 2403 192 -> 157, A^T B 1288 x 3985 x 767 85 -> 65.
 // Bound: 256x128 tiles, power with every CU at work (zeros for operands 65 and 224 us in place of 82 and 288 at 2000 x 4096 x 1024 and 2048 x 4096 x 4096; the matrix core is busy 63 and 81 % of
 // the cycles); 128x64 ones, what L2 hands to the CUs (36 KiB per tile and 32 k: 2000 x 3072 x 1024 906 MB in 59 us, 15.4 TB/s, 936 MB by its counter, the matrix core busy 51 %;

@@ -68,3 +68,18 @@ def test_pairs(hip, BH, S, dk, form):
         size = np.maximum(1.0, np.abs(want[fine]).max() * 2) if h in (1, 6) else 1.0
         assert np.abs(got[fine] - want[fine]).max() <= 2 * SDPA_TOL * size, h
         assert np.nanmax(np.abs(l_got - l_want)) <= 1e-5 * max(1.0, np.nanmax(np.abs(l_want))), h
+
+
+@pytest.mark.parametrize("causal", [0, 1])
+def test_more_tiles_than_a_grid_holds(hip, causal):
+    """2^24 workgroups of 256 threads are one launch too many threads: the heads go in two pieces.  One key a head: O is V but for the left-out terms, three roundings and the
+    others' own (2^-24 each and 2^-8 of that), L the scaled product of Q and K."""
+    BH = 2 ** 24 + 1021
+    say("causal tiles in pieces", causal)
+    rng = np.random.default_rng(BH)
+    q, k, v = (rng.random((BH, 1, 4), np.float32) + 1 for _ in range(3))
+    dq, dk_, dv, do, dl = hip.array(q), hip.array(k), hip.array(v), hip.array(np.full((BH, 1, 4), np.nan, np.float32)), hip.array(np.full((BH, 1), np.nan, np.float32))
+    hip.check(hip.L.axhip_sdpa_fwd(dq.ptr, dk_.ptr, dv.ptr, do.ptr, dl.ptr, BH, 1, 4, 0.5, causal))
+    assert (np.abs(do.numpy() - v) <= 2.0 ** -24 * (4 + 7 / 128) * v).all()
+    want = 0.5 * (q * k).sum(-1)
+    assert (np.abs(dl.numpy() - want) <= 1e-6 * want).all()
