@@ -307,7 +307,9 @@ namespace axhip {
 // workgroups of eight waves each wait for memory through their strip.  us, before -> here: 100 x 10 x 4096 10.8 -> 7.9, 128 x 10 x 1024 8.6 -> 5.7, 64 x
 // 256 x 2048 A^T B 8.7 -> 7.7, 100 x 100 x 4096 9.2 -> 8.9 (on the 16-byte grid with whole K from fp32 instructions: fewer bits in a sum of one product, 1.7 in place of 1 unit of 2^-24).  Geometric means over 800 random products, before over here, and the error over that of before: up to 32 tiles
 // K = 761..960 1.18 to 1.28 (four ranges of four waves, 1.00 of the strips' and 0.7 of the others' error), ..1300 1.36 to 1.45 (eight), ..4608 1.14 to 1.43
-// (eight of eight waves, 0.6 to 0.8); 33 to 64 tiles ..1024 1.07 to 1.36, ..2600 1.12 to 1.31; 65 to 100 tiles 961..2600 1.08 to 1.17.  Below K = 760 the parts are
+// (eight of eight waves, 0.6 to 0.8); 33 to 64 tiles ..1024 1.07 to 1.36, ..2600 1.03 to 1.31; 65 to 100 tiles, cached and
+// from HBM, A B 961..1600 1.12 and 1.07, A^T B ..1950 1.13 and 1.10 (on the grid ..2600 1.10 and 1.08), A B^T ..1280 1.05 and 1.06; past these A B 0.94 to 1.1 and 0.87 to 1.06, A^T B off the grid 0.86 to 1.1, A B^T 0.78 to 1.0
+// and 0.70 to 0.88 (86 tiles, K = 2322 10.7 -> 13.9, from HBM 12.5 -> 17.5: three workgroups a CU, each with a turn through LDS).  Below K = 760 the parts are
 // so short that adding them costs accuracy (1.01 to 1.05 for 1.0 to 1.2 of the speed), past 100 tiles the chip is full (0.7 to 1.0); sixteen ranges 0.8 to 1.0 of eight.  A longer K on
 // 33 to 100 tiles is behind (2610 to 3320 0.92 to 1.09, 4700 to 8000 0.72 to 0.93); up to 32 tiles it is ahead still (49 of 50 up to 15900 1.06 to 1.45), but its error is not compared there.
 // On fp32 instructions up to K = 63 off the grid and 112 on it, where the kernels before are on them too: there is little to multiply and nothing to
@@ -332,10 +334,11 @@ int strips_f32(const StagedArgs &g, int transa, int transb, bool on_grid) {
     const bool strips = (one && g.K <= most) || (two && !transb && g.K <= (third ? 640 : 800));
     // Few tiles and a long K: ranges of it, four to eight workgroups a tile.
     const int64_t waves = tiles <= 32 ? (g.K > 1300 ? 8 : 4) : tiles <= 64 && g.K > 1024 ? 8 : 4;
+    const int64_t farthest = transb ? 1280 : !transa ? 1600 : on_grid ? 2600 : 1950;
     const int64_t ranges = g.K <= 760                ? 1
                            : tiles <= 32             ? (g.K <= 960 ? 4 : g.K <= 4608 ? 8 : 1)
                            : tiles <= 64             ? (g.K <= 2600 ? 4 : 1)
-                           : tiles <= 100            ? (g.K > 960 && g.K <= 2600 ? 8 : 1)
+                           : tiles <= 100            ? (g.K > 960 && g.K <= farthest ? 8 : 1)
                                                      : 1;
     if (ranges > 1) {
         const char *name = transa ? "sgemm_tn_ranges32x3" : transb ? "sgemm_nt_ranges32x3" : "sgemm_nn_ranges32x3";

@@ -1,4 +1,5 @@
-"""Which single fp32 products go over planes of terms (gemm_planes.hip), on the host (256 CUs): sizes on both sides of the rule's lines.  Without a GPU."""
+"""Which single fp32 products go over planes of terms (gemm_planes.hip) and which in ranges of K in one launch (gemm_strips.hip), on the host (256 CUs): sizes on both sides of
+the rules' lines.  Without a GPU."""
 import pytest
 
 from test_host_runtime import run, stub  # noqa: F401  (stub is a fixture)
@@ -23,3 +24,21 @@ hip.check(L.axhip_sgemm(ta, tb, M, N, K, 1.0, A, M if ta else K, B, K if tb else
 assert ("planes" in hip.last_kernel()) == planes, hip.last_kernel()
 assert not planes or [x.kernel.decode().count("k_cut_planes") for x in launched()] == [1, 0]
 """ % ((order, M, N, K, planes),))
+
+
+# (order, M, N, K, whether in ranges): 65 to 100 tiles, on and off the 16-byte grid
+RANGES = [("nn", 96, 1024, 1600, True), ("nn", 96, 1024, 1604, False), ("nn", 123, 601, 1600, True), ("nn", 123, 601, 1601, False), ("nt", 1360, 64, 1280, True), ("nt", 1360, 64, 1284, False),
+          ("nt", 335, 205, 1279, True), ("nt", 335, 205, 2200, False), ("nt", 1368, 34, 2322, False), ("tn", 96, 1056, 2600, True), ("tn", 96, 1056, 2601, False), ("tn", 123, 601, 1950, True),
+          ("tn", 123, 601, 1951, False), ("nt", 64, 1024, 2600, True), ("nt", 64, 1024, 2604, False), ("nt", 100, 10, 4608, True), ("nt", 100, 10, 4612, False)]
+
+
+@pytest.mark.parametrize("order,M,N,K,ranges", RANGES)
+def test_ranges_are_taken(stub, order, M, N, K, ranges):  # noqa: F811
+    run(stub, """
+order, M, N, K, ranges = %r
+hip.check(L.axhip_init())
+ta, tb = order[0] == "t", order[1] == "t"
+hip.check(L.axhip_sgemm(ta, tb, M, N, K, 1.0, A, M if ta else K, B, K if tb else N, 0.0, D, N, None, 0))
+assert (hip.last_kernel() == "sgemm_%%s_ranges32x3" %% order) == ranges, hip.last_kernel()
+assert len(launched()) == 1 or not ranges
+""" % ((order, M, N, K, ranges),))
