@@ -710,7 +710,7 @@ int launch_sdpa(const float *Q, const float *K, const float *V, float *O, float 
                 float scale, int causal, int64_t H, int64_t ld, int64_t ldo, int dkr) {
     // Eight waves on 256 queries cut half as much of K and V for each of them, four on 128 waste less of a short head and
     // of the diagonal.  us, four waves -> eight: 64 heads of [1024, 128] 191 -> 174, 64 of [1024, 96]
-    // 141 -> 126, 96 causal ones of [1000, 80] 116 -> 108, 512 of [512, 64] 201 -> 194; but causal 128 -> 142, 512 of [256, 32]
+    // 141 -> 126, 85 causal ones of [1099, 80] 154 -> 149, 512 of [512, 64] 201 -> 194; but causal 128 -> 142, 512 of [256, 32]
     // 33 -> 37, 256 causal ones of [333, 48] 40 -> 44.  Geometry
     // 128 has the registers of one wave per SIMD with four waves, so it takes eight as soon as there is more than one tile a CU.
     if constexpr (DK > 32) {
